@@ -89,6 +89,10 @@ def _declare(lib):
         "nhp_rmsnorm_partial_fwd": ([vp, vp, vp, vp, vp, f32, ci, i64, i64, i64, ci, ci, vp], ci),
         "nhp_rmsnorm_partial_bwd": ([vp, vp, vp, vp, vp, vp, vp, vp, f32, ci, i64, i64, i64, ci, ci, vp], ci),
         "nhp_norm_bwd_workspace_bytes": ([i64, i64, ci], i64),
+        "nhp_attention_mask_bits": ([vp, vp, i64, i64, i64, vp], ci),
+        "nhp_attention_fwd": ([vp] * 6 + [i64, f32, f32] + [i64] * 7 + [p64] * 4 + [ci, vp], ci),
+        "nhp_attention_bwd": ([vp] * 10 + [f32] + [i64] * 7 + [p64] * 8 + [ci, vp], ci),
+        "nhp_attention_bwd_workspace_bytes": ([i64] * 6, i64),
         "nhp_layernorm_bwd_noalloc": ([vp, vp, vp, vp, vp, vp, vp, vp, i64, i64, ci, ci, vp], ci),
     }
     for name, (args, res) in sigs.items():

@@ -31,6 +31,7 @@ import math
 
 import torch
 
+from . import fused_attention
 from .fused_softmax import FusedScaleMaskSoftmax, SoftmaxFusionTypes
 from .utils import get_fusion_type  # noqa: F401  (also reachable from here, where its caller lives)
 
@@ -232,6 +233,12 @@ class CoreAttention(torch.nn.Module):
         projection, written by the context GEMM itself."""
         b, np_, sq, sk = query_layer.size(1), query_layer.size(2), query_layer.size(0), key_layer.size(0)
         hn = query_layer.size(3)
+        if self.use_cache and attention_mask is not None:
+            with torch.no_grad():
+                attention_mask = attention_mask[..., :sk, :sk]
+        fused = self._one_kernel(query_layer, key_layer, value_layer, attention_mask, key_lengths, merged_heads)
+        if fused is not None:
+            return fused
         if key_layer.size(2) != np_:
             return self._forward_grouped(query_layer, key_layer, value_layer, attention_mask, key_lengths, merged_heads)
         # [sq, b, np, hn] -> [sq, b * np, hn]
@@ -259,9 +266,6 @@ class CoreAttention(torch.nn.Module):
             scores = torch.empty((b * np_, sq, sk), dtype=q.dtype, device=q.device)
             scores = torch.baddbmm(scores, q.transpose(0, 1), k.transpose(0, 1).transpose(1, 2), beta=0.0,
                                    alpha=self.gemm_alpha).view(b, np_, sq, sk)
-        if self.use_cache and attention_mask is not None:
-            with torch.no_grad():
-                attention_mask = attention_mask[..., :sk, :sk]
         bias = self.rpe(sq, sk) if self.rpe is not None else None
         probs = self.scale_mask_softmax(scores, attention_mask, bias=bias, key_lengths=key_lengths)
         # [sk, b, np, hn] -> [sk, b * np, hn]; context [b * np, sq, hn]
@@ -270,6 +274,39 @@ class CoreAttention(torch.nn.Module):
             return _ContextGemm.apply(probs.view(b * np_, sq, sk), v).view(sq, b, np_ * value_layer.size(3))
         context = torch.bmm(probs.view(b * np_, sq, sk), v.transpose(0, 1))
         return context.view(b, np_, sq, value_layer.size(3))
+
+    def _one_kernel(self, query, key, value, mask, key_lengths, merged_heads):
+        """The context from the attention kernels, which keep the scores on the chip, or None where something is added
+        to the scores, dropped, or not provided by them. Which keys a query sees is decided as by the softmax module:
+        by index where that would run its causal kernel, otherwise by the mask (forward only; with the fill value of the
+        padding-mask kernel where that would run, and of the mask function where the torch branch would)."""
+        softmax = self.scale_mask_softmax
+        if (key_lengths is not None or self.rpe is not None or softmax.alibi_slopes is not None or not softmax.fusion
+                or softmax.narrow_forward_scale or mask is None or (softmax.training and softmax.attention_dropout > 0.0)):
+            return None
+        if not fused_attention.supported(query, key, value) or not softmax.input_in_float16:
+            return None
+        scale = self.gemm_alpha * (1.0 if softmax.scale is None else softmax.scale)
+        if not scale > 0.0:
+            return None
+        b, np_, sq, sk = query.size(1), query.size(2), query.size(0), key.size(0)
+        if softmax.upper_triang_mask_fusion and sq == sk:
+            if softmax.is_kernel_available(mask, b, np_, sq, sk):
+                window = softmax.sliding_window_width
+                window = None if window is None or window < 0 else int(window)
+                return fused_attention.causal_attention(query, key, value, scale, window, merged_heads)
+            kernel = False
+        elif softmax.upper_triang_mask_fusion:
+            kernel = softmax._rectangular_kernel_available(mask, b, np_, sq, sk)
+        else:
+            kernel = softmax.is_kernel_available(mask, b, np_, sq, sk)
+        fill = -10000.0 if kernel else softmax.mask_fill
+        if (fill is None or sk > 65536 or mask.dtype != torch.bool or mask.device != query.device
+                or mask.shape not in ((1, 1, sq, sk), (b, 1, sq, sk))):
+            return None
+        if torch.is_grad_enabled() and (query.requires_grad or key.requires_grad or value.requires_grad):
+            return None
+        return fused_attention.masked_attention(query, key, value, mask, scale, fill, merged_heads)
 
     def _causal_block(self, attention_mask, b, np_, sq, sk, like):
         """Block size for the blocked causal GEMMs, 0 when the scores do not go to the causal kernel (which is what
@@ -304,9 +341,6 @@ class CoreAttention(torch.nn.Module):
             scores = torch.empty((b * nkv, group * sq, sk), dtype=q.dtype, device=q.device)
             scores = torch.baddbmm(scores, q, k.transpose(1, 2), beta=0.0, alpha=self.gemm_alpha)
         scores = scores.view(b, np_, sq, sk)
-        if self.use_cache and attention_mask is not None:
-            with torch.no_grad():
-                attention_mask = attention_mask[..., :sk, :sk]
         bias = self.rpe(sq, sk) if self.rpe is not None else None
         probs = self.scale_mask_softmax(scores, attention_mask, bias=bias, key_lengths=key_lengths)
         context = torch.bmm(probs.view(b * nkv, group * sq, sk), v).view(b, np_, sq, hv)

@@ -1,0 +1,128 @@
+"""Scores -> probabilities -> context in one kernel on MI355X.
+
+What ``ParallelSelfAttention.attention`` (megatron/model/transformer.py:526-625) computes with two batched GEMMs and
+the fused softmax between them, for the cases in which nothing is added to the scores and nothing is dropped: the
+kernels of ``csrc/attention.hip`` form scores, row statistics and context on the matrix cores tile by tile, so the
+``[b, np, sq, sk]`` tensors (scores, probabilities and their gradients) do not exist. Scores, statistics and sums are
+fp32; the probabilities are rounded to the storage type before the second product, as they are between the GEMMs.
+
+Layouts as in ``CoreAttention``: q ``[sq, b, np, hn]``, k and v ``[sk, b, nkv, hn]`` with ``nkv`` dividing ``np``, any
+strides with contiguous features.
+"""
+import ctypes
+
+import torch
+
+from ..fused_kernels import _hotpath as _hp
+
+HEAD_DIMS = (64, 80, 96, 128)
+_I64x3 = ctypes.c_int64 * 3
+
+
+def _strides(t):
+    """Element strides of the first three dimensions; that of a dimension of one entry means nothing and is 0."""
+    return tuple(st if n > 1 else 0 for st, n in zip(t.stride()[:3], t.shape))
+
+
+def _readable(t):
+    """``t``, or a copy where the kernels cannot read it: they want contiguous features and 16-byte aligned rows."""
+    s = _strides(t)
+    if t.stride(3) == 1 and (s[0] | s[1] | s[2]) % 8 == 0 and t.data_ptr() % 16 == 0 and s[0] < 1 << 24:
+        return t
+    return t.clone(memory_format=torch.contiguous_format)
+
+
+def _strides3(t):
+    return _I64x3(*_strides(t))
+
+
+def supported(q, k, v):
+    """Whether the kernels take these operands (dtype, device, head size, sizes)."""
+    return (q.is_cuda and q.dtype in (torch.bfloat16, torch.float16) and k.dtype == q.dtype and v.dtype == q.dtype
+            and q.size(3) in HEAD_DIMS and v.size(3) == q.size(3) and q.numel() > 0 and k.numel() > 0
+            and k.shape == v.shape and q.size(0) <= k.size(0) < 1 << 24)
+
+
+def _new_context(q, merged):
+    sq, b, np_, hn = q.shape
+    if merged:
+        return torch.empty((sq, b, np_, hn), dtype=q.dtype, device=q.device)
+    return torch.empty((b, np_, sq, hn), dtype=q.dtype, device=q.device).permute(2, 0, 1, 3)
+
+
+def _finished(out, merged):
+    """``[sq, b, np, hn]`` in the layout that the caller of ``CoreAttention`` gets."""
+    if merged:
+        return out.view(out.size(0), out.size(1), -1)
+    return out.permute(1, 2, 0, 3)
+
+
+def _launch(out, lse, q, k, v, bits, mask_batches, fill, scale, window, who):
+    sq, b, np_, hn = q.shape
+    with _hp.device_guard(q):
+        rc = _hp.lib().nhp_attention_fwd(
+            out.data_ptr(), None if lse is None else lse.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
+            None if bits is None else bits.data_ptr(), mask_batches, fill, scale, -1 if window is None else window, b, np_,
+            k.size(2), sq, k.size(0), hn, _strides3(q), _strides3(k), _strides3(v), _strides3(out), _hp.dtype_code(q, who),
+            _hp.stream_of(q))
+    _hp.check(rc, who)
+
+
+class CausalAttention(torch.autograd.Function):
+    """``softmax(scale * q k^T) v`` under the causal mask (by index, with an optional sliding window)."""
+
+    @staticmethod
+    def forward(ctx, q, k, v, scale, window, merged):
+        q, k, v = _readable(q), _readable(k), _readable(v)
+        out = _new_context(q, merged)
+        need = any(ctx.needs_input_grad[:3])
+        lse = torch.empty((q.size(1) * q.size(2), q.size(0)), dtype=torch.float32, device=q.device) if need else None
+        _launch(out, lse, q, k, v, None, 1, 0.0, scale, window, "CausalAttention")
+        if need:
+            ctx.save_for_backward(q, k, v, out, lse)
+            ctx.conf = (scale, window, merged)
+        return _finished(out, merged)
+
+    @staticmethod
+    def backward(ctx, grad):
+        who = "CausalAttention backward"
+        q, k, v, out, lse = ctx.saved_tensors
+        scale, window, merged = ctx.conf
+        sq, b, np_, hn = q.shape
+        sk, nkv = k.size(0), k.size(2)
+        g = _readable(grad.view(sq, b, np_, hn) if merged and grad.is_contiguous() else
+                      grad.reshape(sq, b, np_, hn) if merged else grad.permute(2, 0, 1, 3))
+        dq, dk, dv = torch.empty_like(q, memory_format=torch.contiguous_format), torch.empty_like(
+            k, memory_format=torch.contiguous_format), torch.empty_like(v, memory_format=torch.contiguous_format)
+        lib = _hp.lib()
+        workspace = torch.empty(lib.nhp_attention_bwd_workspace_bytes(b, np_, nkv, sq, sk, hn), dtype=torch.uint8, device=q.device)
+        with _hp.device_guard(q):
+            rc = lib.nhp_attention_bwd(
+                dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), g.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
+                out.data_ptr(), lse.data_ptr(), workspace.data_ptr(), scale, -1 if window is None else window, b, np_, nkv,
+                sq, sk, hn, _strides3(dq), _strides3(dk), _strides3(dv), _strides3(g), _strides3(q), _strides3(k), _strides3(v),
+                _strides3(out), _hp.dtype_code(q, who), _hp.stream_of(q))
+        _hp.check(rc, who)
+        needs = ctx.needs_input_grad
+        return dq if needs[0] else None, dk if needs[1] else None, dv if needs[2] else None, None, None, None
+
+
+def causal_attention(q, k, v, scale, window=None, merged=False):
+    """Context of q ``[s, b, np, hn]`` over k, v ``[s, b, nkv, hn]``: ``[b, np, s, hn]``, or with ``merged``
+    ``[s, b, np * hn]``. Query i attends to keys ``i - window .. i``."""
+    return CausalAttention.apply(q, k, v, float(scale), window, merged)
+
+
+def masked_attention(q, k, v, mask, scale, fill, merged=False):
+    """Inference only: the context under a boolean mask ``[1 or b, 1, sq, sk]`` (True = masked), whose scores are
+    replaced by ``fill`` after scaling."""
+    q, k, v = _readable(q), _readable(k), _readable(v)
+    sq, sk = q.size(0), k.size(0)
+    mask = mask.contiguous()
+    bits = torch.empty((mask.size(0), sq, (sk + 63) // 64), dtype=torch.int64, device=q.device)
+    out = _new_context(q, merged)
+    with _hp.device_guard(q):
+        rc = _hp.lib().nhp_attention_mask_bits(bits.data_ptr(), mask.data_ptr(), mask.size(0), sq, sk, _hp.stream_of(q))
+    _hp.check(rc, "masked_attention")
+    _launch(out, None, q, k, v, bits, mask.size(0), fill, float(scale), None, "masked_attention")
+    return _finished(out, merged)

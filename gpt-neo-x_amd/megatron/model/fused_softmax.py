@@ -223,6 +223,17 @@ class ScaledMaskedSoftmaxDropout(torch.autograd.Function):
         return grad, None, None, None, None, None, grad_bias, None, None
 
 
+def _fill_value(mask_func):
+    """The value that ``mask_func(scores, mask)`` puts in place of masked scores if that is what it does, leaving the
+    others alone, and if it is so low that they count for nothing beside any other; otherwise None. Found out on one
+    masked and one other score."""
+    try:
+        kept, filled = mask_func(torch.tensor([[[[0.5, 1.5]]]]), torch.tensor([[[[False, True]]]])).flatten().tolist()
+    except Exception:
+        return None
+    return filled if kept == 0.5 and filled <= -10000.0 else None
+
+
 class FusedScaleMaskSoftmax(nn.Module):
     """Scaling, masking and softmax of attention scores ``[b, np, sq, sk]``.
 
@@ -282,6 +293,23 @@ class FusedScaleMaskSoftmax(nn.Module):
             self.alibi_slopes = None
         else:
             self.register_buffer("alibi_slopes", alibi_slopes.detach().float().clone(), persistent=False)
+
+    # ------------------------------------------------------------------ mask function
+    @property
+    def mask_func(self):
+        return self._mask_func
+
+    @mask_func.setter
+    def mask_func(self, func):
+        self._mask_func = func
+        self._mask_fill = ()
+
+    @property
+    def mask_fill(self):
+        """What ``mask_func`` fills masked scores with, None if that is not what it does (found out at first use)."""
+        if self._mask_fill == ():
+            self._mask_fill = _fill_value(self._mask_func)
+        return self._mask_fill
 
     # ------------------------------------------------------------------ dispatch
     def forward(self, input, mask, bias=None, key_lengths=None):

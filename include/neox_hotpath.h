@@ -707,6 +707,39 @@ int nhp_rmsnorm_partial_bwd(void* dx, void* dscale, void* doffset, const void* d
 
 int64_t nhp_norm_bwd_workspace_bytes(int64_t rows, int64_t cols, int dtype);
 
+/* ---------------------------------------------------------------- attention
+ * softmax(scale * q k^T, masked) v in one kernel, 16-bit storage, fp32 scores, statistics and accumulation
+ * (what megatron/model/transformer.py:526-625 computes with two GEMMs and the fused softmax between them).
+ * q [sq, batch, heads, head_dim], k and v [sk, batch, kv_heads, head_dim] (kv_heads divides heads: query head h uses
+ * head h / (heads / kv_heads)), out like q: each a pointer and three element strides {sequence, batch, head}; features
+ * are contiguous, pointers 16-byte aligned, strides multiples of 8. head_dim 64, 80, 96 or 128. scale > 0.
+ *
+ * Without mask_bits: key k is visible to query q when q + (sk - sq) - window <= k <= q + (sk - sq) (window < 0: no lower
+ * limit). With mask_bits (from nhp_attention_mask_bits, mask_batches 1 or batch): masked scores are replaced by
+ * mask_fill (-10000, or the lowest float), rows without a visible key are averages, as a softmax over a row of equal
+ * fill values gives.
+ *
+ * lse (may be NULL): [batch * heads, sq] floats, base-2 logarithm of each row's sum of exponentials of scale * score;
+ * the backward takes it. */
+int nhp_attention_mask_bits(void* bits, const void* mask, int64_t batches, int64_t sq, int64_t sk, void* stream);
+int nhp_attention_fwd(void* out, float* lse, const void* q, const void* k, const void* v, const void* mask_bits,
+                      int64_t mask_batches, float mask_fill, float scale, int64_t window, int64_t batch, int64_t heads,
+                      int64_t kv_heads, int64_t sq, int64_t sk, int64_t head_dim, const int64_t* q_strides,
+                      const int64_t* k_strides, const int64_t* v_strides, const int64_t* out_strides, int dtype,
+                      void* stream);
+
+/* Gradients of nhp_attention_fwd without mask_bits, from its operands, its result and its lse (in the reference the
+ * backward of the two GEMMs and of the softmax, megatron/model/transformer.py:526-625). workspace:
+ * nhp_attention_bwd_workspace_bytes, 16-byte aligned. The same sums in the same order on every run. */
+int64_t nhp_attention_bwd_workspace_bytes(int64_t batch, int64_t heads, int64_t kv_heads, int64_t sq, int64_t sk,
+                                          int64_t head_dim);
+int nhp_attention_bwd(void* dq, void* dk, void* dv, const void* d_out, const void* q, const void* k, const void* v,
+                      const void* out, const float* lse, void* workspace, float scale, int64_t window, int64_t batch,
+                      int64_t heads, int64_t kv_heads, int64_t sq, int64_t sk, int64_t head_dim,
+                      const int64_t* dq_strides, const int64_t* dk_strides, const int64_t* dv_strides,
+                      const int64_t* d_out_strides, const int64_t* q_strides, const int64_t* k_strides,
+                      const int64_t* v_strides, const int64_t* out_strides, int dtype, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,131 @@
+"""The attention kernels (csrc/attention.hip) through ``megatron.model.fused_attention`` and ``CoreAttention``, against
+textbook attention in fp32 torch ops: edges of the 64-key tiles and of the 128-query blocks, head sizes that fill a tile
+row and ones that do not, grouped heads, sliding windows, and bit masks with rows that see nothing.
+
+Tolerance: a rounding to the storage type is off by at most u = 2^-8 (bf16) or 2^-11 (fp16), u / sqrt(3) in the mean
+square; n of them in a row by sqrt(n / 3) u relative to the 2-norm. A context goes through two (probability, result), a
+gradient of v as well. A gradient of q or k goes through two (gradient of the score, result) and through that of the
+context, which enters as dP - dO . context: a difference that is half as large as its members when a query sees only two
+keys (window 1), so the rounding counts twice, in squares four times. Gradients of shared heads are rounded once more
+before they are summed."""
+import math
+
+import pytest
+import torch
+
+import util
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+DTYPES = pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+
+
+def limit(dtype, roundings):
+    return math.sqrt(roundings / 3) * (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11)
+
+
+def rel_err(a, b):
+    return ((a.float() - b.float()).norm() / b.float().norm()).item()
+
+
+def textbook(q, k, v, mask, fill=torch.finfo(torch.float32).min):
+    """[sq, b, np, hn] in fp32; mask broadcastable to [b, np, sq, sk]."""
+    group = q.size(2) // k.size(2)
+    k, v = (torch.repeat_interleave(t.float(), group, dim=2).permute(1, 2, 0, 3) for t in (k, v))
+    scores = torch.matmul(q.float().permute(1, 2, 0, 3).contiguous(), k.transpose(-1, -2).contiguous()) / math.sqrt(q.size(-1))
+    probs = torch.softmax(scores.masked_fill(mask, fill), dim=-1)
+    return torch.matmul(probs, v.contiguous()).permute(2, 0, 1, 3)
+
+
+def hidden(sq, sk, window=None):
+    q = torch.arange(sq, device=DEV).view(sq, 1) + sk - sq
+    k = torch.arange(sk, device=DEV).view(1, sk)
+    return (k > q) if window is None else (k > q) | (k < q - window)
+
+
+def operands(dtype, sq, sk, b, np_, nkv, hn, seed):
+    return [util.randn((s, b, n, hn), dtype, seed=seed + i).to(DEV) for i, (s, n) in enumerate(((sq, np_), (sk, nkv), (sk, nkv)))]
+
+
+@DTYPES
+@pytest.mark.parametrize("hn", [64, 80, 96, 128])
+@pytest.mark.parametrize("s,b,np_,nkv,window", [(20, 1, 4, 4, None), (64, 1, 4, 4, None), (65, 2, 4, 2, None), (128, 1, 8, 2, 1),
+                                                (260, 3, 3, 3, None), (700, 1, 4, 1, 37), (513, 1, 9, 3, 128)])
+def test_causal_forward_and_gradients(dtype, hn, s, b, np_, nkv, window):
+    from megatron.model.fused_attention import causal_attention
+
+    q, k, v = (t.requires_grad_(True) for t in operands(dtype, s, s, b, np_, nkv, hn, 1))
+    out = causal_attention(q, k, v, 1 / math.sqrt(hn), window, merged=True)
+    g = util.randn((s, b, np_ * hn), dtype, seed=9).to(DEV)
+    out.backward(g)
+    qr, kr, vr = (t.detach().float().requires_grad_(True) for t in (q, k, v))
+    ref = textbook(qr, kr, vr, hidden(s, s, window))
+    ref.backward(g.float().view(s, b, np_, hn))
+    assert rel_err(out.view(s, b, np_, hn), ref) <= limit(dtype, 2)
+    for got, want, n in ((q.grad, qr.grad, 6), (k.grad, kr.grad, 6 + (np_ != nkv)), (v.grad, vr.grad, 2 + (np_ != nkv))):
+        assert rel_err(got, want) <= limit(dtype, n)
+    # the other layout, strided operands and a second run: the same bits
+    wide = torch.stack((q.detach(), k.detach().expand_as(q) if nkv == np_ else q.detach()), dim=3).flatten(3)[..., :hn]
+    again = causal_attention(wide, k.detach(), v.detach(), 1 / math.sqrt(hn), window).permute(2, 0, 1, 3)
+    assert torch.equal(util.raw_bits(again.reshape(s, b, np_ * hn)), util.raw_bits(out.detach()))
+
+
+@DTYPES
+@pytest.mark.parametrize("hn", [64, 80, 128])
+@pytest.mark.parametrize("sq,sk,b,np_,nkv", [(1, 1, 1, 4, 4), (1, 200, 2, 4, 2), (5, 64, 1, 4, 4), (130, 333, 2, 4, 4)])
+def test_masked_forward(dtype, hn, sq, sk, b, np_, nkv):
+    """Random masks, a whole tile hidden from every query, and rows that see nothing: those are averages over all keys."""
+    from megatron.model.fused_attention import masked_attention
+
+    q, k, v = operands(dtype, sq, sk, b, np_, nkv, hn, 21)
+    mask = torch.rand((b, 1, sq, sk), generator=torch.Generator().manual_seed(3)).to(DEV) < 0.6
+    mask[:, :, :, 64:128] = True
+    mask[0, :, -1] = True
+    for m in (mask, mask[:1], hidden(sq, sk).view(1, 1, sq, sk)):
+        for fill in (-10000.0, torch.finfo(torch.float32).min):
+            out = masked_attention(q, k, v, m, 1 / math.sqrt(hn), fill, merged=True)
+            assert rel_err(out.view(sq, b, np_, hn), textbook(q, k, v, m, fill)) <= limit(dtype, 2)
+
+
+def test_masked_scores_as_low_as_the_fill_value_count():
+    """With visible scores around -10000 the masked keys of the padding-mask kernel take part in the softmax."""
+    from megatron.model.fused_attention import masked_attention
+
+    q, k, v = operands(torch.bfloat16, 96, 192, 1, 4, 4, 64, 5)
+    q[..., 0], k[..., 0] = 250.0, -320.0   # every score is near -80000 / 8
+    mask = hidden(96, 192).view(1, 1, 96, 192)
+    out = masked_attention(q, k, v, mask, 1 / 8, -10000.0, merged=True)
+    want = textbook(q, k, v, mask, -10000.0)
+    assert rel_err(want, textbook(q, k, v, mask)) > 0.1   # the masked keys matter
+    # scores of 1e4 carry an fp32 rounding of up to 2^-11 here and in the reference: 1e-3 of a probability
+    assert rel_err(out.view(96, 1, 4, 64), want) <= limit(torch.bfloat16, 2) + 2e-3
+
+
+def test_the_caller_takes_the_kernels_and_the_mask_where_it_counts():
+    """``CoreAttention``: a prompt of a length that the softmax gate rejects (forward only) attends by the mask it is
+    given; with a gradient wanted, or a mask function that does not fill, the reference's torch branch stays."""
+    from megatron.model import fused_attention
+    from megatron.model.attention_core import CoreAttention
+    from megatron.model.fused_softmax import SoftmaxFusionTypes as T
+
+    def fills(scores, mask):
+        return scores.masked_fill_(mask, torch.finfo(scores.dtype).min)
+
+    def penalises(scores, mask):
+        return scores - 2.0 * mask.to(scores.dtype)
+
+    s, b, np_, hn = 77, 2, 4, 64
+    q, k, v = operands(torch.bfloat16, s, s, b, np_, np_, hn, 31)
+    mask = hidden(s, s).view(1, 1, s, s).repeat(b, 1, 1, 1)
+    mask[1, :, :, :20] = True   # left padding: the first rows of the second entry see nothing
+    want = textbook(q, k, v, mask)
+    core = CoreAttention(hn, 1, False, True, T.upper_triang, fills, attention_softmax_in_fp32=True)
+    soft = CoreAttention(hn, 1, False, True, T.upper_triang, penalises, attention_softmax_in_fp32=True)
+    assert soft.scale_mask_softmax.mask_fill is None and core.scale_mask_softmax.mask_fill == torch.finfo(torch.float32).min
+    assert core._one_kernel(q, k, v, mask, None, False) is not None
+    assert soft._one_kernel(q, k, v, mask, None, False) is None
+    assert core._one_kernel(q.clone().requires_grad_(True), k, v, mask, None, False) is None
+    assert rel_err(core(q, k, v, mask).permute(2, 0, 1, 3), want) <= limit(torch.bfloat16, 2)
+    # the torch branch rounds the scores to bf16 first: one more rounding, of a score of up to 4 instead of a value
+    assert rel_err(core(q.clone().requires_grad_(True), k, v, mask).permute(2, 0, 1, 3), want) <= 2.0 ** -7
+    assert not fused_attention.supported(q[..., :40], k[..., :40], v[..., :40])

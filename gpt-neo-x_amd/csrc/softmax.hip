@@ -13,7 +13,9 @@
 //   n <= 65536      : W = 1..8 (16 beyond 32768) waves per row with K = 1..8
 //                     chunks per lane; partial max / sum are exchanged through
 //                     2*W floats of LDS (see plan_row for the choice)
-//   otherwise, or if n % 8 != 0 or a pointer is not 16-byte aligned:
+//   n % 8 != 0 or a pointer is not 16-byte aligned:
+//                     the kernels of softmax_ragged.hip
+//   what neither takes (n > 65536, n < 8, n > 16384 where n % 8 != 0 or a pointer is not aligned):
 //                     a scalar three-pass kernel (one workgroup per row).
 //
 // Arithmetic (fp32): z = x*scale, m = max z, e = 2^((z-m)*log2(e) + 64),
@@ -33,12 +35,10 @@
 // backward first applies the dropout backward to dy; the keep mask is
 // regenerated from a counter-based generator, never stored.
 
-#include "common.hpp"
+#include "softmax_ragged.hpp"
 
 namespace nhp {
 
-constexpr float kExpBias = 64.0f;
-constexpr float kMaskFill = -10000.0f;  // scaled_masked_softmax.h:180-184 of the reference
 // Row blocks of one head that are taken for every batch entry in turn when a bias tensor is shared by the
 // batch (batch_interleaved_block); 0: all row blocks of a matrix.
 constexpr int kBiasShareGroup = 0;
@@ -201,14 +201,6 @@ __device__ __forceinline__ Band written_range(uint32_t q, uint32_t window, uint3
         b.lo = r0 > window ? ((r0 - window) >> zshift) << zshift : 0u;
     }
     return b;
-}
-
-// Number of real keys of matrix `mat` ([batch * heads] matrices, one length per batch entry).
-__device__ __forceinline__ uint32_t key_limit(const int32_t* key_lengths, uint32_t mat, uint32_t heads)
-{
-    if (key_lengths == nullptr) return 0xffffffffu;
-    const int32_t len = key_lengths[mat / heads];
-    return len < 0 ? 0u : (uint32_t)len;
 }
 
 // Bit k set: register slot k of wave-slot w holds at least one column of the
@@ -807,8 +799,8 @@ softmax_bwd_kernel(uint16_t* dx, const uint16_t* dy, const uint16_t* y, float sc
 }
 
 // ---------------------------------------------------------------------------
-// Scalar kernels for rows the chunked layout cannot take (n % 8 != 0,
-// unaligned pointers, n > 65536). One workgroup of 256 threads per row,
+// Scalar kernels for rows that neither the chunked layout nor the kernels of
+// softmax_ragged.hip take (see the top of the file). One workgroup of 256 threads per row,
 // the row is re-read from global memory (L2) for every pass.
 // ---------------------------------------------------------------------------
 constexpr int kScalarThreads = 256;
@@ -1118,6 +1110,10 @@ static int causal_fwd(void* y, const void* x, float scale, int64_t batches, int6
     }
         NHP_FOR_PLAN(p);
 #undef CALL
+    } else if (ragged_rows(n)) {
+        const RaggedArgs a{yp, xp, nullptr, nullptr, slopes, bp, kl, scale, (uint32_t)n, (uint32_t)n, heads,
+                           (uint32_t)rows, window, 0, dp, dk};
+        return ragged_causal_fwd<DT>(a, st);
     } else {
         if (!launch_fits(rows, kScalarThreads)) return NHP_ERR_SHAPE;
         scalar_fwd_kernel<DT, 0><<<(uint32_t)rows, kScalarThreads, 0, st>>>(
@@ -1163,6 +1159,10 @@ static int softmax_bwd(void* dx, const void* dy, const void* y, float scale, int
     }
         NHP_FOR_PLAN(p);
 #undef CALL
+    } else if (ragged_rows(n)) {
+        const RaggedArgs a{dxp, dyp, yp, nullptr, nullptr, nullptr, CAUSAL ? kl : nullptr, scale, (uint32_t)n,
+                           (uint32_t)rows_per_matrix, heads, (uint32_t)rows, window, 0, nullptr, dk};
+        return ragged_bwd<DT, CAUSAL>(a, dropout, st);
     } else {
         if (!launch_fits(rows, kScalarThreads)) return NHP_ERR_SHAPE;
         scalar_bwd_kernel<DT, CAUSAL><<<(uint32_t)rows, kScalarThreads, 0, st>>>(
@@ -1235,6 +1235,10 @@ static int masked_fwd(void* y, const void* x, const uint8_t* mask, float scale, 
         NHP_FOR_PLAN(p);
 #undef CALL
 #undef LAUNCH_MASKED
+    } else if (ragged_rows(n)) {
+        const RaggedArgs a{yp, xp, nullptr, mask, ex.slopes, bp, ex.key_lengths, scale, (uint32_t)n, (uint32_t)sq,
+                           (uint32_t)np, (uint32_t)(b * np * sq), kNoWindow, per_batch, dp, dk};
+        return ragged_masked_fwd<DT>(a, st);
     } else {
         if (!launch_fits(b * np * sq, kScalarThreads)) return NHP_ERR_SHAPE;
         scalar_fwd_kernel<DT, 1><<<(uint32_t)(b * np * sq), kScalarThreads, 0, st>>>(

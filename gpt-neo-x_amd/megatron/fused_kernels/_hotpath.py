@@ -93,6 +93,9 @@ def _declare(lib):
         "nhp_attention_fwd": ([vp] * 6 + [i64, f32, f32] + [i64] * 7 + [p64] * 4 + [ci, vp], ci),
         "nhp_attention_bwd": ([vp] * 10 + [f32] + [i64] * 7 + [p64] * 8 + [ci, vp], ci),
         "nhp_attention_bwd_workspace_bytes": ([i64] * 6, i64),
+        "nhp_attention_decode": ([vp] * 8 + [i64, i64, f32, vp, f32] + [i64] * 6 + [p64] * 6 + [ci, vp], ci),
+        "nhp_attention_decode_workspace_bytes": ([i64] * 6, i64),
+        "nhp_kv_cache_append": ([vp] * 5 + [i64] * 5 + [p64] * 4 + [ci, vp], ci),
         "nhp_layernorm_bwd_noalloc": ([vp, vp, vp, vp, vp, vp, vp, vp, i64, i64, ci, ci, vp], ci),
     }
     for name, (args, res) in sigs.items():
@@ -156,6 +159,14 @@ def forward_scale(scale_factor, t, narrow):
 def require_gpu(t, what):
     if t.device.type != "cuda":
         raise RuntimeError(f"{what}: expected a tensor on the GPU, got device {t.device}")
+
+
+def followed(*tensors):
+    """Whether torch follows the operations on any of these beyond autograd (vmap and the other function transforms,
+    forward-mode derivatives, tracing, tensor subclasses): a launch outside of an autograd function would escape it."""
+    return (torch.autograd.forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None
+            or any((type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter)
+                   or torch._C._functorch.is_functorch_wrapped_tensor(t) for t in tensors))
 
 
 # torch's direct accessor of the current stream's handle (what its own launchers use): about a microsecond

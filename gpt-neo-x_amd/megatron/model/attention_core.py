@@ -227,10 +227,17 @@ class CoreAttention(torch.nn.Module):
             softmax_in_fp32=attention_softmax_in_fp32, scale=softmax_scale, sliding_window_width=sliding_window_width,
             alibi_slopes=alibi_slopes, attention_dropout=attention_dropout)
 
-    def forward(self, query_layer, key_layer, value_layer, attention_mask, key_lengths=None, merged_heads=False):
+    def forward(self, query_layer, key_layer, value_layer, attention_mask, key_lengths=None, merged_heads=False,
+                layer_past=None):
         """Returns the context as ``[b, np, sq, hn]`` (what ``ParallelSelfAttention.attention`` returns), or with
         ``merged_heads`` as ``[sq, b, np * hn]``, the layout its caller brings it into before the output
-        projection, written by the context GEMM itself."""
+        projection, written by the context GEMM itself. ``layer_past``: the cached keys and values
+        ``[2, past, b, nkv, hn]``, ``key_layer`` and ``value_layer`` then being those of the new positions alone; the
+        result is ``(context, present)``, both from one pass over the cache, or None where that kernel does not apply
+        (a gradient is wanted, something else than the mask is in play, too many new positions): the caller then
+        concatenates."""
+        if layer_past is not None:
+            return self._cached_step(query_layer, key_layer, value_layer, attention_mask, merged_heads, layer_past)
         b, np_, sq, sk = query_layer.size(1), query_layer.size(2), query_layer.size(0), key_layer.size(0)
         hn = query_layer.size(3)
         if self.use_cache and attention_mask is not None:
@@ -280,6 +287,23 @@ class CoreAttention(torch.nn.Module):
         to the scores, dropped, or not provided by them. Which keys a query sees is decided as by the softmax module:
         by index where that would run its causal kernel, otherwise by the mask (forward only; with the fill value of the
         padding-mask kernel where that would run, and of the mask function where the torch branch would)."""
+        scale = self._plain_scale(query, key, value, mask, key_lengths)
+        if scale is None:
+            return None
+        softmax = self.scale_mask_softmax
+        b, np_, sq, sk = query.size(1), query.size(2), query.size(0), key.size(0)
+        if softmax.upper_triang_mask_fusion and sq == sk and softmax.is_kernel_available(mask, b, np_, sq, sk):
+            window = softmax.sliding_window_width
+            window = None if window is None or window < 0 else int(window)
+            return fused_attention.causal_attention(query, key, value, scale, window, merged_heads)
+        fill = self._fill_by_mask(mask, b, np_, sq, sk, query.device)
+        if fill is None or not fused_attention.plain(query, key, value):
+            return None
+        return fused_attention.masked_attention(query, key, value, mask, scale, fill, merged_heads)
+
+    def _plain_scale(self, query, key, value, mask, key_lengths):
+        """The factor of the scores where they are scaled, masked and nothing else, and the operands are the attention
+        kernels'; otherwise None."""
         softmax = self.scale_mask_softmax
         if (key_lengths is not None or self.rpe is not None or softmax.alibi_slopes is not None or not softmax.fusion
                 or softmax.narrow_forward_scale or mask is None or (softmax.training and softmax.attention_dropout > 0.0)):
@@ -287,26 +311,40 @@ class CoreAttention(torch.nn.Module):
         if not fused_attention.supported(query, key, value) or not softmax.input_in_float16:
             return None
         scale = self.gemm_alpha * (1.0 if softmax.scale is None else softmax.scale)
-        if not scale > 0.0:
-            return None
-        b, np_, sq, sk = query.size(1), query.size(2), query.size(0), key.size(0)
-        if softmax.upper_triang_mask_fusion and sq == sk:
-            if softmax.is_kernel_available(mask, b, np_, sq, sk):
-                window = softmax.sliding_window_width
-                window = None if window is None or window < 0 else int(window)
-                return fused_attention.causal_attention(query, key, value, scale, window, merged_heads)
-            kernel = False
-        elif softmax.upper_triang_mask_fusion:
-            kernel = softmax._rectangular_kernel_available(mask, b, np_, sq, sk)
+        return scale if scale > 0.0 else None
+
+    def _fill_by_mask(self, mask, b, np_, sq, sk, device):
+        """What masked scores are replaced by where the mask decides, None if the kernels cannot follow it."""
+        softmax = self.scale_mask_softmax
+        if softmax.upper_triang_mask_fusion:
+            kernel = sq != sk and softmax._rectangular_kernel_available(mask, b, np_, sq, sk)
         else:
             kernel = softmax.is_kernel_available(mask, b, np_, sq, sk)
         fill = -10000.0 if kernel else softmax.mask_fill
-        if (fill is None or sk > 65536 or mask.dtype != torch.bool or mask.device != query.device
+        if (fill is None or sk > 65536 or mask.dtype != torch.bool or mask.device != device
                 or mask.shape not in ((1, 1, sq, sk), (b, 1, sq, sk))):
             return None
-        if torch.is_grad_enabled() and (query.requires_grad or key.requires_grad or value.requires_grad):
+        return fill
+
+    def _cached_call(self, query, key, value, mask, layer_past):
+        """``(mask, scale, fill)`` for the decoding kernel, or None where it does not apply."""
+        if not fused_attention.decode_supported(query, key, value, layer_past):
             return None
-        return fused_attention.masked_attention(query, key, value, mask, scale, fill, merged_heads)
+        b, np_, sq, sk = query.size(1), query.size(2), query.size(0), layer_past.size(1) + key.size(0)
+        if self.use_cache and mask is not None:
+            mask = mask[..., :sk, :sk]
+        scale = self._plain_scale(query, key, value, mask, None)
+        if scale is None:
+            return None
+        fill = self._fill_by_mask(mask, b, np_, sq, sk, query.device)
+        return None if fill is None else (mask, scale, fill)
+
+    def _cached_step(self, query, key, value, mask, merged_heads, layer_past):
+        call = self._cached_call(query, key, value, mask, layer_past)
+        if call is None:
+            return None
+        mask, scale, fill = call
+        return fused_attention.decode_attention(query, key, value, layer_past, mask, scale, fill, merged_heads)
 
     def _causal_block(self, attention_mask, b, np_, sq, sk, like):
         """Block size for the blocked causal GEMMs, 0 when the scores do not go to the causal kernel (which is what

@@ -126,3 +126,78 @@ def masked_attention(q, k, v, mask, scale, fill, merged=False):
     _hp.check(rc, "masked_attention")
     _launch(out, None, q, k, v, bits, mask.size(0), fill, float(scale), None, "masked_attention")
     return _finished(out, merged)
+
+
+MAX_DECODE_ROWS = 32   # queries that share a key/value head, in nhp_attention_decode
+
+
+def plain(*tensors):
+    """Whether nobody differentiates these or otherwise follows what is done with them."""
+    return not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors)) and not _hp.followed(*tensors)
+
+
+def cache_supported(key, value, layer_past):
+    """Whether ``append_to_cache`` takes these: 16-bit tensors on the GPU that nobody differentiates; ``layer_past``
+    (None: no cached positions) of their type and shape."""
+    if not (key.is_cuda and key.dtype in (torch.bfloat16, torch.float16) and key.dim() == 4 and value.shape == key.shape
+            and value.dtype == key.dtype and value.device == key.device and key.numel() > 0 and key.size(3) % 8 == 0
+            and plain(key, value)):
+        return False
+    sk, width = key.size(0), key.numel() // key.size(0)
+    if layer_past is not None:
+        if not (isinstance(layer_past, torch.Tensor) and layer_past.dim() == 5 and layer_past.size(0) == 2
+                and layer_past.shape[2:] == key.shape[1:] and layer_past.dtype == key.dtype
+                and layer_past.device == key.device and plain(layer_past)):
+            return False
+        sk += layer_past.size(1)
+    return width < 1 << 24 and sk < 1 << 24 and sk * width // key.size(3) < 1 << 31
+
+
+def append_to_cache(key, value, layer_past):
+    """``torch.stack((cat(past keys, key), cat(past values, value)))`` in one launch: ``[2, past + sq, b, nkv, hn]``."""
+    key, value = _readable(key), _readable(value)
+    past_k, past_v = (None, None) if layer_past is None else (_readable(t) for t in layer_past)
+    past = 0 if past_k is None else past_k.size(0)
+    sq, b, nkv, hn = key.shape
+    present = torch.empty((2, past + sq, b, nkv, hn), dtype=key.dtype, device=key.device)
+    with _hp.device_guard(key):
+        rc = _hp.lib().nhp_kv_cache_append(
+            present.data_ptr(), key.data_ptr(), value.data_ptr(), past_k.data_ptr() if past else None,
+            past_v.data_ptr() if past else None, b, nkv, sq, past, hn, _strides3(key), _strides3(value),
+            _strides3(past_k) if past else None, _strides3(past_v) if past else None, _hp.dtype_code(key, "append_to_cache"),
+            _hp.stream_of(key))
+    _hp.check(rc, "append_to_cache")
+    return present
+
+
+def decode_supported(query, key, value, layer_past):
+    """Whether ``decode_attention`` takes these (beside what ``cache_supported`` asks for): some cached positions, and
+    few enough queries for each key/value head."""
+    return (supported(query, key, value) and layer_past is not None and cache_supported(key, value, layer_past) and plain(query)
+            and layer_past.size(1) > 0 and layer_past.size(1) + key.size(0) >= 4 and query.size(1) * query.size(2) <= 1 << 24
+            and query.size(2) % key.size(2) == 0 and query.size(0) * (query.size(2) // key.size(2)) <= MAX_DECODE_ROWS)
+
+
+def decode_attention(query, key, value, layer_past, mask, scale, fill, merged=False):
+    """``masked_attention`` of new positions over the cached ones and themselves, and ``append_to_cache``, in one pass
+    over the cache: ``(context, present)``. ``mask`` ``[1 or b, 1, sq, past + sq]``, True = masked."""
+    query, key, value = _readable(query), _readable(key), _readable(value)
+    past_k, past_v = (_readable(t) for t in layer_past)
+    sq, b, np_, hn = query.shape
+    nkv, past = key.size(2), past_k.size(0)
+    if mask.stride(3) != 1:
+        mask = mask.contiguous()
+    out = _new_context(query, merged)
+    present = torch.empty((2, past + sq, b, nkv, hn), dtype=key.dtype, device=key.device)
+    lib = _hp.lib()
+    scratch = lib.nhp_attention_decode_workspace_bytes(b, np_, nkv, sq, past, hn)
+    workspace = torch.empty(scratch, dtype=torch.uint8, device=query.device) if scratch else None
+    with _hp.device_guard(query):
+        rc = lib.nhp_attention_decode(
+            out.data_ptr(), present.data_ptr(), query.data_ptr(), key.data_ptr(), value.data_ptr(), past_k.data_ptr(),
+            past_v.data_ptr(), mask.data_ptr(), mask.stride(0) if mask.size(0) > 1 else 0, mask.stride(2), fill,
+            None if workspace is None else workspace.data_ptr(), scale, b, np_, nkv, sq, past, hn, _strides3(out), _strides3(query),
+            _strides3(key), _strides3(value), _strides3(past_k), _strides3(past_v), _hp.dtype_code(query, "decode_attention"),
+            _hp.stream_of(query))
+    _hp.check(rc, "decode_attention")
+    return _finished(out, merged), present

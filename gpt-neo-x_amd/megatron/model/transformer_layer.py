@@ -25,6 +25,7 @@ mixture of experts, flash and sparse attention, Transformer Engine layers.
 import torch
 import torch.nn.functional as F
 
+from . import fused_attention
 from .activations import Gated_Activation, get_activation
 from .attention_core import (CoreAttention, apply_rotary_to_query_key, get_fusion_type, split_gqa_and_rotate,
                              split_qkv_and_rotate)
@@ -149,13 +150,25 @@ class SelfAttention(torch.nn.Module):
                 if self.rotary_emb is not None:
                     query, key = apply_rotary_to_query_key(query, key, self.rotary_emb, rotary_ndims=self.rotary_ndims,
                                                            rope_fusion=False, bf16=self.bf16, layer_past=layer_past)
-        if layer_past is not None and layer_past.numel() > 0:
-            past_key, past_value = layer_past
-            key = torch.cat((past_key.type_as(key), key), dim=0)
-            value = torch.cat((past_value.type_as(value), value), dim=0)
-        present = torch.stack((key, value)) if self.use_cache else None
-        # [sq, b, np * hn], written in that layout by the context GEMM
-        context = self.core(query, key, value, attention_mask, merged_heads=True)
+        past = layer_past if layer_past is not None and layer_past.numel() > 0 else None
+        step = None
+        if self.use_cache and past is not None and isinstance(self.core, CoreAttention):
+            step = self.core(query, key, value, attention_mask, merged_heads=True, layer_past=past)
+        if step is not None:
+            context, present = step
+        else:
+            if self.use_cache and fused_attention.cache_supported(key, value, past):
+                present = fused_attention.append_to_cache(key, value, past)
+                if past is not None:
+                    key, value = present
+            else:
+                if past is not None:
+                    past_key, past_value = past
+                    key = torch.cat((past_key.type_as(key), key), dim=0)
+                    value = torch.cat((past_value.type_as(value), value), dim=0)
+                present = torch.stack((key, value)) if self.use_cache else None
+            # [sq, b, np * hn], written in that layout by the attention kernel or the context GEMM
+            context = self.core(query, key, value, attention_mask, merged_heads=True)
         output, bias = self.dense(context)
         return ([output, present] if self.use_cache else output), bias
 

@@ -740,6 +740,28 @@ int nhp_attention_bwd(void* dq, void* dk, void* dv, const void* d_out, const voi
                       const int64_t* d_out_strides, const int64_t* q_strides, const int64_t* k_strides,
                       const int64_t* v_strides, const int64_t* out_strides, int dtype, void* stream);
 
+/* One decoding step (what megatron/model/transformer.py:916-958 does with two concatenations, a stack and the attention of
+ * :526-625): the context of sq new positions over `past` >= 1 cached ones and themselves, and the next cache
+ * cache_out [2, past + sq, batch, kv_heads, head_dim] (contiguous), in one pass over the cache. Operands as in
+ * nhp_attention_fwd; the new keys and values have sq rows, the cached ones `past`. mask: bytes, not zero = masked (replaced
+ * by mask_fill), element (b, s, k) at b * mask_batch_stride + s * mask_row_stride + k for k < past + sq; past + sq >= 4.
+ * sq * (heads / kv_heads) <= 32. workspace (may be NULL where its size is 0): nhp_attention_decode_workspace_bytes,
+ * 16-byte aligned; nothing has to be cleared in it. */
+int64_t nhp_attention_decode_workspace_bytes(int64_t batch, int64_t heads, int64_t kv_heads, int64_t sq, int64_t past,
+                                             int64_t head_dim);
+int nhp_attention_decode(void* out, void* cache_out, const void* q, const void* k_new, const void* v_new, const void* k_past,
+                         const void* v_past, const void* mask, int64_t mask_batch_stride, int64_t mask_row_stride,
+                         float mask_fill, void* workspace, float scale, int64_t batch, int64_t heads, int64_t kv_heads,
+                         int64_t sq, int64_t past, int64_t head_dim, const int64_t* out_strides, const int64_t* q_strides,
+                         const int64_t* k_new_strides, const int64_t* v_new_strides, const int64_t* k_past_strides,
+                         const int64_t* v_past_strides, int dtype, void* stream);
+
+/* cache_out as above without the attention (megatron/model/transformer.py:916-935): past may be 0, head_dim any multiple of 8. */
+int nhp_kv_cache_append(void* cache_out, const void* k_new, const void* v_new, const void* k_past, const void* v_past,
+                        int64_t batch, int64_t kv_heads, int64_t sq, int64_t past, int64_t head_dim,
+                        const int64_t* k_new_strides, const int64_t* v_new_strides, const int64_t* k_past_strides,
+                        const int64_t* v_past_strides, int dtype, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -3,8 +3,8 @@
 The data flow of GPT-NeoX's ``ParallelTransformerLayer`` (megatron/model/transformer.py:962-1321)
 with ``ParallelSelfAttention`` (:326-959) and ``ParallelMLP`` (:93-196) inside, without the
 model-parallel layers: every linear layer is a plain ``torch.nn.functional.linear`` (library
-GEMM) that hands its bias on instead of adding it (``skip_bias_add``), and everything between
-the GEMMs is one of the fused kernels:
+GEMM; for the few rows of a decoding step nhp_linear_decode) that hands its bias on instead of
+adding it (``skip_bias_add``), and everything between the GEMMs is one of the fused kernels:
 
     norm                      nhp_layernorm / nhp_rmsnorm (the two norms of the parallel-residual layout: nhp_layernorm_pair)
     qkv projection            GEMM (bias added by the GEMM, as ColumnParallelLinear does for qkv)
@@ -23,7 +23,6 @@ next call continues after them (inference, :916-935). Left out: tensor / sequenc
 mixture of experts, flash and sparse attention, Transformer Engine layers.
 """
 import torch
-import torch.nn.functional as F
 
 from . import fused_attention
 from .activations import Gated_Activation, get_activation
@@ -31,6 +30,7 @@ from .attention_core import (CoreAttention, apply_rotary_to_query_key, get_fusio
                              split_qkv_and_rotate)
 from .fused_bias_dropout import (bias_add_residual_pair, bias_dropout_add_fused_inference, bias_dropout_add_fused_train,
                                  get_bias_dropout_add)
+from .fused_linear import linear
 from .norms import get_norm, layer_norm_pair
 from .positional_embeddings import AliBi, RotaryEmbedding
 
@@ -49,8 +49,8 @@ class Linear(torch.nn.Module):
 
     def forward(self, x):
         if self.skip_bias_add:
-            return F.linear(x, self.weight), self.bias
-        return F.linear(x, self.weight, self.bias), None
+            return linear(x, self.weight), self.bias
+        return linear(x, self.weight, self.bias), None
 
 
 class MLP(torch.nn.Module):

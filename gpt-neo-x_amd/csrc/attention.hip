@@ -13,10 +13,10 @@
 // each recomputing the scores: seven products instead of five, but no atomic sums, so results are the same on every run.
 //
 // Measured (us, causal, forward / backward; products and softmax separately before, both per pass of the module):
-//   [8192, 1, 32 heads, 8 of keys, 128] bf16   552 / 1836 (986 / 1048 TFLOP/s)   whole pass 5786 -> 2322
-//   [2048, 8, 16, 128] bf16                    189 / 702  (729 / 686)            about 1930 -> 890
+//   [8192, 1, 32 heads, 8 of keys, 128] bf16   544 / 1770 (1011 / 1087 TFLOP/s)   whole pass 5786 -> 2322
+//   [2048, 8, 16, 128] bf16                    175 / 585  (788 / 823)            about 1930 -> 890
 //   [1024, 4, 12, 64] fp16                     26 / 65    (251 / 350)            whole pass 428 -> 172
-//   [1531, 1, 32, 128] bf16, by mask           54 + 6 for the bits               650 -> 60
+//   [1531, 1, 32, 128] bf16, by mask           57 + 7 for the bits               650 -> 60
 #include "attention.hpp"
 
 namespace nhp {
@@ -111,6 +111,10 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_kernel(AttnFwdArgs a)
             const bool active = MODE == kBits || (key0 <= wave_hi && key0 + 63 >= wave_lo);
             if (active) {
                 f32x16 s[2] = {f32x16{}, f32x16{}};
+                // the wave that multiplies goes first, so that the other one of the SIMD is left with its softmax
+                // (4 to 5 % of the kernel at 64, 80 and 128 features: 568 -> 544 us at 8192 positions, 32 heads of 128;
+                // no gain in the kernels of the gradients)
+                __builtin_amdgcn_s_setprio(1);
 #pragma unroll
                 for (int t = 0; t < G::kSteps; ++t) {
 #pragma unroll
@@ -119,6 +123,7 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_kernel(AttnFwdArgs a)
                         s[n] = F::mma(kf, qf[t], s[n]);
                     }
                 }
+                __builtin_amdgcn_s_setprio(0);
                 if constexpr (MODE == kBits) {
                     const uint64_t w = bits[(int64_t)qi * kt_hi + kt];
 #pragma unroll
@@ -170,6 +175,7 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_kernel(AttnFwdArgs a)
                         sum += s[n][i];
                     }
                 l += sum;
+                __builtin_amdgcn_s_setprio(1);
 #pragma unroll
                 for (int ks = 0; ks < 4; ++ks) {
                     const u32x4 pf = F::pack8(s[ks >> 1], (ks & 1) * 8);
@@ -180,6 +186,7 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_kernel(AttnFwdArgs a)
                         o[d] = F::mma(vf, pf, o[d]);
                     }
                 }
+                __builtin_amdgcn_s_setprio(0);
             }
             kt = following;
             buf ^= 1;
@@ -212,10 +219,18 @@ __global__ void __launch_bounds__(256) pack_mask_kernel(uint64_t* out, const uin
     if (row >= rows) return;
     const int lane = threadIdx.x & 63;
     const uint8_t* p = mask + row * sk;
-    for (int w = 0; w < words; ++w) {
-        const int key = w * 64 + lane;
-        const uint64_t word = __ballot(key >= sk || p[min(key, sk - 1)] != 0);
-        if (lane == 0) out[row * words + w] = word;
+    // eight words at a time: one after the other, a row of 1531 keys waited for memory 24 times (12.8 -> 7.5 us for 1531 rows)
+    for (int w0 = 0; w0 < words; w0 += 8) {
+        uint8_t v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = p[min((w0 + j) * 64 + lane, sk - 1)];
+        uint64_t mine = 0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const uint64_t word = __ballot((w0 + j) * 64 + lane >= sk || v[j] != 0);
+            mine = lane == j ? word : mine;
+        }
+        if (lane < min(8, words - w0)) out[row * words + w0 + lane] = mine;
     }
 }
 

@@ -1,4 +1,4 @@
-// y = x W^T (+ bias) for the few rows of a decoding step (at most 16), 16-bit storage, fp32 sums.
+// y = x W^T (+ bias) for the few rows of a decoding step (at most 32), 16-bit storage, fp32 sums.
 //
 // Such a product reads every weight once for a handful of rows: the weights' bytes are its time, and the matrix cores idle.
 // What a CU can have on the way is the limit, so x must not take much of it: read again for every 16 weight rows it costs
@@ -34,12 +34,13 @@ __device__ __forceinline__ f32x4v linear_mma(u32x4 a, u32x4 b, f32x4v c)
     else return __builtin_amdgcn_mfma_f32_16x16x32_f16(bitcast<f16x8>(a), bitcast<f16x8>(b), c, 0, 0, 0);
 }
 
-template <int DT>
+// MT: tiles of 16 rows of x
+template <int DT, int MT>
 __global__ void __launch_bounds__(64 * kLinearWaves) linear_decode_kernel(LinearArgs a)
 {
     constexpr int kParts = kLinearSteps / kLinearPart;
     static_assert(kParts * kLinearPart == kLinearSteps && kParts % 2 == 0, "an even number of parts");
-    __shared__ float sums[2][kLinearWaves][16][17];
+    __shared__ float sums[2][kLinearWaves][16 * MT][17];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g = lane >> 4;
     const int split = blockIdx.x % a.splits, first_tile = blockIdx.x / a.splits, stride = gridDim.x / a.splits;
@@ -58,24 +59,34 @@ __global__ void __launch_bounds__(64 * kLinearWaves) linear_decode_kernel(Linear
         asm volatile("" ::: "memory");   // not put off until they are needed
     };
     load(part[0], first_tile, 0);
-    u32x4 x[kLinearSteps];
-    const uint16_t* xp = a.x + (int64_t)min(r16, a.m - 1) * a.k + lo * 32 + g * 8;
+    u32x4 x[MT][kLinearSteps];
 #pragma unroll
-    for (int s = 0; s < kLinearSteps; ++s) x[s] = s < count ? load16(xp + s * 32) : u32x4{0, 0, 0, 0};
+    for (int i = 0; i < MT; ++i) {
+        const uint16_t* xp = a.x + (int64_t)min(i * 16 + r16, a.m - 1) * a.k + lo * 32 + g * 8;
+#pragma unroll
+        for (int s = 0; s < kLinearSteps; ++s) x[i][s] = s < count ? load16(xp + s * 32) : u32x4{0, 0, 0, 0};
+    }
 
     int buf = 0;
     for (int tile = first_tile; tile < tiles; tile += stride) {
-        f32x4v acc{};
+        f32x4v acc[MT];
+#pragma unroll
+        for (int r = 0; r < MT; ++r) acc[r] = f32x4v{};
 #pragma unroll
         for (int i = 0; i < kParts; ++i) {
             if (i + 1 < kParts) load(part[(i + 1) & 1], tile, (i + 1) * kLinearPart);
             else if (tile + stride < tiles) load(part[0], tile + stride, 0);
 #pragma unroll
             for (int s = 0; s < kLinearPart; ++s)
-                if (i * kLinearPart + s < count) acc = linear_mma<DT>(part[i & 1][s], x[i * kLinearPart + s], acc);
+                if (i * kLinearPart + s < count) {
+#pragma unroll
+                    for (int r = 0; r < MT; ++r) acc[r] = linear_mma<DT>(part[i & 1][s], x[r][i * kLinearPart + s], acc[r]);
+                }
         }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) sums[buf][wave][r16][4 * g + j] = acc[j];
+        for (int r = 0; r < MT; ++r)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) sums[buf][wave][r * 16 + r16][4 * g + j] = acc[r][j];
         __syncthreads();
         // (a wave is at most one tile ahead of those that add up here: the other half of the sums is free)
         const int row = tid >> 4, col = tid & 15;
@@ -115,7 +126,9 @@ static int launch_linear(const LinearArgs& a, hipStream_t st)
 {
     launch_prepare();
     const int tiles = a.n / 16, most = kLinearBlocks / a.splits;
-    linear_decode_kernel<DT><<<dim3((unsigned)((tiles < most ? tiles : most) * a.splits)), dim3(64 * kLinearWaves), 0, st>>>(a);
+    const dim3 blocks((unsigned)((tiles < most ? tiles : most) * a.splits)), threads(64 * kLinearWaves);
+    if (a.m <= 16) linear_decode_kernel<DT, 1><<<blocks, threads, 0, st>>>(a);
+    else linear_decode_kernel<DT, 2><<<blocks, threads, 0, st>>>(a);
     if (a.splits > 1) linear_merge_kernel<DT><<<dim3((unsigned)(((int64_t)a.m * a.n / 4 + 255) / 256)), dim3(256), 0, st>>>(a);
     return launch_result();
 }
@@ -135,7 +148,7 @@ int nhp_linear_decode(void* y, const void* x, const void* weight, const void* bi
 {
     using namespace nhp;
     if (!y || !x || !weight) return NHP_ERR_NULL;
-    if (rows < 1 || rows > 16 || out_features < 16 || out_features % 16 || in_features < 32 || in_features % 32) return NHP_ERR_SHAPE;
+    if (rows < 1 || rows > 32 || out_features < 16 || out_features % 16 || in_features < 32 || in_features % 32) return NHP_ERR_SHAPE;
     if (in_features > kLinearWhole * kLinearSplits || out_features > (1 << 24)) return NHP_ERR_SHAPE;
     if (!ptr_aligned16(x) || !ptr_aligned16(weight) || !ptr_aligned16(y)) return NHP_ERR_SHAPE;
     const int splits = in_features > kLinearWhole ? kLinearSplits : 1;

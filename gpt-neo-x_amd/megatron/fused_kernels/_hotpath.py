@@ -165,8 +165,10 @@ def require_gpu(t, what):
 
 def followed(*tensors):
     """Whether torch follows the operations on any of these beyond autograd (vmap and the other function transforms,
-    forward-mode derivatives, tracing, tensor subclasses): a launch outside of an autograd function would escape it."""
-    return (torch.autograd.forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None
+    forward-mode derivatives, tracing, compilation, tensor subclasses): a launch outside of an autograd function would
+    escape it."""
+    return (torch.compiler.is_compiling() or torch.autograd.forward_ad._current_level >= 0
+            or torch._C._get_tracing_state() is not None
             or any((type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter)
                    or torch._C._functorch.is_functorch_wrapped_tensor(t) for t in tensors))
 

@@ -10,6 +10,9 @@ parallel layers around it:
     probs   = dropout(probs)                                 same kernel on the causal branch
     context = bmm(probs, v)                                  library GEMM
 
+Where nothing is added to the scores and nothing dropped, the three are one kernel (``fused_attention``); what follows is
+about the other calls.
+
 ``norm_factor = sqrt(head_dim) * coeff`` and ``coeff = max(1, layer_number)`` with
 ``apply_query_key_layer_scaling``, otherwise ``coeff`` is None and the softmax does not
 scale: the two factors cancel in exact arithmetic and only keep fp16 scores in range.

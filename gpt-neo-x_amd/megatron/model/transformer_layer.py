@@ -10,7 +10,8 @@ adding it (``skip_bias_add``), and everything between the GEMMs is one of the fu
     qkv projection            GEMM (bias added by the GEMM, as ColumnParallelLinear does for qkv)
     rotary on q and k         nhp_rope_cached_qk on the two views of the projection output; its backward writes
                               into the gradient of the projection output (no concatenation)
-    scores / probs / context  CoreAttention: GEMM, fused softmax (+ dropout), GEMM
+    scores / probs / context  CoreAttention: nhp_attention_fwd / _bwd, with cached positions nhp_attention_decode; with
+                              dropout or an additive term GEMM, fused softmax, GEMM
     output projection         GEMM, bias handed on
     bias + dropout + residual nhp_bias_add_residual / nhp_bias_dropout_add
     MLP                       GEMM, bias+GeLU or gated activation kernel, GEMM, bias handed on

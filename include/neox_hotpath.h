@@ -762,7 +762,7 @@ int nhp_kv_cache_append(void* cache_out, const void* k_new, const void* v_new, c
                         const int64_t* k_new_strides, const int64_t* v_new_strides, const int64_t* k_past_strides,
                         const int64_t* v_past_strides, int dtype, void* stream);
 
-/* y [rows, out_features] = x [rows, in_features] weight^T (+ bias, may be NULL) for 1 to 16 rows, 16-bit storage, fp32 sums:
+/* y [rows, out_features] = x [rows, in_features] weight^T (+ bias, may be NULL) for 1 to 32 rows, 16-bit storage, fp32 sums:
  * the linear layers of a decoding step (the ParallelLinear layers of megatron/model/transformer.py:120-196 and :370-415). All
  * contiguous, x, weight and y 16-byte aligned, out_features a multiple of 16, in_features of 32 and at most 16384.
  * workspace (may be NULL where its size is 0): nhp_linear_decode_workspace_bytes, 16-byte aligned. */

@@ -1,4 +1,4 @@
-"""The few-row linear layer (csrc/linear_decode.hip) against fp64: one and sixteen rows, weight tiles fewer and more than
+"""The few-row linear layer (csrc/linear_decode.hip) against fp64: one and two tiles of sixteen rows, weight tiles fewer and more than
 workgroups, contractions that do not divide evenly among the waves, and the split ones.
 
 Tolerance: one rounding of the result, at most u = 2^-8 (bf16) or 2^-11 (fp16), u / sqrt(3) in the mean square of a 2-norm;
@@ -16,13 +16,13 @@ DEV = "cuda"
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("n,k", [(16, 32), (48, 544), (4112, 96), (2304, 768), (6160, 4096), (80, 4128), (1040, 11008), (32, 16384)])
-@pytest.mark.parametrize("rows", [1, 7, 16])
+@pytest.mark.parametrize("rows", [1, 7, 16, 17, 32])
 def test_against_fp64(dtype, n, k, rows):
     from megatron.model import fused_linear
 
     x, w = util.randn((rows, 1, k), dtype, seed=1).to(DEV), util.randn((n, k), dtype, seed=2).to(DEV)
     b = util.randn((n,), dtype, seed=3, std=math.sqrt(k)).to(DEV)
-    assert fused_linear._few_rows(x, w, b)
+    assert fused_linear._few_rows(x, w, b) == (rows <= 16 or min(n, k) <= 2048)
     for bias in (None, b):
         got = fused_linear.linear(x, w, bias)
         want = x.double() @ w.double().t() + (0.0 if bias is None else bias.double())
@@ -52,7 +52,7 @@ def test_everything_else_goes_to_the_library():
     assert g.grad is not None
     with torch.no_grad():
         assert fused_linear._few_rows(x, g, None)
-    for a, b in ((x.repeat(5, 1), w), (x.float(), w.float()), (x[:, :40], w[:, :40]), (x, w[:24]), (x[:0], w), (x.cpu(), w.cpu()),
+    for a, b in ((x.repeat(9, 1), w), (x.float(), w.float()), (x[:, :40], w[:, :40]), (x, w[:24]), (x[:0], w), (x.cpu(), w.cpu()),
                  (torch.cat((x, x), 1)[:, ::2], w)):
         assert not fused_linear._few_rows(a, b, None)
         assert linear(a, b).shape == (a.size(0), b.size(0))

@@ -5,8 +5,10 @@
 // wave's kilobyte touches nine 128-byte lines instead of eight). The last chunk of a row is read as the eight elements
 // that end the row and shifted into place, so nothing beyond a row is read; it is written in pieces of 8, 4 and 2 bytes.
 //
-// Bounded by memory, as the aligned kernels are: [8, 12, 380, 1021] fp16 with a padding mask, forward 151 -> 32 us
-// (149 MB of scores and probabilities), backward 113 -> 36 us (224 MB, 6.3 TB/s). The scalar kernels (2-byte accesses, three passes over a row), which
+// Bounded by memory, as the aligned kernels are: [8, 12, 380, 1021] fp16 with a padding mask, forward 151 -> 28 us
+// (149 MB of scores and probabilities), backward 113 -> 36 us (224 MB, 6.3 TB/s). Non-temporal accesses, as there, although
+// the lines at the ends of a row are shared with its neighbours: [4, 16, 1000, 2047] forward 108 -> 100 us, backward 145
+// -> 134. The scalar kernels (2-byte accesses, three passes over a row), which
 // took these rows before, remain for rows of fewer than 8 or more than 16384 elements.
 #include "softmax_ragged.hpp"
 
@@ -29,7 +31,7 @@ struct RaggedGeo {
 __device__ __forceinline__ u32x4 load_chunk(const uint16_t* row, uint32_t col, uint32_t n)
 {
     const uint32_t at = min(col, n - 8);
-    const u32x4 raw = *reinterpret_cast<const u32x4_any*>(row + at);
+    const u32x4 raw = __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(row + at));
     if (col == at) return raw;
     uint64_t lo = (uint64_t)raw[1] << 32 | raw[0], hi = (uint64_t)raw[3] << 32 | raw[2];
     uint32_t shift = (col - at) * 16;   // 16 .. 112
@@ -48,7 +50,7 @@ __device__ __forceinline__ void store_chunk(uint16_t* row, uint32_t col, uint32_
     uint16_t* p = row + col;
     const uint32_t left = n - col;
     if (left >= 8) {
-        *reinterpret_cast<u32x4_any*>(p) = v;
+        __builtin_nontemporal_store(v, reinterpret_cast<u32x4_any*>(p));
         return;
     }
     if (left & 4) {
@@ -136,18 +138,33 @@ __global__ void __launch_bounds__(256) ragged_fwd_kernel(RaggedArgs a)
         }
     }
 
-    for (uint32_t head = hg * kHeads; head < min(np, hg * kHeads + kHeads); ++head) {
+    // rows of up to 1024 elements: the scores of both heads are asked for before those of the first are used (37.3 -> 35.2 us
+    // at [4, 12, 1023, 1023], 34.8 -> 31.9 at [8, 12, 512, 701]; no gain with more chunks under way anyway)
+    constexpr bool kBoth = MODE == 1 && K <= 2;
+    u32x4 ahead[kBoth ? K : 1];
+    auto fetch = [&](u32x4* to, uint32_t head) {
+        const uint16_t* xr = a.in + ((uint64_t)(bi * np + head) * sq + q) * n;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            to[k] = u32x4{0, 0, 0, 0};
+            if (skip[k] != 0xffu) to[k] = load_chunk(xr, (uint32_t)((k * W + w) * L + l) * 8u, n);
+        }
+    };
+    const uint32_t head_end = min(np, hg * kHeads + kHeads);
+    for (uint32_t head = hg * kHeads; head < head_end; ++head) {
         const uint64_t row = (uint64_t)(bi * np + head) * sq + q;
-        const uint16_t* xr = a.in + row * n;
         uint16_t* yr = a.out + row * n;
         const uint16_t* br = EXTRA && a.bias ? a.bias + ((uint64_t)head * sq + q) * n : nullptr;
         float z[K][8];
         u32x4 raw[K];
+        if (kBoth && head != hg * kHeads) {
 #pragma unroll
-        for (int k = 0; k < K; ++k) {
-            const uint32_t col = (uint32_t)((k * W + w) * L + l) * 8u;
-            raw[k] = u32x4{0, 0, 0, 0};
-            if (skip[k] != 0xffu) raw[k] = load_chunk(xr, col, n);
+            for (int k = 0; k < K; ++k) raw[k] = ahead[kBoth ? k : 0];
+        } else {
+            fetch(raw, head);
+            if constexpr (kBoth) {
+                if (head + 1 < head_end) fetch(ahead, head + 1);
+            }
         }
         float m = kNegInf;
 #pragma unroll
@@ -291,7 +308,8 @@ __global__ void __launch_bounds__(256) ragged_bwd_kernel(RaggedArgs a)
 
 bool ragged_rows(int64_t n) { return n >= 8 && n <= kMaxRaggedRow; }
 
-// One wave per row up to 2048 elements (no barrier), four beyond; short rows share a wave.
+// One wave per row up to 2048 elements (no barrier), four beyond; short rows share a wave. Three chunks per lane for 4099
+// elements instead of four half empty: forward 54 -> 45 us at [2, 8, 700, 4099], backward 63 -> 55.
 #define NHP_RAGGED_PLAN(CALL)                          \
     do {                                               \
         const uint32_t chunks = (a.n + 7) / 8;         \
@@ -303,7 +321,9 @@ bool ragged_rows(int64_t n) { return n >= 8 && n <= kMaxRaggedRow; }
         else if (chunks <= 192) { CALL(64, 3, 1); }    \
         else if (chunks <= 256) { CALL(64, 4, 1); }    \
         else if (chunks <= 512) { CALL(64, 2, 4); }    \
+        else if (chunks <= 768) { CALL(64, 3, 4); }    \
         else if (chunks <= 1024) { CALL(64, 4, 4); }   \
+        else if (chunks <= 1536) { CALL(64, 6, 4); }   \
         else { CALL(64, 8, 4); }                       \
     } while (0)
 

@@ -38,10 +38,10 @@ class Guarded:
         return bool(self.buf[:start].isnan().all() and self.buf[start + n:].isnan().all())
 
 
-# edges of the geometries: 64, 128, 256, 512, 1024, 1536, 2048, 4096, 8192, 16384 elements; offsets in elements
+# edges of the geometries: 64, 128, 256, 512, 1024, 1536, 2048, 4096, 6144, 8192, 12288, 16384 elements; offsets in elements
 MASKED = [(2, 3, 5, 9, 0), (1, 2, 3, 63, 3), (2, 1, 7, 64, 1), (1, 4, 3, 65, 0), (2, 3, 4, 129, 5), (1, 2, 2, 257, 7), (1, 5, 6, 511, 0),
           (2, 2, 3, 513, 2), (1, 3, 3, 1021, 0), (1, 2, 2, 1025, 1), (1, 2, 2, 1537, 0), (1, 2, 3, 2047, 4), (1, 2, 2, 2049, 0),
-          (1, 3, 2, 4099, 6), (1, 2, 2, 8191, 0), (1, 2, 2, 8200, 1), (1, 1, 2, 16383, 0)]
+          (1, 3, 2, 4099, 6), (1, 2, 2, 6145, 0), (1, 2, 2, 8191, 0), (1, 1, 2, 12289, 3), (1, 2, 2, 8200, 1), (1, 1, 2, 16383, 0)]
 
 
 @DTYPES

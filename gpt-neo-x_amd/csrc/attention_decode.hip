@@ -13,8 +13,9 @@
 // registers in the order in which the instruction wants them (16 rows x 64 bytes per load); values are transposed
 // through LDS, whose rows are padded so that the 8 rows of a transposing read fall on different banks.
 //
-// Measured (past 2047, 16 sequences, 32 heads, 128 features, bf16; 1.07 GB read and written): 204 us, 5.3 TB/s, which is
-// what a copy of that size reaches; concatenations 949 us and attention 118 us before. A whole layer's step 1174 -> 373 us.
+// Measured (past 2047, 16 sequences, 32 heads, 128 features, bf16; 1.07 GB read and written): 204 to 230 us on different
+// cards, 4.7 to 5.3 TB/s, about what a copy of that size reaches; concatenations 949 us and attention 118 us before. A whole
+// layer's step 1174 -> 365 us.
 #include "attention.hpp"
 
 namespace nhp {

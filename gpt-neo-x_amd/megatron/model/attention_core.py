@@ -324,10 +324,7 @@ class CoreAttention(torch.nn.Module):
         else:
             kernel = softmax.is_kernel_available(mask, b, np_, sq, sk)
         fill = -10000.0 if kernel else softmax.mask_fill
-        if (fill is None or sk > 65536 or mask.dtype != torch.bool or mask.device != device
-                or mask.shape not in ((1, 1, sq, sk), (b, 1, sq, sk))):
-            return None
-        return fill
+        return fill if fused_attention.mask_supported(mask, b, sq, sk, device) else None
 
     def _cached_call(self, query, key, value, mask, layer_past):
         """``(mask, scale, fill)`` for the decoding kernel, or None where it does not apply."""
@@ -347,7 +344,7 @@ class CoreAttention(torch.nn.Module):
         if call is None:
             return None
         mask, scale, fill = call
-        return fused_attention.decode_attention(query, key, value, layer_past, mask, scale, fill, merged_heads)
+        return fused_attention.checked_decode_attention(query, key, value, layer_past, mask, scale, fill, merged_heads)
 
     def _causal_block(self, attention_mask, b, np_, sq, sk, like):
         """Block size for the blocked causal GEMMs, 0 when the scores do not go to the causal kernel (which is what

@@ -37,10 +37,25 @@ def _strides3(t):
 
 
 def supported(q, k, v):
-    """Whether the kernels take these operands (dtype, device, head size, sizes)."""
+    """Whether the kernels take these operands. They get addresses and the sizes of q alone, so everything that makes q, k
+    and v belong together is checked here: one device and type, one batch, heads that divide, a head size there is a kernel
+    for, no more queries than keys."""
     return (q.is_cuda and q.dtype in (torch.bfloat16, torch.float16) and k.dtype == q.dtype and v.dtype == q.dtype
-            and q.size(3) in HEAD_DIMS and v.size(3) == q.size(3) and q.numel() > 0 and k.numel() > 0
-            and k.shape == v.shape and q.size(0) <= k.size(0) < 1 << 24)
+            and k.device == q.device and v.device == q.device and q.dim() == 4 and k.dim() == 4 and k.shape == v.shape
+            and q.size(3) in HEAD_DIMS and k.size(3) == q.size(3) and k.size(1) == q.size(1)
+            and q.numel() > 0 and k.numel() > 0 and q.size(2) % k.size(2) == 0 and q.size(0) <= k.size(0) < 1 << 24)
+
+
+def mask_supported(mask, b, sq, sk, device):
+    """Whether the kernels take ``mask`` for ``sq`` queries over ``sk`` keys of ``b`` batch entries."""
+    return (mask.dtype == torch.bool and mask.device == device and mask.shape in ((1, 1, sq, sk), (b, 1, sq, sk))
+            and sk <= 65536)
+
+
+def _refuse_unless(taken, who, *tensors):
+    if not taken:
+        raise RuntimeError(f"{who}: the kernels do not take these operands: "
+                           + ", ".join(f"{tuple(t.shape)} {t.dtype} on {t.device}" for t in tensors))
 
 
 def _new_context(q, merged):
@@ -73,6 +88,7 @@ class CausalAttention(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, v, scale, window, merged):
+        _refuse_unless(supported(q, k, v), "CausalAttention", q, k, v)
         q, k, v = _readable(q), _readable(k), _readable(v)
         out = _new_context(q, merged)
         need = any(ctx.needs_input_grad[:3])
@@ -116,6 +132,8 @@ def causal_attention(q, k, v, scale, window=None, merged=False):
 def masked_attention(q, k, v, mask, scale, fill, merged=False):
     """Inference only: the context under a boolean mask ``[1 or b, 1, sq, sk]`` (True = masked), whose scores are
     replaced by ``fill`` after scaling."""
+    _refuse_unless(supported(q, k, v) and mask_supported(mask, q.size(1), q.size(0), k.size(0), q.device), "masked_attention",
+                   q, k, v, mask)
     q, k, v = _readable(q), _readable(k), _readable(v)
     sq, sk = q.size(0), k.size(0)
     mask = mask.contiguous()
@@ -136,27 +154,45 @@ def plain(*tensors):
     return not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors)) and not _hp.followed(*tensors)
 
 
-def cache_supported(key, value, layer_past):
-    """Whether ``append_to_cache`` takes these: 16-bit tensors on the GPU that nobody differentiates; ``layer_past``
-    (None: no cached positions) of their type and shape."""
+def _cache_fits(key, value, past):
+    """Whether these are 16-bit keys and values on one GPU, of one shape and a size that the kernels can address after ``past``
+    cached positions."""
     if not (key.is_cuda and key.dtype in (torch.bfloat16, torch.float16) and key.dim() == 4 and value.shape == key.shape
-            and value.dtype == key.dtype and value.device == key.device and key.numel() > 0 and key.size(3) % 8 == 0
-            and plain(key, value)):
+            and value.dtype == key.dtype and value.device == key.device and key.numel() > 0 and key.size(3) % 8 == 0):
         return False
-    sk, width = key.size(0), key.numel() // key.size(0)
-    if layer_past is not None:
-        if not (isinstance(layer_past, torch.Tensor) and layer_past.dim() == 5 and layer_past.size(0) == 2
-                and layer_past.shape[2:] == key.shape[1:] and layer_past.dtype == key.dtype
-                and layer_past.device == key.device and plain(layer_past)):
-            return False
-        sk += layer_past.size(1)
+    sk, width = past + key.size(0), key.numel() // key.size(0)
     return width < 1 << 24 and sk < 1 << 24 and sk * width // key.size(3) < 1 << 31
+
+
+def _continues(cached, key):
+    """Whether cached keys or values, ``[.., past, b, nkv, hn]``, are followed by ``key``."""
+    return cached.shape[-3:] == key.shape[1:] and cached.dtype == key.dtype and cached.device == key.device
+
+
+def cache_supported(key, value, layer_past):
+    """Whether a layer can use ``append_to_cache`` for these: what the kernel takes, and nobody differentiates; ``layer_past``
+    (None: no cached positions) ``[2, past, b, nkv, hn]``."""
+    if layer_past is None:
+        return _cache_fits(key, value, 0) and plain(key, value)
+    return (isinstance(layer_past, torch.Tensor) and layer_past.dim() == 5 and layer_past.size(0) == 2
+            and _cache_fits(key, value, layer_past.size(1)) and _continues(layer_past, key) and plain(key, value, layer_past))
+
+
+def _past_fits(key, value, past_key, past_value):
+    """``cache_supported`` for a direct call, whoever differentiates."""
+    return (past_key.dim() == 4 and past_value.shape == past_key.shape and _cache_fits(key, value, past_key.size(0))
+            and _continues(past_key, key) and _continues(past_value, key))
 
 
 def append_to_cache(key, value, layer_past):
     """``torch.stack((cat(past keys, key), cat(past values, value)))`` in one launch: ``[2, past + sq, b, nkv, hn]``."""
+    past_k, past_v = (None, None) if layer_past is None else layer_past
+    if layer_past is None:
+        _refuse_unless(_cache_fits(key, value, 0), "append_to_cache", key, value)
+    else:
+        _refuse_unless(_past_fits(key, value, past_k, past_v), "append_to_cache", key, value, past_k, past_v)
+        past_k, past_v = _readable(past_k), _readable(past_v)
     key, value = _readable(key), _readable(value)
-    past_k, past_v = (None, None) if layer_past is None else (_readable(t) for t in layer_past)
     past = 0 if past_k is None else past_k.size(0)
     sq, b, nkv, hn = key.shape
     present = torch.empty((2, past + sq, b, nkv, hn), dtype=key.dtype, device=key.device)
@@ -170,17 +206,31 @@ def append_to_cache(key, value, layer_past):
     return present
 
 
+def _decode_fits(query, key, value, past):
+    """A key for every query, some cached positions, and few enough queries for each key/value head."""
+    return (supported(query, key, value) and query.size(0) == key.size(0) and past > 0 and past + key.size(0) >= 4
+            and query.size(0) * (query.size(2) // key.size(2)) <= MAX_DECODE_ROWS)
+
+
 def decode_supported(query, key, value, layer_past):
-    """Whether ``decode_attention`` takes these (beside what ``cache_supported`` asks for): some cached positions, and
-    few enough queries for each key/value head."""
-    return (supported(query, key, value) and layer_past is not None and cache_supported(key, value, layer_past) and plain(query)
-            and layer_past.size(1) > 0 and layer_past.size(1) + key.size(0) >= 4 and query.size(1) * query.size(2) <= 1 << 24
-            and query.size(2) % key.size(2) == 0 and query.size(0) * (query.size(2) // key.size(2)) <= MAX_DECODE_ROWS)
+    """Whether ``decode_attention`` takes these, and nobody differentiates."""
+    return (layer_past is not None and cache_supported(key, value, layer_past) and _decode_fits(query, key, value, layer_past.size(1))
+            and plain(query))
 
 
 def decode_attention(query, key, value, layer_past, mask, scale, fill, merged=False):
     """``masked_attention`` of new positions over the cached ones and themselves, and ``append_to_cache``, in one pass
     over the cache: ``(context, present)``. ``mask`` ``[1 or b, 1, sq, past + sq]``, True = masked."""
+    past_k, past_v = layer_past
+    fits = (_past_fits(key, value, past_k, past_v) and _decode_fits(query, key, value, past_k.size(0))
+            and mask_supported(mask, query.size(1), query.size(0), past_k.size(0) + key.size(0), query.device))
+    _refuse_unless(fits, "decode_attention", query, key, value, past_k, past_v, mask)
+    return checked_decode_attention(query, key, value, layer_past, mask, scale, fill, merged)
+
+
+def checked_decode_attention(query, key, value, layer_past, mask, scale, fill, merged):
+    """``decode_attention`` for a caller that has asked ``decode_supported`` and ``mask_supported`` already: a step of a small
+    model waits for the host, and the checks cost it several microseconds a layer."""
     query, key, value = _readable(query), _readable(key), _readable(value)
     past_k, past_v = (_readable(t) for t in layer_past)
     sq, b, np_, hn = query.shape

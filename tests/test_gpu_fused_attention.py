@@ -129,3 +129,20 @@ def test_the_caller_takes_the_kernels_and_the_mask_where_it_counts():
     # the torch branch rounds the scores to bf16 first: one more rounding, of a score of up to 4 instead of a value
     assert rel_err(core(q.clone().requires_grad_(True), k, v, mask).permute(2, 0, 1, 3), want) <= 2.0 ** -7
     assert not fused_attention.supported(q[..., :40], k[..., :40], v[..., :40])
+
+
+def test_the_caller_refuses_operands_that_do_not_belong_together():
+    """``CoreAttention`` leaves them to the products, which raise (the checks themselves: test_attention_operands.py)."""
+    from megatron.model.attention_core import CoreAttention
+    from megatron.model.fused_softmax import SoftmaxFusionTypes as T
+
+    core = CoreAttention(64, 1, False, True, T.upper_triang, lambda s, m: s.masked_fill_(m, -1e4), attention_softmax_in_fp32=True)
+    q, k, v = operands(torch.bfloat16, 128, 128, 4, 4, 4, 64, 1)
+    mask = hidden(128, 128).view(1, 1, 128, 128)
+    for grad in (False, True):
+        for key, value in ((k[:, :2], v[:, :2]), (k[:, :1], v[:, :1]), (k.repeat(1, 2, 1, 1), v.repeat(1, 2, 1, 1)), (k.cpu(), v.cpu()),
+                           (k, v.cpu()), (k[:, :, :3], v[:, :, :3])):
+            with pytest.raises((RuntimeError, AssertionError)):
+                core(q.clone().requires_grad_(grad), key, value, mask)
+        with pytest.raises(RuntimeError):
+            core(q.cpu().requires_grad_(grad), k, v, mask)

@@ -39,17 +39,25 @@ def _strides3(t):
 def supported(q, k, v):
     """Whether the kernels take these operands. They get addresses and the sizes of q alone, so everything that makes q, k
     and v belong together is checked here: one device and type, one batch, heads that divide, a head size there is a kernel
-    for, no more queries than keys."""
+    for, no more queries than keys, and sizes that the kernels can address."""
     return (q.is_cuda and q.dtype in (torch.bfloat16, torch.float16) and k.dtype == q.dtype and v.dtype == q.dtype
             and k.device == q.device and v.device == q.device and q.dim() == 4 and k.dim() == 4 and k.shape == v.shape
             and q.size(3) in HEAD_DIMS and k.size(3) == q.size(3) and k.size(1) == q.size(1)
-            and q.numel() > 0 and k.numel() > 0 and q.size(2) % k.size(2) == 0 and q.size(0) <= k.size(0) < 1 << 24)
+            and q.numel() > 0 and k.numel() > 0 and q.size(2) % k.size(2) == 0 and q.size(0) <= k.size(0)
+            and _addressable(q.size(0), k.size(0), q.size(1), q.size(2), k.size(2), q.size(3)))
+
+
+def _addressable(sq, sk, b, np_, nkv, hn):
+    """The limits of the entry points (fill_operand and the grids in csrc/attention.hip): a row of a contiguous copy, of
+    the result or of a gradient is below 2^24 elements, and a grid of 256 work-items a workgroup below 2^32."""
+    return (sk < 1 << 24 and (sq == 1 or b * np_ * hn < 1 << 24) and (sk == 1 or b * nkv * hn < 1 << 24)
+            and (b * np_ + 7) // 8 * 8 * ((sk + 127) // 128) < 1 << 24 and sk * b * nkv * hn < 1 << 35)
 
 
 def mask_supported(mask, b, sq, sk, device):
     """Whether the kernels take ``mask`` for ``sq`` queries over ``sk`` keys of ``b`` batch entries."""
     return (mask.dtype == torch.bool and mask.device == device and mask.shape in ((1, 1, sq, sk), (b, 1, sq, sk))
-            and sk <= 65536)
+            and sk <= 65536 and mask.size(0) * sq < 1 << 26)
 
 
 def _refuse_unless(taken, who, *tensors):

@@ -59,6 +59,9 @@ STRANGERS = {
     "three dimensions in q": (Standin(8, 4, 64), K, V),
     "a head size without a kernel": operands(hn=72),
     "more queries than keys": operands(sq=9),
+    "rows of 2^24 elements": operands(sq=2, sk=2, b=2048, np_=64, nkv=64, hn=128),
+    "rows of 2^24 elements in k and v alone": operands(sq=1, sk=2, b=2048, np_=64, nkv=64, hn=128),
+    "2^24 workgroups": operands(sq=128, sk=128, b=1 << 24, np_=1, nkv=1),
 }
 
 
@@ -90,6 +93,7 @@ def test_masks_that_do_not_fit():
         with pytest.raises(RuntimeError, match="do not take these operands"):
             fa.masked_attention(Q, K, V, m, 0.1, -1e4)
     assert not fa.mask_supported(mask(4, 65537), 1, 4, 65537, Q.device)
+    assert not fa.mask_supported(mask(512, 512, 1 << 17), 1 << 17, 512, 512, Q.device)
 
 
 def test_caches_that_do_not_fit():

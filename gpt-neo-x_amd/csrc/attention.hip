@@ -206,8 +206,8 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_kernel(AttnFwdArgs a)
     if (qw + ql < a.sq) {
         const float inv = 1.0f / l;
         if (a.lse && half == 0) a.lse[(int64_t)bh * a.sq + qw + ql] = m + __log2f(l);
-        uint16_t* op = a.o + b * a.o_b + h * a.o_h + (int64_t)(qw + ql) * a.o_s;
-        store_transposed<DT, HD>(op, o, inv, half);
+        const int64_t at = b * a.o_b + h * a.o_h + (int64_t)(qw + ql) * a.o_s;
+        store_transposed<DT, HD>(a.o + at, a.kept ? a.kept + at : nullptr, o, inv, half);
     }
 }
 
@@ -370,7 +370,7 @@ __global__ void __launch_bounds__(256, 2) attn_dq_kernel(AttnBwdArgs a)
         }
     }
     if (qw + ql < a.sq)
-        store_transposed<DT, HD>(a.dq + b * a.dq_b + h * a.dq_h + (int64_t)(qw + ql) * a.dq_s, dq, a.scale, half);
+        store_transposed<DT, HD>(a.dq + b * a.dq_b + h * a.dq_h + (int64_t)(qw + ql) * a.dq_s, nullptr, dq, a.scale, half);
 }
 
 // Gradients of k and v: 32 keys per wave as columns, their k and v rows in registers; Q and dO tiles of 64 queries (and
@@ -486,8 +486,8 @@ __global__ void __launch_bounds__(256, 2) attn_dkv_kernel(AttnBwdArgs a)
         }
     }
     if (kw + kl < a.sk) {
-        store_transposed<DT, HD>(a.dk + b * a.dk_b + h * a.dk_h + (int64_t)(kw + kl) * a.dk_s, dk, a.scale, half);
-        store_transposed<DT, HD>(a.dv + b * a.dv_b + h * a.dv_h + (int64_t)(kw + kl) * a.dv_s, dv, 1.0f, half);
+        store_transposed<DT, HD>(a.dk + b * a.dk_b + h * a.dk_h + (int64_t)(kw + kl) * a.dk_s, nullptr, dk, a.scale, half);
+        store_transposed<DT, HD>(a.dv + b * a.dv_b + h * a.dv_h + (int64_t)(kw + kl) * a.dv_s, nullptr, dv, 1.0f, half);
     }
 }
 
@@ -572,10 +572,10 @@ int nhp_attention_mask_bits(void* bits, const void* mask, int64_t batches, int64
     return launch_result();
 }
 
-int nhp_attention_fwd(void* out, float* lse, const void* q, const void* k, const void* v, const void* mask_bits,
-                      int64_t mask_batches, float mask_fill, float scale, int64_t window, int64_t batch, int64_t heads,
-                      int64_t kv_heads, int64_t sq, int64_t sk, int64_t head_dim, const int64_t* q_strides,
-                      const int64_t* k_strides, const int64_t* v_strides, const int64_t* out_strides, int dtype, void* stream)
+int nhp_attention_fwd_keep(void* out, void* kept, float* lse, const void* q, const void* k, const void* v, const void* mask_bits,
+                           int64_t mask_batches, float mask_fill, float scale, int64_t window, int64_t batch, int64_t heads,
+                           int64_t kv_heads, int64_t sq, int64_t sk, int64_t head_dim, const int64_t* q_strides,
+                           const int64_t* k_strides, const int64_t* v_strides, const int64_t* out_strides, int dtype, void* stream)
 {
     using namespace nhp;
     if (!out || !q || !k || !v || !q_strides || !k_strides || !v_strides || !out_strides) return NHP_ERR_NULL;
@@ -592,7 +592,9 @@ int nhp_attention_fwd(void* out, float* lse, const void* q, const void* k, const
     const uint16_t* o = nullptr;
     if (rc == NHP_OK) rc = fill_operand(o, a.o_s, a.o_b, a.o_h, out, out_strides);
     if (rc != NHP_OK) return rc;
+    if (!ptr_aligned16(kept)) return NHP_ERR_SHAPE;
     a.o = static_cast<uint16_t*>(out);
+    a.kept = static_cast<uint16_t*>(kept);
     a.lse = lse;
     a.bits = static_cast<const uint64_t*>(mask_bits);
     a.bits_batches = (int)mask_batches;
@@ -610,6 +612,15 @@ int nhp_attention_fwd(void* out, float* lse, const void* q, const void* k, const
     if (dtype == NHP_BF16) return launch_fwd_hd<NHP_BF16>(a, (int)head_dim, mode, static_cast<hipStream_t>(stream));
     if (dtype == NHP_F16) return launch_fwd_hd<NHP_F16>(a, (int)head_dim, mode, static_cast<hipStream_t>(stream));
     return NHP_ERR_DTYPE;
+}
+
+int nhp_attention_fwd(void* out, float* lse, const void* q, const void* k, const void* v, const void* mask_bits,
+                      int64_t mask_batches, float mask_fill, float scale, int64_t window, int64_t batch, int64_t heads,
+                      int64_t kv_heads, int64_t sq, int64_t sk, int64_t head_dim, const int64_t* q_strides,
+                      const int64_t* k_strides, const int64_t* v_strides, const int64_t* out_strides, int dtype, void* stream)
+{
+    return nhp_attention_fwd_keep(out, nullptr, lse, q, k, v, mask_bits, mask_batches, mask_fill, scale, window, batch, heads,
+                                  kv_heads, sq, sk, head_dim, q_strides, k_strides, v_strides, out_strides, dtype, stream);
 }
 
 int64_t nhp_attention_bwd_workspace_bytes(int64_t batch, int64_t heads, int64_t kv_heads, int64_t sq, int64_t sk, int64_t head_dim)

@@ -31,7 +31,7 @@ constexpr float kLazy = 8.0f;
 
 struct AttnFwdArgs {
     const uint16_t *q, *k, *v;
-    uint16_t* o;
+    uint16_t *o, *kept;   // the result, and a second copy with the same strides or null
     float* lse;   // [batch * heads, sq], base-2 logarithm of the row's sum of exponentials; may be null
     const uint64_t* bits;
     int64_t q_s, q_b, q_h, k_s, k_b, k_h, v_s, v_b, v_h, o_s, o_b, o_h;   // element strides
@@ -200,9 +200,9 @@ __device__ __forceinline__ float sum_halves(float v)
 }
 
 // Stores the feature-major accumulators of one row (lane pair l, l + 32), times `f`: lane half 0 of a pair ends up
-// with features 16 j .. 16 j + 7, half 1 with the next eight.
+// with features 16 j .. 16 j + 7, half 1 with the next eight. `second`: another row that gets the same, or null.
 template <int DT, int HD>
-__device__ __forceinline__ void store_transposed(uint16_t* row, const f32x16 (&o)[AttnGeo<HD>::kDTiles], float f, int half)
+__device__ __forceinline__ void store_transposed(uint16_t* row, uint16_t* second, const f32x16 (&o)[AttnGeo<HD>::kDTiles], float f, int half)
 {
 #pragma unroll
     for (int d = 0; d < AttnGeo<HD>::kDTiles; ++d)
@@ -215,7 +215,9 @@ __device__ __forceinline__ void store_transposed(uint16_t* row, const f32x16 (&o
             const uint32_t y1 = Half2<DT>::pack(o[d][8 * j + 6] * f, o[d][8 * j + 7] * f);
             const auto r0 = __builtin_amdgcn_permlane32_swap(x0, y0, false, false);
             const auto r1 = __builtin_amdgcn_permlane32_swap(x1, y1, false, false);
-            *reinterpret_cast<u32x4*>(row + d * 32 + j * 16 + half * 8) = u32x4{(uint32_t)r0[0], (uint32_t)r1[0], (uint32_t)r0[1], (uint32_t)r1[1]};
+            const u32x4 chunk = {(uint32_t)r0[0], (uint32_t)r1[0], (uint32_t)r0[1], (uint32_t)r1[1]};
+            *reinterpret_cast<u32x4*>(row + d * 32 + j * 16 + half * 8) = chunk;
+            if (second) *reinterpret_cast<u32x4*>(second + d * 32 + j * 16 + half * 8) = chunk;
         }
 }
 

@@ -91,6 +91,7 @@ def _declare(lib):
         "nhp_norm_bwd_workspace_bytes": ([i64, i64, ci], i64),
         "nhp_attention_mask_bits": ([vp, vp, i64, i64, i64, vp], ci),
         "nhp_attention_fwd": ([vp] * 6 + [i64, f32, f32] + [i64] * 7 + [p64] * 4 + [ci, vp], ci),
+        "nhp_attention_fwd_keep": ([vp] * 7 + [i64, f32, f32] + [i64] * 7 + [p64] * 4 + [ci, vp], ci),
         "nhp_attention_bwd": ([vp] * 10 + [f32] + [i64] * 7 + [p64] * 8 + [ci, vp], ci),
         "nhp_attention_bwd_workspace_bytes": ([i64] * 6, i64),
         "nhp_attention_decode": ([vp] * 8 + [i64, i64, f32, vp, f32] + [i64] * 6 + [p64] * 6 + [ci, vp], ci),

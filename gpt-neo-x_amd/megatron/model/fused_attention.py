@@ -67,32 +67,39 @@ def _refuse_unless(taken, who, *tensors):
 
 
 def _new_context(q, merged):
+    """Memory for the context, ``[sq, b, np, hn]`` with ``merged`` and ``[b, np, sq, hn]`` without."""
     sq, b, np_, hn = q.shape
-    if merged:
-        return torch.empty((sq, b, np_, hn), dtype=q.dtype, device=q.device)
-    return torch.empty((b, np_, sq, hn), dtype=q.dtype, device=q.device).permute(2, 0, 1, 3)
+    return torch.empty((sq, b, np_, hn) if merged else (b, np_, sq, hn), dtype=q.dtype, device=q.device)
+
+
+def _by_position(out, merged):
+    """``_new_context`` as ``[sq, b, np, hn]``, the order of dimensions in which the kernels take their operands."""
+    return out if merged else out.permute(2, 0, 1, 3)
 
 
 def _finished(out, merged):
-    """``[sq, b, np, hn]`` in the layout that the caller of ``CoreAttention`` gets."""
-    if merged:
-        return out.view(out.size(0), out.size(1), -1)
-    return out.permute(1, 2, 0, 3)
+    """``_new_context`` in the layout that the caller of ``CoreAttention`` gets."""
+    return out.view(out.size(0), out.size(1), -1) if merged else out
 
 
-def _launch(out, lse, q, k, v, bits, mask_batches, fill, scale, window, who):
+def _launch(out, kept, lse, q, k, v, bits, mask_batches, fill, scale, window, who):
+    """``out`` (and ``kept``, laid out alike, or None) ``[sq, b, np, hn]``."""
     sq, b, np_, hn = q.shape
     with _hp.device_guard(q):
-        rc = _hp.lib().nhp_attention_fwd(
-            out.data_ptr(), None if lse is None else lse.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
-            None if bits is None else bits.data_ptr(), mask_batches, fill, scale, -1 if window is None else window, b, np_,
-            k.size(2), sq, k.size(0), hn, _strides3(q), _strides3(k), _strides3(v), _strides3(out), _hp.dtype_code(q, who),
-            _hp.stream_of(q))
+        rc = _hp.lib().nhp_attention_fwd_keep(
+            out.data_ptr(), None if kept is None else kept.data_ptr(), None if lse is None else lse.data_ptr(), q.data_ptr(),
+            k.data_ptr(), v.data_ptr(), None if bits is None else bits.data_ptr(), mask_batches, fill, scale,
+            -1 if window is None else window, b, np_, k.size(2), sq, k.size(0), hn, _strides3(q), _strides3(k), _strides3(v),
+            _strides3(out), _hp.dtype_code(q, who), _hp.stream_of(q))
     _hp.check(rc, who)
 
 
 class CausalAttention(torch.autograd.Function):
-    """``softmax(scale * q k^T) v`` under the causal mask (by index, with an optional sliding window)."""
+    """``softmax(scale * q k^T) v`` under the causal mask (by index, with an optional sliding window): ``[sq, b, np, hn]``
+    with ``merged``, ``[b, np, sq, hn]`` without.
+
+    The backward needs the context. The caller may change it in place (the products would not mind: their backward does not
+    use it), so the result is no view made in here and the kernel stores it a second time for the backward."""
 
     @staticmethod
     def forward(ctx, q, k, v, scale, window, merged):
@@ -100,12 +107,13 @@ class CausalAttention(torch.autograd.Function):
         q, k, v = _readable(q), _readable(k), _readable(v)
         out = _new_context(q, merged)
         need = any(ctx.needs_input_grad[:3])
+        kept = torch.empty_like(out) if need else None
         lse = torch.empty((q.size(1) * q.size(2), q.size(0)), dtype=torch.float32, device=q.device) if need else None
-        _launch(out, lse, q, k, v, None, 1, 0.0, scale, window, "CausalAttention")
+        _launch(_by_position(out, merged), kept, lse, q, k, v, None, 1, 0.0, scale, window, "CausalAttention")
         if need:
-            ctx.save_for_backward(q, k, v, out, lse)
+            ctx.save_for_backward(q, k, v, kept, lse)
             ctx.conf = (scale, window, merged)
-        return _finished(out, merged)
+        return out
 
     @staticmethod
     def backward(ctx, grad):
@@ -114,8 +122,7 @@ class CausalAttention(torch.autograd.Function):
         scale, window, merged = ctx.conf
         sq, b, np_, hn = q.shape
         sk, nkv = k.size(0), k.size(2)
-        g = _readable(grad.view(sq, b, np_, hn) if merged and grad.is_contiguous() else
-                      grad.reshape(sq, b, np_, hn) if merged else grad.permute(2, 0, 1, 3))
+        g, out = _readable(_by_position(grad, merged)), _by_position(out, merged)
         dq, dk, dv = torch.empty_like(q, memory_format=torch.contiguous_format), torch.empty_like(
             k, memory_format=torch.contiguous_format), torch.empty_like(v, memory_format=torch.contiguous_format)
         lib = _hp.lib()
@@ -134,7 +141,7 @@ class CausalAttention(torch.autograd.Function):
 def causal_attention(q, k, v, scale, window=None, merged=False):
     """Context of q ``[s, b, np, hn]`` over k, v ``[s, b, nkv, hn]``: ``[b, np, s, hn]``, or with ``merged``
     ``[s, b, np * hn]``. Query i attends to keys ``i - window .. i``."""
-    return CausalAttention.apply(q, k, v, float(scale), window, merged)
+    return _finished(CausalAttention.apply(q, k, v, float(scale), window, merged), merged)
 
 
 def masked_attention(q, k, v, mask, scale, fill, merged=False):
@@ -150,7 +157,7 @@ def masked_attention(q, k, v, mask, scale, fill, merged=False):
     with _hp.device_guard(q):
         rc = _hp.lib().nhp_attention_mask_bits(bits.data_ptr(), mask.data_ptr(), mask.size(0), sq, sk, _hp.stream_of(q))
     _hp.check(rc, "masked_attention")
-    _launch(out, None, q, k, v, bits, mask.size(0), fill, float(scale), None, "masked_attention")
+    _launch(_by_position(out, merged), None, None, q, k, v, bits, mask.size(0), fill, float(scale), None, "masked_attention")
     return _finished(out, merged)
 
 
@@ -254,7 +261,7 @@ def checked_decode_attention(query, key, value, layer_past, mask, scale, fill, m
         rc = lib.nhp_attention_decode(
             out.data_ptr(), present.data_ptr(), query.data_ptr(), key.data_ptr(), value.data_ptr(), past_k.data_ptr(),
             past_v.data_ptr(), mask.data_ptr(), mask.stride(0) if mask.size(0) > 1 else 0, mask.stride(2), fill,
-            None if workspace is None else workspace.data_ptr(), scale, b, np_, nkv, sq, past, hn, _strides3(out), _strides3(query),
+            None if workspace is None else workspace.data_ptr(), scale, b, np_, nkv, sq, past, hn, _strides3(_by_position(out, merged)), _strides3(query),
             _strides3(key), _strides3(value), _strides3(past_k), _strides3(past_v), _hp.dtype_code(query, "decode_attention"),
             _hp.stream_of(query))
     _hp.check(rc, "decode_attention")

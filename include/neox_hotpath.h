@@ -727,6 +727,13 @@ int nhp_attention_fwd(void* out, float* lse, const void* q, const void* k, const
                       int64_t kv_heads, int64_t sq, int64_t sk, int64_t head_dim, const int64_t* q_strides,
                       const int64_t* k_strides, const int64_t* v_strides, const int64_t* out_strides, int dtype,
                       void* stream);
+/* The same with a second copy of the result, laid out like out (may be NULL): for a caller that hands the result to code that
+ * may change it in place, as that of the bmm of megatron/model/transformer.py:616 may be, and needs it for the backward. */
+int nhp_attention_fwd_keep(void* out, void* kept, float* lse, const void* q, const void* k, const void* v,
+                           const void* mask_bits, int64_t mask_batches, float mask_fill, float scale, int64_t window,
+                           int64_t batch, int64_t heads, int64_t kv_heads, int64_t sq, int64_t sk, int64_t head_dim,
+                           const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides,
+                           const int64_t* out_strides, int dtype, void* stream);
 
 /* Gradients of nhp_attention_fwd without mask_bits, from its operands, its result and its lse (in the reference the
  * backward of the two GEMMs and of the softmax, megatron/model/transformer.py:526-625). workspace:

@@ -146,3 +146,20 @@ def test_the_caller_refuses_operands_that_do_not_belong_together():
                 core(q.clone().requires_grad_(grad), key, value, mask)
         with pytest.raises(RuntimeError):
             core(q.cpu().requires_grad_(grad), k, v, mask)
+
+
+@pytest.mark.parametrize("merged", [True, False], ids=["merged", "bnsh"])
+def test_the_context_may_be_changed_in_place(merged):
+    """As the product's result may be: the gradients are those of the same change into new memory, bit for bit."""
+    from megatron.model.attention_core import CoreAttention
+    from megatron.model.fused_softmax import SoftmaxFusionTypes as T
+
+    core = CoreAttention(64, 1, False, True, T.upper_triang, lambda s, m: s.masked_fill_(m, -1e4), attention_softmax_in_fp32=True)
+    mask = hidden(128, 128).view(1, 1, 128, 128)
+    results = []
+    for change in (lambda t: t.mul_(0.5).add_(1.0), lambda t: t.mul(0.5).add(1.0)):
+        leaves = [t.requires_grad_(True) for t in operands(torch.bfloat16, 128, 128, 2, 4, 2, 64, 1)]
+        out = change(core(*leaves, mask, merged_heads=merged))
+        out.square().sum().backward()
+        results.append([util.raw_bits(t) for t in (out.detach(), *(leaf.grad for leaf in leaves))])
+    assert all(torch.equal(a, b) for a, b in zip(*results))

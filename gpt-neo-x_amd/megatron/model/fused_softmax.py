@@ -294,22 +294,10 @@ class FusedScaleMaskSoftmax(nn.Module):
         else:
             self.register_buffer("alibi_slopes", alibi_slopes.detach().float().clone(), persistent=False)
 
-    # ------------------------------------------------------------------ mask function
-    @property
-    def mask_func(self):
-        return self._mask_func
-
-    @mask_func.setter
-    def mask_func(self, func):
-        self._mask_func = func
-        self._mask_fill = ()
-
     @property
     def mask_fill(self):
-        """What ``mask_func`` fills masked scores with, None if that is not what it does (found out at first use)."""
-        if self._mask_fill == ():
-            self._mask_fill = _fill_value(self._mask_func)
-        return self._mask_fill
+        """What ``mask_func`` fills masked scores with, None if that is not what it does."""
+        return _fill_value(self.mask_func)
 
     # ------------------------------------------------------------------ dispatch
     def forward(self, input, mask, bias=None, key_lengths=None):

@@ -584,3 +584,30 @@ def test_forward_scale_narrowing_helper_and_constructor_flag():
     assert m.narrow_forward_scale is False
     m = FusedScaleMaskSoftmax(True, False, SoftmaxFusionTypes.none, lambda s, k: s, True, s128, narrow_forward_scale=True)
     assert m.narrow_forward_scale is True
+
+
+def test_a_mask_function_is_an_attribute_like_any_other():
+    """It may be a module, may be replaced, and comes back from a state that was saved as a whole module."""
+    import copy
+
+    from megatron.model.fused_softmax import SoftmaxFusionTypes as T
+
+    class Fill(torch.nn.Module):
+        def __init__(self, value):
+            super().__init__()
+            self.value = value
+
+        def forward(self, scores, mask):
+            return scores.masked_fill(mask, self.value)
+
+    m = make(T.none)
+    assert m.__dict__["mask_func"] is mask_func and m.mask_fill == torch.finfo(torch.float32).min
+    m.__setstate__(copy.copy(m.__dict__))   # what unpickling a whole module does
+    assert m.mask_func is mask_func
+    x, mask = torch.randn(1, 1, 2, 4), torch.tensor([[[[False, True, False, True]] * 2]])
+    from megatron.model.fused_softmax import FusedScaleMaskSoftmax
+    sm = FusedScaleMaskSoftmax(False, False, T.none, Fill(-20000.0), True, None)
+    assert sm.mask_fill == -20000.0 and [n for n, _ in sm.named_children()] == ["mask_func"]
+    sm.mask_func = Fill(-30000.0)
+    assert sm.mask_fill == -30000.0
+    assert torch.equal(sm(x, mask), torch.softmax(x.masked_fill(mask, -30000.0), -1))

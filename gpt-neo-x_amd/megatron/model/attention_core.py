@@ -299,8 +299,8 @@ class CoreAttention(torch.nn.Module):
             window = softmax.sliding_window_width
             window = None if window is None or window < 0 else int(window)
             return fused_attention.causal_attention(query, key, value, scale, window, merged_heads)
-        fill = self._fill_by_mask(mask, b, np_, sq, sk, query.device)
-        if fill is None or not fused_attention.plain(query, key, value):
+        fill = self._fill_by_mask(mask, b, np_, sq, sk, query.device) if fused_attention.plain(query, key, value) else None
+        if fill is None:
             return None
         return fused_attention.masked_attention(query, key, value, mask, scale, fill, merged_heads)
 
@@ -318,13 +318,14 @@ class CoreAttention(torch.nn.Module):
 
     def _fill_by_mask(self, mask, b, np_, sq, sk, device):
         """What masked scores are replaced by where the mask decides, None if the kernels cannot follow it."""
+        if not fused_attention.mask_supported(mask, b, sq, sk, device):
+            return None
         softmax = self.scale_mask_softmax
         if softmax.upper_triang_mask_fusion:
             kernel = sq != sk and softmax._rectangular_kernel_available(mask, b, np_, sq, sk)
         else:
             kernel = softmax.is_kernel_available(mask, b, np_, sq, sk)
-        fill = -10000.0 if kernel else softmax.mask_fill
-        return fill if fused_attention.mask_supported(mask, b, sq, sk, device) else None
+        return -10000.0 if kernel else softmax.mask_fill
 
     def _cached_call(self, query, key, value, mask, layer_past):
         """``(mask, scale, fill)`` for the decoding kernel, or None where it does not apply."""

@@ -35,6 +35,8 @@ all of it widening:
   then not apply its own dropout.
 """
 import enum
+import functools
+import math
 
 import torch
 from torch import nn
@@ -223,15 +225,37 @@ class ScaledMaskedSoftmaxDropout(torch.autograd.Function):
         return grad, None, None, None, None, None, grad_bias, None, None
 
 
-def _fill_value(mask_func):
-    """The value that ``mask_func(scores, mask)`` puts in place of masked scores if that is what it does, leaving the
-    others alone, and if it is so low that they count for nothing beside any other; otherwise None. Found out on one
-    masked and one other score."""
+# What a mask function is tried on: two batch entries, two heads, three queries (one sees nothing, one everything), scores of
+# both signs and many sizes, all of them the same in every 16-bit type. On the CPU whatever the default device is: the answer
+# is read on the host, also while a graph is being captured.
+_TRIAL_ROWS = [[0.5, -96.0, 0.0, 1.5], [-0.03125, 7.0, 1024.0, -3.0], [-20480.0, 2.0, -1.0, 12288.0]]
+_TRIAL_SCORES = [[_TRIAL_ROWS, _TRIAL_ROWS[1:] + _TRIAL_ROWS[:1]], [_TRIAL_ROWS[2:] + _TRIAL_ROWS[:2], _TRIAL_ROWS[::-1]]]
+_TRIAL_MASK = [[[[True, True, True, True], [False, True, False, True], [False, False, False, False]]],
+               [[[True, True, False, True], [True, True, True, True], [False, False, True, False]]]]
+_HIGHEST_FILL = -9984.0   # -10000 in bfloat16
+_TRIAL_HIDDEN = torch.tensor(_TRIAL_MASK, device="cpu")
+_TRIAL = {dtype: torch.tensor(_TRIAL_SCORES, dtype=dtype, device="cpu") for dtype in (torch.float32, torch.float16, torch.bfloat16)}
+
+
+@functools.lru_cache(maxsize=16)
+def _trial_filled(fill):
+    return [[[[fill if masked else score for score, masked in zip(row, hidden)] for row, hidden in zip(head, mask[0])]
+             for head in entry] for entry, mask in zip(_TRIAL_SCORES, _TRIAL_MASK)]
+
+
+def _fill_value(mask_func, dtype=torch.float32):
+    """The value that ``mask_func(scores, mask)`` puts in place of masked scores of ``dtype`` if that is what it does, leaving
+    the others alone, and if it is finite and no higher than -10000; otherwise None.
+
+    It is asked again for every call that relies on the answer (about 10 us): a function may be anything, and behave
+    differently from one call to the next."""
     try:
-        kept, filled = mask_func(torch.tensor([[[[0.5, 1.5]]]]), torch.tensor([[[[False, True]]]])).flatten().tolist()
-    except Exception:
+        filled = mask_func(_TRIAL[dtype].clone(), _TRIAL_HIDDEN.clone()).tolist()   # (it may write into either)
+        fill = filled[0][0][0][0]
+        taken = -math.inf < fill <= _HIGHEST_FILL and filled == _trial_filled(fill)
+    except Exception:   # whatever such a function raises here it raises, or does not, where it is really used
         return None
-    return filled if kept == 0.5 and filled <= -10000.0 else None
+    return fill if taken else None
 
 
 class FusedScaleMaskSoftmax(nn.Module):
@@ -296,8 +320,9 @@ class FusedScaleMaskSoftmax(nn.Module):
 
     @property
     def mask_fill(self):
-        """What ``mask_func`` fills masked scores with, None if that is not what it does."""
-        return _fill_value(self.mask_func)
+        """What ``mask_func`` fills masked scores with on the torch branch, None if that is not what it does."""
+        narrow = self.input_in_float16 and not self.softmax_in_fp32
+        return _fill_value(self.mask_func, torch.float32 if not narrow else torch.float16 if self.input_in_fp16 else torch.bfloat16)
 
     # ------------------------------------------------------------------ dispatch
     def forward(self, input, mask, bias=None, key_lengths=None):

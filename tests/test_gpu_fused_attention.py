@@ -163,3 +163,23 @@ def test_the_context_may_be_changed_in_place(merged):
         out.square().sum().backward()
         results.append([util.raw_bits(t) for t in (out.detach(), *(leaf.grad for leaf in leaves))])
     assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
+@pytest.mark.parametrize("kind", ["subtracts 1e5", "-inf"])
+def test_rows_that_see_nothing_follow_the_mask_function(kind):
+    """A function that subtracts leaves the softmax of the scores in a row that sees nothing, -inf leaves NaN; a fill leaves
+    the average. Left padding, without a gradient, a length that the softmax gate refuses."""
+    from megatron.model.attention_core import CoreAttention
+    from megatron.model.fused_softmax import SoftmaxFusionTypes as T
+
+    func = {"subtracts 1e5": lambda s, m: s - 1e5 * m.to(s.dtype), "-inf": lambda s, m: s.masked_fill(m, float("-inf"))}[kind]
+    q, k, v = operands(torch.bfloat16, 77, 77, 1, 4, 4, 64, 31)
+    mask = hidden(77, 77).view(1, 1, 77, 77).clone()
+    mask[:, :, :, :20] = True
+    core = CoreAttention(64, 1, False, True, T.upper_triang, func, attention_softmax_in_fp32=True)
+    got = core(q, k, v, mask).float()
+    scores = torch.matmul(q.float().permute(1, 2, 0, 3).contiguous(), k.float().permute(1, 2, 3, 0).contiguous()) / 8
+    want = torch.matmul(torch.softmax(func(scores, mask), -1), v.float().permute(1, 2, 0, 3).contiguous())
+    assert torch.equal(got.isnan(), want.isnan()) and bool(want[:, :, :20].isnan().all()) == (kind == "-inf")
+    # scores of up to 4 are rounded to bf16 first; beside 1e5 an fp32 score keeps 2^-7
+    assert rel_err(got[~want.isnan()], want[~want.isnan()]) <= 2.0 ** -6

@@ -611,3 +611,62 @@ def test_a_mask_function_is_an_attribute_like_any_other():
     sm.mask_func = Fill(-30000.0)
     assert sm.mask_fill == -30000.0
     assert torch.equal(sm(x, mask), torch.softmax(x.masked_fill(mask, -30000.0), -1))
+
+
+FILLS = {
+    "lowest of the type": lambda s, m: s.masked_fill_(m, torch.finfo(s.dtype).min),
+    "constant": lambda s, m: s.masked_fill(m, -10000.0),
+    "where": lambda s, m: torch.where(m, torch.full((), -16384.0, dtype=s.dtype, device=s.device), s),
+}
+OTHERS = {
+    "-inf, which leaves NaN in rows that see nothing": lambda s, m: s.masked_fill_(m, float("-inf")),
+    "subtracts": lambda s, m: s - 1e5 * m.to(s.dtype),
+    "subtracts little": lambda s, m: s - 2.0 * m.to(s.dtype),
+    "a fill that competes with scores": lambda s, m: s.masked_fill(m, -100.0),
+    "clamps the others": lambda s, m: s.clamp(-50.0, 50.0).masked_fill(m, -10000.0),
+    "by position": lambda s, m: s.masked_fill(m, -10000.0) + 0.5 * torch.arange(s.size(-1), device=s.device),
+    "by head": lambda s, m: (s + torch.arange(s.size(1), device=s.device).view(1, -1, 1, 1)).masked_fill(m, -10000.0),
+    "by query": lambda s, m: s.masked_fill(m, -10000.0) * torch.arange(1, s.size(2) + 1, device=s.device).view(1, 1, -1, 1),
+    "one entry only": lambda s, m: torch.cat((s[:1].masked_fill(m[:1], -10000.0), s[1:])),
+    "the other way round": lambda s, m: s.masked_fill(~m, -10000.0),
+    "several values": lambda s, m: torch.where(m, -20000.0 - s.abs(), s),
+    "NaN": lambda s, m: s.masked_fill(m, float("nan")),
+    "none": None,
+}
+
+
+@pytest.mark.parametrize("fp32", [True, False])
+@pytest.mark.parametrize("kind", [*FILLS, *OTHERS])
+def test_mask_functions_that_are_a_fill_and_others(kind, fp32):
+    """What the attention kernels may rely on; a function that is anything else keeps the torch branch."""
+    from megatron.model.fused_softmax import SoftmaxFusionTypes as T
+
+    for fp16, dtype in ((True, torch.float16), (False, torch.bfloat16)):
+        m = make(T.none, fp16=fp16, bf16=not fp16, fp32=fp32)
+        m.mask_func = {**FILLS, **OTHERS}[kind]
+        if kind in OTHERS:
+            assert m.mask_fill is None
+            continue
+        work = torch.zeros((1, 1, 1, 1), dtype=torch.float32 if fp32 else dtype)
+        fill = m.mask_func(work, torch.ones_like(work, dtype=torch.bool)).item()
+        assert fill <= -9984.0 and m.mask_fill == fill   # (-10000 in bfloat16)
+
+
+def test_a_mask_function_is_asked_again():
+    """Its behaviour may change, it may write into what it is given, and the default device may be another one."""
+    from megatron.model.fused_softmax import SoftmaxFusionTypes as T
+
+    m, value = make(T.none), [-10000.0]
+
+    def changes(scores, mask):
+        mask.logical_or_(torch.zeros_like(mask))
+        return scores.masked_fill_(mask, value[0])
+
+    m.mask_func = changes
+    for value[0] in (-10000.0, -30000.0, float("-inf"), -20000.0):
+        assert m.mask_fill == (value[0] if math.isfinite(value[0]) else None)
+    m.mask_func = lambda s, mask: s.masked_fill_(mask.logical_not_(), -10000.0)
+    assert m.mask_fill is None
+    m.mask_func = mask_func
+    with torch.device("meta"):
+        assert m.mask_fill == torch.finfo(torch.float32).min

@@ -35,13 +35,33 @@ def rel_err(a, b):
     return ((a.float() - b.float()).norm() / b.float().norm()).item()
 
 
+@pytest.fixture(params=["kernel", "products"])
+def route(request, monkeypatch):
+    """Which way ``CoreAttention`` goes where nothing but a mask is in play: the attention kernels, or the two products around
+    the softmax, which stay for other head sizes, dropout and additive terms."""
+    if request.param == "products":
+        products_only(monkeypatch)
+    return request.param
+
+
+def products_only(monkeypatch):
+    from megatron.model import fused_attention
+
+    monkeypatch.setattr(fused_attention, "supported", lambda q, k, v: False)
+
+
+def goes(core, route, q, k, v, mask):
+    """Whether ``core`` takes that way for this call."""
+    return (core._one_kernel(q, k, v, mask, None, False) is not None) == (route == "kernel")
+
+
 def qkv(dtype, sq, b, np_, hn, seed):
     return [util.randn((sq, b, np_, hn), dtype, seed=seed + i).to(DEV).requires_grad_(True) for i in range(3)]
 
 
 @pytest.mark.parametrize("layer_scaling", [False, True], ids=["plain", "qk-layer-scaling"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
-def test_causal_attention_matches_textbook(dtype, layer_scaling):
+def test_causal_attention_matches_textbook(dtype, layer_scaling, route):
     from megatron.model.attention_core import CoreAttention
     from megatron.model.fused_softmax import SoftmaxFusionTypes as T
 
@@ -58,7 +78,7 @@ def test_causal_attention_matches_textbook(dtype, layer_scaling):
         assert core.scale_mask_softmax.scale == pytest.approx(1 / math.sqrt(hn))
     q, k, v = qkv(dtype, sq, b, np_, hn, 1)
     mask = fb.causal_mask(sq, DEV)
-    assert core.scale_mask_softmax.is_kernel_available(mask, b, np_, sq, sq)
+    assert core.scale_mask_softmax.is_kernel_available(mask, b, np_, sq, sq) and goes(core, route, q, k, v, mask)
     out = core(q, k, v, mask)
     assert out.shape == (b, np_, sq, hn) and out.dtype == dtype
     g = util.randn((b, np_, sq, hn), dtype, seed=9).to(DEV)
@@ -81,7 +101,7 @@ def test_causal_attention_matches_textbook(dtype, layer_scaling):
     assert rel_err(plain(q.detach(), k.detach(), v.detach(), mask), out) <= lim
 
 
-def test_padding_mask_alibi_window_and_rpe_inside_the_caller():
+def test_padding_mask_alibi_window_and_rpe_inside_the_caller(route):
     from megatron.model.attention_core import CoreAttention
     from megatron.model.fused_softmax import SoftmaxFusionTypes as T
     from megatron.model.positional_embeddings import AliBi
@@ -235,7 +255,7 @@ def test_split_and_rotate_matches_split_then_rotate(rotary_ndims):
     assert torch.equal(util.raw_bits(qd), util.raw_bits(qe)) and torch.equal(util.raw_bits(kd), util.raw_bits(ke))
 
 
-def test_merged_heads_output_equals_the_permuted_context():
+def test_merged_heads_output_equals_the_permuted_context(route):
     """CoreAttention(..., merged_heads=True) returns permute(2, 0, 1, 3) of the default result, reshaped to
     [sq, b, np * hn] (megatron/model/transformer.py:941-947), bit for bit, with the same gradients."""
     from megatron.model.attention_core import CoreAttention
@@ -246,6 +266,7 @@ def test_merged_heads_output_equals_the_permuted_context():
     mask = fb.causal_mask(sq, DEV)
     qa, ka, va = qkv(dtype, sq, b, np_, hn, 31)
     qb, kb, vb = (t.detach().clone().requires_grad_(True) for t in (qa, ka, va))
+    assert goes(core, route, qa, ka, va, mask)
     merged = core(qa, ka, va, mask, merged_heads=True)
     plain = core(qb, kb, vb, mask).permute(2, 0, 1, 3).contiguous().view(sq, b, np_ * hn)
     assert merged.shape == (sq, b, np_ * hn) and merged.is_contiguous()
@@ -259,8 +280,8 @@ def test_merged_heads_output_equals_the_permuted_context():
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("merged", [False, True], ids=["bnsh", "merged"])
-def test_grouped_query_attention_equals_attention_with_repeated_heads(dtype, merged):
-    """k and v with fewer heads than q: the grouped GEMMs against what the reference does, repeat_interleave of
+def test_grouped_query_attention_equals_attention_with_repeated_heads(dtype, merged, route):
+    """k and v with fewer heads than q: the grouped GEMMs (the kernel's shared heads) against what the reference does, repeat_interleave of
     the k/v heads (gqa_project, megatron/model/transformer.py:820-837) followed by ordinary attention; textbook
     fp32 attention on the repeated heads as the arbiter. The gradients of k and v are the sums over the query heads
     that share them."""
@@ -275,6 +296,7 @@ def test_grouped_query_attention_equals_attention_with_repeated_heads(dtype, mer
     q = util.randn((sq, b, np_, hn), dtype, seed=41).to(DEV).requires_grad_(True)
     k = util.randn((sq, b, nkv, hn), dtype, seed=42).to(DEV).requires_grad_(True)
     v = util.randn((sq, b, nkv, hn), dtype, seed=43).to(DEV).requires_grad_(True)
+    assert goes(core, route, q, k, v, mask)
     out = core(q, k, v, mask, merged_heads=merged)
     shape = (sq, b, np_ * hn) if merged else (b, np_, sq, hn)
     assert out.shape == shape and out.dtype == dtype
@@ -349,6 +371,7 @@ def test_blocked_causal_gemms_equal_the_dense_ones(case, monkeypatch):
     from megatron.model.attention_core import CoreAttention
     from megatron.model.fused_softmax import SoftmaxFusionTypes as T
 
+    products_only(monkeypatch)   # the attention kernels would take four of the cases
     dtype = torch.float16 if case == "fp16-alpha" else torch.bfloat16
     sq, b, np_, hn = (2048, 1, 4, 64) if case == "2048" else (328, 2, 4, 64)
     if case != "2048":
@@ -385,7 +408,7 @@ def test_blocked_causal_gemms_equal_the_dense_ones(case, monkeypatch):
     q, k, v = qkv(dtype, sq, b, np_, hn, 51)
     q2, k2, v2 = (t.detach().clone().requires_grad_(True) for t in (q, k, v))
     assert blocked._causal_block(mask, b, np_, sq, sq, q) == (512 if case == "2048" else 128)
-    assert dense._causal_block(mask, b, np_, sq, sq, q) == 0
+    assert dense._causal_block(mask, b, np_, sq, sq, q) == 0 and goes(blocked, "products", q, k, v, mask)
     g = util.randn((sq, b, np_ * hn), dtype, seed=55).to(DEV)
     torch.manual_seed(7)
     monkeypatch.setattr(attention_core.torch, "empty", poisoned_empty)

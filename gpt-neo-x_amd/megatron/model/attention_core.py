@@ -197,6 +197,8 @@ class CoreAttention(torch.nn.Module):
             (and the four of the backward) only on and below the diagonal blocks. The skipped parts of the score
             and probability tensors and of their gradients stay uninitialised; switch this off for tools that
             inspect those tensors (e.g. autograd's anomaly detection would report the stale NaN patterns in them).
+            Off, the attention kernels, which form none of these tensors, are not used either; nor are they while
+            ``scale_mask_softmax`` has hooks, is a subclass or has a method replaced.
     """
 
     def __init__(self, head_dim, layer_number, fp16, bf16, fusion_type, mask_func, attention_softmax_in_fp32=False,
@@ -305,9 +307,11 @@ class CoreAttention(torch.nn.Module):
         return fused_attention.masked_attention(query, key, value, mask, scale, fill, merged_heads)
 
     def _plain_scale(self, query, key, value, mask, key_lengths):
-        """The factor of the scores where they are scaled, masked and nothing else, and the operands are the attention
-        kernels'; otherwise None."""
+        """The factor of the scores where they are scaled, masked and nothing else, nobody looks at them or at the
+        probabilities, and the operands are the attention kernels'; otherwise None."""
         softmax = self.scale_mask_softmax
+        if not (self.causal_gemm_blocks and fused_attention.untouched(softmax, FusedScaleMaskSoftmax)):
+            return None
         if (key_lengths is not None or self.rpe is not None or softmax.alibi_slopes is not None or not softmax.fusion
                 or softmax.narrow_forward_scale or mask is None or (softmax.training and softmax.attention_dropout > 0.0)):
             return None

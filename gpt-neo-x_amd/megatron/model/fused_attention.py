@@ -10,8 +10,10 @@ Layouts as in ``CoreAttention``: q ``[sq, b, np, hn]``, k and v ``[sk, b, nkv, h
 strides with contiguous features.
 """
 import ctypes
+import functools
 
 import torch
+from torch.nn.modules.module import _has_any_global_hook
 
 from ..fused_kernels import _hotpath as _hp
 
@@ -167,6 +169,19 @@ MAX_DECODE_ROWS = 32   # queries that share a key/value head, in nhp_attention_d
 def plain(*tensors):
     """Whether nobody differentiates these or otherwise follows what is done with them."""
     return not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors)) and not _hp.followed(*tensors)
+
+
+@functools.lru_cache(maxsize=8)
+def _methods(cls):
+    return frozenset(name for name, member in vars(cls).items() if callable(member) or isinstance(member, (property, staticmethod)))
+
+
+def untouched(module, cls):
+    """Whether ``module`` is a ``cls`` as it stands: no subclass, none of its methods replaced, no hooks. Whoever put such a
+    thing there wants the tensors that pass through the module, so it has to be called, with those tensors."""
+    return (type(module) is cls and module.__dict__.keys().isdisjoint(_methods(cls))
+            and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
+                     or _has_any_global_hook()))
 
 
 def _cache_fits(key, value, past):

@@ -183,3 +183,20 @@ def test_rows_that_see_nothing_follow_the_mask_function(kind):
     assert torch.equal(got.isnan(), want.isnan()) and bool(want[:, :, :20].isnan().all()) == (kind == "-inf")
     # scores of up to 4 are rounded to bf16 first; beside 1e5 an fp32 score keeps 2^-7
     assert rel_err(got[~want.isnan()], want[~want.isnan()]) <= 2.0 ** -6
+
+
+def test_a_hook_on_the_softmax_module_sees_the_probabilities():
+    """While it is there the probabilities are formed; the result agrees with the kernel's."""
+    from megatron.model.attention_core import CoreAttention
+    from megatron.model.fused_softmax import SoftmaxFusionTypes as T
+
+    core = CoreAttention(64, 1, False, True, T.upper_triang, lambda s, m: s.masked_fill_(m, -1e4), attention_softmax_in_fp32=True)
+    q, k, v = operands(torch.bfloat16, 128, 128, 2, 4, 4, 64, 1)
+    mask, seen = hidden(128, 128).view(1, 1, 128, 128), []
+    handle = core.scale_mask_softmax.register_forward_hook(lambda module, args, out: seen.append(out))
+    with_hook = core(q, k, v, mask)
+    handle.remove()
+    without = core(q, k, v, mask)
+    assert len(seen) == 1 and seen[0].shape == (2, 4, 128, 128) and core._one_kernel(q, k, v, mask, None, False) is not None
+    # the products round the scores (up to 4, instead of a value of 1) once more
+    assert rel_err(with_hook, without) <= 2.0 ** -7

@@ -152,11 +152,11 @@ class SelfAttention(torch.nn.Module):
                     query, key = apply_rotary_to_query_key(query, key, self.rotary_emb, rotary_ndims=self.rotary_ndims,
                                                            rope_fusion=False, bf16=self.bf16, layer_past=layer_past)
         past = layer_past if layer_past is not None and layer_past.numel() > 0 else None
-        step = None
-        if self.use_cache and past is not None and isinstance(self.core, CoreAttention):
-            step = self.core(query, key, value, attention_mask, merged_heads=True, layer_past=past)
-        if step is not None:
-            context, present = step
+        call = None
+        if self.use_cache and past is not None and fused_attention.untouched(self.core, CoreAttention):
+            call = self.core._cached_call(query, key, value, attention_mask, past)
+        if call is not None:
+            context, present = fused_attention.checked_decode_attention(query, key, value, past, *call, merged=True)
         else:
             if self.use_cache and fused_attention.cache_supported(key, value, past):
                 present = fused_attention.append_to_cache(key, value, past)

@@ -63,3 +63,35 @@ def test_a_watched_softmax_is_called(who, monkeypatch):
 
 def test_the_switch_for_tools_that_inspect_the_tensors(monkeypatch):
     assert scale(core(causal_gemm_blocks=False), monkeypatch) is None
+
+
+def test_a_hook_on_the_attention_of_a_layer_with_cached_positions():
+    """It fires once a step, with the keys of all positions and the context."""
+    import types
+
+    from megatron.model.transformer_layer import SelfAttention
+
+    args = types.SimpleNamespace(hidden_size=128, num_attention_heads=2, num_kv_heads=None, seq_length=16, precision="fp32", pos_emb="rotary",
+                                 rotary_pct=1.0, rope_fusion=False, attention_softmax_in_fp32=False, attention_dropout=0.0,
+                                 scaled_upper_triang_masked_softmax_fusion=False, scaled_masked_softmax_fusion=False)
+    attention = SelfAttention(args, fb.fill_masked_with_dtype_min, 1, rotary=True, use_cache=True)
+    seen = []
+    attention.core.register_forward_hook(lambda module, inputs, out: seen.append((inputs[1].size(0), tuple(out.shape))))
+    x, mask = torch.randn(5, 1, 128), fb.causal_mask(5)
+    with torch.no_grad():
+        (_, present), _ = attention(x[:4], mask[..., :4, :4])
+        attention(x[4:], mask[..., 4:, :], layer_past=present)
+    assert seen == [(4, (4, 1, 128)), (5, (1, 1, 128))]
+
+
+def test_a_watched_attention_takes_no_step_of_its_own(monkeypatch):
+    c = core(use_cache=True)
+    assert fused_attention.untouched(c, CoreAttention)
+    for watch in (lambda: c.register_forward_hook(lambda m, i, o: None), lambda: c.register_forward_pre_hook(lambda m, i: None)):
+        handle = watch()
+        assert not fused_attention.untouched(c, CoreAttention)
+        handle.remove()
+    assert fused_attention.untouched(c, CoreAttention)
+    c.forward = lambda *a, **k: None
+    assert not fused_attention.untouched(c, CoreAttention)
+    assert not fused_attention.untouched(type("Own", (CoreAttention,), {})(64, 1, False, True, T.none, None), CoreAttention)

@@ -292,30 +292,30 @@ class CoreAttention(torch.nn.Module):
         to the scores, dropped, or not provided by them. Which keys a query sees is decided as by the softmax module:
         by index where that would run its causal kernel, otherwise by the mask (forward only; with the fill value of the
         padding-mask kernel where that would run, and of the mask function where the torch branch would)."""
-        scale = self._plain_scale(query, key, value, mask, key_lengths)
-        if scale is None:
+        scale = self._plain_scale(mask, key_lengths)
+        if scale is None or not fused_attention.supported(query, key, value):
             return None
         softmax = self.scale_mask_softmax
         b, np_, sq, sk = query.size(1), query.size(2), query.size(0), key.size(0)
         if softmax.upper_triang_mask_fusion and sq == sk and softmax.is_kernel_available(mask, b, np_, sq, sk):
             window = softmax.sliding_window_width
             window = None if window is None or window < 0 else int(window)
-            return fused_attention.causal_attention(query, key, value, scale, window, merged_heads)
+            return fused_attention.causal_attention(query, key, value, scale, window, merged_heads, checked=True)
         fill = self._fill_by_mask(mask, b, np_, sq, sk, query.device) if fused_attention.plain(query, key, value) else None
         if fill is None:
             return None
         return fused_attention.masked_attention(query, key, value, mask, scale, fill, merged_heads)
 
-    def _plain_scale(self, query, key, value, mask, key_lengths):
-        """The factor of the scores where they are scaled, masked and nothing else, nobody looks at them or at the
-        probabilities, and the operands are the attention kernels'; otherwise None."""
+    def _plain_scale(self, mask, key_lengths):
+        """The factor of the scores where they are scaled, masked and nothing else, and nobody looks at them or at the
+        probabilities; otherwise None."""
         softmax = self.scale_mask_softmax
         if not (self.causal_gemm_blocks and fused_attention.untouched(softmax, FusedScaleMaskSoftmax)):
             return None
         if (key_lengths is not None or self.rpe is not None or softmax.alibi_slopes is not None or not softmax.fusion
                 or softmax.narrow_forward_scale or mask is None or (softmax.training and softmax.attention_dropout > 0.0)):
             return None
-        if not fused_attention.supported(query, key, value) or not softmax.input_in_float16:
+        if not softmax.input_in_float16:
             return None
         scale = self.gemm_alpha * (1.0 if softmax.scale is None else softmax.scale)
         return scale if scale > 0.0 else None
@@ -333,14 +333,12 @@ class CoreAttention(torch.nn.Module):
 
     def _cached_call(self, query, key, value, mask, layer_past):
         """``(mask, scale, fill)`` for the decoding kernel, or None where it does not apply."""
-        if not fused_attention.decode_supported(query, key, value, layer_past):
+        scale = self._plain_scale(mask, None)
+        if scale is None or not fused_attention.decode_supported(query, key, value, layer_past):
             return None
-        b, np_, sq, sk = query.size(1), query.size(2), query.size(0), layer_past.size(1) + key.size(0)
-        if self.use_cache and mask is not None:
+        (sq, b, np_, _), sk = query.shape, layer_past.size(1) + key.size(0)
+        if self.use_cache and (mask.size(-1) > sk or mask.size(-2) > sk):
             mask = mask[..., :sk, :sk]
-        scale = self._plain_scale(query, key, value, mask, None)
-        if scale is None:
-            return None
         fill = self._fill_by_mask(mask, b, np_, sq, sk, query.device)
         return None if fill is None else (mask, scale, fill)
 

@@ -42,11 +42,14 @@ def supported(q, k, v):
     """Whether the kernels take these operands. They get addresses and the sizes of q alone, so everything that makes q, k
     and v belong together is checked here: one device and type, one batch, heads that divide, a head size there is a kernel
     for, no more queries than keys, and sizes that the kernels can address."""
-    return (q.is_cuda and q.dtype in (torch.bfloat16, torch.float16) and k.dtype == q.dtype and v.dtype == q.dtype
-            and k.device == q.device and v.device == q.device and q.dim() == 4 and k.dim() == 4 and k.shape == v.shape
-            and q.size(3) in HEAD_DIMS and k.size(3) == q.size(3) and k.size(1) == q.size(1)
-            and q.numel() > 0 and k.numel() > 0 and q.size(2) % k.size(2) == 0 and q.size(0) <= k.size(0)
-            and _addressable(q.size(0), k.size(0), q.size(1), q.size(2), k.size(2), q.size(3)))
+    device, dtype, shape, kv_shape = q.device, q.dtype, q.shape, k.shape
+    if not (q.is_cuda and (dtype is torch.bfloat16 or dtype is torch.float16) and k.dtype is dtype and v.dtype is dtype
+            and k.device == device and v.device == device and len(shape) == 4 and len(kv_shape) == 4 and v.shape == kv_shape):
+        return False
+    sq, b, np_, hn = shape
+    sk, kv_b, nkv, kv_hn = kv_shape
+    return (hn in HEAD_DIMS and kv_hn == hn and kv_b == b > 0 and nkv > 0 < np_ and np_ % nkv == 0 and 0 < sq <= sk
+            and _addressable(sq, sk, b, np_, nkv, hn))
 
 
 def _addressable(sq, sk, b, np_, nkv, hn):
@@ -69,62 +72,56 @@ def _refuse_unless(taken, who, *tensors):
 
 
 def _new_context(q, merged):
-    """Memory for the context, ``[sq, b, np, hn]`` with ``merged`` and ``[b, np, sq, hn]`` without."""
+    """Memory for the context in the layout that the caller of ``CoreAttention`` gets, ``[sq, b, np * hn]`` with ``merged`` and
+    ``[b, np, sq, hn]`` without, and its strides over position, batch entry and head. (Made in that shape, not as a view of
+    another: a view inside an autograd function is closed to changes in place, one outside costs a node of the graph.)"""
     sq, b, np_, hn = q.shape
-    return torch.empty((sq, b, np_, hn) if merged else (b, np_, sq, hn), dtype=q.dtype, device=q.device)
+    if merged:
+        return torch.empty((sq, b, np_ * hn), dtype=q.dtype, device=q.device), _I64x3(b * np_ * hn if sq > 1 else 0, np_ * hn, hn)
+    return torch.empty((b, np_, sq, hn), dtype=q.dtype, device=q.device), _I64x3(hn, np_ * sq * hn, sq * hn)
 
 
-def _by_position(out, merged):
-    """``_new_context`` as ``[sq, b, np, hn]``, the order of dimensions in which the kernels take their operands."""
-    return out if merged else out.permute(2, 0, 1, 3)
-
-
-def _finished(out, merged):
-    """``_new_context`` in the layout that the caller of ``CoreAttention`` gets."""
-    return out.view(out.size(0), out.size(1), -1) if merged else out
-
-
-def _launch(out, kept, lse, q, k, v, bits, mask_batches, fill, scale, window, who):
-    """``out`` (and ``kept``, laid out alike, or None) ``[sq, b, np, hn]``."""
+def _launch(out, out_strides, kept, lse, q, k, v, bits, mask_batches, fill, scale, window, who):
+    """``out`` and ``out_strides`` from ``_new_context``; ``kept`` laid out like ``out``, or None."""
     sq, b, np_, hn = q.shape
     with _hp.device_guard(q):
         rc = _hp.lib().nhp_attention_fwd_keep(
             out.data_ptr(), None if kept is None else kept.data_ptr(), None if lse is None else lse.data_ptr(), q.data_ptr(),
             k.data_ptr(), v.data_ptr(), None if bits is None else bits.data_ptr(), mask_batches, fill, scale,
             -1 if window is None else window, b, np_, k.size(2), sq, k.size(0), hn, _strides3(q), _strides3(k), _strides3(v),
-            _strides3(out), _hp.dtype_code(q, who), _hp.stream_of(q))
+            out_strides, _hp.dtype_code(q, who), _hp.stream_of(q))
     _hp.check(rc, who)
 
 
 class CausalAttention(torch.autograd.Function):
-    """``softmax(scale * q k^T) v`` under the causal mask (by index, with an optional sliding window): ``[sq, b, np, hn]``
-    with ``merged``, ``[b, np, sq, hn]`` without.
+    """``softmax(scale * q k^T) v`` under the causal mask (by index, with an optional sliding window).
 
     The backward needs the context. The caller may change it in place (the products would not mind: their backward does not
-    use it), so the result is no view made in here and the kernel stores it a second time for the backward."""
+    use it), so the kernel stores it a second time for the backward."""
 
     @staticmethod
-    def forward(ctx, q, k, v, scale, window, merged):
-        _refuse_unless(supported(q, k, v), "CausalAttention", q, k, v)
+    def forward(ctx, q, k, v, scale, window, merged, checked=False):
+        """``checked``: the caller has asked ``supported`` already (twice would cost a short call 8 of 155 us)."""
+        _refuse_unless(checked or supported(q, k, v), "CausalAttention", q, k, v)
         q, k, v = _readable(q), _readable(k), _readable(v)
-        out = _new_context(q, merged)
+        out, out_strides = _new_context(q, merged)
         need = any(ctx.needs_input_grad[:3])
         kept = torch.empty_like(out) if need else None
         lse = torch.empty((q.size(1) * q.size(2), q.size(0)), dtype=torch.float32, device=q.device) if need else None
-        _launch(_by_position(out, merged), kept, lse, q, k, v, None, 1, 0.0, scale, window, "CausalAttention")
+        _launch(out, out_strides, kept, lse, q, k, v, None, 1, 0.0, scale, window, "CausalAttention")
         if need:
             ctx.save_for_backward(q, k, v, kept, lse)
-            ctx.conf = (scale, window, merged)
+            ctx.conf = (scale, window, merged, out_strides)
         return out
 
     @staticmethod
     def backward(ctx, grad):
         who = "CausalAttention backward"
         q, k, v, out, lse = ctx.saved_tensors
-        scale, window, merged = ctx.conf
+        scale, window, merged, out_strides = ctx.conf
         sq, b, np_, hn = q.shape
         sk, nkv = k.size(0), k.size(2)
-        g, out = _readable(_by_position(grad, merged)), _by_position(out, merged)
+        g = _readable(grad.reshape(sq, b, np_, hn) if merged else grad.permute(2, 0, 1, 3))
         dq, dk, dv = torch.empty_like(q, memory_format=torch.contiguous_format), torch.empty_like(
             k, memory_format=torch.contiguous_format), torch.empty_like(v, memory_format=torch.contiguous_format)
         lib = _hp.lib()
@@ -134,16 +131,17 @@ class CausalAttention(torch.autograd.Function):
                 dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), g.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
                 out.data_ptr(), lse.data_ptr(), workspace.data_ptr(), scale, -1 if window is None else window, b, np_, nkv,
                 sq, sk, hn, _strides3(dq), _strides3(dk), _strides3(dv), _strides3(g), _strides3(q), _strides3(k), _strides3(v),
-                _strides3(out), _hp.dtype_code(q, who), _hp.stream_of(q))
+                out_strides, _hp.dtype_code(q, who), _hp.stream_of(q))
         _hp.check(rc, who)
         needs = ctx.needs_input_grad
-        return dq if needs[0] else None, dk if needs[1] else None, dv if needs[2] else None, None, None, None
+        return dq if needs[0] else None, dk if needs[1] else None, dv if needs[2] else None, None, None, None, None
 
 
-def causal_attention(q, k, v, scale, window=None, merged=False):
+def causal_attention(q, k, v, scale, window=None, merged=False, checked=False):
     """Context of q ``[s, b, np, hn]`` over k, v ``[s, b, nkv, hn]``: ``[b, np, s, hn]``, or with ``merged``
-    ``[s, b, np * hn]``. Query i attends to keys ``i - window .. i``."""
-    return _finished(CausalAttention.apply(q, k, v, float(scale), window, merged), merged)
+    ``[s, b, np * hn]``. Query i attends to keys ``i - window .. i``. ``checked``: the caller has asked
+    ``supported`` already."""
+    return CausalAttention.apply(q, k, v, float(scale), window, merged, checked)
 
 
 def masked_attention(q, k, v, mask, scale, fill, merged=False):
@@ -155,12 +153,12 @@ def masked_attention(q, k, v, mask, scale, fill, merged=False):
     sq, sk = q.size(0), k.size(0)
     mask = mask.contiguous()
     bits = torch.empty((mask.size(0), sq, (sk + 63) // 64), dtype=torch.int64, device=q.device)
-    out = _new_context(q, merged)
+    out, out_strides = _new_context(q, merged)
     with _hp.device_guard(q):
         rc = _hp.lib().nhp_attention_mask_bits(bits.data_ptr(), mask.data_ptr(), mask.size(0), sq, sk, _hp.stream_of(q))
     _hp.check(rc, "masked_attention")
-    _launch(_by_position(out, merged), None, None, q, k, v, bits, mask.size(0), fill, float(scale), None, "masked_attention")
-    return _finished(out, merged)
+    _launch(out, out_strides, None, None, q, k, v, bits, mask.size(0), fill, float(scale), None, "masked_attention")
+    return out
 
 
 MAX_DECODE_ROWS = 32   # queries that share a key/value head, in nhp_attention_decode
@@ -187,11 +185,13 @@ def untouched(module, cls):
 def _cache_fits(key, value, past):
     """Whether these are 16-bit keys and values on one GPU, of one shape and a size that the kernels can address after ``past``
     cached positions."""
-    if not (key.is_cuda and key.dtype in (torch.bfloat16, torch.float16) and key.dim() == 4 and value.shape == key.shape
-            and value.dtype == key.dtype and value.device == key.device and key.numel() > 0 and key.size(3) % 8 == 0):
+    dtype, shape = key.dtype, key.shape
+    if not (key.is_cuda and (dtype is torch.bfloat16 or dtype is torch.float16) and len(shape) == 4 and value.shape == shape
+            and value.dtype is dtype and value.device == key.device):
         return False
-    sk, width = past + key.size(0), key.numel() // key.size(0)
-    return width < 1 << 24 and sk < 1 << 24 and sk * width // key.size(3) < 1 << 31
+    sq, b, nkv, hn = shape
+    sk, heads = past + sq, b * nkv
+    return sq > 0 < heads and hn > 0 and hn % 8 == 0 and heads * hn < 1 << 24 and sk < 1 << 24 and sk * heads < 1 << 31
 
 
 def _continues(cached, key):
@@ -244,8 +244,23 @@ def _decode_fits(query, key, value, past):
 
 def decode_supported(query, key, value, layer_past):
     """Whether ``decode_attention`` takes these, and nobody differentiates."""
-    return (layer_past is not None and cache_supported(key, value, layer_past) and _decode_fits(query, key, value, layer_past.size(1))
-            and plain(query))
+    return (isinstance(layer_past, torch.Tensor) and layer_past.dim() == 5 and layer_past.size(0) == 2
+            and _cache_fits(key, value, layer_past.size(1)) and _continues(layer_past, key)
+            and _decode_fits(query, key, value, layer_past.size(1)) and plain(query, key, value, layer_past))
+
+
+def _cached_rows(layer_past):
+    """Address and strides of the cached keys and of the values, their number, and what has to live until the launch. Of one
+    tensor without making two of it, which takes the host 5 us."""
+    if isinstance(layer_past, torch.Tensor):
+        pair, past, b, nkv, hn = layer_past.stride()
+        if hn == 1 and (pair | past | b | nkv) % 8 == 0 and past < 1 << 24 and layer_past.data_ptr() % 16 == 0:
+            n = layer_past.shape
+            strides = _I64x3(past if n[1] > 1 else 0, b if n[2] > 1 else 0, nkv if n[3] > 1 else 0)
+            keys = layer_past.data_ptr()
+            return (keys, strides), (keys + 2 * pair, strides), n[1], layer_past
+    keys, values = (_readable(t) for t in layer_past)
+    return (keys.data_ptr(), _strides3(keys)), (values.data_ptr(), _strides3(values)), keys.size(0), (keys, values)
 
 
 def decode_attention(query, key, value, layer_past, mask, scale, fill, merged=False):
@@ -262,22 +277,22 @@ def checked_decode_attention(query, key, value, layer_past, mask, scale, fill, m
     """``decode_attention`` for a caller that has asked ``decode_supported`` and ``mask_supported`` already: a step of a small
     model waits for the host, and the checks cost it several microseconds a layer."""
     query, key, value = _readable(query), _readable(key), _readable(value)
-    past_k, past_v = (_readable(t) for t in layer_past)
+    (keys, key_strides), (values, value_strides), past, _alive = _cached_rows(layer_past)
     sq, b, np_, hn = query.shape
-    nkv, past = key.size(2), past_k.size(0)
+    nkv = key.size(2)
     if mask.stride(3) != 1:
         mask = mask.contiguous()
-    out = _new_context(query, merged)
+    out, out_strides = _new_context(query, merged)
     present = torch.empty((2, past + sq, b, nkv, hn), dtype=key.dtype, device=key.device)
     lib = _hp.lib()
     scratch = lib.nhp_attention_decode_workspace_bytes(b, np_, nkv, sq, past, hn)
     workspace = torch.empty(scratch, dtype=torch.uint8, device=query.device) if scratch else None
     with _hp.device_guard(query):
         rc = lib.nhp_attention_decode(
-            out.data_ptr(), present.data_ptr(), query.data_ptr(), key.data_ptr(), value.data_ptr(), past_k.data_ptr(),
-            past_v.data_ptr(), mask.data_ptr(), mask.stride(0) if mask.size(0) > 1 else 0, mask.stride(2), fill,
-            None if workspace is None else workspace.data_ptr(), scale, b, np_, nkv, sq, past, hn, _strides3(_by_position(out, merged)), _strides3(query),
-            _strides3(key), _strides3(value), _strides3(past_k), _strides3(past_v), _hp.dtype_code(query, "decode_attention"),
-            _hp.stream_of(query))
+            out.data_ptr(), present.data_ptr(), query.data_ptr(), key.data_ptr(), value.data_ptr(), keys,
+            values, mask.data_ptr(), mask.stride(0) if mask.size(0) > 1 else 0, mask.stride(2), fill,
+            None if workspace is None else workspace.data_ptr(), scale, b, np_, nkv, sq, past, hn,
+            out_strides, _strides3(query), _strides3(key), _strides3(value), key_strides, value_strides,
+            _hp.dtype_code(query, "decode_attention"), _hp.stream_of(query))
     _hp.check(rc, "decode_attention")
-    return _finished(out, merged), present
+    return out, present

@@ -1,6 +1,5 @@
 """Whoever looks at the modules of the attention keeps seeing what passes through them: hooks, subclasses and replaced methods of
-the softmax module, hooks on ``CoreAttention`` in a layer with cached positions. On the CPU; which route a call takes is asked
-with the operand checks answered for a GPU."""
+the softmax module, hooks on ``CoreAttention`` in a layer with cached positions. On the CPU."""
 import pytest
 import torch
 
@@ -20,10 +19,9 @@ def core(**kw):
     return CoreAttention(64, 1, False, True, T.upper_triang, fb.fill_masked_with_dtype_min, attention_softmax_in_fp32=True, **kw)
 
 
-def scale(c, monkeypatch):
-    monkeypatch.setattr(fused_attention, "supported", lambda q, k, v: True)
-    t = torch.zeros((8, 1, 4, 64), dtype=torch.bfloat16)
-    return c._plain_scale(t, t, t, fb.causal_mask(8), None)
+def scale(c):
+    """What the attention kernels would scale the scores by, None where ``c`` takes the products."""
+    return c._plain_scale(fb.causal_mask(8), None)
 
 
 def subclass(c):
@@ -49,20 +47,20 @@ WATCHERS = {
 
 
 @pytest.mark.parametrize("who", WATCHERS)
-def test_a_watched_softmax_is_called(who, monkeypatch):
+def test_a_watched_softmax_is_called(who):
     c = core()
-    assert scale(c, monkeypatch) == pytest.approx(0.125)
+    assert scale(c) == pytest.approx(0.125)
     handle = WATCHERS[who](c)
     try:
-        assert scale(c, monkeypatch) is None
+        assert scale(c) is None
     finally:
         if hasattr(handle, "remove"):
             handle.remove()
-            assert scale(c, monkeypatch) == pytest.approx(0.125)
+            assert scale(c) == pytest.approx(0.125)
 
 
-def test_the_switch_for_tools_that_inspect_the_tensors(monkeypatch):
-    assert scale(core(causal_gemm_blocks=False), monkeypatch) is None
+def test_the_switch_for_tools_that_inspect_the_tensors():
+    assert scale(core(causal_gemm_blocks=False)) is None
 
 
 def test_a_hook_on_the_attention_of_a_layer_with_cached_positions():
@@ -84,7 +82,7 @@ def test_a_hook_on_the_attention_of_a_layer_with_cached_positions():
     assert seen == [(4, (4, 1, 128)), (5, (1, 1, 128))]
 
 
-def test_a_watched_attention_takes_no_step_of_its_own(monkeypatch):
+def test_a_watched_attention_takes_no_step_of_its_own():
     c = core(use_cache=True)
     assert fused_attention.untouched(c, CoreAttention)
     for watch in (lambda: c.register_forward_hook(lambda m, i, o: None), lambda: c.register_forward_pre_hook(lambda m, i: None)):

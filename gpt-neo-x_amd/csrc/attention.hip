@@ -375,7 +375,8 @@ __global__ void __launch_bounds__(256, 2) attn_dq_kernel(AttnBwdArgs a)
 
 // Gradients of k and v: 32 keys per wave as columns, their k and v rows in registers; Q and dO tiles of 64 queries (and
 // their row statistics) in LDS. Per 32 queries: S = Q k^T, dP = dO v^T, dS = P (dP - delta), dv^T += dO^T P,
-// dk^T += Q^T dS.
+// dk^T += Q^T dS. A workgroup goes over the queries of `fold` heads that share its keys, one after the other into the same
+// accumulators; what remains to be added up (fold < group) it leaves in fp32.
 template <int DT, int HD>
 __global__ void __launch_bounds__(256, 2) attn_dkv_kernel(AttnBwdArgs a)
 {
@@ -390,9 +391,9 @@ __global__ void __launch_bounds__(256, 2) attn_dkv_kernel(AttnBwdArgs a)
     const int kl = lane & 31, half = lane >> 5;
     const int nkb = (a.sk + kFwdRows - 1) / kFwdRows;
     const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
-    const int bh = xcd * a.heads_per_xcd + idx / nkb;
-    if (bh >= a.batch * a.heads) return;
-    const int b = bh / a.heads, h = bh % a.heads, hk = h / a.group;
+    const int units = a.heads / a.fold, unit = xcd * a.heads_per_xcd + idx / nkb;   // (batch entry, `fold` heads)
+    if (unit >= a.batch * units) return;
+    const int b = unit / units, h0 = unit % units * a.fold, hk = h0 / a.group;
     const int k0 = (idx % nkb) * kFwdRows, kw = k0 + wave * 32;
     const int ki = min(kw + kl, a.sk - 1);
 
@@ -414,30 +415,35 @@ __global__ void __launch_bounds__(256, 2) attn_dkv_kernel(AttnBwdArgs a)
     const int q_lo = max(0, k0 - a.shift), q_hi = min(a.sq, k0 + kFwdRows - a.shift + a.window);
     const int qt_lo = q_lo >> 6, qt_hi = (q_hi + 63) >> 6;
     const int wave_lo = kw - a.shift, wave_hi = min(kw + 31, a.sk - 1) - a.shift + a.window;
-    const uint16_t* qbase = a.q + b * a.q_b + h * a.q_h;
-    const uint16_t* gbase = a.d_o + b * a.do_b + h * a.do_h;
-    const float* lse = a.lse + (int64_t)bh * a.sq;
-    const float* delta = a.delta + (int64_t)bh * a.sq;
+    const uint16_t* qbase = a.q + b * a.q_b;
+    const uint16_t* gbase = a.d_o + b * a.do_b;
     TileLoader<HD, kLean> qload(a.q_s, lane, wave), gload(a.do_s, lane, wave);
     const int row = G::row_addr(kl, half), tr = G::tr_addr(lane);
-    auto fetch = [&](int qt, int buf) {
+    auto fetch = [&](int h, int qt, int buf) {
         const int left = a.sq - qt * 64;
-        qload.load(qbase + (int64_t)qt * 64 * a.q_s, lds + buf * G::kTileBytes, left);
-        gload.load(gbase + (int64_t)qt * 64 * a.do_s, lds + (2 + buf) * G::kTileBytes, left);
-        if (wave == 0) load_floats(lse + qt * 64, stats + buf * 512, lane, left);
-        if (wave == 1) load_floats(delta + qt * 64, stats + buf * 512 + 256, lane, left);
+        const int64_t row0 = ((int64_t)b * a.heads + h) * a.sq + qt * 64;
+        qload.load(qbase + h * a.q_h + (int64_t)qt * 64 * a.q_s, lds + buf * G::kTileBytes, left);
+        gload.load(gbase + h * a.do_h + (int64_t)qt * 64 * a.do_s, lds + (2 + buf) * G::kTileBytes, left);
+        if (wave == 0) load_floats(a.lse + row0, stats + buf * 512, lane, left);
+        if (wave == 1) load_floats(a.delta + row0, stats + buf * 512 + 256, lane, left);
     };
 
     f32x16 dk[G::kDTiles], dv[G::kDTiles];
 #pragma unroll
     for (int d = 0; d < G::kDTiles; ++d) dk[d] = dv[d] = f32x16{};
-    if (qt_lo < qt_hi) fetch(qt_lo, 0);
-    for (int qt = qt_lo; qt < qt_hi; ++qt) {
-        const int buf = (qt - qt_lo) & 1;
+    // the tiles of all heads in one sequence: the first one of a head is on its way during the last one of the head before
+    int buf = 1, h = h0, qt = qt_lo;
+    if (qt_lo < qt_hi) fetch(h, qt, 0);
+    for (int left = (qt_hi - qt_lo) * a.fold; left > 0; --left) {
+        const int r0 = qt * 64;
+        buf ^= 1;
         wait_lds_loads();
         __syncthreads();
-        if (qt + 1 < qt_hi) fetch(qt + 1, buf ^ 1);
-        const int r0 = qt * 64;
+        if (++qt == qt_hi) {
+            qt = qt_lo;
+            ++h;
+        }
+        if (left > 1) fetch(h, qt, buf ^ 1);
         if (r0 + 63 < wave_lo || r0 > wave_hi) continue;
         const char* qt_lds = lds + buf * G::kTileBytes;
         const char* gt_lds = lds + (2 + buf) * G::kTileBytes;
@@ -485,18 +491,21 @@ __global__ void __launch_bounds__(256, 2) attn_dkv_kernel(AttnBwdArgs a)
             }
         }
     }
-    if (kw + kl < a.sk) {
-        store_transposed<DT, HD>(a.dk + b * a.dk_b + h * a.dk_h + (int64_t)(kw + kl) * a.dk_s, nullptr, dk, a.scale, half);
-        store_transposed<DT, HD>(a.dv + b * a.dv_b + h * a.dv_h + (int64_t)(kw + kl) * a.dv_s, nullptr, dv, 1.0f, half);
+    if (kw + kl < a.sk && a.dk_parts) {
+        const int64_t at = ((int64_t)unit * a.sk + kw + kl) * HD;
+        store_transposed<HD>(a.dk_parts + at, dk, a.scale, half);
+        store_transposed<HD>(a.dv_parts + at, dv, 1.0f, half);
+    } else if (kw + kl < a.sk) {
+        store_transposed<DT, HD>(a.dk + b * a.dk_b + hk * a.dk_h + (int64_t)(kw + kl) * a.dk_s, nullptr, dk, a.scale, half);
+        store_transposed<DT, HD>(a.dv + b * a.dv_b + hk * a.dv_h + (int64_t)(kw + kl) * a.dv_s, nullptr, dv, 1.0f, half);
     }
 }
 
-// Sums the gradients of the query heads that share a key/value head: `parts` [rows, kv_heads * group, hd] (contiguous)
-// -> out with strides. blockIdx.z picks dk or dv.
+// Adds up what the workgroups of a key/value head have left and rounds the sums. blockIdx.z picks dk or dv.
 template <int DT>
-__global__ void __launch_bounds__(256) attn_group_sum_kernel(AttnBwdArgs a, const uint16_t* dk_parts, const uint16_t* dv_parts, int hd)
+__global__ void __launch_bounds__(256) attn_group_sum_kernel(AttnBwdArgs a, int hd)
 {
-    const int kv_heads = a.heads / a.group, chunks = hd / 8;
+    const int kv_heads = a.heads / a.group, parts = a.group / a.fold, chunks = hd / 8;
     const int64_t items = (int64_t)a.sk * a.batch * kv_heads * chunks;
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= items) return;
@@ -507,50 +516,63 @@ __global__ void __launch_bounds__(256) attn_group_sum_kernel(AttnBwdArgs a, cons
     const int b = (int)(r % a.batch);
     const int64_t s = r / a.batch;
     const bool second = blockIdx.z != 0;
-    const uint16_t* p = (second ? dv_parts : dk_parts) + ((s * a.batch + b) * a.heads + (int64_t)hk * a.group) * hd + c * 8;
+    const float* p = (second ? a.dv_parts : a.dk_parts) + (((int64_t)b * kv_heads + hk) * parts * a.sk + s) * hd + c * 8;
     float sum[8] = {};
-    for (int g = 0; g < a.group; ++g) {
-        float f[8];
-        unpack8<DT>(load16_stream(p + (int64_t)g * hd), f);
+    for (int g = 0; g < parts; ++g) {
+        const f32x4* x = reinterpret_cast<const f32x4*>(p + (int64_t)g * a.sk * hd);
+        const f32x4 lo = __builtin_nontemporal_load(x), hi = __builtin_nontemporal_load(x + 1);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) sum[j] += f[j];
+        for (int j = 0; j < 4; ++j) {
+            sum[j] += lo[j];
+            sum[4 + j] += hi[j];
+        }
     }
     uint16_t* o = second ? a.dv + s * a.dv_s + b * a.dv_b + hk * a.dv_h : a.dk + s * a.dk_s + b * a.dk_b + hk * a.dk_h;
     *reinterpret_cast<u32x4*>(o + c * 8) = pack8<DT>(sum);
 }
 
+// Query heads that a workgroup of the second gradient kernel goes over: as many as leave enough workgroups. Every head that is
+// not added up in registers costs 8 bytes written and read again per element of k and v, but causal key blocks differ in
+// length by up to a factor of 2 * blocks, and with few workgroups the longest one is what the launch takes. Two workgroups
+// fit on a CU: 512 at once, which is enough where a row is at most eight blocks long, between 1024 and 8192 keys it takes
+// 2048, and 1024 beyond (where the products outweigh the rest). Both kernels, us, fold 1 / 2 / 4 of a group of 4, 128 features:
+//   [1024, 8, 16 heads] 240 / 217 / 256 (1024 / 512 / 256 workgroups), [1024, 16, 16] 435 / 403 / 365,
+//   [2048, 8, 16] 651 / 657 / 658 (2048 / 1024 / 512), [4096, 4, 16] 1094 / 1142 / 1240, [4096, 8, 16] 2151 / 2071 / 2177,
+//   [8192, 1, 32] 1886 / 1865 / 2226 (2048 / 1024 / 512), [8192, 4, 16] 3795 / 3736 / 3714, [512, 1, 32] 52 / 58 / 75.
+static int bwd_fold(int64_t batch, int64_t heads, int64_t kv_heads, int64_t sk)
+{
+    const int64_t group = heads / kv_heads, blocks = batch * heads * ((sk + kFwdRows - 1) / kFwdRows);
+    const int64_t least = sk <= 1024 ? 512 : sk < 8192 ? 2048 : 1024;
+    for (int64_t fold = group < blocks / least ? group : blocks / least; fold > 1; --fold)
+        if (group % fold == 0) return (int)fold;
+    return 1;
+}
+
 template <int DT, int HD>
-static int launch_bwd(AttnBwdArgs a, uint16_t* parts, hipStream_t st)
+static int launch_bwd(AttnBwdArgs a, hipStream_t st)
 {
     const int64_t nqb = (a.sq + kFwdRows - 1) / kFwdRows, nkb = (a.sk + kFwdRows - 1) / kFwdRows;
     const int64_t per = 8 * (int64_t)a.heads_per_xcd;
+    AttnBwdArgs w = a;
+    w.heads_per_xcd = (a.batch * (a.heads / a.fold) + 7) / 8;
     const int64_t sum_blocks = ((int64_t)a.sk * a.batch * (a.heads / a.group) * (HD / 8) + 255) / 256;
-    if (!grid_fits(per * nqb, 256) || !grid_fits(per * nkb, 256) || !grid_fits(sum_blocks, 256)) return NHP_ERR_SHAPE;
+    const int64_t dkv_blocks = 8 * (int64_t)w.heads_per_xcd * nkb;
+    if (!grid_fits(per * nqb, 256) || !grid_fits(dkv_blocks, 256) || !grid_fits(sum_blocks, 256)) return NHP_ERR_SHAPE;
     launch_prepare();
     attn_dq_kernel<DT, HD><<<dim3((unsigned)(per * nqb)), dim3(256), 0, st>>>(a);
-    AttnBwdArgs w = a;
-    uint16_t* dv_parts = nullptr;
-    if (a.group > 1) {
-        dv_parts = parts + (int64_t)a.sk * a.batch * a.heads * HD;
-        w.dk = parts;
-        w.dv = dv_parts;
-        w.dk_s = w.dv_s = (int64_t)a.batch * a.heads * HD;
-        w.dk_b = w.dv_b = (int64_t)a.heads * HD;
-        w.dk_h = w.dv_h = HD;
-    }
-    attn_dkv_kernel<DT, HD><<<dim3((unsigned)(per * nkb)), dim3(256), 0, st>>>(w);
-    if (a.group > 1) attn_group_sum_kernel<DT><<<dim3((unsigned)sum_blocks, 1, 2), dim3(256), 0, st>>>(a, parts, dv_parts, HD);
+    attn_dkv_kernel<DT, HD><<<dim3((unsigned)dkv_blocks), dim3(256), 0, st>>>(w);
+    if (a.fold < a.group) attn_group_sum_kernel<DT><<<dim3((unsigned)sum_blocks, 1, 2), dim3(256), 0, st>>>(a, HD);
     return launch_result();
 }
 
 template <int DT>
-static int launch_bwd_hd(const AttnBwdArgs& a, uint16_t* parts, int hd, hipStream_t st)
+static int launch_bwd_hd(const AttnBwdArgs& a, int hd, hipStream_t st)
 {
     switch (hd) {
-    case 64: return launch_bwd<DT, 64>(a, parts, st);
-    case 80: return launch_bwd<DT, 80>(a, parts, st);
-    case 96: return launch_bwd<DT, 96>(a, parts, st);
-    case 128: return launch_bwd<DT, 128>(a, parts, st);
+    case 64: return launch_bwd<DT, 64>(a, st);
+    case 80: return launch_bwd<DT, 80>(a, st);
+    case 96: return launch_bwd<DT, 96>(a, st);
+    case 128: return launch_bwd<DT, 128>(a, st);
     }
     return NHP_ERR_SHAPE;
 }
@@ -626,8 +648,10 @@ int nhp_attention_fwd(void* out, float* lse, const void* q, const void* k, const
 int64_t nhp_attention_bwd_workspace_bytes(int64_t batch, int64_t heads, int64_t kv_heads, int64_t sq, int64_t sk, int64_t head_dim)
 {
     if (batch <= 0 || heads <= 0 || kv_heads <= 0 || sq <= 0 || sk <= 0 || head_dim <= 0) return 0;
+    if (heads % kv_heads) return 0;
     const int64_t delta = (batch * heads * sq * 4 + 255) / 256 * 256;
-    return delta + (heads > kv_heads ? 2 * sk * batch * heads * head_dim * 2 : 0);
+    const int64_t fold = nhp::bwd_fold(batch, heads, kv_heads, sk);
+    return delta + (fold * kv_heads < heads ? 2 * sk * batch * (heads / fold) * head_dim * 4 : 0);
 }
 
 int nhp_attention_bwd(void* dq, void* dk, void* dv, const void* d_out, const void* q, const void* k, const void* v,
@@ -661,7 +685,11 @@ int nhp_attention_bwd(void* dq, void* dk, void* dv, const void* d_out, const voi
     a.dv = static_cast<uint16_t*>(dv);
     a.lse = lse;
     a.delta = static_cast<float*>(workspace);
-    auto* parts = reinterpret_cast<uint16_t*>(static_cast<char*>(workspace) + (batch * heads * sq * 4 + 255) / 256 * 256);
+    a.fold = bwd_fold(batch, heads, kv_heads, sk);
+    if (a.fold * kv_heads < heads) {
+        a.dk_parts = reinterpret_cast<float*>(static_cast<char*>(workspace) + (batch * heads * sq * 4 + 255) / 256 * 256);
+        a.dv_parts = a.dk_parts + sk * batch * (heads / a.fold) * head_dim;
+    }
     a.scale = scale;
     a.scale_log2 = scale * kLog2e;
     a.batch = (int)batch;
@@ -672,8 +700,8 @@ int nhp_attention_bwd(void* dq, void* dk, void* dv, const void* d_out, const voi
     a.shift = (int)(sk - sq);
     a.window = window < 0 || window > sk ? (int)sk : (int)window;
     a.heads_per_xcd = (int)((batch * heads + 7) / 8);
-    if (dtype == NHP_BF16) return launch_bwd_hd<NHP_BF16>(a, parts, (int)head_dim, static_cast<hipStream_t>(stream));
-    if (dtype == NHP_F16) return launch_bwd_hd<NHP_F16>(a, parts, (int)head_dim, static_cast<hipStream_t>(stream));
+    if (dtype == NHP_BF16) return launch_bwd_hd<NHP_BF16>(a, (int)head_dim, static_cast<hipStream_t>(stream));
+    if (dtype == NHP_F16) return launch_bwd_hd<NHP_F16>(a, (int)head_dim, static_cast<hipStream_t>(stream));
     return NHP_ERR_DTYPE;
 }
 

@@ -41,13 +41,15 @@ struct AttnFwdArgs {
 
 struct AttnBwdArgs {
     const uint16_t *q, *k, *v, *o, *d_o;
-    uint16_t *dq, *dk, *dv;   // dk, dv: one head per QUERY head when heads share keys (summed up by a second kernel)
+    uint16_t *dq, *dk, *dv;
+    float *dk_parts, *dv_parts;   // [batch * heads / fold][sk][head size], summed up by a second kernel; null without one
     const float* lse;
     float* delta;   // [batch * heads, sq]: sum over features of out * d_out, written by the first kernel for the second
     int64_t q_s, q_b, q_h, k_s, k_b, k_h, v_s, v_b, v_h, o_s, o_b, o_h, do_s, do_b, do_h;
     int64_t dq_s, dq_b, dq_h, dk_s, dk_b, dk_h, dv_s, dv_b, dv_h;
     float scale, scale_log2;
     int batch, heads, group, sq, sk, shift, window, heads_per_xcd;
+    int fold;   // query heads that a workgroup of the second kernel goes over; they share a key/value head
 };
 
 template <int DT>
@@ -218,6 +220,20 @@ __device__ __forceinline__ void store_transposed(uint16_t* row, uint16_t* second
             const u32x4 chunk = {(uint32_t)r0[0], (uint32_t)r1[0], (uint32_t)r0[1], (uint32_t)r1[1]};
             *reinterpret_cast<u32x4*>(row + d * 32 + j * 16 + half * 8) = chunk;
             if (second) *reinterpret_cast<u32x4*>(second + d * 32 + j * 16 + half * 8) = chunk;
+        }
+}
+
+// The same as floats.
+template <int HD>
+__device__ __forceinline__ void store_transposed(float* row, const f32x16 (&o)[AttnGeo<HD>::kDTiles], float f, int half)
+{
+#pragma unroll
+    for (int d = 0; d < AttnGeo<HD>::kDTiles; ++d)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            if (d * 32 + g * 8 >= HD) continue;
+            *reinterpret_cast<f32x4*>(row + d * 32 + g * 8 + half * 4) =
+                f32x4{o[d][4 * g] * f, o[d][4 * g + 1] * f, o[d][4 * g + 2] * f, o[d][4 * g + 3] * f};
         }
 }
 

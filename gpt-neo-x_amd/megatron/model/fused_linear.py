@@ -3,10 +3,26 @@
 The reference's Column / RowParallelLinear (megatron/mpu/layers.py) call the library GEMM whatever the number of rows. With
 few of them the product is a single read of the weights, and the library's call alone takes the host 25 us (this one 8).
 
-Where the line lies, library -> here on the GPU: 16 rows [4096, 4096] 14.9 -> 11.5 us, [22016, 4096] 51.7 -> 43.5,
-[4096, 11008] 38.2 -> 27.6, [2048, 8192] 12.6 -> 13.2, [2560, 10240] 16.9 -> 22.1; one row [2304, 768] 7.2 -> 3.6. 32 rows
-[2304, 768] 6.9 -> 4.9, [8192, 2048] 12.9 -> 13.4, [2048, 2048] 11.3 -> 8.3, [1024, 4096] 11.8 -> 14.3, but [4096, 4096]
-12.6 -> 15.4, [7680, 2560] 12.0 -> 18.5. Layers up to 2048 features wait for the host in either case."""
+Where the line lies. On the GPU, weights not in any cache, us here / library:
+    rows           1            4            16            32
+    [2304, 768]    3.7 / 8.6    3.8 / 6.7    4.1 / 6.7     5.0 / 9.5
+    [2048, 2048]   5.1 / 13.0   5.5 / 11.3   6.4 / 11.3    8.3 / 11.5
+    [1024, 4096]   7.3 / 16.5   7.9 / 14.7   10.0 / 14.7   13.7 / 12.1
+    [4096, 4096]   9.7 / 17.6   9.7 / 15.8   11.8 / 15.7   15.4 / 13.3
+    [22016, 4096]  39.5 / 51.5  39.7 / 50.0  40.9 / 50.8   45.3 / 41.5
+    [4096, 11008]  25.4 / 40.1  24.4 / 37.6  26.2 / 37.6   29.1 / 29.8
+    [6144, 4096]   14.4 / 16.3  14.9 / 14.5  16.9 / 14.4   20.8 / 15.3
+    [5120, 5120]   14.8 / 15.6  15.1 / 14.0  16.0 / 15.4   18.3 / 18.2
+    [4096, 14336]  31.2 / 28.2  30.1 / 25.2  32.1 / 25.8   35.6 / 30.9
+    [7680, 2560]   12.8 / 13.3  13.1 / 11.4  14.4 / 11.5   16.9 / 12.1
+    [2560, 10240]  19.4 / 21.5  18.9 / 16.8  20.6 / 17.2   23.3 / 21.5
+Where a side has at most 2048 features the kernel is ahead up to about 24 rows. Larger ones are mixed: with 2560 features a
+wave has five of its eight steps to do and the tiles do not divide among the workgroups (160 for 64, 480 for 256). They are
+taken all the same up to 16 rows, because it is the host that a step waits for until its cache is long: a layer of 2560
+features called step by step takes 222 us here and 272 to 282 with those products in the library, with 1 to 8 sequences of up
+to 2000 positions, and 16 of 200. Where the GPU is what is waited for the library is ahead there: 16 sequences of 2000 positions
+336 / 320 us, and in a captured graph 71 / 76 us with one sequence, 90 / 91 with four, 195 / 176 with eight of 2000, 336 / 314
+with 16. With 4096 features, 8 heads of keys: 247 / 274 us step by step, 178 / 175 in a graph (16 of 2000)."""
 import torch
 import torch.nn.functional as F
 

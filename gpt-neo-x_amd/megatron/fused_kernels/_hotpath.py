@@ -166,9 +166,9 @@ def require_gpu(t, what):
 
 def followed(*tensors):
     """Whether torch follows the operations on any of these beyond autograd (vmap and the other function transforms,
-    forward-mode derivatives, tracing, compilation, tensor subclasses): a launch outside of an autograd function would
-    escape it."""
-    return (torch.compiler.is_compiling() or torch.autograd.forward_ad._current_level >= 0
+    forward-mode derivatives, tracing, compilation, dispatch modes such as a counter of operations, tensor subclasses): a
+    launch outside of an autograd function would escape it."""
+    return (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0 or torch.autograd.forward_ad._current_level >= 0
             or torch._C._get_tracing_state() is not None
             or any((type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter)
                    or torch._C._functorch.is_functorch_wrapped_tensor(t) for t in tensors))

@@ -1,5 +1,5 @@
 """Whoever looks at the modules of the attention keeps seeing what passes through them: hooks, subclasses and replaced methods of
-the softmax module, hooks on ``CoreAttention`` in a layer with cached positions. On the CPU."""
+the softmax module, hooks on ``CoreAttention`` in a layer with cached positions, dispatch modes. On the CPU."""
 import pytest
 import torch
 
@@ -93,3 +93,15 @@ def test_a_watched_attention_takes_no_step_of_its_own():
     c.forward = lambda *a, **k: None
     assert not fused_attention.untouched(c, CoreAttention)
     assert not fused_attention.untouched(type("Own", (CoreAttention,), {})(64, 1, False, True, T.none, None), CoreAttention)
+
+
+def test_a_dispatch_mode_follows_what_is_done():
+    """Launches past torch would escape it: a count of operations, a trace over real tensors."""
+    from torch.utils.flop_counter import FlopCounterMode
+
+    from megatron.fused_kernels import _hotpath
+
+    t, c = torch.zeros(2), core()
+    assert not _hotpath.followed(t) and scale(c) is not None
+    with FlopCounterMode(display=False):
+        assert _hotpath.followed(t) and scale(c) is None

@@ -293,7 +293,7 @@ class CoreAttention(torch.nn.Module):
         by index where that would run its causal kernel, otherwise by the mask (forward only; with the fill value of the
         padding-mask kernel where that would run, and of the mask function where the torch branch would)."""
         scale = self._plain_scale(mask, key_lengths)
-        if scale is None or not fused_attention.supported(query, key, value):
+        if scale is None or fused_attention.recast(query) or not fused_attention.supported(query, key, value):
             return None
         softmax = self.scale_mask_softmax
         b, np_, sq, sk = query.size(1), query.size(2), query.size(0), key.size(0)
@@ -335,7 +335,7 @@ class CoreAttention(torch.nn.Module):
     def _cached_call(self, query, key, value, mask, layer_past):
         """``(mask, scale, fill)`` for the decoding kernel, or None where it does not apply."""
         scale = self._plain_scale(mask, None)
-        if scale is None or not fused_attention.decode_supported(query, key, value, layer_past):
+        if scale is None or fused_attention.recast(query) or not fused_attention.decode_supported(query, key, value, layer_past):
             return None
         (sq, b, np_, _), sk = query.shape, layer_past.size(1) + key.size(0)
         if self.use_cache and (mask.size(-1) > sk or mask.size(-2) > sk):

@@ -182,6 +182,11 @@ def untouched(module, cls):
                      or _has_any_global_hook()))
 
 
+def recast(t):
+    """Whether autocast would hand the products another type than that of ``t``."""
+    return torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") is not t.dtype
+
+
 def _cache_fits(key, value, past):
     """Whether these are 16-bit keys and values on one GPU, of one shape and a size that the kernels can address after ``past``
     cached positions."""

@@ -218,3 +218,23 @@ def test_a_hook_on_the_softmax_module_sees_the_probabilities():
     assert len(seen) == 1 and seen[0].shape == (2, 4, 128, 128) and core._one_kernel(q, k, v, mask, None, False) is not None
     # the products round the scores (up to 4, instead of a value of 1) once more
     assert rel_err(with_hook, without) <= 2.0 ** -7
+
+
+@pytest.mark.parametrize("s", [128, 77], ids=["causal", "by mask"])
+def test_autocast_to_another_type_keeps_its_result(s, monkeypatch):
+    """The products take the type that autocast gives them, and so does the result; to their own type it changes nothing."""
+    from megatron.model import fused_attention
+    from megatron.model.attention_core import CoreAttention
+    from megatron.model.fused_softmax import SoftmaxFusionTypes as T
+
+    core = CoreAttention(64, 1, True, False, T.upper_triang, lambda s, m: s.masked_fill_(m, -1e4), attention_softmax_in_fp32=True)
+    q, k, v = operands(torch.bfloat16, s, s, 1, 4, 4, 64, 1)
+    mask = hidden(s, s).view(1, 1, s, s)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert core._one_kernel(q, k, v, mask, None, False) is not None
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert core._one_kernel(q, k, v, mask, None, False) is None
+        got = core(q, k, v, mask)
+        monkeypatch.setattr(fused_attention, "supported", lambda *a: False)
+        want = core(q, k, v, mask)
+    assert got.dtype == want.dtype == torch.float16 and torch.equal(got, want)

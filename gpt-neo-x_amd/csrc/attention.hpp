@@ -178,7 +178,7 @@ struct TileLoader {
     // tile over. (A scalar write of m0 needs one wait state before its use here.)
     static __device__ __forceinline__ void issue(const char* tile, uint32_t offset, uint32_t dst)
     {
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(offset), "s"(tile) : "memory");
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(offset), "s"(tile) : "memory", "m0");
     }
 };
 
@@ -187,7 +187,7 @@ __device__ __forceinline__ void load_floats(const float* src, const char* dst, i
 {
     const uint32_t offset = min(lane, count - 1) * 4;
     const uint32_t d = __builtin_amdgcn_readfirstlane(lds_address(dst));
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(d), "v"(offset), "s"(src) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(d), "v"(offset), "s"(src) : "memory", "m0");
 }
 
 __device__ __forceinline__ float max_halves(float v)

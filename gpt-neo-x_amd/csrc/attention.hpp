@@ -83,6 +83,14 @@ struct Frag<NHP_F16> {
     }
 };
 
+// The 16 x 16 x 32 instruction, for few rows.
+template <int DT>
+__device__ __forceinline__ f32x4 mma16(u32x4 x, u32x4 y, f32x4 c)
+{
+    if constexpr (DT == NHP_BF16) return __builtin_amdgcn_mfma_f32_16x16x32_bf16(bitcast<bf16x8>(x), bitcast<bf16x8>(y), c, 0, 0, 0);
+    else return __builtin_amdgcn_mfma_f32_16x16x32_f16(bitcast<f16x8>(x), bitcast<f16x8>(y), c, 0, 0, 0);
+}
+
 // Geometry of a tile of 64 rows of HD elements in LDS.
 template <int HD>
 struct AttnGeo {

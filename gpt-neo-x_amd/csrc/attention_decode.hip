@@ -20,7 +20,6 @@
 
 namespace nhp {
 
-typedef float f32x4v __attribute__((ext_vector_type(4)));
 typedef uint32_t u32_byte __attribute__((aligned(1)));
 
 struct AttnDecodeArgs {
@@ -33,13 +32,6 @@ struct AttnDecodeArgs {
     float scale_log2, fill_log2;
     int batch, kv_heads, group, sq, past, splits, keys_per_split;
 };
-
-template <int DT>
-__device__ __forceinline__ f32x4v mma16(u32x4 x, u32x4 y, f32x4v c)
-{
-    if constexpr (DT == NHP_BF16) return __builtin_amdgcn_mfma_f32_16x16x32_bf16(bitcast<bf16x8>(x), bitcast<bf16x8>(y), c, 0, 0, 0);
-    else return __builtin_amdgcn_mfma_f32_16x16x32_f16(bitcast<f16x8>(x), bitcast<f16x8>(y), c, 0, 0, 0);
-}
 
 // Combines the lanes l, l ^ 16, l ^ 32, l ^ 48.
 template <typename Op>
@@ -107,14 +99,14 @@ __global__ void __launch_bounds__(256, NQ == 1 ? 3 : 2) attn_decode_kernel(AttnD
         else return base + (value_row(i) * st + value_col(i));
     };
 
-    f32x4v o[NQ][G::kTiles];
+    f32x4 o[NQ][G::kTiles];
     float m[NQ], l[NQ];
 #pragma unroll
     for (int n = 0; n < NQ; ++n) {
         m[n] = kFarBelow;
         l[n] = 0.0f;
 #pragma unroll
-        for (int d = 0; d < G::kTiles; ++d) o[n][d] = f32x4v{};
+        for (int d = 0; d < G::kTiles; ++d) o[n][d] = f32x4{};
     }
 
     for (int next = key_lo + wave * 32; next < key_hi; next += 128) {
@@ -182,7 +174,7 @@ __global__ void __launch_bounds__(256, NQ == 1 ? 3 : 2) attn_decode_kernel(AttnD
         u32x4 pf[NQ];
 #pragma unroll
         for (int n = 0; n < NQ; ++n) {
-            f32x4v s[2] = {f32x4v{}, f32x4v{}};
+            f32x4 s[2] = {f32x4{}, f32x4{}};
 #pragma unroll
             for (int t = 0; t < G::kSteps; ++t)
 #pragma unroll
@@ -244,7 +236,7 @@ __global__ void __launch_bounds__(256, NQ == 1 ? 3 : 2) attn_decode_kernel(AttnD
         __syncthreads();
         float* sums = reinterpret_cast<float*>(mine);
 #pragma unroll
-        for (int d = 0; d < G::kTiles; ++d) *reinterpret_cast<f32x4v*>(sums + r16 * G::kSumRow + d * 16 + 4 * g) = o[n][d];
+        for (int d = 0; d < G::kTiles; ++d) *reinterpret_cast<f32x4*>(sums + r16 * G::kSumRow + d * 16 + 4 * g) = o[n][d];
         __syncthreads();
         const int r = tid >> 4, c = tid & 15, row = n * 16 + r;
         if (c >= G::kChunks || row >= rows) continue;
@@ -267,8 +259,8 @@ __global__ void __launch_bounds__(256, NQ == 1 ? 3 : 2) attn_decode_kernel(AttnD
             *reinterpret_cast<u32x4*>(op + c * 8) = pack8<DT>(acc);
         } else {
             const int64_t at = ((int64_t)split * pairs + pair) * rows + row;
-            *reinterpret_cast<f32x4v*>(a.part_o + at * HD + c * 8) = f32x4v{acc[0], acc[1], acc[2], acc[3]};
-            *reinterpret_cast<f32x4v*>(a.part_o + at * HD + c * 8 + 4) = f32x4v{acc[4], acc[5], acc[6], acc[7]};
+            *reinterpret_cast<f32x4*>(a.part_o + at * HD + c * 8) = f32x4{acc[0], acc[1], acc[2], acc[3]};
+            *reinterpret_cast<f32x4*>(a.part_o + at * HD + c * 8 + 4) = f32x4{acc[4], acc[5], acc[6], acc[7]};
             if (c == 0) *reinterpret_cast<f32x2*>(a.part_ml + at * 2) = f32x2{big, total};
         }
     }
@@ -288,8 +280,8 @@ __global__ void __launch_bounds__(256) attn_decode_merge_kernel(AttnDecodeArgs a
         const int64_t at = s * count + at0;
         const float f = exp2_raw(a.part_ml[at * 2] - big);
         total = fmaf(a.part_ml[at * 2 + 1], f, total);
-        const f32x4v x = *reinterpret_cast<const f32x4v*>(a.part_o + at * HD + c * 8);
-        const f32x4v y = *reinterpret_cast<const f32x4v*>(a.part_o + at * HD + c * 8 + 4);
+        const f32x4 x = *reinterpret_cast<const f32x4*>(a.part_o + at * HD + c * 8);
+        const f32x4 y = *reinterpret_cast<const f32x4*>(a.part_o + at * HD + c * 8 + 4);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             acc[j] = fmaf(x[j], f, acc[j]);

@@ -15,8 +15,6 @@
 
 namespace nhp {
 
-typedef float f32x4v __attribute__((ext_vector_type(4)));
-
 struct LinearArgs {
     uint16_t* y;
     const uint16_t *x, *w, *bias;
@@ -26,13 +24,6 @@ struct LinearArgs {
 
 constexpr int kLinearWaves = 16, kLinearBlocks = 256, kLinearSteps = 8, kLinearPart = 4;
 constexpr int kLinearWhole = kLinearSteps * kLinearWaves * 32, kLinearSplits = 4;   // features of an unsplit product; splits beyond
-
-template <int DT>
-__device__ __forceinline__ f32x4v linear_mma(u32x4 a, u32x4 b, f32x4v c)
-{
-    if constexpr (DT == NHP_BF16) return __builtin_amdgcn_mfma_f32_16x16x32_bf16(bitcast<bf16x8>(a), bitcast<bf16x8>(b), c, 0, 0, 0);
-    else return __builtin_amdgcn_mfma_f32_16x16x32_f16(bitcast<f16x8>(a), bitcast<f16x8>(b), c, 0, 0, 0);
-}
 
 // MT: tiles of 16 rows of x
 template <int DT, int MT>
@@ -69,9 +60,9 @@ __global__ void __launch_bounds__(64 * kLinearWaves) linear_decode_kernel(Linear
 
     int buf = 0;
     for (int tile = first_tile; tile < tiles; tile += stride) {
-        f32x4v acc[MT];
+        f32x4 acc[MT];
 #pragma unroll
-        for (int r = 0; r < MT; ++r) acc[r] = f32x4v{};
+        for (int r = 0; r < MT; ++r) acc[r] = f32x4{};
 #pragma unroll
         for (int i = 0; i < kParts; ++i) {
             if (i + 1 < kParts) load(part[(i + 1) & 1], tile, (i + 1) * kLinearPart);
@@ -80,7 +71,7 @@ __global__ void __launch_bounds__(64 * kLinearWaves) linear_decode_kernel(Linear
             for (int s = 0; s < kLinearPart; ++s)
                 if (i * kLinearPart + s < count) {
 #pragma unroll
-                    for (int r = 0; r < MT; ++r) acc[r] = linear_mma<DT>(part[i & 1][s], x[r][i * kLinearPart + s], acc[r]);
+                    for (int r = 0; r < MT; ++r) acc[r] = mma16<DT>(part[i & 1][s], x[r][i * kLinearPart + s], acc[r]);
                 }
         }
 #pragma unroll
@@ -112,9 +103,9 @@ __global__ void __launch_bounds__(256) linear_merge_kernel(LinearArgs a)
 {
     const int64_t size = (int64_t)a.m * a.n, at = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
     if (at >= size) return;
-    f32x4v v{};
+    f32x4 v{};
 #pragma unroll
-    for (int s = 0; s < kLinearSplits; ++s) v += *reinterpret_cast<const f32x4v*>(a.parts + s * size + at);
+    for (int s = 0; s < kLinearSplits; ++s) v += *reinterpret_cast<const f32x4*>(a.parts + s * size + at);
     if (a.bias)
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[j] += Half2<DT>::from_bits(a.bias[(int)(at % a.n) + j]);

@@ -48,7 +48,7 @@ def operands(dtype, sq, sk, b, np_, nkv, hn, seed):
 
 @DTYPES
 @pytest.mark.parametrize("hn", [64, 80, 96, 128])
-@pytest.mark.parametrize("s,b,np_,nkv,window", [(20, 1, 4, 4, None), (64, 1, 4, 4, None), (65, 2, 4, 2, None), (128, 1, 8, 2, 1),
+@pytest.mark.parametrize("s,b,np_,nkv,window", [(20, 1, 4, 4, None), (2113, 1, 2, 1, None), (1600, 1, 3, 3, 700), (64, 1, 4, 4, None), (65, 2, 4, 2, None), (128, 1, 8, 2, 1),
                                                 (260, 3, 3, 3, None), (700, 1, 4, 1, 37), (513, 1, 9, 3, 128),
                                                 # shared heads: two of four, all four, all three in one workgroup
                                                 (65, 64, 16, 4, None), (65, 128, 16, 4, 7), (131, 64, 12, 4, None)])
@@ -71,6 +71,68 @@ def test_causal_forward_and_gradients(dtype, hn, s, b, np_, nkv, window):
     assert torch.equal(util.raw_bits(again.reshape(s, b, np_ * hn)), util.raw_bits(out.detach()))
 
 
+@DTYPES
+@pytest.mark.parametrize("hn", [64, 96])
+@pytest.mark.parametrize("sq,sk,b,np_,nkv,window", [(1, 2, 1, 4, 4, None), (1, 130, 2, 4, 2, 5), (63, 129, 1, 4, 4, None), (128, 192, 1, 8, 2, 64),
+                                                    (200, 1301, 1, 3, 1, None), (129, 1000, 2, 4, 4, 300), (500, 501, 1, 2, 2, 3)])
+def test_fewer_queries_than_keys(dtype, hn, sq, sk, b, np_, nkv, window):
+    """The queries are the last ones: query i attends to keys up to ``i + sk - sq``, forward and gradients; keys before every
+    window get none."""
+    from megatron.model.fused_attention import causal_attention
+
+    q, k, v = (t.requires_grad_(True) for t in operands(dtype, sq, sk, b, np_, nkv, hn, 61))
+    g = util.randn((b, np_, sq, hn), dtype, seed=9).to(DEV)
+    causal_attention(q, k, v, 1 / math.sqrt(hn), window).backward(g)
+    qr, kr, vr = (t.detach().float().requires_grad_(True) for t in (q, k, v))
+    ref = textbook(qr, kr, vr, hidden(sq, sk, window))
+    ref.backward(g.float().permute(2, 0, 1, 3))
+    out = causal_attention(q, k, v, 1 / math.sqrt(hn), window).permute(2, 0, 1, 3)
+    # one query has one score gradient for each key and head, whose rounding all features share: the largest and not the mean
+    # square of a rounding, a factor of sqrt(3)
+    few = math.sqrt(3) if sq == 1 else 1.0
+    assert rel_err(out, ref) <= limit(dtype, 2) * few
+    for got, want, n in ((q.grad, qr.grad, 6), (k.grad, kr.grad, 6), (v.grad, vr.grad, 2)):
+        assert rel_err(got, want) <= limit(dtype, n) * few
+    if window is not None and sk - sq - window > 0:
+        assert not k.grad[:sk - sq - window].any() and not v.grad[:sk - sq - window].any()
+
+
+def test_values_that_are_not_finite_stay_with_what_sees_them():
+    """In the causal kernels: a NaN in a query reaches that query, in a key the queries that see it, an infinite value one
+    feature of theirs; a NaN in the gradient of one context reaches its query and the keys that it sees. (Positions at the
+    edge of a tile: within one, a product with an exact zero spreads them, as the products over whole rows do.)"""
+    from megatron.model.fused_attention import causal_attention
+
+    def apart(value, *where):
+        expected = torch.zeros(value.shape, dtype=torch.bool, device=DEV)
+        for at in where:
+            expected[at] = True
+        assert torch.equal(~torch.isfinite(value), expected)
+
+    q, k, v = operands(torch.bfloat16, 200, 200, 1, 4, 2, 64, 71)
+    q2, k2, v2 = q.clone(), k.clone(), v.clone()
+    q2[70, 0, 1, 3], k2[90, 0, 1, 5], v2[128, 0, 0, 7] = float("nan"), float("nan"), float("inf")
+    out = causal_attention(q2, k2, v2, 1 / 8, merged=True).view(200, 1, 4, 64)
+    apart(out, (70, 0, 1), (slice(90, None), 0, slice(2, 4)), (slice(128, None), 0, slice(0, 2), 7))
+    # a score of -inf: that key counts for nothing
+    q3, k3 = q.clone(), k.clone()
+    q3[..., 0] = q3[..., 0].abs() + 0.125
+    k3[50, 0, 1, 0] = float("-inf")
+    out = causal_attention(q3, k3, v, 1 / 8, merged=True).view(200, 1, 4, 64)
+    mask = hidden(200, 200).expand(1, 4, 200, 200).clone()
+    mask[:, 2:, :, 50] = True
+    k3[50, 0, 1, 0] = 0.0
+    want = textbook(q3, k3, v, mask)
+    assert rel_err(out, want) <= limit(torch.bfloat16, 2)
+    leaves = [t.requires_grad_(True) for t in (q, k, v)]
+    g = util.randn((200, 1, 4, 64), torch.bfloat16, seed=9).to(DEV)
+    g[127, 0, 3, 9] = float("nan")
+    causal_attention(*leaves, 1 / 8, merged=True).backward(g.view(200, 1, 256))
+    apart(q.grad, (127, 0, 3))
+    apart(k.grad, (slice(0, 128), 0, 1))
+    apart(v.grad, (slice(0, 128), 0, 1, 9))
+
+
 @pytest.mark.parametrize("b", [1, 64, 128], ids=["apart", "in pairs", "together"])
 def test_gradients_of_shared_heads_are_summed_before_they_are_rounded(b):
     """A query head's part may lie beyond the range of fp16 where the sum does not. With q, k and v zero the probabilities are
@@ -90,7 +152,8 @@ def test_gradients_of_shared_heads_are_summed_before_they_are_rounded(b):
 
 @DTYPES
 @pytest.mark.parametrize("hn", [64, 80, 128])
-@pytest.mark.parametrize("sq,sk,b,np_,nkv", [(1, 1, 1, 4, 4), (1, 200, 2, 4, 2), (5, 64, 1, 4, 4), (130, 333, 2, 4, 4)])
+@pytest.mark.parametrize("sq,sk,b,np_,nkv", [(1, 1, 1, 4, 4), (1, 200, 2, 4, 2), (5, 64, 1, 4, 4), (130, 333, 2, 4, 4), (1531, 1531, 1, 2, 1),
+                                             (300, 4100, 1, 2, 2)])
 def test_masked_forward(dtype, hn, sq, sk, b, np_, nkv):
     """Random masks, a whole tile hidden from every query, and rows that see nothing: those are averages over all keys."""
     from megatron.model.fused_attention import masked_attention

@@ -12,11 +12,12 @@
 // The gradients take two kernels, one over blocks of queries (gradient of q) and one over blocks of keys (of k and v),
 // each recomputing the scores: seven products instead of five, but no atomic sums, so results are the same on every run.
 //
-// Measured (us, causal, forward / backward; products and softmax separately before, both per pass of the module):
-//   [8192, 1, 32 heads, 8 of keys, 128] bf16   544 / 1770 (1011 / 1087 TFLOP/s)   whole pass 5786 -> 2322
+// Measured (us, causal, forward / backward; products and softmax separately before, both per pass of the module; cards differ
+// by up to 8 %):
+//   [8192, 1, 32 heads, 8 of keys, 128] bf16   591 / 1876 (931 / 1026 TFLOP/s)   whole pass 5786 -> 2357
 //   [2048, 8, 16, 128] bf16                    175 / 585  (788 / 823)            about 1930 -> 890
-//   [1024, 4, 12, 64] fp16                     26 / 65    (251 / 350)            whole pass 428 -> 172
-//   [1531, 1, 32, 128] bf16, by mask           57 + 7 for the bits               650 -> 60
+//   [1024, 4, 12, 64] fp16                     29 / 73    (224 / 312)            whole pass 428 -> 126 to 163, with the host
+//   [1531, 1, 32, 128] bf16, by mask           68 + 5 for the bits               650 -> 73
 #include "attention.hpp"
 
 namespace nhp {

@@ -247,7 +247,7 @@ def _fill_value(mask_func, dtype=torch.float32):
     """The value that ``mask_func(scores, mask)`` puts in place of masked scores of ``dtype`` if that is what it does, leaving
     the others alone, and if it is finite and no higher than -10000; otherwise None.
 
-    It is asked again for every call that relies on the answer (about 10 us): a function may be anything, and behave
+    It is asked again for every call that relies on the answer (10 to 15 us): a function may be anything, and behave
     differently from one call to the next."""
     try:
         filled = mask_func(_TRIAL[dtype].clone(), _TRIAL_HIDDEN.clone()).tolist()   # (it may write into either)

@@ -176,8 +176,9 @@ def _methods(cls):
 
 def untouched(module, cls):
     """Whether ``module`` is a ``cls`` as it stands: no subclass, none of its methods replaced, no hooks. Whoever put such a
-    thing there wants the tensors that pass through the module, so it has to be called, with those tensors."""
-    return (type(module) is cls and module.__dict__.keys().isdisjoint(_methods(cls))
+    thing there wants the tensors that pass through the module, so it has to be called, with those tensors; so does torch
+    while it compiles."""
+    return (not torch.compiler.is_compiling() and type(module) is cls and module.__dict__.keys().isdisjoint(_methods(cls))
             and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
                      or _has_any_global_hook()))
 

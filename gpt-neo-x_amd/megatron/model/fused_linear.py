@@ -23,6 +23,8 @@ features called step by step takes 222 us here and 272 to 282 with those product
 to 2000 positions, and 16 of 200. Where the GPU is what is waited for the library is ahead there: 16 sequences of 2000 positions
 336 / 320 us, and in a captured graph 71 / 76 us with one sequence, 90 / 91 with four, 195 / 176 with eight of 2000, 336 / 314
 with 16. With 4096 features, 8 heads of keys: 247 / 274 us step by step, 178 / 175 in a graph (16 of 2000)."""
+from typing import Optional
+
 import torch
 import torch.nn.functional as F
 
@@ -46,10 +48,19 @@ def _few_rows(x, weight, bias):
             and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
 
 
-def linear(x, weight, bias=None):
+def linear(x, weight, bias: Optional[torch.Tensor] = None):
     """``torch.nn.functional.linear``; in inference with few rows of a 16-bit type by one kernel (two with more than 4096
-    features)."""
-    if weight.dim() != 2 or not _few_rows(x, weight, bias):
+    features). Scripted, compiled, exported or traced over proxies it is torch's: the sizes below would become conditions."""
+    if torch.jit.is_scripting():
+        return F.linear(x, weight, bias)
+    else:
+        return _linear(x, weight, bias)
+
+
+@torch.jit.unused
+def _linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> torch.Tensor:
+    if (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None or not isinstance(x, torch.Tensor)
+            or not isinstance(weight, torch.Tensor) or weight.dim() != 2 or not _few_rows(x, weight, bias)):
         return F.linear(x, weight, bias)
     n, k = weight.shape
     rows = x.numel() // k

@@ -1,5 +1,8 @@
 """Whoever looks at the modules of the attention keeps seeing what passes through them: hooks, subclasses and replaced methods of
-the softmax module, hooks on ``CoreAttention`` in a layer with cached positions, dispatch modes. On the CPU."""
+the softmax module, hooks on ``CoreAttention`` in a layer with cached positions, dispatch modes,
+tracers and compilers. On the CPU."""
+import types
+
 import pytest
 import torch
 
@@ -63,16 +66,18 @@ def test_the_switch_for_tools_that_inspect_the_tensors():
     assert scale(core(causal_gemm_blocks=False)) is None
 
 
-def test_a_hook_on_the_attention_of_a_layer_with_cached_positions():
-    """It fires once a step, with the keys of all positions and the context."""
-    import types
-
+def cpu_attention(use_cache, num_kv_heads=None):
     from megatron.model.transformer_layer import SelfAttention
 
-    args = types.SimpleNamespace(hidden_size=128, num_attention_heads=2, num_kv_heads=None, seq_length=16, precision="fp32", pos_emb="rotary",
-                                 rotary_pct=1.0, rope_fusion=False, attention_softmax_in_fp32=False, attention_dropout=0.0,
+    args = types.SimpleNamespace(hidden_size=128, num_attention_heads=2, num_kv_heads=num_kv_heads, seq_length=16, precision="fp32",
+                                 pos_emb="rotary", rotary_pct=1.0, rope_fusion=False, attention_softmax_in_fp32=False, attention_dropout=0.0,
                                  scaled_upper_triang_masked_softmax_fusion=False, scaled_masked_softmax_fusion=False)
-    attention = SelfAttention(args, fb.fill_masked_with_dtype_min, 1, rotary=True, use_cache=True)
+    return SelfAttention(args, lambda s, m: s.masked_fill(m, -10000.0), 1, rotary=True, use_cache=use_cache)
+
+
+def test_a_hook_on_the_attention_of_a_layer_with_cached_positions():
+    """It fires once a step, with the keys of all positions and the context."""
+    attention = cpu_attention(use_cache=True)
     seen = []
     attention.core.register_forward_hook(lambda module, inputs, out: seen.append((inputs[1].size(0), tuple(out.shape))))
     x, mask = torch.randn(5, 1, 128), fb.causal_mask(5)
@@ -105,3 +110,26 @@ def test_a_dispatch_mode_follows_what_is_done():
     assert not _hotpath.followed(t) and scale(c) is not None
     with FlopCounterMode(display=False):
         assert _hotpath.followed(t) and scale(c) is None
+
+
+@pytest.mark.parametrize("skip_bias_add", [False, True])
+def test_a_linear_layer_can_be_traced_scripted_and_exported(skip_bias_add):
+    from megatron.model.transformer_layer import Linear
+
+    layer, x = Linear(64, 32, skip_bias_add=skip_bias_add), torch.randn(5, 64)
+    want = layer(x)
+    exported = torch.export.export(layer, (x,), dynamic_shapes={"x": {0: torch.export.Dim("rows", min=2, max=4096)}}).module()
+    for other in (torch.fx.symbolic_trace(layer), torch.jit.script(layer), exported):
+        for got, expected in zip(other(x), want):
+            assert got is expected or torch.equal(got, expected)
+
+
+@pytest.mark.parametrize("past", [None, 3])
+def test_a_layer_attention_compiles_whole(past):
+    attention = cpu_attention(use_cache=True, num_kv_heads=1).eval()
+    cached = None if past is None else torch.randn(2, past, 1, 1, 64)
+    args = torch.randn(4, 1, 128), torch.zeros((1, 1, 4, 4 + (past or 0)), dtype=torch.bool), cached
+    with torch.no_grad():
+        (want, want_present), _ = attention(*args)
+        (got, present), _ = torch.compile(attention, fullgraph=True, backend="eager")(*args)
+    assert torch.allclose(got, want, atol=1e-6) and torch.equal(present, want_present)

@@ -28,14 +28,20 @@ def _strides(t):
 
 def _readable(t):
     """``t``, or a copy where the kernels cannot read it: they want contiguous features and 16-byte aligned rows."""
-    s = _strides(t)
-    if t.stride(3) == 1 and (s[0] | s[1] | s[2]) % 8 == 0 and t.data_ptr() % 16 == 0 and s[0] < 1 << 24:
-        return t
-    return t.clone(memory_format=torch.contiguous_format)
+    return _operand(t)[0]
 
 
 def _strides3(t):
     return _I64x3(*_strides(t))
+
+
+def _operand(t):
+    """``_readable`` and the strides that the entry points take."""
+    s = _strides(t)
+    if t.stride(3) == 1 and (s[0] | s[1] | s[2]) % 8 == 0 and t.data_ptr() % 16 == 0 and s[0] < 1 << 24:
+        return t, _I64x3(*s)
+    t = t.clone(memory_format=torch.contiguous_format)
+    return t, _strides3(t)
 
 
 def supported(q, k, v):
@@ -81,15 +87,15 @@ def _new_context(q, merged):
     return torch.empty((b, np_, sq, hn), dtype=q.dtype, device=q.device), _I64x3(hn, np_ * sq * hn, sq * hn)
 
 
-def _launch(out, out_strides, kept, lse, q, k, v, bits, mask_batches, fill, scale, window, who):
-    """``out`` and ``out_strides`` from ``_new_context``; ``kept`` laid out like ``out``, or None."""
+def _launch(out, out_strides, kept, lse, q, k, v, strides, bits, mask_batches, fill, scale, window, who):
+    """``out`` and ``out_strides`` from ``_new_context``, ``kept`` laid out like ``out``, or None; q, k, v and ``strides`` from
+    ``_operand``."""
     sq, b, np_, hn = q.shape
     with _hp.device_guard(q):
         rc = _hp.lib().nhp_attention_fwd_keep(
             out.data_ptr(), None if kept is None else kept.data_ptr(), None if lse is None else lse.data_ptr(), q.data_ptr(),
             k.data_ptr(), v.data_ptr(), None if bits is None else bits.data_ptr(), mask_batches, fill, scale,
-            -1 if window is None else window, b, np_, k.size(2), sq, k.size(0), hn, _strides3(q), _strides3(k), _strides3(v),
-            out_strides, _hp.dtype_code(q, who), _hp.stream_of(q))
+            -1 if window is None else window, b, np_, k.size(2), sq, k.size(0), hn, *strides, out_strides, _hp.dtype_code(q, who), _hp.stream_of(q))
     _hp.check(rc, who)
 
 
@@ -103,12 +109,12 @@ class CausalAttention(torch.autograd.Function):
     def forward(ctx, q, k, v, scale, window, merged, checked=False):
         """``checked``: the caller has asked ``supported`` already (twice would cost a short call 8 of 155 us)."""
         _refuse_unless(checked or supported(q, k, v), "CausalAttention", q, k, v)
-        q, k, v = _readable(q), _readable(k), _readable(v)
+        (q, q_strides), (k, k_strides), (v, v_strides) = _operand(q), _operand(k), _operand(v)
         out, out_strides = _new_context(q, merged)
         need = any(ctx.needs_input_grad[:3])
         kept = torch.empty_like(out) if need else None
         lse = torch.empty((q.size(1) * q.size(2), q.size(0)), dtype=torch.float32, device=q.device) if need else None
-        _launch(out, out_strides, kept, lse, q, k, v, None, 1, 0.0, scale, window, "CausalAttention")
+        _launch(out, out_strides, kept, lse, q, k, v, (q_strides, k_strides, v_strides), None, 1, 0.0, scale, window, "CausalAttention")
         if need:
             ctx.save_for_backward(q, k, v, kept, lse)
             ctx.conf = (scale, window, merged, out_strides)
@@ -117,11 +123,14 @@ class CausalAttention(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad):
         who = "CausalAttention backward"
+        # (a hook on saved tensors may hand them back laid out otherwise)
         q, k, v, out, lse = ctx.saved_tensors
+        (q, q_strides), (k, k_strides), (v, v_strides) = _operand(q), _operand(k), _operand(v)
+        out, lse = out.contiguous(), lse.contiguous()
         scale, window, merged, out_strides = ctx.conf
         sq, b, np_, hn = q.shape
         sk, nkv = k.size(0), k.size(2)
-        g = _readable(grad.reshape(sq, b, np_, hn) if merged else grad.permute(2, 0, 1, 3))
+        g, g_strides = _operand(grad.reshape(sq, b, np_, hn) if merged else grad.permute(2, 0, 1, 3))
         dq, dk, dv = torch.empty_like(q, memory_format=torch.contiguous_format), torch.empty_like(
             k, memory_format=torch.contiguous_format), torch.empty_like(v, memory_format=torch.contiguous_format)
         lib = _hp.lib()
@@ -130,8 +139,8 @@ class CausalAttention(torch.autograd.Function):
             rc = lib.nhp_attention_bwd(
                 dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), g.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
                 out.data_ptr(), lse.data_ptr(), workspace.data_ptr(), scale, -1 if window is None else window, b, np_, nkv,
-                sq, sk, hn, _strides3(dq), _strides3(dk), _strides3(dv), _strides3(g), _strides3(q), _strides3(k), _strides3(v),
-                out_strides, _hp.dtype_code(q, who), _hp.stream_of(q))
+                sq, sk, hn, _strides3(dq), _strides3(dk), _strides3(dv), g_strides, q_strides, k_strides, v_strides, out_strides,
+                _hp.dtype_code(q, who), _hp.stream_of(q))
         _hp.check(rc, who)
         needs = ctx.needs_input_grad
         return dq if needs[0] else None, dk if needs[1] else None, dv if needs[2] else None, None, None, None, None
@@ -149,7 +158,7 @@ def masked_attention(q, k, v, mask, scale, fill, merged=False):
     replaced by ``fill`` after scaling."""
     _refuse_unless(supported(q, k, v) and mask_supported(mask, q.size(1), q.size(0), k.size(0), q.device), "masked_attention",
                    q, k, v, mask)
-    q, k, v = _readable(q), _readable(k), _readable(v)
+    (q, q_strides), (k, k_strides), (v, v_strides) = _operand(q), _operand(k), _operand(v)
     sq, sk = q.size(0), k.size(0)
     mask = mask.contiguous()
     bits = torch.empty((mask.size(0), sq, (sk + 63) // 64), dtype=torch.int64, device=q.device)
@@ -157,7 +166,7 @@ def masked_attention(q, k, v, mask, scale, fill, merged=False):
     with _hp.device_guard(q):
         rc = _hp.lib().nhp_attention_mask_bits(bits.data_ptr(), mask.data_ptr(), mask.size(0), sq, sk, _hp.stream_of(q))
     _hp.check(rc, "masked_attention")
-    _launch(out, out_strides, None, None, q, k, v, bits, mask.size(0), fill, float(scale), None, "masked_attention")
+    _launch(out, out_strides, None, None, q, k, v, (q_strides, k_strides, v_strides), bits, mask.size(0), fill, float(scale), None, "masked_attention")
     return out
 
 

@@ -301,3 +301,26 @@ def test_autocast_to_another_type_keeps_its_result(s, monkeypatch):
         monkeypatch.setattr(fused_attention, "supported", lambda *a: False)
         want = core(q, k, v, mask)
     assert got.dtype == want.dtype == torch.float16 and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("merged", [True, False], ids=["merged", "bnsh"])
+def test_hooks_on_saved_tensors(merged):
+    """They may keep them anywhere and hand them back in another layout: the same gradients, bit for bit."""
+    from megatron.model.fused_attention import causal_attention
+
+    def elsewhere(t):
+        return t.cpu().transpose(0, -1).contiguous()   # the last dimension outermost
+
+    g = None
+    results = []
+    for hooks in (None, (elsewhere, lambda t: t.to(DEV).transpose(0, -1))):
+        leaves = [t.requires_grad_(True) for t in operands(torch.bfloat16, 136, 136, 2, 8, 2, 64, 1)]
+        if hooks is None:
+            out = causal_attention(*leaves, 1 / 8, merged=merged)
+            g = util.randn(tuple(out.shape), torch.bfloat16, seed=9).to(DEV)
+        else:
+            with torch.autograd.graph.saved_tensors_hooks(*hooks):
+                out = causal_attention(*leaves, 1 / 8, merged=merged)
+        out.backward(g)
+        results.append([util.raw_bits(leaf.grad) for leaf in leaves])
+    assert all(torch.equal(a, b) for a, b in zip(*results))

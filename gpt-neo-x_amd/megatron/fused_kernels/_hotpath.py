@@ -164,14 +164,21 @@ def require_gpu(t, what):
         raise RuntimeError(f"{what}: expected a tensor on the GPU, got device {t.device}")
 
 
+# (looked up once: a decoding layer asks a dozen times and waits for the host)
+_is_compiling, _tracing_state, _dispatch_modes = torch.compiler.is_compiling, torch._C._get_tracing_state, torch._C._len_torch_dispatch_stack
+_forward_ad, _is_wrapped = torch.autograd.forward_ad, torch._C._functorch.is_functorch_wrapped_tensor
+
+
 def followed(*tensors):
     """Whether torch follows the operations on any of these beyond autograd (vmap and the other function transforms,
     forward-mode derivatives, tracing, compilation, dispatch modes such as a counter of operations, tensor subclasses): a
     launch outside of an autograd function would escape it."""
-    return (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0 or torch.autograd.forward_ad._current_level >= 0
-            or torch._C._get_tracing_state() is not None
-            or any((type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter)
-                   or torch._C._functorch.is_functorch_wrapped_tensor(t) for t in tensors))
+    if _is_compiling() or _dispatch_modes() > 0 or _forward_ad._current_level >= 0 or _tracing_state() is not None:
+        return True
+    for t in tensors:
+        if (type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter) or _is_wrapped(t):
+            return True
+    return False
 
 
 # torch's direct accessor of the current stream's handle (what its own launchers use): about a microsecond

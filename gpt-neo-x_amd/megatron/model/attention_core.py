@@ -304,17 +304,18 @@ class CoreAttention(torch.nn.Module):
         fill = self._fill_by_mask(mask, b, np_, sq, sk, query.device) if fused_attention.plain(query, key, value) else None
         if fill is None:
             return None
-        return fused_attention.masked_attention(query, key, value, mask, scale, fill, merged_heads)
+        return fused_attention.masked_attention(query, key, value, mask, scale, fill, merged_heads, checked=True)
 
     def _plain_scale(self, mask, key_lengths):
         """The factor of the scores where they are scaled, masked and nothing else, and nobody looks at them or at the
         probabilities; otherwise None."""
         softmax = self.scale_mask_softmax
-        if (not (self.causal_gemm_blocks and fused_attention.untouched(softmax, FusedScaleMaskSoftmax))
+        if (not self.causal_gemm_blocks or mask is None or key_lengths is not None or self.rpe is not None
+                or not fused_attention.untouched(softmax, FusedScaleMaskSoftmax)
                 or torch._C._len_torch_dispatch_stack() > 0):   # a dispatch mode sees the products, not a launch
             return None
-        if (key_lengths is not None or self.rpe is not None or softmax.alibi_slopes is not None or not softmax.fusion
-                or softmax.narrow_forward_scale or mask is None or (softmax.training and softmax.attention_dropout > 0.0)):
+        if (softmax.alibi_slopes is not None or not softmax.fusion or softmax.narrow_forward_scale
+                or (softmax.training and softmax.attention_dropout > 0.0)):
             return None
         if not softmax.input_in_float16:
             return None

@@ -153,11 +153,11 @@ def causal_attention(q, k, v, scale, window=None, merged=False, checked=False):
     return CausalAttention.apply(q, k, v, float(scale), window, merged, checked)
 
 
-def masked_attention(q, k, v, mask, scale, fill, merged=False):
+def masked_attention(q, k, v, mask, scale, fill, merged=False, checked=False):
     """Inference only: the context under a boolean mask ``[1 or b, 1, sq, sk]`` (True = masked), whose scores are
-    replaced by ``fill`` after scaling."""
-    _refuse_unless(supported(q, k, v) and mask_supported(mask, q.size(1), q.size(0), k.size(0), q.device), "masked_attention",
-                   q, k, v, mask)
+    replaced by ``fill`` after scaling. ``checked``: the caller has asked ``supported`` and ``mask_supported`` already."""
+    _refuse_unless(checked or supported(q, k, v) and mask_supported(mask, q.size(1), q.size(0), k.size(0), q.device),
+                   "masked_attention", q, k, v, mask)
     (q, q_strides), (k, k_strides), (v, v_strides) = _operand(q), _operand(k), _operand(v)
     sq, sk = q.size(0), k.size(0)
     mask = mask.contiguous()
@@ -187,8 +187,9 @@ def untouched(module, cls):
     """Whether ``module`` is a ``cls`` as it stands: no subclass, none of its methods replaced, no hooks. Whoever put such a
     thing there wants the tensors that pass through the module, so it has to be called, with those tensors; so does torch
     while it compiles."""
-    return (not torch.compiler.is_compiling() and type(module) is cls and module.__dict__.keys().isdisjoint(_methods(cls))
-            and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
+    own = module.__dict__
+    return (not _hp._is_compiling() and type(module) is cls and own.keys().isdisjoint(_methods(cls))
+            and not (own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or own["_backward_pre_hooks"]
                      or _has_any_global_hook()))
 
 
@@ -229,13 +230,14 @@ def _past_fits(key, value, past_key, past_value):
             and _continues(past_key, key) and _continues(past_value, key))
 
 
-def append_to_cache(key, value, layer_past):
-    """``torch.stack((cat(past keys, key), cat(past values, value)))`` in one launch: ``[2, past + sq, b, nkv, hn]``."""
+def append_to_cache(key, value, layer_past, checked=False):
+    """``torch.stack((cat(past keys, key), cat(past values, value)))`` in one launch: ``[2, past + sq, b, nkv, hn]``.
+    ``checked``: the caller has asked ``cache_supported`` already."""
     past_k, past_v = (None, None) if layer_past is None else layer_past
     if layer_past is None:
-        _refuse_unless(_cache_fits(key, value, 0), "append_to_cache", key, value)
+        _refuse_unless(checked or _cache_fits(key, value, 0), "append_to_cache", key, value)
     else:
-        _refuse_unless(_past_fits(key, value, past_k, past_v), "append_to_cache", key, value, past_k, past_v)
+        _refuse_unless(checked or _past_fits(key, value, past_k, past_v), "append_to_cache", key, value, past_k, past_v)
         past_k, past_v = _readable(past_k), _readable(past_v)
     key, value = _readable(key), _readable(value)
     past = 0 if past_k is None else past_k.size(0)

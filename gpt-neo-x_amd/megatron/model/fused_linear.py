@@ -38,13 +38,13 @@ MAX_FEATURES = 16384
 
 def _few_rows(x, weight, bias):
     n, k = weight.shape
+    dtype = x.dtype
     return (x.numel() <= (MAX_ROWS_NARROW if min(n, k) <= 2048 else MAX_ROWS) * k and x.is_cuda and x.dim() > 0 and x.size(-1) == k and x.numel() > 0
-            and x.dtype in (torch.bfloat16, torch.float16) and weight.dtype == x.dtype and weight.device == x.device
+            and (dtype is torch.bfloat16 or dtype is torch.float16) and weight.dtype is dtype and weight.device == x.device
             and k % 32 == 0 and k <= MAX_FEATURES and n % 16 == 0 and 0 < n <= 1 << 24 and weight.is_contiguous()
             and x.is_contiguous()
-            and (bias is None or (bias.dtype == x.dtype and bias.device == x.device and bias.shape == (n,) and bias.is_contiguous()
-                                  and plain(bias)))
-            and plain(x, weight) and not torch.is_autocast_enabled("cuda")
+            and (bias is None or (bias.dtype is dtype and bias.device == x.device and bias.shape == (n,) and bias.is_contiguous()))
+            and (plain(x, weight) if bias is None else plain(x, weight, bias)) and not torch.is_autocast_enabled("cuda")
             and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
 
 
@@ -59,8 +59,8 @@ def linear(x, weight, bias: Optional[torch.Tensor] = None):
 
 @torch.jit.unused
 def _linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> torch.Tensor:
-    if (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None or not isinstance(x, torch.Tensor)
-            or not isinstance(weight, torch.Tensor) or weight.dim() != 2 or not _few_rows(x, weight, bias)):
+    if (_hp._is_compiling() or _hp._tracing_state() is not None or not isinstance(x, torch.Tensor) or not isinstance(weight, torch.Tensor)
+            or weight.dim() != 2 or not _few_rows(x, weight, bias)):
         return F.linear(x, weight, bias)
     n, k = weight.shape
     rows = x.numel() // k

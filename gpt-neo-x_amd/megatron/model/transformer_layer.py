@@ -159,7 +159,7 @@ class SelfAttention(torch.nn.Module):
             context, present = fused_attention.checked_decode_attention(query, key, value, past, *call, merged=True)
         else:
             if self.use_cache and fused_attention.cache_supported(key, value, past):
-                present = fused_attention.append_to_cache(key, value, past)
+                present = fused_attention.append_to_cache(key, value, past, checked=True)
                 if past is not None:
                     key, value = present
             else:

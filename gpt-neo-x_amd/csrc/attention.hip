@@ -539,7 +539,7 @@ __global__ void __launch_bounds__(256) attn_group_sum_kernel(AttnBwdArgs a, int 
 // 2048, and 1024 beyond (where the products outweigh the rest). Both kernels, us, fold 1 / 2 / 4 of a group of 4, 128 features:
 //   [1024, 8, 16 heads] 240 / 217 / 256 (1024 / 512 / 256 workgroups), [1024, 16, 16] 435 / 403 / 365,
 //   [2048, 8, 16] 651 / 657 / 658 (2048 / 1024 / 512), [4096, 4, 16] 1094 / 1142 / 1240, [4096, 8, 16] 2151 / 2071 / 2177,
-//   [8192, 1, 32] 1886 / 1865 / 2226 (2048 / 1024 / 512), [8192, 4, 16] 3795 / 3736 / 3714, [512, 1, 32] 52 / 58 / 75.
+//   [8192, 1, 32] 1886 / 1865 / 2226 (2048 / 1024 / 512), [8192, 4, 16] 3795 / 3736 / 3714, [300, 1, 32] 44 / 55 / 76.
 static int bwd_fold(int64_t batch, int64_t heads, int64_t kv_heads, int64_t sk)
 {
     const int64_t group = heads / kv_heads, blocks = batch * heads * ((sk + kFwdRows - 1) / kFwdRows);

@@ -36,12 +36,9 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_kernel(AttnFwdArgs a)
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int ql = lane & 31, half = lane >> 5;
 
-    // workgroups of one head stay on one XCD (its K and V then live in that L2), long rows first
     const int nqb = (a.sq + kFwdRows - 1) / kFwdRows;
-    const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
-    const int bh = xcd * a.heads_per_xcd + idx / nqb;
-    if (bh >= a.batch * a.heads) return;
-    const int qb = nqb - 1 - idx % nqb;
+    const Place at_block = place(a.batch * a.heads);
+    const int bh = at_block.unit, qb = nqb - 1 - at_block.block;
     const int b = bh / a.heads, h = bh % a.heads, hk = h / a.group;
     const int q0 = qb * kFwdRows, qw = q0 + wave * 32;
     const int qi = min(qw + ql, a.sq - 1);
@@ -239,7 +236,7 @@ template <int DT, int HD>
 static int launch_fwd(const AttnFwdArgs& a, int mode, hipStream_t st)
 {
     const int64_t nqb = (a.sq + kFwdRows - 1) / kFwdRows;
-    const int64_t grid = 8 * (int64_t)a.heads_per_xcd * nqb;
+    const int64_t grid = (int64_t)a.batch * a.heads * nqb;
     if (!grid_fits(grid, 256)) return NHP_ERR_SHAPE;
     launch_prepare();
     if (mode == kCausal)
@@ -273,10 +270,8 @@ __global__ void __launch_bounds__(256, 2) attn_dq_kernel(AttnBwdArgs a)
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int ql = lane & 31, half = lane >> 5;
     const int nqb = (a.sq + kFwdRows - 1) / kFwdRows;
-    const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
-    const int bh = xcd * a.heads_per_xcd + idx / nqb;
-    if (bh >= a.batch * a.heads) return;
-    const int qb = nqb - 1 - idx % nqb;
+    const Place at_block = place(a.batch * a.heads);
+    const int bh = at_block.unit, qb = nqb - 1 - at_block.block;
     const int b = bh / a.heads, h = bh % a.heads, hk = h / a.group;
     const int q0 = qb * kFwdRows, qw = q0 + wave * 32;
     const int qi = min(qw + ql, a.sq - 1);
@@ -390,12 +385,11 @@ __global__ void __launch_bounds__(256, 2) attn_dkv_kernel(AttnBwdArgs a)
     char* const stats = lds + 4 * G::kTileBytes;   // [2 buffers][lse, delta][64]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int kl = lane & 31, half = lane >> 5;
-    const int nkb = (a.sk + kFwdRows - 1) / kFwdRows;
-    const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
-    const int units = a.heads / a.fold, unit = xcd * a.heads_per_xcd + idx / nkb;   // (batch entry, `fold` heads)
-    if (unit >= a.batch * units) return;
+    const int units = a.heads / a.fold;
+    const Place at_block = place(a.batch * units);   // (batch entry, `fold` heads); the first keys are seen by most queries
+    const int unit = at_block.unit;
     const int b = unit / units, h0 = unit % units * a.fold, hk = h0 / a.group;
-    const int k0 = (idx % nkb) * kFwdRows, kw = k0 + wave * 32;
+    const int k0 = at_block.block * kFwdRows, kw = k0 + wave * 32;
     const int ki = min(kw + kl, a.sk - 1);
 
     const uint16_t* kp = a.k + b * a.k_b + hk * a.k_h + (int64_t)ki * a.k_s + half * 8;
@@ -535,15 +529,16 @@ __global__ void __launch_bounds__(256) attn_group_sum_kernel(AttnBwdArgs a, int 
 // Query heads that a workgroup of the second gradient kernel goes over: as many as leave enough workgroups. Every head that is
 // not added up in registers costs 8 bytes written and read again per element of k and v, but causal key blocks differ in
 // length by up to a factor of 2 * blocks, and with few workgroups the longest one is what the launch takes. Two workgroups
-// fit on a CU: 512 at once, which is enough where a row is at most eight blocks long, between 1024 and 8192 keys it takes
-// 2048, and 1024 beyond (where the products outweigh the rest). Both kernels, us, fold 1 / 2 / 4 of a group of 4, 128 features:
-//   [1024, 8, 16 heads] 240 / 217 / 256 (1024 / 512 / 256 workgroups), [1024, 16, 16] 435 / 403 / 365,
-//   [2048, 8, 16] 651 / 657 / 658 (2048 / 1024 / 512), [4096, 4, 16] 1094 / 1142 / 1240, [4096, 8, 16] 2151 / 2071 / 2177,
-//   [8192, 1, 32] 1886 / 1865 / 2226 (2048 / 1024 / 512), [8192, 4, 16] 3795 / 3736 / 3714, [300, 1, 32] 44 / 55 / 76.
+// fit on a CU: 512 at once, which is enough where a row is at most eight blocks long; beyond, twice that. All kernels of the
+// backward, us, fold 1 / 2 / 4 of a group of 4, 128 features:
+//   [1024, 4, 32 heads] 198 / 183 / 239 (1024 / 512 / 256 workgroups), [1024, 16, 16] 405 / 327 / 318,
+//   [2048, 1, 32] 181 / 249 / 401 (512 / 256 / 128), [2048, 8, 16] 569 / 515 / 570 (2048 / 1024 / 512),
+//   [4096, 1, 32] 497 / 577 / 862, [4096, 2, 32 of 80] 678 / 677 / 748, [8192, 1, 32] 1743 / 1727 / 2144,
+//   [8192, 4, 16] 3545 / 3478 / 3513, [300, 1, 32] 44 / 55 / 77.
 static int bwd_fold(int64_t batch, int64_t heads, int64_t kv_heads, int64_t sk)
 {
     const int64_t group = heads / kv_heads, blocks = batch * heads * ((sk + kFwdRows - 1) / kFwdRows);
-    const int64_t least = sk <= 1024 ? 512 : sk < 8192 ? 2048 : 1024;
+    const int64_t least = sk <= 1024 ? 512 : 1024;
     for (int64_t fold = group < blocks / least ? group : blocks / least; fold > 1; --fold)
         if (group % fold == 0) return (int)fold;
     return 1;
@@ -553,15 +548,12 @@ template <int DT, int HD>
 static int launch_bwd(AttnBwdArgs a, hipStream_t st)
 {
     const int64_t nqb = (a.sq + kFwdRows - 1) / kFwdRows, nkb = (a.sk + kFwdRows - 1) / kFwdRows;
-    const int64_t per = 8 * (int64_t)a.heads_per_xcd;
-    AttnBwdArgs w = a;
-    w.heads_per_xcd = (a.batch * (a.heads / a.fold) + 7) / 8;
     const int64_t sum_blocks = ((int64_t)a.sk * a.batch * (a.heads / a.group) * (HD / 8) + 255) / 256;
-    const int64_t dkv_blocks = 8 * (int64_t)w.heads_per_xcd * nkb;
-    if (!grid_fits(per * nqb, 256) || !grid_fits(dkv_blocks, 256) || !grid_fits(sum_blocks, 256)) return NHP_ERR_SHAPE;
+    const int64_t dq_blocks = (int64_t)a.batch * a.heads * nqb, dkv_blocks = (int64_t)a.batch * (a.heads / a.fold) * nkb;
+    if (!grid_fits(dq_blocks, 256) || !grid_fits(dkv_blocks, 256) || !grid_fits(sum_blocks, 256)) return NHP_ERR_SHAPE;
     launch_prepare();
-    attn_dq_kernel<DT, HD><<<dim3((unsigned)(per * nqb)), dim3(256), 0, st>>>(a);
-    attn_dkv_kernel<DT, HD><<<dim3((unsigned)dkv_blocks), dim3(256), 0, st>>>(w);
+    attn_dq_kernel<DT, HD><<<dim3((unsigned)dq_blocks), dim3(256), 0, st>>>(a);
+    attn_dkv_kernel<DT, HD><<<dim3((unsigned)dkv_blocks), dim3(256), 0, st>>>(a);
     if (a.fold < a.group) attn_group_sum_kernel<DT><<<dim3((unsigned)sum_blocks, 1, 2), dim3(256), 0, st>>>(a, HD);
     return launch_result();
 }
@@ -630,7 +622,6 @@ int nhp_attention_fwd_keep(void* out, void* kept, float* lse, const void* q, con
     a.sk = (int)sk;
     a.shift = (int)(sk - sq);
     a.window = window < 0 || window > sk ? (int)sk : (int)window;
-    a.heads_per_xcd = (int)((batch * heads + 7) / 8);
     const int mode = mask_bits ? kBits : kCausal;
     if (dtype == NHP_BF16) return launch_fwd_hd<NHP_BF16>(a, (int)head_dim, mode, static_cast<hipStream_t>(stream));
     if (dtype == NHP_F16) return launch_fwd_hd<NHP_F16>(a, (int)head_dim, mode, static_cast<hipStream_t>(stream));
@@ -700,7 +691,6 @@ int nhp_attention_bwd(void* dq, void* dk, void* dv, const void* d_out, const voi
     a.sk = (int)sk;
     a.shift = (int)(sk - sq);
     a.window = window < 0 || window > sk ? (int)sk : (int)window;
-    a.heads_per_xcd = (int)((batch * heads + 7) / 8);
     if (dtype == NHP_BF16) return launch_bwd_hd<NHP_BF16>(a, (int)head_dim, static_cast<hipStream_t>(stream));
     if (dtype == NHP_F16) return launch_bwd_hd<NHP_F16>(a, (int)head_dim, static_cast<hipStream_t>(stream));
     return NHP_ERR_DTYPE;

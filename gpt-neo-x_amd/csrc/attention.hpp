@@ -36,7 +36,7 @@ struct AttnFwdArgs {
     const uint64_t* bits;
     int64_t q_s, q_b, q_h, k_s, k_b, k_h, v_s, v_b, v_h, o_s, o_b, o_h;   // element strides
     float scale_log2, fill_log2;
-    int bits_batches, batch, heads, group, sq, sk, shift, window, heads_per_xcd;
+    int bits_batches, batch, heads, group, sq, sk, shift, window;
 };
 
 struct AttnBwdArgs {
@@ -48,9 +48,30 @@ struct AttnBwdArgs {
     int64_t q_s, q_b, q_h, k_s, k_b, k_h, v_s, v_b, v_h, o_s, o_b, o_h, do_s, do_b, do_h;
     int64_t dq_s, dq_b, dq_h, dk_s, dk_b, dk_h, dv_s, dv_b, dv_h;
     float scale, scale_log2;
-    int batch, heads, group, sq, sk, shift, window, heads_per_xcd;
+    int batch, heads, group, sq, sk, shift, window;
     int fold;   // query heads that a workgroup of the second kernel goes over; they share a key/value head
 };
+
+// Which block of which matrix ((batch entry, head), or several heads of one batch entry) a workgroup takes; one workgroup
+// for each. Under a causal mask blocks differ in length by up to their number, and they are handed out longest first (the
+// caller counts them that way), the longest of all matrices ahead of the next shorter ones: matrix by matrix the last ones
+// started with their longest blocks while the rest of the chip had run dry, and two long ones could meet on a CU. A matrix
+// stays on one XCD, whose L2 then holds its keys and values, where the matrices divide among the XCDs; dealt out to all of
+// them otherwise (12 matrices left two XCDs idle). One pass each, us, matrix by matrix -> here, forward / backward:
+//   [1024, 4, 12 heads, 64] 26.4 -> 21.5 / 67.1 -> 54.5, [2048, 8, 16, 128] 188 -> 159 / 599 -> 525,
+//   [3000, 1, 32 on 8, 128] 111 -> 84 / 371 -> 293, [4096, 4, 16, 128] 324 -> 292 / 1016 -> 920,
+//   [8192, 1, 12, 64] 211 -> 152 / 544 -> 404 (on one XCD each 170 / 500), [8192, 1, 32 on 8, 128] 547 -> 528 / 1799 -> 1739.
+struct Place {
+    int unit, block;
+};
+__device__ __forceinline__ Place place(int units)
+{
+    if (units % 8 == 0) {
+        const int per_xcd = units / 8, idx = blockIdx.x >> 3;
+        return {(int)(blockIdx.x & 7) * per_xcd + idx % per_xcd, idx / per_xcd};
+    }
+    return {(int)(blockIdx.x % units), (int)(blockIdx.x / units)};
+}
 
 template <int DT>
 struct Frag;

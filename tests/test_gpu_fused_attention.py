@@ -71,6 +71,25 @@ def test_causal_forward_and_gradients(dtype, hn, s, b, np_, nkv, window):
     assert torch.equal(util.raw_bits(again.reshape(s, b, np_ * hn)), util.raw_bits(out.detach()))
 
 
+@pytest.mark.parametrize("b,np_", [(1, 1), (1, 7), (1, 8), (2, 8), (3, 4), (1, 24)])
+@pytest.mark.parametrize("s", [128, 129, 700])
+def test_a_matrix_is_the_same_among_others(b, np_, s):
+    """Matrices that divide among the XCDs and ones that do not, of one block and of several: the bits that each has alone."""
+    from megatron.model.fused_attention import causal_attention
+
+    leaves = [t.requires_grad_(True) for t in operands(torch.bfloat16, s, s, b, np_, np_, 64, 31)]
+    g = util.randn((b, np_, s, 64), torch.bfloat16, seed=9).to(DEV)
+    out = causal_attention(*leaves, 0.125)
+    grads = torch.autograd.grad(out, leaves, g)
+    for i in range(b):
+        for h in range(np_):
+            one = [t.detach()[:, i:i + 1, h:h + 1].requires_grad_(True) for t in leaves]
+            alone = causal_attention(*one, 0.125)
+            assert torch.equal(alone[0, 0], out[i, h])
+            for got, want in zip(torch.autograd.grad(alone, one, g[i:i + 1, h:h + 1]), grads):
+                assert torch.equal(got[:, 0, 0], want[:, i, h])
+
+
 @DTYPES
 @pytest.mark.parametrize("hn", [64, 96])
 @pytest.mark.parametrize("sq,sk,b,np_,nkv,window", [(1, 2, 1, 4, 4, None), (1, 130, 2, 4, 2, 5), (63, 129, 1, 4, 4, None), (128, 192, 1, 8, 2, 64),

@@ -6,16 +6,22 @@
 // them while it has them, so they are read once and written once. That traffic is the bound; the matrix instructions and
 // the softmax take a tenth of its time.
 //
-// Split. Rows of the matrix instruction (16 x 16 x 32) are keys, its columns the queries that share a key/value head
-// (new positions x heads of the group, at most 32). The four waves of a workgroup take 32 keys each in turn and share
-// nothing until the end, where their sums are merged; a (batch entry, key/value head) pair is cut into as many
-// workgroups as it takes to have one on every CU, and a second kernel merges those. Keys go from memory into the
-// registers in the order in which the instruction wants them (16 rows x 64 bytes per load); values are transposed
-// through LDS, whose rows are padded so that the 8 rows of a transposing read fall on different banks.
+// Rows of the matrix instruction (16 x 16 x 32) are keys, its columns the queries that share a key/value head (new positions
+// x heads of the group, at most 32). A workgroup is four waves, each with 32 keys at a time, which share nothing until the
+// end, where their sums are merged. Keys go from memory into the registers in the order in which the instruction wants them
+// (16 rows x 64 bytes per load); values are transposed through LDS, whose rows are padded so that the 8 rows of a transposing
+// read fall on different banks. The next 32 keys and values are on their way while the wave stores and multiplies these.
 //
-// Measured (past 2047, 16 sequences, 32 heads, 128 features, bf16; 1.07 GB read and written): 204 to 230 us on different
-// cards, 4.7 to 5.3 TB/s, about what a copy of that size reaches; concatenations 949 us and attention 118 us before. A whole
-// layer's step 1174 -> 365 us.
+// Split. What the memory rewards is one workgroup on every CU and long runs of addresses. So where there are many (batch entry,
+// key/value head) pairs the waves of a workgroup take two or four neighbouring heads, whose rows of a position lie side by
+// side, and with fewer of them the keys of a pair are cut into parts, which a second kernel merges (decode_plan).
+//
+// Measured (us, bf16, without the prefetch and with one head per workgroup before; copy: read and written bytes at 5.1 TB/s):
+//   16 sequences of 2047, 32 heads of 128      221 -> 204 (copy 210)     32 of 1000, 32 heads of 128   221 -> 192 (206)
+//   32 of 2000, 8 heads of keys of 128          90 -> 85 (103)           20 of 2000, 32 heads of 80    328 -> 231 (161)
+//   9 of 2000, 32 heads of 128                 163 -> 119 (116)          5 of 3000, 32 heads of 128    119 -> 91 (96)
+//   1 of 8000, 32 heads of 128                  58 -> 57 (51)            4 of 300, 8 heads of keys      14 -> 11 (2)
+// (Concatenations 949 us and attention 118 us for the first of them, before there was such a kernel.)
 #include "attention.hpp"
 
 namespace nhp {
@@ -30,7 +36,14 @@ struct AttnDecodeArgs {
     int64_t q_s, q_b, q_h, kn_s, kn_b, kn_h, vn_s, vn_b, vn_h, kp_s, kp_b, kp_h, vp_s, vp_b, vp_h;
     int64_t out_s, out_b, out_h, o_s, o_b, o_h, mask_b, mask_q;
     float scale_log2, fill_log2;
-    int batch, kv_heads, group, sq, past, splits, keys_per_split;
+    int batch, kv_heads, group, sq, past, splits, keys_per_split, heads_per_block;
+};
+
+struct Yes {
+    static constexpr bool value = true;
+};
+struct No {
+    static constexpr bool value = false;
 };
 
 // Combines the lanes l, l ^ 16, l ^ 32, l ^ 48.
@@ -55,17 +68,20 @@ struct DecodeGeo {
     static constexpr int kWaveBytes = kValueBytes > kSumBytes ? kValueBytes : kSumBytes;
 };
 
-// NQ: tiles of 16 queries
-template <int DT, int HD, int NQ>
-__global__ void __launch_bounds__(256, NQ == 1 ? 3 : 2) attn_decode_kernel(AttnDecodeArgs a)
+// NQ: tiles of 16 queries; NH: key/value heads of a workgroup, one or several waves each. (With two tiles of queries the
+// registers for what is on its way are there for one workgroup per CU only.)
+template <int DT, int HD, int NQ, int NH>
+__global__ void __launch_bounds__(256, NQ == 1 ? 2 : 1) attn_decode_kernel(AttnDecodeArgs a)
 {
     using G = DecodeGeo<HD>;
+    constexpr int kKeyWaves = 4 / NH, kKeys = 32 * kKeyWaves;   // waves that share a head's keys, and what they take in a round
     __shared__ __attribute__((aligned(1024))) char lds[4 * G::kWaveBytes];
     __shared__ float wave_m[4][NQ * 16], wave_l[4][NQ * 16];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g = lane >> 4;
     const int pairs = a.batch * a.kv_heads;
-    const int pair = blockIdx.x % pairs, split = blockIdx.x / pairs;
+    const int groups = pairs / NH, pair0 = blockIdx.x % groups * NH;
+    const int pair = pair0 + wave % NH, split = blockIdx.x / groups;
     const int b = pair / a.kv_heads, hk = pair % a.kv_heads;
     const int rows = a.sq * a.group, sk = a.past + a.sq;
     const int key_lo = split * a.keys_per_split, key_hi = min(sk, key_lo + a.keys_per_split);
@@ -109,39 +125,8 @@ __global__ void __launch_bounds__(256, NQ == 1 ? 3 : 2) attn_decode_kernel(AttnD
         for (int d = 0; d < G::kTiles; ++d) o[n][d] = f32x4{};
     }
 
-    for (int next = key_lo + wave * 32; next < key_hi; next += 128) {
-        // opaque, so that the addresses are formed here as base + lane offset; kept as running pointers, one for each
-        // access, they would not fit into the registers
-        int key0 = next;
-        asm volatile("" : "+s"(key0));
-        u32x4 kf[2][G::kSteps], vf[G::kLoads];
-        if (key0 + 32 <= a.past) {
-            const uint16_t *kt = kp + (int64_t)key0 * a.kp_s, *vt = vp + (int64_t)key0 * a.vp_s;
-#pragma unroll
-            for (int t2 = 0; t2 < 2; ++t2)
-#pragma unroll
-                for (int t = 0; t < G::kSteps; ++t)
-                    kf[t2][t] = 4 * t + g < G::kChunks ? load16(kt + (uint64_t)(t2 * 16) * kps + t * 32 + (r16 * kps + g * 8)) : u32x4{0, 0, 0, 0};
-#pragma unroll
-            for (int i = 0; i < G::kLoads; ++i) vf[i] = load16_stream(value_at(vt, vps, i));
-        } else {   // the last ones: cached, new, or beyond the end (the last one again)
-#pragma unroll
-            for (int t2 = 0; t2 < 2; ++t2) {
-                const int key = min(key0 + t2 * 16 + r16, sk - 1);
-                const uint16_t* p = key < a.past ? kp + key * a.kp_s : kn + (key - a.past) * a.kn_s;
-#pragma unroll
-                for (int t = 0; t < G::kSteps; ++t)
-                    kf[t2][t] = 4 * t + g < G::kChunks ? load16(p + (4 * t + g) * 8) : u32x4{0, 0, 0, 0};
-            }
-#pragma unroll
-            for (int i = 0; i < G::kLoads; ++i) {
-                const int key = min(key0 + (int)value_row(i), sk - 1);
-                vf[i] = load16((key < a.past ? vp + key * a.vp_s : vn + (key - a.past) * a.vn_s) + value_col(i));
-            }
-        }
-        // bytes 4 g .. 4 g + 3 of each 16 keys of this lane's query; the last ones of a row are read as the four bytes that
-        // end it
-        uint32_t hidden[NQ][2];
+    // bytes 4 g .. 4 g + 3 of each 16 keys of this lane's query; the last ones of a row are read as the four bytes that end it
+    auto read_mask = [&](int key0, uint32_t (&hidden)[NQ][2]) {
 #pragma unroll
         for (int n = 0; n < NQ; ++n)
 #pragma unroll
@@ -150,11 +135,50 @@ __global__ void __launch_bounds__(256, NQ == 1 ? 3 : 2) attn_decode_kernel(AttnD
                 const uint32_t w = *reinterpret_cast<const u32_byte*>(mrow[n] + at);
                 hidden[n][t2] = key - at < 4 ? w >> (8 * (key - at)) : 0u;
             }
-
+    };
+    using Keys = u32x4[2][G::kSteps];
+    using Values = u32x4[G::kLoads];
+    using Hidden = uint32_t[NQ][2];
+    // 32 cached keys and values
+    auto load = [&](int key0, Keys& kf, Values& vf, Hidden& hidden) {
+        // opaque, so that the addresses are formed here as base + lane offset; kept as running pointers, one for each
+        // access, they would not fit into the registers
+        asm volatile("" : "+s"(key0));
+        const uint16_t *kt = kp + (int64_t)key0 * a.kp_s, *vt = vp + (int64_t)key0 * a.vp_s;
+#pragma unroll
+        for (int t2 = 0; t2 < 2; ++t2)
+#pragma unroll
+            for (int t = 0; t < G::kSteps; ++t)
+                kf[t2][t] = 4 * t + g < G::kChunks ? load16(kt + (uint64_t)(t2 * 16) * kps + t * 32 + (r16 * kps + g * 8)) : u32x4{0, 0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < G::kLoads; ++i) vf[i] = load16_stream(value_at(vt, vps, i));
+        read_mask(key0, hidden);
+        asm volatile("" ::: "memory");   // not put off until they are needed
+    };
+    // the last ones: cached, new, or beyond the end (the last one again)
+    auto load_last = [&](int key0, Keys& kf, Values& vf, Hidden& hidden) {
+#pragma unroll
+        for (int t2 = 0; t2 < 2; ++t2) {
+            const int key = min(key0 + t2 * 16 + r16, sk - 1);
+            const uint16_t* p = key < a.past ? kp + key * a.kp_s : kn + (key - a.past) * a.kn_s;
+#pragma unroll
+            for (int t = 0; t < G::kSteps; ++t) kf[t2][t] = 4 * t + g < G::kChunks ? load16(p + (4 * t + g) * 8) : u32x4{0, 0, 0, 0};
+        }
+#pragma unroll
+        for (int i = 0; i < G::kLoads; ++i) {
+            const int key = min(key0 + (int)value_row(i), sk - 1);
+            vf[i] = load16((key < a.past ? vp + key * a.vp_s : vn + (key - a.past) * a.vn_s) + value_col(i));
+        }
+        read_mask(key0, hidden);
+    };
+    // Stores and multiplies them; `whole`: all 32 exist.
+    auto use = [&](auto whole, int key0, Keys& kf, Values& vf, Hidden& hidden) {
+        constexpr bool kWhole = decltype(whole)::value;
+        asm volatile("" : "+s"(key0));
         uint16_t *kd = ko + (int64_t)key0 * a.out_s, *vd = vo + (int64_t)key0 * a.out_s;
 #pragma unroll
         for (int t2 = 0; t2 < 2; ++t2) {
-            if (key0 + t2 * 16 + r16 >= key_hi) continue;
+            if (!kWhole && key0 + t2 * 16 + r16 >= key_hi) continue;
 #pragma unroll
             for (int t = 0; t < G::kSteps; ++t)
                 if (4 * t + g < G::kChunks) *reinterpret_cast<u32x4*>(kd + (uint64_t)(t2 * 16) * outs + t * 32 + (r16 * outs + g * 8)) = kf[t2][t];
@@ -165,7 +189,7 @@ __global__ void __launch_bounds__(256, NQ == 1 ? 3 : 2) attn_decode_kernel(AttnD
 #pragma unroll
         for (int i = 0; i < G::kLoads; ++i) {
             *reinterpret_cast<u32x4*>(mine + value_row(i) * G::kRowBytes + value_col(i) * 2) = vf[i];
-            if (key0 + (int)value_row(i) < key_hi) store16_stream(value_at(vd, outs, i), vf[i]);
+            if (kWhole || key0 + (int)value_row(i) < key_hi) store16_stream(value_at(vd, outs, i), vf[i]);
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -186,7 +210,7 @@ __global__ void __launch_bounds__(256, NQ == 1 ? 3 : 2) attn_decode_kernel(AttnD
                 for (int i = 0; i < 4; ++i) {
                     const int key = key0 + t2 * 16 + 4 * g + i;
                     float x = hidden[n][t2] >> (8 * i) & 0xffu ? a.fill_log2 : s[t2][i] * a.scale_log2;
-                    x = key < key_hi ? x : kNegInf;
+                    if (!kWhole) x = key < key_hi ? x : kNegInf;
                     s[t2][i] = x;
                     mx = fmaxf(mx, x);
                 }
@@ -220,6 +244,28 @@ __global__ void __launch_bounds__(256, NQ == 1 ? 3 : 2) attn_decode_kernel(AttnD
 #pragma unroll
             for (int n = 0; n < NQ; ++n) o[n][d] = mma16<DT>(vt, pf[n], o[n][d]);
         }
+    };
+    int key0 = key_lo + wave / NH * 32;
+    const int last_whole = min(a.past, key_hi) - 32;
+    Keys kf[2];
+    Values vf[2];
+    Hidden hidden[2];
+    if (key0 <= last_whole) {
+        load(key0, kf[0], vf[0], hidden[0]);
+        for (;;) {
+            if (key0 + kKeys <= last_whole) load(key0 + kKeys, kf[1], vf[1], hidden[1]);
+            use(Yes{}, key0, kf[0], vf[0], hidden[0]);
+            key0 += kKeys;
+            if (key0 > last_whole) break;
+            if (key0 + kKeys <= last_whole) load(key0 + kKeys, kf[0], vf[0], hidden[0]);
+            use(Yes{}, key0, kf[1], vf[1], hidden[1]);
+            key0 += kKeys;
+            if (key0 > last_whole) break;
+        }
+    }
+    for (; key0 < key_hi; key0 += kKeys) {
+        load_last(key0, kf[0], vf[0], hidden[0]);
+        use(No{}, key0, kf[0], vf[0], hidden[0]);
     }
 
     // the four waves' sums, 16 queries at a time
@@ -238,30 +284,33 @@ __global__ void __launch_bounds__(256, NQ == 1 ? 3 : 2) attn_decode_kernel(AttnD
 #pragma unroll
         for (int d = 0; d < G::kTiles; ++d) *reinterpret_cast<f32x4*>(sums + r16 * G::kSumRow + d * 16 + 4 * g) = o[n][d];
         __syncthreads();
-        const int r = tid >> 4, c = tid & 15, row = n * 16 + r;
-        if (c >= G::kChunks || row >= rows) continue;
-        float big = kFarBelow, total = 0.0f, acc[8] = {};
+        for (int item = tid; item < NH * 256; item += 256) {
+            const int hh = item >> 8, r = (item >> 4) & 15, c = item & 15, row = n * 16 + r;
+            if (c >= G::kChunks || row >= rows) continue;
+            const int pr = pair0 + hh, b2 = pr / a.kv_heads, hk2 = pr % a.kv_heads;
+            float big = kFarBelow, total = 0.0f, acc[8] = {};
 #pragma unroll
-        for (int w = 0; w < 4; ++w) big = fmaxf(big, wave_m[w][row]);
+            for (int w = 0; w < kKeyWaves; ++w) big = fmaxf(big, wave_m[w * NH + hh][row]);
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const float f = exp2_raw(wave_m[w][row] - big);
-            total = fmaf(wave_l[w][row], f, total);
-            const float* p = reinterpret_cast<const float*>(lds + w * G::kWaveBytes) + r * G::kSumRow + c * 8;
+            for (int w = 0; w < kKeyWaves; ++w) {
+                const float f = exp2_raw(wave_m[w * NH + hh][row] - big);
+                total = fmaf(wave_l[w * NH + hh][row], f, total);
+                const float* p = reinterpret_cast<const float*>(lds + (w * NH + hh) * G::kWaveBytes) + r * G::kSumRow + c * 8;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) acc[j] = fmaf(p[j], f, acc[j]);
-        }
-        if (a.splits == 1) {
-            const float inv = 1.0f / total;
+                for (int j = 0; j < 8; ++j) acc[j] = fmaf(p[j], f, acc[j]);
+            }
+            if (a.splits == 1) {
+                const float inv = 1.0f / total;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) acc[j] *= inv;
-            uint16_t* op = a.o + row / a.group * a.o_s + b * a.o_b + (hk * a.group + row % a.group) * a.o_h;
-            *reinterpret_cast<u32x4*>(op + c * 8) = pack8<DT>(acc);
-        } else {
-            const int64_t at = ((int64_t)split * pairs + pair) * rows + row;
-            *reinterpret_cast<f32x4*>(a.part_o + at * HD + c * 8) = f32x4{acc[0], acc[1], acc[2], acc[3]};
-            *reinterpret_cast<f32x4*>(a.part_o + at * HD + c * 8 + 4) = f32x4{acc[4], acc[5], acc[6], acc[7]};
-            if (c == 0) *reinterpret_cast<f32x2*>(a.part_ml + at * 2) = f32x2{big, total};
+                for (int j = 0; j < 8; ++j) acc[j] *= inv;
+                uint16_t* op = a.o + row / a.group * a.o_s + b2 * a.o_b + (hk2 * a.group + row % a.group) * a.o_h;
+                *reinterpret_cast<u32x4*>(op + c * 8) = pack8<DT>(acc);
+            } else {
+                const int64_t at = ((int64_t)split * pairs + pr) * rows + row;
+                *reinterpret_cast<f32x4*>(a.part_o + at * HD + c * 8) = f32x4{acc[0], acc[1], acc[2], acc[3]};
+                *reinterpret_cast<f32x4*>(a.part_o + at * HD + c * 8 + 4) = f32x4{acc[4], acc[5], acc[6], acc[7]};
+                if (c == 0) *reinterpret_cast<f32x2*>(a.part_ml + at * 2) = f32x2{big, total};
+            }
         }
     }
 }
@@ -320,23 +369,54 @@ __global__ void __launch_bounds__(256) cache_append_kernel(CacheArgs a)
     *reinterpret_cast<u32x4*>(a.out + (value ? a.items * 8 : 0) + i * 8) = load16(p + c * 8);
 }
 
-// Workgroups per (batch entry, key/value head) pair: one for each CU in all, and 256 keys at least for each. More of them
-// cost the cache's bandwidth (one sequence of 8000 keys, 32 heads of 128: 58 us with 8 each, 64 with 24; 16 sequences of
-// 2048: 221 with one, 228 with two), and a second one for 200 keys costs the merge (12 heads of 64: 6.2 -> 7.4 us).
-static int decode_splits(int64_t pairs, int64_t sk)
+// Heads of a workgroup and workgroups of a pair of batch entry and key/value head.
+//
+// Heads: four or two where that leaves about one workgroup for each CU (1024 pairs of 128 features, 4 / 2 / 1 heads: 192 / 212
+// / 217 us, 768: 161 / 164 / 172, 512: 199 / 204 / 221, of which the first needs a second kernel, 384: 165 / 162 / 171, 288: 147
+// / 125 / 121), earlier where rows of 160 or 192 bytes end within a cache line (640 pairs of 80 features: 231 / 251 / 304).
+//
+// Workgroups: few, but so many that they go evenly on 256 CUs, with 256 keys at least (128 where there are less workgroups than
+// CUs). More of them cost the cache's bandwidth and the second kernel (256 pairs of 2000 keys: 85 us with one each, 89 with two;
+// 12 pairs of 200 keys: 6.2, 7.4), uneven ones leave CUs idle (288 pairs: 154 us with one each, 130 with two, 121 with four;
+// 160: 115 with two, 96 with four; 32 of 300: 14 with two, 11 with three).
+struct DecodePlan {
+    int heads_per_block, splits, keys_per_split;
+};
+static DecodePlan decode_plan(int64_t batch, int64_t kv_heads, int64_t rows, int64_t sk, int64_t hd)
 {
-    const int64_t most = (sk + 255) / 256, wanted = (256 + pairs - 1) / pairs;
-    return (int)(wanted < most ? wanted : most);
+    const int64_t pairs = batch * kv_heads;
+    const bool whole_lines = hd % 64 == 0;
+    int heads = 1;
+    if (rows <= 16 && kv_heads % 4 == 0 && pairs >= (whole_lines ? 640 : 512)) heads = 4;
+    else if (rows <= 16 && kv_heads % 2 == 0 && pairs >= 384) heads = 2;
+    const int64_t groups = pairs / heads, most = sk <= 256 ? 1 : (sk + 127) / 128;
+    int64_t splits = 1, best = 0;
+    for (int64_t s = 1; s <= most && s <= 256; ++s) {
+        const int64_t blocks = groups * s, rounds = (blocks + 255) / 256;
+        if (s > 1 && rounds > 1 && sk < s * 256) break;
+        // rounds of workgroups against their number (192 of them, or 160 with four heads, need no second kernel), and in
+        // hundredths 3 for the second kernel and 1 for each split
+        const bool full = s == 1 && rounds == 1 && blocks >= (heads == 4 ? 160 : 192);
+        const int64_t cost = (full ? 1000 : rounds * 256 * 1000 / blocks) * (100 + (s > 1 ? 3 + s : 0));
+        if (s == 1 || cost < best) {
+            best = cost;
+            splits = s;
+        }
+    }
+    const int64_t keys = ((sk + splits - 1) / splits + 127) / 128 * 128;
+    return {heads, (int)((sk + keys - 1) / keys), (int)keys};   // no empty split
 }
 
 template <int DT, int HD>
 static int launch_decode(const AttnDecodeArgs& a, hipStream_t st)
 {
-    const int64_t pairs = (int64_t)a.batch * a.kv_heads, grid = pairs * a.splits, rows = (int64_t)a.sq * a.group;
+    const int64_t pairs = (int64_t)a.batch * a.kv_heads, grid = pairs / a.heads_per_block * a.splits, rows = (int64_t)a.sq * a.group;
     if (!grid_fits(grid, 256) || !grid_fits((pairs * rows + 15) / 16, 256)) return NHP_ERR_SHAPE;
     launch_prepare();
-    if (rows <= 16) attn_decode_kernel<DT, HD, 1><<<dim3((unsigned)grid), dim3(256), 0, st>>>(a);
-    else attn_decode_kernel<DT, HD, 2><<<dim3((unsigned)grid), dim3(256), 0, st>>>(a);
+    if (rows > 16) attn_decode_kernel<DT, HD, 2, 1><<<dim3((unsigned)grid), dim3(256), 0, st>>>(a);
+    else if (a.heads_per_block == 1) attn_decode_kernel<DT, HD, 1, 1><<<dim3((unsigned)grid), dim3(256), 0, st>>>(a);
+    else if (a.heads_per_block == 2) attn_decode_kernel<DT, HD, 1, 2><<<dim3((unsigned)grid), dim3(256), 0, st>>>(a);
+    else attn_decode_kernel<DT, HD, 1, 4><<<dim3((unsigned)grid), dim3(256), 0, st>>>(a);
     if (a.splits > 1) attn_decode_merge_kernel<DT, HD><<<dim3((unsigned)((pairs * rows + 15) / 16)), dim3(256), 0, st>>>(a);
     return launch_result();
 }
@@ -368,7 +448,7 @@ int64_t nhp_attention_decode_workspace_bytes(int64_t batch, int64_t heads, int64
 {
     using namespace nhp;
     if (!decode_sizes_ok(batch, heads, kv_heads, sq, past, head_dim)) return 0;
-    const int64_t splits = decode_splits(batch * kv_heads, past + sq);
+    const int64_t splits = decode_plan(batch, kv_heads, sq * (heads / kv_heads), past + sq, head_dim).splits;
     return splits == 1 ? 0 : splits * batch * heads * sq * (head_dim + 2) * 4;
 }
 
@@ -412,9 +492,10 @@ int nhp_attention_decode(void* out, void* cache_out, const void* q, const void* 
     a.group = (int)(heads / kv_heads);
     a.sq = (int)sq;
     a.past = (int)past;
-    a.splits = decode_splits(batch * kv_heads, sk);
-    a.keys_per_split = (int)(((sk + a.splits - 1) / a.splits + 127) / 128 * 128);
-    a.splits = (int)((sk + a.keys_per_split - 1) / a.keys_per_split);   // none of them empty
+    const DecodePlan plan = decode_plan(batch, kv_heads, sq * a.group, sk, head_dim);
+    a.splits = plan.splits;
+    a.keys_per_split = plan.keys_per_split;
+    a.heads_per_block = plan.heads_per_block;
     if (a.splits > 1) {
         if (!workspace || !ptr_aligned16(workspace)) return NHP_ERR_NULL;
         a.part_o = static_cast<float*>(workspace);

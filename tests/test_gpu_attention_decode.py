@@ -44,6 +44,20 @@ def test_decode(dtype, hn, past, sq, b, np_, nkv):
     assert torch.equal(append_to_cache(k.transpose(0, 1).contiguous().transpose(0, 1), v, None), torch.stack((k, v)))
 
 
+@pytest.mark.parametrize("hn", [64, 80, 96, 128])
+@pytest.mark.parametrize("past", [3, 31, 32, 63, 64, 65, 97, 128, 161, 300])
+@pytest.mark.parametrize("sq,b,np_,nkv", [(1, 160, 4, 4), (1, 128, 4, 4), (2, 97, 8, 4), (1, 192, 2, 2), (9, 192, 4, 2), (1, 131, 3, 3)])
+def test_many_sequences(hn, past, sq, b, np_, nkv):
+    """One, two and four heads of keys per workgroup; rounds of 32 keys that a wave has one, two or several of."""
+    from megatron.model.fused_attention import decode_attention
+
+    q, k, v, layer_past = cached(torch.bfloat16, past, sq, b, np_, nkv, hn)
+    mask = hidden(sq, past + sq).view(1, 1, sq, past + sq)
+    out, present = decode_attention(q, k[past:], v[past:], layer_past, mask, 1 / math.sqrt(hn), -10000.0, merged=True)
+    assert torch.equal(present, torch.stack((k, v)))
+    assert rel_err(out.view(sq, b, np_, hn), textbook(q, k, v, mask, -10000.0)) <= limit(torch.bfloat16, 2)
+
+
 def test_nan_and_infinite_keys_stay_where_they_are():
     """A value that is not finite reaches the queries that see it and no others; the cache keeps it."""
     from megatron.model.fused_attention import decode_attention

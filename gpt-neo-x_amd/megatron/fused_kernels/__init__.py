@@ -3,7 +3,7 @@
 Keeps the two entry points of GPT-NeoX's ``megatron/fused_kernels/__init__.py``
 (``load`` at :35-143, ``load_fused_kernels`` at :167-181). Instead of JIT-building
 three pybind11 extensions, ``load`` makes sure ``libneox_hotpath.so`` (hand-written
-gfx950 kernels behind a C ABI) is built and importable; the three extension
+gfx950 kernels behind a C ABI) and ``_native.so`` (the host side of the most frequent calls) are built and importable; the three extension
 module names of the reference (``scaled_upper_triang_masked_softmax_cuda``,
 ``scaled_masked_softmax_cuda``, ``fused_rotary_positional_embedding``) are thin
 modules over that library and are registered in ``sys.modules`` here.
@@ -38,7 +38,7 @@ def load(neox_args=None):
     reference. Raises if the build or the load fails.
     """
     verbose = True if neox_args is None else (getattr(neox_args, "rank", 0) == 0)
-    if not os.path.exists(_hotpath.LIB_PATH):
+    if not (os.path.exists(_hotpath.LIB_PATH) and os.path.exists(_hotpath.NATIVE_PATH)):
         if verbose:
             print(f"building {_hotpath.LIB_PATH} for gfx950 ...", flush=True)
         _hotpath.build(verbose=verbose)

@@ -12,6 +12,7 @@ import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libneox_hotpath.so")
+NATIVE_PATH = os.path.join(_HERE, "_native.so")
 CSRC_DIR = os.path.normpath(os.path.join(_HERE, "..", "..", "csrc"))
 
 F16, BF16, F32 = 0, 1, 2
@@ -133,6 +134,23 @@ def lib():
                     )
                 _lib = handle
     return _lib
+
+
+_native = None
+
+
+def native():
+    """The extension module with the host side of the most frequent calls (csrc/native.cpp); raises ImportError when it is
+    absent. Its functions return NotImplemented for operands that they leave to the caller. Not to be called while torch
+    compiles: it does not see through them."""
+    global _native
+    if _native is None:
+        try:
+            from . import _native as module   # links libneox_hotpath.so beside it
+        except ImportError as e:
+            raise ImportError(f"cannot load {NATIVE_PATH}: {e}") from e
+        _native = module
+    return _native
 
 
 def check(status, what):

@@ -100,7 +100,13 @@ class GeLUFunction(torch.autograd.Function):
         return dx, dbias
 
 
-bias_gelu_impl = GeLUFunction.apply
+def bias_gelu_impl(input, bias):
+    """``GeLUFunction.apply(input, bias)``."""
+    if not _hp._is_compiling():
+        y = _hp.native().bias_gelu(input, bias)
+        if y is not NotImplemented:
+            return y
+    return GeLUFunction.apply(input, bias)
 
 
 # ---------------------------------------------------------------------------
@@ -219,4 +225,8 @@ class Gated_Activation(torch.nn.Module):
         self._code = _GATE_CODE[activation_func]
 
     def forward(self, x, bias=None):
+        if bias is None and not _hp._is_compiling():
+            y = _hp.native().gated(x, self._code)
+            if y is not NotImplemented:
+                return y
         return _GatedActivationFunction.apply(x, bias, self._code)

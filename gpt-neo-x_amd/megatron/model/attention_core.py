@@ -34,6 +34,7 @@ import math
 
 import torch
 
+from ..fused_kernels import _hotpath as _hp
 from . import fused_attention
 from .fused_softmax import FusedScaleMaskSoftmax, SoftmaxFusionTypes
 from .utils import get_fusion_type  # noqa: F401  (also reachable from here, where its caller lives)
@@ -536,6 +537,10 @@ def split_gqa_and_rotate(mixed_x_layer, rotary_emb, num_heads, num_kv_heads, lay
     if layer_past is not None and layer_past.numel() > 0:
         offset = layer_past[0].shape[0]
     cos, sin = rotary_emb(mixed_x_layer, seq_len=seq_len + offset)
+    if not _hp._is_compiling():
+        parts = _hp.native().split_rotary(mixed_x_layer, cos, sin, offset, num_heads, num_kv_heads)
+        if parts is not NotImplemented:
+            return parts
     rows = slice(offset, offset + seq_len)
     return _SplitRotaryGQA.apply(mixed_x_layer, cos[rows], sin[rows], num_heads, num_kv_heads)
 
@@ -550,5 +555,9 @@ def split_qkv_and_rotate(mixed_x_layer, rotary_emb, layer_past=None):
     if layer_past is not None and layer_past.numel() > 0:
         offset = layer_past[0].shape[0]
     cos, sin = rotary_emb(mixed_x_layer, seq_len=seq_len + offset)
+    if not _hp._is_compiling():
+        parts = _hp.native().split_rotary(mixed_x_layer, cos, sin, offset, 0, 0)
+        if parts is not NotImplemented:
+            return parts
     rows = slice(offset, offset + seq_len)
     return _SplitRotaryQKV.apply(mixed_x_layer, cos[rows], sin[rows])

@@ -150,6 +150,10 @@ def causal_attention(q, k, v, scale, window=None, merged=False, checked=False):
     """Context of q ``[s, b, np, hn]`` over k, v ``[s, b, nkv, hn]``: ``[b, np, s, hn]``, or with ``merged``
     ``[s, b, np * hn]``. Query i attends to keys ``i - window .. i``. ``checked``: the caller has asked
     ``supported`` already."""
+    if not _hp._is_compiling():
+        out = _hp.native().causal_attention(q, k, v, float(scale), -1 if window is None else window, merged)
+        if out is not NotImplemented:
+            return out
     return CausalAttention.apply(q, k, v, float(scale), window, merged, checked)
 
 
@@ -158,6 +162,10 @@ def masked_attention(q, k, v, mask, scale, fill, merged=False, checked=False):
     replaced by ``fill`` after scaling. ``checked``: the caller has asked ``supported`` and ``mask_supported`` already."""
     _refuse_unless(checked or supported(q, k, v) and mask_supported(mask, q.size(1), q.size(0), k.size(0), q.device),
                    "masked_attention", q, k, v, mask)
+    if not _hp._is_compiling():
+        out = _hp.native().masked_attention(q, k, v, mask, float(scale), float(fill), merged)
+        if out is not NotImplemented:
+            return out
     (q, q_strides), (k, k_strides), (v, v_strides) = _operand(q), _operand(k), _operand(v)
     sq, sk = q.size(0), k.size(0)
     mask = mask.contiguous()
@@ -233,6 +241,10 @@ def _past_fits(key, value, past_key, past_value):
 def append_to_cache(key, value, layer_past, checked=False):
     """``torch.stack((cat(past keys, key), cat(past values, value)))`` in one launch: ``[2, past + sq, b, nkv, hn]``.
     ``checked``: the caller has asked ``cache_supported`` already."""
+    if checked and not _hp._is_compiling():
+        present = _hp.native().append_to_cache(key, value, layer_past)
+        if present is not NotImplemented:
+            return present
     past_k, past_v = (None, None) if layer_past is None else layer_past
     if layer_past is None:
         _refuse_unless(checked or _cache_fits(key, value, 0), "append_to_cache", key, value)
@@ -293,6 +305,10 @@ def decode_attention(query, key, value, layer_past, mask, scale, fill, merged=Fa
 def checked_decode_attention(query, key, value, layer_past, mask, scale, fill, merged):
     """``decode_attention`` for a caller that has asked ``decode_supported`` and ``mask_supported`` already: a step of a small
     model waits for the host, and the checks cost it several microseconds a layer."""
+    if not _hp._is_compiling():
+        both = _hp.native().decode_attention(query, key, value, layer_past, mask, float(scale), float(fill), merged)
+        if both is not NotImplemented:
+            return both
     query, key, value = _readable(query), _readable(key), _readable(value)
     (keys, key_strides), (values, value_strides), past, _alive = _cached_rows(layer_past)
     sq, b, np_, hn = query.shape

@@ -153,6 +153,10 @@ def bias_add_residual_pair(x1: Tensor, bias1: Optional[Tensor], x2: Tensor, bias
     attention and MLP branches (three ``bias_dropout_add`` calls in ParallelTransformerLayer.forward,
     megatron/model/transformer.py:1229-1250) when dropout is off, in one kernel and with the reference's
     roundings."""
+    if not _hp._is_compiling():
+        out = _hp.native().add_residual_pair(x1, bias1, x2, bias2, residual)
+        if out is not NotImplemented:
+            return out
     return _BiasAddResidualPair.apply(x1, bias1, x2, bias2, residual)
 
 
@@ -202,6 +206,10 @@ def bias_dropout_add(x: Tensor, bias: Tensor, residual: Optional[Tensor], prob: 
         if not prob < 1.0:
             raise ValueError(f"dropout probability has to be between 0 and 1, but got {prob}")
         return _BiasDropoutAdd.apply(x, bias, residual, prob, _fresh_seed(x.device))
+    if not _hp._is_compiling():
+        out = _hp.native().add_residual(x, bias, residual)
+        if out is not NotImplemented:
+            return out
     return _BiasAddResidual.apply(x, bias, residual)
 
 

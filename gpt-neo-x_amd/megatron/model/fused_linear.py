@@ -59,6 +59,10 @@ def linear(x, weight, bias: Optional[torch.Tensor] = None):
 
 @torch.jit.unused
 def _linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> torch.Tensor:
+    if not _hp._is_compiling():
+        y = _hp.native().linear(x, weight, bias, MAX_ROWS, MAX_ROWS_NARROW)
+        if y is not NotImplemented:
+            return y
     if (_hp._is_compiling() or _hp._tracing_state() is not None or not isinstance(x, torch.Tensor) or not isinstance(weight, torch.Tensor)
             or weight.dim() != 2 or not _few_rows(x, weight, bias)):
         return F.linear(x, weight, bias)

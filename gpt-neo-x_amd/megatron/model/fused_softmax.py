@@ -41,6 +41,7 @@ import math
 import torch
 from torch import nn
 
+from ..fused_kernels import _hotpath as _hp
 from ..fused_kernels import load_fused_kernels
 from . import dropout_rng
 
@@ -404,6 +405,11 @@ class FusedScaleMaskSoftmax(nn.Module):
         if key_lengths is not None:
             assert key_lengths.shape == (b,), "key_lengths must be [b]"
         slopes = self._slopes_on(input.device)
+        if dropout == 0.0 and slopes is None and bias is None and key_lengths is None and not self.narrow_forward_scale \
+                and not _hp._is_compiling():
+            probs = _hp.native().masked_softmax(input, mask, factor)
+            if probs is not NotImplemented:
+                return probs
         if dropout > 0.0:
             return ScaledMaskedSoftmaxDropout.apply(input, mask, factor, dropout, self._dropout_seed(input.device), slopes, bias,
                                                     key_lengths, self.narrow_forward_scale)
@@ -417,6 +423,11 @@ class FusedScaleMaskSoftmax(nn.Module):
 
         assert sq == sk, "causal mask is only for self attention"
         slopes = self._slopes_on(input.device)
+        if dropout == 0.0 and slopes is None and bias is None and key_lengths is None and zero_block == 0 \
+                and not self.narrow_forward_scale and not _hp._is_compiling():
+            probs = _hp.native().causal_softmax(input, factor, -1 if self.sliding_window_width is None else self.sliding_window_width)
+            if probs is not NotImplemented:
+                return probs
         # the kernel takes [attn_batches, sq, sk]; the causal mask is implied by the indices
         flat = input.view(b * np, sq, sk)
         if bias is not None:

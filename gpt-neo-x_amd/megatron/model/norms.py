@@ -179,6 +179,10 @@ def layer_norm_pair(x, norm_a, norm_b):
             and x.size(-1) * x.element_size() <= 16384)
     if not same:
         return norm_a(x), norm_b(x)
+    if not _hp._is_compiling():
+        y = _hp.native().layer_norm_pair(x, norm_a.weight, norm_a.bias, norm_b.weight, norm_b.bias, norm_a.eps)
+        if y is not NotImplemented:
+            return y
     return _LayerNormPairFunction.apply(x, norm_a.weight, norm_a.bias, norm_b.weight, norm_b.bias, norm_a.eps)
 
 
@@ -210,6 +214,10 @@ class LayerNorm(torch.nn.Module):
         if input.device.type != "cuda":
             # off the GPU: torch's own LayerNorm, which is the reference's class (megatron/model/norms.py:16)
             return torch.nn.functional.layer_norm(input, self.normalized_shape, self.weight, self.bias, self.eps)
+        if not _hp._is_compiling():
+            y = _hp.native().layer_norm(input, self.weight, self.bias, self.eps)
+            if y is not NotImplemented:
+                return y
         return _LayerNormFunction.apply(input, self.weight, self.bias, self.eps)
 
     def extra_repr(self):
@@ -299,8 +307,12 @@ class RMSNorm(torch.nn.Module):
             raise RuntimeError(f"RMSNorm: expected last dimension {self.d}, got {x.size(-1)}")
         if x.device.type != "cuda":
             return self._forward_torch(x)
-        return _RMSNormFunction.apply(x, self.scale, self.offset, self.eps, 0 if self.fused_eps else 1,
-                                      self.partial_size)
+        mode = 0 if self.fused_eps else 1
+        if not _hp._is_compiling():
+            y = _hp.native().rms_norm(x, self.scale, self.offset, self.eps, mode, self.d if self.partial_size is None else self.partial_size)
+            if y is not NotImplemented:
+                return y
+        return _RMSNormFunction.apply(x, self.scale, self.offset, self.eps, mode, self.partial_size)
 
     def _forward_torch(self, x):
         """Off the GPU: the statements of the reference's ``RMSNorm.forward`` (megatron/model/norms.py:82-107), every

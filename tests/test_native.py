@@ -1,0 +1,44 @@
+"""What the host side in csrc/native.cpp leaves to Python, on the CPU: everything that is not a plain tensor on a GPU, and calls
+of another form."""
+import pytest
+import torch
+
+from megatron.fused_kernels import _hotpath as hp
+
+X = torch.ones((4, 4))
+
+
+class Sub(torch.Tensor):
+    pass
+
+
+OPERANDS = {"on the cpu": X, "subclass": X.as_subclass(Sub), "meta": torch.empty((4, 4), device="meta"), "none": None, "number": 3.0,
+            "sparse": X.to_sparse(), "parameter": torch.nn.Parameter(X)}
+CALLS = {"layer_norm": ("x", None, None, 1e-5), "layer_norm_pair": ("x", None, None, None, None, 1e-5), "rms_norm": ("x", None, None, 1e-5, 0, 4),
+         "bias_gelu": ("x", None), "gated": ("x", 0), "causal_softmax": ("x", 1.0, -1), "masked_softmax": ("x", "x", 1.0),
+         "rotary": ("x", "x", "x", "x", 0), "split_rotary": ("x", "x", "x", 0, 0, 0), "add_residual": ("x", None, None),
+         "add_residual_pair": ("x", None, "x", None, "x"), "causal_attention": ("x", "x", "x", 1.0, -1, True),
+         "masked_attention": ("x", "x", "x", "x", 1.0, -1e4, True), "decode_attention": ("x", "x", "x", "x", "x", 1.0, -1e4, True),
+         "append_to_cache": ("x", "x", None), "linear": ("x", "x", None, 16, 32)}
+
+
+@pytest.mark.parametrize("name", CALLS)
+def test_left_to_python(name):
+    call = getattr(hp.native(), name)
+    for operand in OPERANDS.values():
+        assert call(*(operand if a == "x" else a for a in CALLS[name])) is NotImplemented
+    assert call() is NotImplemented and call(*CALLS[name]) is NotImplemented
+    assert call(*(X if a == "x" else a for a in CALLS[name]), None) is NotImplemented
+    assert call(*(X if a == "x" else 2 ** 80 for a in CALLS[name])) is NotImplemented
+    with pytest.raises(TypeError):
+        call(x=X)
+
+
+def test_a_missing_module_is_an_error(monkeypatch):
+    import sys
+
+    monkeypatch.setattr(hp, "_native", None)
+    monkeypatch.setitem(sys.modules, "megatron.fused_kernels._native", None)
+    monkeypatch.delattr(sys.modules["megatron.fused_kernels"], "_native", raising=False)
+    with pytest.raises(ImportError, match="_native.so"):
+        hp.native()

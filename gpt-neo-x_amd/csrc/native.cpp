@@ -940,7 +940,7 @@ PyObject* py_append_to_cache(PyObject*, PyObject* const* args, Py_ssize_t count)
     END_HANDLE_TH_ERRORS
 }
 
-// linear(x, weight, bias, most rows, most rows of a narrow layer): x W^T (+ bias) of few rows that nobody differentiates
+// linear(x, weight, bias, most rows, most rows of a layer that is narrow or split): x W^T (+ bias) of few rows that nobody differentiates
 PyObject* py_linear(PyObject*, PyObject* const* args, Py_ssize_t count)
 {
     HANDLE_TH_ERRORS
@@ -949,7 +949,7 @@ PyObject* py_linear(PyObject*, PyObject* const* args, Py_ssize_t count)
     int64_t most, most_narrow;
     if (!take_all(args, count, x, w, b, most, most_narrow) || followed() || at::autocast::is_autocast_enabled(at::kCUDA) || x.dim() < 1 || w.dim() != 2 || !is_half(x) || !alike(x, w)) return not_here();
     const int64_t n = w.size(0), k = w.size(1);
-    if (x.size(-1) != k || x.numel() > (std::min(n, k) <= 2048 ? most_narrow : most) * k || k % 32 || k > 16384 || n % 16 || n > (1 << 24) ||
+    if (x.size(-1) != k || x.numel() > (std::min(n, k) <= 2048 || k > 4096 ? most_narrow : most) * k || k % 32 || k > 16384 || n % 16 || n > (1 << 24) ||
         !w.is_contiguous() || !x.is_contiguous() || reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 ||
         reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 || (b && (b->dim() != 1 || b->size(0) != n || !alike(*b, x) || !b->is_contiguous())) ||
         wants_grad({&x, &w}) || (b && wants_grad({&*b})))

@@ -1,28 +1,24 @@
 """``y = x W^T (+ b)`` for the few rows of a decoding step, on the kernel of csrc/linear_decode.hip.
 
 The reference's Column / RowParallelLinear (megatron/mpu/layers.py) call the library GEMM whatever the number of rows. With
-few of them the product is a single read of the weights, and the library's call alone takes the host 25 us (this one 8).
+few of them the product is a single read of the weights, and the library's call alone takes the host 25 us (this one 4).
 
 Where the line lies. On the GPU, weights not in any cache, us here / library:
-    rows           1            4            16            32
-    [2304, 768]    3.7 / 8.6    3.8 / 6.7    4.1 / 6.7     5.0 / 9.5
-    [2048, 2048]   5.1 / 13.0   5.5 / 11.3   6.4 / 11.3    8.3 / 11.5
-    [1024, 4096]   7.3 / 16.5   7.9 / 14.7   10.0 / 14.7   13.7 / 12.1
-    [4096, 4096]   9.7 / 17.6   9.7 / 15.8   11.8 / 15.7   15.4 / 13.3
-    [22016, 4096]  39.5 / 51.5  39.7 / 50.0  40.9 / 50.8   45.3 / 41.5
-    [4096, 11008]  25.4 / 40.1  24.4 / 37.6  26.2 / 37.6   29.1 / 29.8
-    [6144, 4096]   14.4 / 16.3  14.9 / 14.5  16.9 / 14.4   20.8 / 15.3
-    [5120, 5120]   14.8 / 15.6  15.1 / 14.0  16.0 / 15.4   18.3 / 18.2
-    [4096, 14336]  31.2 / 28.2  30.1 / 25.2  32.1 / 25.8   35.6 / 30.9
-    [7680, 2560]   12.8 / 13.3  13.1 / 11.4  14.4 / 11.5   16.9 / 12.1
-    [2560, 10240]  19.4 / 21.5  18.9 / 16.8  20.6 / 17.2   23.3 / 21.5
-Where a side has at most 2048 features the kernel is ahead up to about 24 rows. Larger ones are mixed: with 2560 features a
-wave has five of its eight steps to do and the tiles do not divide among the workgroups (160 for 64, 480 for 256). They are
-taken all the same up to 16 rows, because it is the host that a step waits for until its cache is long: a layer of 2560
-features called step by step takes 222 us here and 272 to 282 with those products in the library, with 1 to 8 sequences of up
-to 2000 positions, and 16 of 200. Where the GPU is what is waited for the library is ahead there: 16 sequences of 2000 positions
-336 / 320 us, and in a captured graph 71 / 76 us with one sequence, 90 / 91 with four, 195 / 176 with eight of 2000, 336 / 314
-with 16. With 4096 features, 8 heads of keys: 247 / 274 us step by step, 178 / 175 in a graph (16 of 2000)."""
+    rows           1            4            16            24            32
+    [2304, 768]    3.7 / 5.1    3.7 / 5.2    3.8 / 5.2     4.3 / 7.0     4.4 / 7.0
+    [2048, 2048]   5.0 / 11.0   4.9 / 11.0   5.7 / 10.9    7.1 / 10.9    7.8 / 11.1
+    [1024, 4096]   6.5 / 14.6   6.6 / 14.4   8.5 / 14.4    11.1 / 14.2   12.6 / 11.8
+    [4096, 4096]   9.4 / 15.5   9.8 / 15.4   10.9 / 15.5   13.1 / 13.2   14.6 / 13.1
+    [12288, 4096]  20.5 / 27.5  21.0 / 28.3  22.7 / 28.3   24.9 / 23.5   26.7 / 24.2
+    [22016, 4096]  34.2 / 51.7  34.9 / 52.1  37.5 / 52.5   40.2 / 43.4   42.1 / 43.9
+    [6144, 4096]   13.1 / 15.6  13.5 / 15.6  15.3 / 15.5   17.5 / 16.0   18.7 / 16.3
+    [7680, 2560]   10.1 / 12.0  10.2 / 12.0  11.6 / 11.9   13.0 / 12.6   14.2 / 12.9
+    [5120, 5120]   14.1 / 14.4  14.4 / 14.9  15.1 / 17.4   16.2 / 20.2   16.8 / 20.6
+    [2560, 10240]  14.3 / 19.5  14.8 / 19.4  15.8 / 19.6   17.8 / 22.3   18.2 / 22.4
+    [4096, 11008]  20.2 / 37.6  20.5 / 37.9  22.2 / 37.9   23.9 / 31.2   24.8 / 30.8
+    [4096, 14336]  24.6 / 25.8  25.2 / 25.9  26.8 / 26.9   28.7 / 31.2   30.7 / 33.4
+Up to 16 rows the kernel is ahead everywhere, up to 32 where a side has at most 2048 features or where four workgroups share the
+contraction (more than 4096 features); in between the library catches up."""
 from typing import Optional
 
 import torch
@@ -32,14 +28,14 @@ from ..fused_kernels import _hotpath as _hp
 from .fused_attention import plain
 
 MAX_ROWS = 16          # of any layer
-MAX_ROWS_NARROW = 32   # where one of its sides has at most 2048 features
+MAX_ROWS_NARROW = 32   # where one of its sides has at most 2048 features, or more than 4096 come in
 MAX_FEATURES = 16384
 
 
 def _few_rows(x, weight, bias):
     n, k = weight.shape
     dtype = x.dtype
-    return (x.numel() <= (MAX_ROWS_NARROW if min(n, k) <= 2048 else MAX_ROWS) * k and x.is_cuda and x.dim() > 0 and x.size(-1) == k and x.numel() > 0
+    return (x.numel() <= (MAX_ROWS_NARROW if min(n, k) <= 2048 or k > 4096 else MAX_ROWS) * k and x.is_cuda and x.dim() > 0 and x.size(-1) == k and x.numel() > 0
             and (dtype is torch.bfloat16 or dtype is torch.float16) and weight.dtype is dtype and weight.device == x.device
             and k % 32 == 0 and k <= MAX_FEATURES and n % 16 == 0 and 0 < n <= 1 << 24 and weight.is_contiguous()
             and x.is_contiguous()

@@ -31,6 +31,21 @@ def test_against_fp64(dtype, n, k, rows):
         assert torch.equal(got, fused_linear.linear(x, w, bias))
 
 
+@pytest.mark.parametrize("n,k", [(20496, 96), (12304, 288), (8208, 2080), (4128, 4064), (272, 4192), (1040, 12320)])
+@pytest.mark.parametrize("rows", [1, 16, 18])
+def test_several_tiles_and_odd_steps(n, k, rows):
+    """Up to six tiles for a workgroup, pieces of one step among those of two, waves with none; a bias that starts in the middle
+    of a word."""
+    from megatron.model import fused_linear
+
+    x, w = util.randn((rows, k), torch.bfloat16, seed=1).to(DEV), util.randn((n, k), torch.bfloat16, seed=2).to(DEV)
+    b = util.randn((n + 1,), torch.bfloat16, seed=3, std=math.sqrt(k)).to(DEV)
+    for bias in (b[1:], b[:-1]):
+        want = x.double() @ w.double().t() + bias.double()
+        got = fused_linear.linear(x, w, bias)
+        assert (got.double() - want).norm() <= 2.0 ** -8 / math.sqrt(3) * want.norm()
+
+
 def test_an_infinite_weight_reaches_its_own_result_only():
     from megatron.model.fused_linear import linear
 

@@ -14,13 +14,26 @@
 //
 // Measured (us, causal, forward / backward; products and softmax separately before, both per pass of the module; cards differ
 // by up to 8 %):
-//   [8192, 1, 32 heads, 8 of keys, 128] bf16   591 / 1876 (931 / 1026 TFLOP/s)   whole pass 5786 -> 2357
-//   [2048, 8, 16, 128] bf16                    175 / 585  (788 / 823)            about 1930 -> 890
-//   [1024, 4, 12, 64] fp16                     29 / 73    (224 / 312)            whole pass 428 -> 126 to 163, with the host
-//   [1531, 1, 32, 128] bf16, by mask           68 + 5 for the bits               650 -> 73
+//   [8192, 1, 32 heads, 8 of keys, 128] bf16   490 / 1738 (1122 / 1107 TFLOP/s)  whole pass 5786 -> 2230
+//   [2048, 8, 16, 128] bf16                    148 / 512  (930 / 940)            about 1930 -> 690
+//   [1024, 4, 12, 64] fp16                     19 / 52    (340 / 435)            whole pass 428 -> 84, with the host
+//   [1531, 1, 32, 128] bf16, by mask           48 + 5 for the bits               650 -> 53
+// Of that the reads ahead of the products and the probabilities between them (forward, us): [8192, 1, 32 on 8, 128] 527 -> 486,
+// [4096, 2, 16, 96] 126 -> 110, [4096, 2, 32, 80] 219 -> 208, [2048, 8, 16, 128] 157 -> 148, [8192, 1, 12, 64] 148 -> 145; by mask
+// (its bits ahead too) [1531, 1, 32, 128] 54 -> 48. Gradient
+// of q the same way: both kernels 1754 -> 1738, [1024, 4, 12, 64] 53.3 -> 51.9. In the kernel of k and v there are no registers
+// for it (one pair of operands ahead: no change, two: 13 registers spilled and 2 % slower).
 #include "attention.hpp"
 
 namespace nhp {
+
+struct First {
+    static constexpr int value = 0;
+};
+struct Second {
+    static constexpr int value = 1;
+};
+constexpr int kReadsAhead = 4;   // reads of keys that are under way in the forward kernel (6: no faster)
 
 // MODE of the forward kernel
 constexpr int kCausal = 0;   // key k is visible to query q when q + shift - window <= k <= q + shift, by index
@@ -96,22 +109,39 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_kernel(AttnFwdArgs a)
             kload.load(kbase + (int64_t)kt * 64 * a.k_s, lds + buf * G::kTileBytes, left);
             vload.load(vbase + (int64_t)kt * 64 * a.v_s, lds + (2 + buf) * G::kTileBytes, left);
         };
-        int kt = next_tile(kt_lo), buf = 0;
-        if (kt < kt_hi) fetch(kt, 0);
-        while (kt < kt_hi) {
+        // Mask bits are asked for a tile ahead, before that tile, and waited for together with it: asked for where they are
+        // needed, they would be waited for behind the tile that is under way.
+        uint64_t word = 0;
+        auto fetch_word = [&](int kt) {
+            if constexpr (MODE == kBits) word = bits[(int64_t)qi * kt_hi + kt];
+        };
+        int kt = next_tile(kt_lo);
+        if (kt < kt_hi) {
+            fetch_word(kt);
+            fetch(kt, 0);
+        }
+        // (two tiles a turn of the loop: the addresses in LDS are then those of the first plus a constant)
+        auto turn = [&](auto which) {
+            constexpr int buf = decltype(which)::value;
             wait_lds_loads();
+            if constexpr (MODE == kBits) asm volatile("" : "+v"(word));
+            const uint64_t w = word;
             __syncthreads();
             const int following = next_tile(kt + 1);
-            if (following < kt_hi) fetch(following, buf ^ 1);
+            if (following < kt_hi) {
+                fetch_word(following);
+                fetch(following, buf ^ 1);
+            }
             const int key0 = kt * 64;
             const char* kt_lds = lds + buf * G::kTileBytes;
             const char* vt_lds = lds + (2 + buf) * G::kTileBytes;
             const bool active = MODE == kBits || (key0 <= wave_hi && key0 + 63 >= wave_lo);
             if (active) {
                 f32x16 s[2] = {f32x16{}, f32x16{}};
-                // the wave that multiplies goes first, so that the other one of the SIMD is left with its softmax
-                // (4 to 5 % of the kernel at 64, 80 and 128 features: 568 -> 544 us at 8192 positions, 32 heads of 128;
-                // no gain in the kernels of the gradients)
+                // The compiler would read two operands, wait for them and multiply them, sixteen times over: the reads are
+                // dealt out here, four of them ahead of the products (sched_group_barrier: 0x100 reads, 0x008 products).
+                // The wave that multiplies goes first, so that the other one of the SIMD is left with its softmax (4 to 5 %
+                // of the kernel, no gain in the kernels of the gradients).
                 __builtin_amdgcn_s_setprio(1);
 #pragma unroll
                 for (int t = 0; t < G::kSteps; ++t) {
@@ -121,9 +151,15 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_kernel(AttnFwdArgs a)
                         s[n] = F::mma(kf, qf[t], s[n]);
                     }
                 }
+                __builtin_amdgcn_sched_group_barrier(0x100, kReadsAhead, 0);
+#pragma unroll
+                for (int i = 0; i < 2 * G::kSteps - kReadsAhead; ++i) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                }
+                __builtin_amdgcn_sched_group_barrier(0x008, kReadsAhead, 0);
                 __builtin_amdgcn_s_setprio(0);
                 if constexpr (MODE == kBits) {
-                    const uint64_t w = bits[(int64_t)qi * kt_hi + kt];
 #pragma unroll
                     for (int n = 0; n < 2; ++n) {
                         const uint32_t wn = (uint32_t)(w >> (32 * n)) >> (4 * half);
@@ -148,6 +184,18 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_kernel(AttnFwdArgs a)
                             if (key > last || (MODE == kCausal && key < first)) s[n][i] = kNegInf;
                         }
                 }
+                // Values by 16 keys: those of the first are read ahead of the softmax, those of the next while one lot is
+                // multiplied, and between those products the next eight probabilities are formed (sched_barrier keeps the
+                // order as it is written).
+                u32x4 vf[2][G::kDTiles];
+                auto read_v = [&](int ks) {
+#pragma unroll
+                    for (int d = 0; d < G::kDTiles; ++d)
+                        vf[ks & 1][d] = lds_read_tr(vt_lds + (vrow ^ (d << 6)) + ks * 16 * G::kRowBytes,
+                                                    vt_lds + (vrow ^ (d << 6 | 32)) + (ks * 16 + 8) * G::kRowBytes);
+                };
+                read_v(0);
+                __builtin_amdgcn_sched_barrier(0);
                 const float c = MODE == kBits ? 1.0f : a.scale_log2;
                 float mx = fmaxf(s[0][0], s[1][0]);
 #pragma unroll
@@ -165,29 +213,40 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_kernel(AttnFwdArgs a)
                         for (int i = 0; i < 16; ++i) o[d][i] *= alpha;
                 }
                 float sum = 0.0f;
+                u32x4 pf;
+                auto element = [&](int i) {
+                    const float x = exp2_raw(fmaf(s[i >> 4][i & 15], c, -m));
+                    s[i >> 4][i & 15] = x;
+                    sum += x;
+                };
 #pragma unroll
-                for (int n = 0; n < 2; ++n)
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) {
-                        s[n][i] = exp2_raw(fmaf(s[n][i], c, -m));
-                        sum += s[n][i];
-                    }
-                l += sum;
+                for (int i = 0; i < 8; ++i) element(i);
+                pf = F::pack8(s[0], 0);
                 __builtin_amdgcn_s_setprio(1);
 #pragma unroll
                 for (int ks = 0; ks < 4; ++ks) {
-                    const u32x4 pf = F::pack8(s[ks >> 1], (ks & 1) * 8);
+                    if (ks < 3) read_v(ks + 1);
+                    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                     for (int d = 0; d < G::kDTiles; ++d) {
-                        const u32x4 vf = lds_read_tr(vt_lds + (vrow ^ (d << 6)) + ks * 16 * G::kRowBytes,
-                                                     vt_lds + (vrow ^ (d << 6 | 32)) + (ks * 16 + 8) * G::kRowBytes);
-                        o[d] = F::mma(vf, pf, o[d]);
+                        o[d] = F::mma(vf[ks & 1][d], pf, o[d]);
+                        if (ks < 3) {
+#pragma unroll
+                            for (int i = 8 * d / G::kDTiles; i < 8 * (d + 1) / G::kDTiles; ++i) element((ks + 1) * 8 + i);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
                     }
+                    if (ks < 3) pf = F::pack8(s[(ks + 1) >> 1], ((ks + 1) & 1) * 8);
                 }
+                l += sum;
                 __builtin_amdgcn_s_setprio(0);
             }
             kt = following;
-            buf ^= 1;
+        };
+        while (kt < kt_hi) {
+            turn(First{});
+            if (kt >= kt_hi) break;
+            turn(Second{});
         }
         if constexpr (MODE == kBits) {
             // A row without a visible key (or with nothing but scores as low as the fill value) is an average over the
@@ -322,24 +381,44 @@ __global__ void __launch_bounds__(256, 2) attn_dq_kernel(AttnBwdArgs a)
 #pragma unroll
     for (int d = 0; d < G::kDTiles; ++d) dq[d] = f32x16{};
     fetch(kt_lo, 0);
-    for (int kt = kt_lo; kt < kt_hi; ++kt) {
-        const int buf = (kt - kt_lo) & 1;
+    auto turn = [&](auto which, int kt) {
+        constexpr int buf = decltype(which)::value;
         wait_lds_loads();
         __syncthreads();
         if (kt + 1 < kt_hi) fetch(kt + 1, buf ^ 1);
         const int key0 = kt * 64;
-        if (key0 > wave_hi || key0 + 63 < wave_lo) continue;
+        if (key0 > wave_hi || key0 + 63 < wave_lo) return;
         const char* kt_lds = lds + buf * G::kTileBytes;
         const char* vt_lds = lds + (2 + buf) * G::kTileBytes;
         const bool edge = key0 + 63 >= a.sk || key0 + 63 > qw + a.shift || key0 < wave_lo + 31;
 #pragma unroll
         for (int n = 0; n < 2; ++n) {
+            // reads ahead of the products and probabilities between them, as in the forward kernel
             f32x16 s{}, dp{};
+            constexpr int kAhead = 3;
+            u32x4 kf[kAhead], vf[kAhead];
+            auto read = [&](int t) {
+                kf[t % kAhead] = lds_read16(kt_lds + (krow ^ (t << 5)) + n * 32 * G::kRowBytes);
+                vf[t % kAhead] = lds_read16(vt_lds + (krow ^ (t << 5)) + n * 32 * G::kRowBytes);
+            };
+            u32x4 tf[2][G::kDTiles];
+            auto read_t = [&](int ks) {
+                const char* base = kt_lds + (n * 32 + ks * 16) * G::kRowBytes;
+#pragma unroll
+                for (int d = 0; d < G::kDTiles; ++d)
+                    tf[ks][d] = lds_read_tr(base + (ktr ^ (d << 6)), base + (ktr ^ (d << 6 | 32)) + 8 * G::kRowBytes);
+            };
+#pragma unroll
+            for (int t = 0; t < kAhead && t < G::kSteps; ++t) read(t);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int t = 0; t < G::kSteps; ++t) {
-                s = F::mma(lds_read16(kt_lds + (krow ^ (t << 5)) + n * 32 * G::kRowBytes), qf[t], s);
-                dp = F::mma(lds_read16(vt_lds + (krow ^ (t << 5)) + n * 32 * G::kRowBytes), gf[t], dp);
+                s = F::mma(kf[t % kAhead], qf[t], s);
+                dp = F::mma(vf[t % kAhead], gf[t], dp);
+                if (t + kAhead < G::kSteps) read(t + kAhead);
+                __builtin_amdgcn_sched_barrier(0);
             }
+            read_t(0);
             if (edge) {
                 const int q = qw + ql + a.shift;
                 const int last = min(a.sk - 1, q) - key0 - 4 * half, first = q - a.window - key0 - 4 * half;
@@ -349,21 +428,30 @@ __global__ void __launch_bounds__(256, 2) attn_dq_kernel(AttnBwdArgs a)
                     if (key > last || key < first) s[i] = kNegInf;
                 }
             }
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
+            auto element = [&](int i) {
                 const float p = exp2_raw(fmaf(s[i], a.scale_log2, -lse));
                 s[i] = p * (dp[i] - delta);
-            }
+            };
 #pragma unroll
-            for (int ks = 0; ks < 2; ++ks) {
-                const u32x4 f = F::pack8(s, ks * 8);
+            for (int i = 0; i < 8; ++i) element(i);
+            u32x4 f = F::pack8(s, 0);
+            read_t(1);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int d = 0; d < G::kDTiles; ++d) {
-                    const char* base = kt_lds + (n * 32 + ks * 16) * G::kRowBytes;
-                    dq[d] = F::mma(lds_read_tr(base + (ktr ^ (d << 6)), base + (ktr ^ (d << 6 | 32)) + 8 * G::kRowBytes), f, dq[d]);
-                }
+            for (int d = 0; d < G::kDTiles; ++d) {
+                dq[d] = F::mma(tf[0][d], f, dq[d]);
+#pragma unroll
+                for (int i = 8 * d / G::kDTiles; i < 8 * (d + 1) / G::kDTiles; ++i) element(8 + i);
+                __builtin_amdgcn_sched_barrier(0);
             }
+            f = F::pack8(s, 8);
+#pragma unroll
+            for (int d = 0; d < G::kDTiles; ++d) dq[d] = F::mma(tf[1][d], f, dq[d]);
         }
+    };
+    for (int kt = kt_lo; kt < kt_hi; kt += 2) {
+        turn(First{}, kt);
+        if (kt + 1 < kt_hi) turn(Second{}, kt + 1);
     }
     if (qw + ql < a.sq)
         store_transposed<DT, HD>(a.dq + b * a.dq_b + h * a.dq_h + (int64_t)(qw + ql) * a.dq_s, nullptr, dq, a.scale, half);

@@ -15,7 +15,7 @@
 // 1 / (1 + e^-v) with the hardware exp2 and reciprocal; erf from the device
 // math library.
 
-#include "common.hpp"
+#include "activation.hpp"
 
 #include <cstdlib>
 
@@ -24,45 +24,6 @@ namespace nhp {
 constexpr int kGatedThreads = 256;
 constexpr int kGatedU = 2;
 constexpr int kGatedMaxTw = 64;
-
-enum GateAct {
-    kActSwish = NHP_GATE_SWISH,
-    kActGelu = NHP_GATE_GELU,
-    kActRelu = NHP_GATE_RELU,
-    kActSigmoid = NHP_GATE_SIGMOID,
-    kActIdentity = NHP_GATE_IDENTITY
-};
-
-__device__ __forceinline__ float sigmoid_fast(float v)
-{
-    return __builtin_amdgcn_rcpf(1.0f + exp2_raw(-v * kLog2e));
-}
-
-// act(g) and d act / d g
-template <int ACT>
-__device__ __forceinline__ void gate_eval(float g, float& act, float& dact)
-{
-    if constexpr (ACT == kActSwish) {
-        const float s = sigmoid_fast(g);
-        act = g * s;
-        dact = s * (1.0f + g * (1.0f - s));
-    } else if constexpr (ACT == kActGelu) {
-        const float cdf = 0.5f * (1.0f + erff(g * 0.70710678118654752f));
-        const float pdf = 0.3989422804014327f * exp2_raw((-0.5f * kLog2e) * g * g);
-        act = g * cdf;
-        dact = cdf + g * pdf;
-    } else if constexpr (ACT == kActRelu) {
-        act = g > 0.0f ? g : 0.0f;
-        dact = g > 0.0f ? 1.0f : 0.0f;
-    } else if constexpr (ACT == kActSigmoid) {
-        const float s = sigmoid_fast(g);
-        act = s;
-        dact = s * (1.0f - s);
-    } else {
-        act = g;
-        dact = 1.0f;
-    }
-}
 
 // ---------------------------------------------------------------------------
 // BWD = false: out[row, c] = act(g) * x

@@ -1,4 +1,5 @@
-// y = x W^T (+ bias) for the few rows of a decoding step (at most 32), 16-bit storage, fp32 sums.
+// y = x W^T (+ bias) for the few rows of a decoding step (at most 32), 16-bit storage, fp32 sums; also with the activation or the
+// residual addition that follows it (LinearEnd).
 //
 // Such a product reads every weight once for a handful of rows: the weights' bytes are its time, and the matrix cores idle.
 // What a CU can have on the way is the limit, so x must not take much of it: read again for every 16 weight rows it costs
@@ -17,6 +18,7 @@
 //
 // Rows of the matrix instruction (16 x 16 x 32) are weight rows, its columns the rows of x. A lane takes 16 consecutive
 // bytes of its row per instruction and x in the same order, which the contraction does not mind.
+#include "activation.hpp"
 #include "attention.hpp"
 
 namespace nhp {
@@ -27,7 +29,15 @@ struct LinearArgs {
     float* parts;   // with splits > 1: [splits][m][n]
     int m, n, k, splits;
     int bias_words;   // the bias starts at a multiple of four bytes
+    int act;          // the gate's function (kGatedRows)
+    const uint16_t *x1, *bias1, *residual;   // kAddRows: [m, n], [n], [m, n], the first two may be null
 };
+
+// What is done with a sum: nothing but the bias; gelu(bias + sum); act(gate) * value, the gate being the sum n / 2 features on;
+// residual + (sum + bias), or residual + ((x1 + bias1) + (sum + bias)). In all of them the sum is rounded to the storage
+// type first and the rest rounded where the kernels for it round (pointwise.hip, gated.hip): the same bits with a launch less
+// (a layer of 768 features, one sequence: a step 100 -> 91 us; 4096 features, gated, 16 sequences: 312 -> 307).
+enum LinearEnd { kPlainRows, kGeluRows, kGatedRows, kAddRows };
 
 constexpr int kLinearWaves = 8, kLinearBlocks = 256, kLinearSteps = 16;   // steps of 32 features that a wave has at most
 constexpr int kLinearWhole = kLinearSteps * kLinearWaves * 32, kLinearSplits = 4;   // features of an unsplit product; splits beyond
@@ -39,8 +49,60 @@ __device__ __forceinline__ void wait_pieces()
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
 }
 
+template <int DT>
+__device__ __forceinline__ float bias_of(const LinearArgs& a, int tile, int col)
+{
+    if (!a.bias) return 0.0f;
+    if (!a.bias_words) return Half2<DT>::from_bits(a.bias[tile * 16 + col]);
+    // by scalar loads (constant memory at a uniform address): a vector load would be waited for behind the pieces that are
+    // under way
+    typedef const __attribute__((address_space(4))) uint32_t* Words;
+    const Words words = (Words)(uintptr_t)(a.bias + __builtin_amdgcn_readfirstlane(tile) * 16);
+    uint32_t w = 0;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        uint32_t word = words[q];
+        asm volatile("" : "+s"(word));   // the value, not its address, is what is picked
+        w = col >> 1 == q ? word : w;
+    }
+    return col & 1 ? Half2<DT>::hi(w) : Half2<DT>::lo(w);
+}
+
+__device__ __forceinline__ float gate_of(int act, float g)
+{
+    float value, slope;
+    switch (act) {
+    case kActSwish: gate_eval<kActSwish>(g, value, slope); break;
+    case kActGelu: gate_eval<kActGelu>(g, value, slope); break;
+    case kActRelu: gate_eval<kActRelu>(g, value, slope); break;
+    case kActSigmoid: gate_eval<kActSigmoid>(g, value, slope); break;
+    default: gate_eval<kActIdentity>(g, value, slope); break;
+    }
+    return value;
+}
+
+// The result of a row and feature; `at`: its place in y, `bias`: that of the feature, `gate`: the second sum of kGatedRows.
+template <int DT, int END>
+__device__ __forceinline__ float finish(const LinearArgs& a, float sum, float bias, float gate, int64_t at, int feature)
+{
+    using H = Half2<DT>;
+    if constexpr (END == kPlainRows) {
+        return a.bias ? sum + bias : sum;
+    } else if constexpr (END == kGeluRows) {
+        return gelu_fwd(bias + H::round(sum));
+    } else if constexpr (END == kGatedRows) {
+        return gate_of(a.act, H::round(gate)) * H::round(sum);
+    } else {
+        const float v = H::round(sum) + bias, residual = H::from_bits(a.residual[at]);
+        if (!a.x1) return residual + v;
+        float t = H::from_bits(a.x1[at]);
+        if (a.bias1) t = H::round(t + H::from_bits(a.bias1[feature]));
+        return residual + H::round(t + v);
+    }
+}
+
 // MT: tiles of 16 rows of x
-template <int DT, int MT>
+template <int DT, int MT, int END>
 __global__ void __launch_bounds__(64 * kLinearWaves) linear_decode_kernel(LinearArgs a)
 {
     __shared__ __attribute__((aligned(1024))) char ring[kLinearWaves * kRing * kPieceBytes];
@@ -51,7 +113,8 @@ __global__ void __launch_bounds__(64 * kLinearWaves) linear_decode_kernel(Linear
     // groups of 32 features are dealt out evenly to the waves of all splits, a wave's being consecutive
     const int groups = a.k / 32, shares = kLinearWaves * a.splits, share = split * kLinearWaves + wave;
     const int lo = __builtin_amdgcn_readfirstlane(groups * share / shares), count = __builtin_amdgcn_readfirstlane(groups * (share + 1) / shares - lo);
-    const int tiles = a.n / 16, pieces = (count + 1) / 2;
+    constexpr int kParts = END == kGatedRows ? 2 : 1;   // tiles of a result: its values, its gates
+    const int tiles = a.n / 16 / kParts, pieces = (count + 1) / 2;
 
     u32x4 x[MT][kLinearSteps];
 #pragma unroll
@@ -79,13 +142,16 @@ __global__ void __launch_bounds__(64 * kLinearWaves) linear_decode_kernel(Linear
             TileLoader<128>::issue(reinterpret_cast<const char*>(w + (int64_t)i * 8 * a.k), offset, mine_at + at * kPieceBytes + i * 1024);
     };
     // all pieces of all tiles, one after the other
-    int left = first_tile < tiles ? ((tiles - 1 - first_tile) / stride + 1) * pieces : 0;
-    int next_tile = first_tile, next_piece = 0, next_at = 0;
+    int left = first_tile < tiles ? ((tiles - 1 - first_tile) / stride + 1) * pieces * kParts : 0;
+    int next_tile = first_tile, next_part = 0, next_piece = 0, next_at = 0;
     auto fetch_next = [&]() {
-        fetch(next_tile, next_piece, next_at);
+        fetch(next_tile + next_part * tiles, next_piece, next_at);
         if (++next_piece == pieces) {
             next_piece = 0;
-            next_tile += stride;
+            if (++next_part == kParts) {
+                next_part = 0;
+                next_tile += stride;
+            }
         }
         next_at = next_at + 1 == kRing ? 0 : next_at + 1;
     };
@@ -95,82 +161,125 @@ __global__ void __launch_bounds__(64 * kLinearWaves) linear_decode_kernel(Linear
 
     int buf = 0, at = 0;
     for (int tile = first_tile; tile < tiles; tile += stride) {
-        f32x4 acc[MT];
+        float value = 0.0f;   // kGatedRows: the first of the two sums
+        for (int part = 0; part < kParts; ++part) {
+            f32x4 acc[MT];
 #pragma unroll
-        for (int r = 0; r < MT; ++r) acc[r] = f32x4{};
+            for (int r = 0; r < MT; ++r) acc[r] = f32x4{};
 #pragma unroll
-        for (int p = 0; p < kLinearSteps / 2; ++p) {
-            if (p >= pieces) continue;
-            if (left >= kRing - 1) wait_pieces<2 * (kRing - 2)>();
-            else wait_pieces<0>();
-            if (left >= kRing) fetch_next();
-            --left;
-            const char* f = frag + at * kPieceBytes;
-            at = at + 1 == kRing ? 0 : at + 1;
-            const u32x4 w_lo = lds_read16(f + ((g ^ sw) << 4)), w_hi = lds_read16(f + (((4 + g) ^ sw) << 4));
+            for (int p = 0; p < kLinearSteps / 2; ++p) {
+                if (p >= pieces) continue;
+                if (left >= kRing - 1) wait_pieces<2 * (kRing - 2)>();
+                else wait_pieces<0>();
+                if (left >= kRing) fetch_next();
+                --left;
+                const char* f = frag + at * kPieceBytes;
+                at = at + 1 == kRing ? 0 : at + 1;
+                const u32x4 w_lo = lds_read16(f + ((g ^ sw) << 4)), w_hi = lds_read16(f + (((4 + g) ^ sw) << 4));
 #pragma unroll
-            for (int r = 0; r < MT; ++r) acc[r] = mma16<DT>(w_lo, x[r][2 * p], acc[r]);
-            if (2 * p + 1 < count)
+                for (int r = 0; r < MT; ++r) acc[r] = mma16<DT>(w_lo, x[r][2 * p], acc[r]);
+                if (2 * p + 1 < count)
 #pragma unroll
-                for (int r = 0; r < MT; ++r) acc[r] = mma16<DT>(w_hi, x[r][2 * p + 1], acc[r]);
-        }
-#pragma unroll
-        for (int r = 0; r < MT; ++r)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) sums[buf][wave][r * 16 + r16][4 * g + j] = acc[r][j];
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        // (a wave is at most one tile ahead of those that add up here: the other half of the sums is free)
-        const int row = tid >> 4, col = tid & 15;
-        if (row < a.m && row < 16 * MT) {
-            float v = 0.0f;
-#pragma unroll
-            for (int s = 0; s < kLinearWaves; ++s) v += sums[buf][s][row][col];
-            const int64_t to = (int64_t)row * a.n + tile * 16 + col;
-            if (a.splits > 1) {
-                a.parts[(int64_t)split * a.m * a.n + to] = v;
-            } else {
-                if (a.bias && a.bias_words) {
-                    // by scalar loads: a vector load would be waited for behind the pieces that are under way
-                    const uint32_t* words = reinterpret_cast<const uint32_t*>(a.bias + tile * 16);
-                    uint32_t w = words[0];
-#pragma unroll
-                    for (int q = 1; q < 8; ++q) w = col >> 1 == q ? words[q] : w;
-                    v += col & 1 ? Half2<DT>::hi(w) : Half2<DT>::lo(w);
-                } else if (a.bias) {
-                    v += Half2<DT>::from_bits(a.bias[tile * 16 + col]);
-                }
-                a.y[to] = Half2<DT>::to_bits(v);
+                    for (int r = 0; r < MT; ++r) acc[r] = mma16<DT>(w_hi, x[r][2 * p + 1], acc[r]);
             }
+#pragma unroll
+            for (int r = 0; r < MT; ++r)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) sums[buf][wave][r * 16 + r16][4 * g + j] = acc[r][j];
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            // (a wave is at most one tile ahead of those that add up here: the other half of the sums is free)
+            const int row = tid >> 4, col = tid & 15;
+            if (row < a.m && row < 16 * MT) {
+                float v = 0.0f;
+#pragma unroll
+                for (int s = 0; s < kLinearWaves; ++s) v += sums[buf][s][row][col];
+                if (a.splits > 1) {
+                    a.parts[((int64_t)split * a.m + row) * a.n + (tile + part * tiles) * 16 + col] = v;
+                } else if (part + 1 < kParts) {
+                    value = v;
+                } else {
+                    const int64_t to = (int64_t)row * (a.n / kParts) + tile * 16 + col;
+                    const float bias = END == kGatedRows ? 0.0f : bias_of<DT>(a, tile, col);
+                    float result = finish<DT, END>(a, kParts == 2 ? value : v, bias, v, to, tile * 16 + col);
+                    asm volatile("" : "+v"(result));   // in fp32, not a product that is rounded to fp16 at once
+                    a.y[to] = Half2<DT>::to_bits(result);
+                }
+            }
+            buf ^= 1;
         }
-        buf ^= 1;
     }
 }
 
 // Adds the splits up, four columns per thread.
-template <int DT>
+template <int DT, int END>
 __global__ void __launch_bounds__(256) linear_merge_kernel(LinearArgs a)
 {
+    constexpr int kParts = END == kGatedRows ? 2 : 1;
+    const int width = a.n / kParts;
     const int64_t size = (int64_t)a.m * a.n, at = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
-    if (at >= size) return;
-    f32x4 v{};
+    if (at >= size / kParts) return;
+    const int row = (int)(at / width), feature = (int)(at % width);
+    f32x4 v[kParts];
 #pragma unroll
-    for (int s = 0; s < kLinearSplits; ++s) v += *reinterpret_cast<const f32x4*>(a.parts + s * size + at);
-    if (a.bias)
+    for (int p = 0; p < kParts; ++p) {
+        v[p] = f32x4{};
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] += Half2<DT>::from_bits(a.bias[(int)(at % a.n) + j]);
-    *reinterpret_cast<u32x2*>(a.y + at) = u32x2{Half2<DT>::pack(v[0], v[1]), Half2<DT>::pack(v[2], v[3])};
+        for (int s = 0; s < kLinearSplits; ++s)
+            v[p] += *reinterpret_cast<const f32x4*>(a.parts + s * size + (int64_t)row * a.n + p * width + feature);
+    }
+    float out[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const float bias = END != kGatedRows && a.bias ? Half2<DT>::from_bits(a.bias[feature + j]) : 0.0f;
+        out[j] = finish<DT, END>(a, v[0][j], bias, v[kParts - 1][j], at + j, feature + j);
+    }
+    *reinterpret_cast<u32x2*>(a.y + at) = u32x2{Half2<DT>::pack(out[0], out[1]), Half2<DT>::pack(out[2], out[3])};
 }
 
-template <int DT>
+template <int DT, int END>
 static int launch_linear(const LinearArgs& a, hipStream_t st)
 {
     launch_prepare();
-    const int tiles = a.n / 16, most = kLinearBlocks / a.splits;
+    const int width = END == kGatedRows ? a.n / 2 : a.n, tiles = width / 16, most = kLinearBlocks / a.splits;
     const dim3 blocks((unsigned)((tiles < most ? tiles : most) * a.splits)), threads(64 * kLinearWaves);
-    if (a.m <= 16) linear_decode_kernel<DT, 1><<<blocks, threads, 0, st>>>(a);
-    else linear_decode_kernel<DT, 2><<<blocks, threads, 0, st>>>(a);
-    if (a.splits > 1) linear_merge_kernel<DT><<<dim3((unsigned)(((int64_t)a.m * a.n / 4 + 255) / 256)), dim3(256), 0, st>>>(a);
+    if (a.m <= 16) linear_decode_kernel<DT, 1, END><<<blocks, threads, 0, st>>>(a);
+    else linear_decode_kernel<DT, 2, END><<<blocks, threads, 0, st>>>(a);
+    if (a.splits > 1) linear_merge_kernel<DT, END><<<dim3((unsigned)(((int64_t)a.m * width / 4 + 255) / 256)), dim3(256), 0, st>>>(a);
     return launch_result();
+}
+
+template <int END>
+static int linear_rows(LinearArgs a, int dtype, void* stream)
+{
+    if (!a.y || !a.x || !a.w) return NHP_ERR_NULL;
+    if (!ptr_aligned16(a.x) || !ptr_aligned16(a.w) || !ptr_aligned16(a.y) || !ptr_aligned16(a.parts)) return NHP_ERR_SHAPE;
+    a.splits = a.k > kLinearWhole ? kLinearSplits : 1;
+    if (a.splits > 1 && !a.parts) return NHP_ERR_NULL;
+    a.bias_words = (reinterpret_cast<uintptr_t>(a.bias) & 3) == 0;
+    if (dtype == NHP_BF16) return launch_linear<NHP_BF16, END>(a, static_cast<hipStream_t>(stream));
+    if (dtype == NHP_F16) return launch_linear<NHP_F16, END>(a, static_cast<hipStream_t>(stream));
+    return NHP_ERR_DTYPE;
+}
+
+static bool linear_sizes_ok(int64_t rows, int64_t out_features, int64_t in_features, int64_t multiple)
+{
+    return rows >= 1 && rows <= 32 && out_features >= multiple && out_features % multiple == 0 && out_features <= (1 << 24) &&
+           in_features >= 32 && in_features % 32 == 0 && in_features <= kLinearWhole * kLinearSplits;
+}
+
+static LinearArgs linear_args(void* y, const void* x, const void* weight, const void* bias, void* workspace, int64_t rows,
+                              int64_t out_features, int64_t in_features)
+{
+    LinearArgs a{};
+    a.y = static_cast<uint16_t*>(y);
+    a.x = static_cast<const uint16_t*>(x);
+    a.w = static_cast<const uint16_t*>(weight);
+    a.bias = static_cast<const uint16_t*>(bias);
+    a.parts = static_cast<float*>(workspace);
+    a.m = (int)rows;
+    a.n = (int)out_features;
+    a.k = (int)in_features;
+    return a;
 }
 
 }  // namespace nhp
@@ -187,19 +296,35 @@ int nhp_linear_decode(void* y, const void* x, const void* weight, const void* bi
                       int64_t out_features, int64_t in_features, int dtype, void* stream)
 {
     using namespace nhp;
+    if (!linear_sizes_ok(rows, out_features, in_features, 16)) return !y || !x || !weight ? NHP_ERR_NULL : NHP_ERR_SHAPE;
+    return linear_rows<kPlainRows>(linear_args(y, x, weight, bias, workspace, rows, out_features, in_features), dtype, stream);
+}
+
+int nhp_linear_decode_act(void* y, const void* x, const void* weight, const void* bias, void* workspace, int64_t rows,
+                          int64_t out_features, int64_t in_features, int act, int dtype, void* stream)
+{
+    using namespace nhp;
+    const bool gelu = act == NHP_LINEAR_BIAS_GELU;
     if (!y || !x || !weight) return NHP_ERR_NULL;
-    if (rows < 1 || rows > 32 || out_features < 16 || out_features % 16 || in_features < 32 || in_features % 32) return NHP_ERR_SHAPE;
-    if (in_features > kLinearWhole * kLinearSplits || out_features > (1 << 24)) return NHP_ERR_SHAPE;
-    if (!ptr_aligned16(x) || !ptr_aligned16(weight) || !ptr_aligned16(y)) return NHP_ERR_SHAPE;
-    const int splits = in_features > kLinearWhole ? kLinearSplits : 1;
-    if (splits > 1 && !workspace) return NHP_ERR_NULL;
-    if (!ptr_aligned16(workspace)) return NHP_ERR_SHAPE;
-    const LinearArgs a{static_cast<uint16_t*>(y), static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(weight),
-                       static_cast<const uint16_t*>(bias), static_cast<float*>(workspace), (int)rows, (int)out_features,
-                       (int)in_features, splits, (reinterpret_cast<uintptr_t>(bias) & 3) == 0};
-    if (dtype == NHP_BF16) return launch_linear<NHP_BF16>(a, static_cast<hipStream_t>(stream));
-    if (dtype == NHP_F16) return launch_linear<NHP_F16>(a, static_cast<hipStream_t>(stream));
-    return NHP_ERR_DTYPE;
+    if (!gelu && (act < NHP_GATE_SWISH || act > NHP_GATE_IDENTITY || bias)) return NHP_ERR_SHAPE;
+    if (!linear_sizes_ok(rows, out_features, in_features, gelu ? 16 : 32)) return NHP_ERR_SHAPE;
+    LinearArgs a = linear_args(y, x, weight, bias, workspace, rows, out_features, in_features);
+    a.act = act;
+    return gelu ? linear_rows<kGeluRows>(a, dtype, stream) : linear_rows<kGatedRows>(a, dtype, stream);
+}
+
+int nhp_linear_decode_add(void* y, const void* x, const void* weight, const void* bias, const void* x1, const void* bias1,
+                          const void* residual, void* workspace, int64_t rows, int64_t out_features, int64_t in_features, int dtype,
+                          void* stream)
+{
+    using namespace nhp;
+    if (!y || !x || !weight || !residual || (bias1 && !x1)) return NHP_ERR_NULL;
+    if (!linear_sizes_ok(rows, out_features, in_features, 16)) return NHP_ERR_SHAPE;
+    LinearArgs a = linear_args(y, x, weight, bias, workspace, rows, out_features, in_features);
+    a.x1 = static_cast<const uint16_t*>(x1);
+    a.bias1 = static_cast<const uint16_t*>(bias1);
+    a.residual = static_cast<const uint16_t*>(residual);
+    return linear_rows<kAddRows>(a, dtype, stream);
 }
 
 }  // extern "C"

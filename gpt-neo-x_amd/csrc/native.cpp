@@ -940,28 +940,84 @@ PyObject* py_append_to_cache(PyObject*, PyObject* const* args, Py_ssize_t count)
     END_HANDLE_TH_ERRORS
 }
 
-// linear(x, weight, bias, most rows, most rows of a layer that is narrow or split): x W^T (+ bias) of few rows that nobody differentiates
+// Whether x W^T is one of few rows that nobody differentiates, the operands as the kernels read them
+bool few_rows(const Tensor& x, const Tensor& w, const MaybeTensor& b, int64_t most, int64_t most_split)
+{
+    if (followed() || at::autocast::is_autocast_enabled(at::kCUDA) || x.dim() < 1 || w.dim() != 2 || !is_half(x) || !alike(x, w)) return false;
+    const int64_t n = w.size(0), k = w.size(1);
+    return x.size(-1) == k && x.numel() <= (std::min(n, k) <= 2048 || k > 4096 ? most_split : most) * k && k % 32 == 0 && k <= 16384 &&
+           n % 16 == 0 && n <= (1 << 24) && w.is_contiguous() && x.is_contiguous() && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
+           reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0 &&
+           (!b || (b->dim() == 1 && b->size(0) == n && alike(*b, x) && b->is_contiguous() && !wants_grad({&*b}))) && !wants_grad({&x, &w});
+}
+
+Tensor new_rows(const Tensor& x, int64_t width)
+{
+    auto shape = x.sizes().vec();
+    shape.back() = width;
+    return at::empty(shape, x.options());
+}
+
+// linear(x, weight, bias, most rows, most rows of a layer that is narrow or split): x W^T (+ bias)
 PyObject* py_linear(PyObject*, PyObject* const* args, Py_ssize_t count)
 {
     HANDLE_TH_ERRORS
     Tensor x, w;
     MaybeTensor b;
-    int64_t most, most_narrow;
-    if (!take_all(args, count, x, w, b, most, most_narrow) || followed() || at::autocast::is_autocast_enabled(at::kCUDA) || x.dim() < 1 || w.dim() != 2 || !is_half(x) || !alike(x, w)) return not_here();
-    const int64_t n = w.size(0), k = w.size(1);
-    if (x.size(-1) != k || x.numel() > (std::min(n, k) <= 2048 || k > 4096 ? most_narrow : most) * k || k % 32 || k > 16384 || n % 16 || n > (1 << 24) ||
-        !w.is_contiguous() || !x.is_contiguous() || reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 ||
-        reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 || (b && (b->dim() != 1 || b->size(0) != n || !alike(*b, x) || !b->is_contiguous())) ||
-        wants_grad({&x, &w}) || (b && wants_grad({&*b})))
-        return not_here();
+    int64_t most, most_split;
+    if (!take_all(args, count, x, w, b, most, most_split) || !few_rows(x, w, b, most, most_split)) return not_here();
     const at::NoGradGuard no_grad;
     const c10::DeviceGuard guard(x.device());
-    const int64_t rows = x.numel() / k;
-    auto shape = x.sizes().vec();
-    shape.back() = n;
-    Tensor y = at::empty(shape, x.options());
+    const int64_t n = w.size(0), k = w.size(1), rows = x.numel() / k;
+    Tensor y = new_rows(x, n);
     const Tensor ws = bytes(nhp_linear_decode_workspace_bytes(rows, n, k), x);
     check(nhp_linear_decode(y.data_ptr(), x.data_ptr(), w.data_ptr(), ptr(b), ptr(ws), rows, n, k, type_code(x.scalar_type()), stream_of(x)), "linear");
+    return THPVariable_Wrap(y);
+    END_HANDLE_TH_ERRORS
+}
+
+// linear_act(x, weight, bias, act, most rows, most rows ..): the activation of x W^T
+PyObject* py_linear_act(PyObject*, PyObject* const* args, Py_ssize_t count)
+{
+    HANDLE_TH_ERRORS
+    Tensor x, w;
+    MaybeTensor b;
+    int64_t act, most, most_split;
+    if (!take_all(args, count, x, w, b, act, most, most_split) || !few_rows(x, w, b, most, most_split)) return not_here();
+    const bool gated = act != NHP_LINEAR_BIAS_GELU;
+    if (gated && (b || w.size(0) % 32 || act < NHP_GATE_SWISH || act > NHP_GATE_IDENTITY)) return not_here();
+    const at::NoGradGuard no_grad;
+    const c10::DeviceGuard guard(x.device());
+    const int64_t n = w.size(0), k = w.size(1), rows = x.numel() / k;
+    Tensor y = new_rows(x, gated ? n / 2 : n);
+    const Tensor ws = bytes(nhp_linear_decode_workspace_bytes(rows, n, k), x);
+    check(nhp_linear_decode_act(y.data_ptr(), x.data_ptr(), w.data_ptr(), ptr(b), ptr(ws), rows, n, k, (int)act, type_code(x.scalar_type()),
+                                stream_of(x)), "linear and activation");
+    return THPVariable_Wrap(y);
+    END_HANDLE_TH_ERRORS
+}
+
+// linear_add(x, weight, bias, x1, bias1, residual, most rows, most rows ..): residual + (x W^T + bias), or with x1
+// residual + ((x1 + bias1) + (x W^T + bias))
+PyObject* py_linear_add(PyObject*, PyObject* const* args, Py_ssize_t count)
+{
+    HANDLE_TH_ERRORS
+    Tensor x, w, r;
+    MaybeTensor b, x1, b1;
+    int64_t most, most_split;
+    if (!take_all(args, count, x, w, b, x1, b1, r, most, most_split) || !few_rows(x, w, b, most, most_split) || (b1 && !x1)) return not_here();
+    const int64_t n = w.size(0), k = w.size(1), rows = x.numel() / k;
+    if (r.dim() != x.dim() || r.size(-1) != n || r.numel() != rows * n || !alike(r, x) || !r.is_contiguous() || wants_grad({&r})) return not_here();
+    for (int64_t i = 0; i + 1 < x.dim(); ++i)
+        if (r.size(i) != x.size(i)) return not_here();
+    if (x1 && (x1->sizes() != r.sizes() || !alike(*x1, x) || !x1->is_contiguous() || wants_grad({&*x1}))) return not_here();
+    if (b1 && (b1->dim() != 1 || b1->size(0) != n || !alike(*b1, x) || !b1->is_contiguous() || wants_grad({&*b1}))) return not_here();
+    const at::NoGradGuard no_grad;
+    const c10::DeviceGuard guard(x.device());
+    Tensor y = new_rows(x, n);
+    const Tensor ws = bytes(nhp_linear_decode_workspace_bytes(rows, n, k), x);
+    check(nhp_linear_decode_add(y.data_ptr(), x.data_ptr(), w.data_ptr(), ptr(b), ptr(x1), ptr(b1), r.data_ptr(), ptr(ws), rows, n, k,
+                                type_code(x.scalar_type()), stream_of(x)), "linear and residual");
     return THPVariable_Wrap(y);
     END_HANDLE_TH_ERRORS
 }
@@ -971,6 +1027,7 @@ PyMethodDef kMethods[] = {NATIVE(layer_norm),       NATIVE(layer_norm_pair),  NA
                           NATIVE(gated),            NATIVE(causal_softmax),   NATIVE(masked_softmax),    NATIVE(rotary),
                           NATIVE(split_rotary),     NATIVE(add_residual),     NATIVE(add_residual_pair), NATIVE(causal_attention),
                           NATIVE(masked_attention), NATIVE(decode_attention), NATIVE(append_to_cache),   NATIVE(linear),
+                          NATIVE(linear_act),       NATIVE(linear_add),
                           {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 

@@ -98,6 +98,8 @@ def _declare(lib):
         "nhp_attention_decode": ([vp] * 8 + [i64, i64, f32, vp, f32] + [i64] * 6 + [p64] * 6 + [ci, vp], ci),
         "nhp_attention_decode_workspace_bytes": ([i64] * 6, i64),
         "nhp_linear_decode": ([vp] * 5 + [i64] * 3 + [ci, vp], ci),
+        "nhp_linear_decode_act": ([vp] * 5 + [i64] * 3 + [ci, ci, vp], ci),
+        "nhp_linear_decode_add": ([vp] * 8 + [i64] * 3 + [ci, vp], ci),
         "nhp_linear_decode_workspace_bytes": ([i64] * 3, i64),
         "nhp_kv_cache_append": ([vp] * 5 + [i64] * 5 + [p64] * 4 + [ci, vp], ci),
         "nhp_layernorm_bwd_noalloc": ([vp, vp, vp, vp, vp, vp, vp, vp, i64, i64, ci, ci, vp], ci),

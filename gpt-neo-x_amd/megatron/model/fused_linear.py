@@ -30,6 +30,7 @@ from .fused_attention import plain
 MAX_ROWS = 16          # of any layer
 MAX_ROWS_NARROW = 32   # where one of its sides has at most 2048 features, or more than 4096 come in
 MAX_FEATURES = 16384
+BIAS_GELU = 16   # NHP_LINEAR_BIAS_GELU; gates go by their codes
 
 
 def _few_rows(x, weight, bias):

@@ -14,7 +14,8 @@ adding it (``skip_bias_add``), and everything between the GEMMs is one of the fu
                               dropout or an additive term GEMM, fused softmax, GEMM
     output projection         GEMM, bias handed on
     bias + dropout + residual nhp_bias_add_residual / nhp_bias_dropout_add
-    MLP                       GEMM, bias+GeLU or gated activation kernel, GEMM, bias handed on
+    MLP                       GEMM, bias+GeLU or gated activation kernel, GEMM, bias handed on; for the few rows of a decoding
+                              step nhp_linear_decode_act and, with the addition, nhp_linear_decode_add
 
 Both residual layouts of the reference are provided: the sequential one
 (``x = x + attn(ln1(x)); x = x + mlp(ln2(x))``, :1254-1318) and the parallel one of the
@@ -25,8 +26,9 @@ mixture of experts, flash and sparse attention, Transformer Engine layers.
 """
 import torch
 
-from . import fused_attention
-from .activations import Gated_Activation, get_activation
+from ..fused_kernels import _hotpath as _hp
+from . import fused_attention, fused_linear
+from .activations import Gated_Activation, bias_gelu_impl, get_activation
 from .attention_core import (CoreAttention, apply_rotary_to_query_key, get_fusion_type, split_gqa_and_rotate,
                              split_qkv_and_rotate)
 from .fused_bias_dropout import (bias_add_residual_pair, bias_dropout_add_fused_inference, bias_dropout_add_fused_train,
@@ -80,7 +82,50 @@ class MLP(torch.nn.Module):
         self.linear1 = Linear(hidden, ffn_dim, bias=use_bias, skip_bias_add=True)
         self.linear2 = Linear(ffn_dim_in, hidden, bias=use_bias, skip_bias_add=True)
 
+    def _activated(self, x):
+        """The activated intermediate for the few rows of a decoding step, in the launch of the first product, or None."""
+        if not fused_attention.untouched(self.linear1, Linear):
+            return None
+        bias = self.linear1.bias
+        if self.is_gated:
+            if not fused_attention.untouched(self.activation_func, Gated_Activation):
+                return None
+            act = self.activation_func._code
+        elif self.activation_func is bias_gelu_impl:
+            act = fused_linear.BIAS_GELU
+        else:
+            return None
+        y = _hp.native().linear_act(x, self.linear1.weight, bias, act, fused_linear.MAX_ROWS, fused_linear.MAX_ROWS_NARROW)
+        return None if y is NotImplemented else y
+
+    def _few_rows(self, x):
+        """Whether ``x`` may be few rows that nobody differentiates (the launches ask closely)."""
+        return (not _hp._is_compiling() and not torch.is_grad_enabled() and isinstance(x, torch.Tensor) and x.dim() > 0
+                and x.numel() <= fused_linear.MAX_ROWS_NARROW * x.size(-1))
+
+    def add_to(self, residual, x, other=None, other_bias=None):
+        """``residual + mlp(x)`` or ``residual + ((other + other_bias) + mlp(x))`` for the few rows of a decoding step, the
+        activation and the addition each in the launch of a product; None for anything else, and where somebody looks at the
+        modules."""
+        if not self._few_rows(x) or not (fused_attention.untouched(self, MLP) and fused_attention.untouched(self.linear2, Linear)):
+            return None
+        intermediate = self._activated(x)
+        if intermediate is None:
+            return None
+        y = _hp.native().linear_add(intermediate, self.linear2.weight, self.linear2.bias, other, other_bias, residual,
+                                    fused_linear.MAX_ROWS, fused_linear.MAX_ROWS_NARROW)
+        if y is not NotImplemented:
+            return y
+        output, bias = self.linear2(intermediate)
+        if other is None:
+            return bias_dropout_add_fused_inference(output, bias, residual, 0.0)
+        return bias_add_residual_pair(other, other_bias, output, bias, residual)
+
     def forward(self, hidden_states):
+        if self._few_rows(hidden_states):
+            intermediate = self._activated(hidden_states)
+            if intermediate is not None:
+                return self.linear2(intermediate)
         intermediate, bias = self.linear1(hidden_states)
         if self.is_gated or (self.activation_type == "gelu" and self.bias_gelu_fusion):
             if bias is None and not self.is_gated:
@@ -211,6 +256,10 @@ class TransformerLayer(torch.nn.Module):
             return bias_dropout_add_fused_train if self.training else bias_dropout_add_fused_inference
         return get_bias_dropout_add(self.training)
 
+    def _mlp_added(self, residual, x, other=None, other_bias=None):
+        mlp = self.mlp
+        return mlp.add_to(residual, x, other, other_bias) if type(mlp) is MLP else None
+
     def _attend(self, x, attention_mask, layer_past):
         output, bias = self.attention(x, attention_mask, layer_past=layer_past)
         if self.use_cache:
@@ -230,6 +279,9 @@ class TransformerLayer(torch.nn.Module):
             attention_output, attention_bias = self._attend(x1, attention_mask, layer_past)
             if self.bias_dropout_fusion and (self.hidden_dropout == 0.0 or not self.training):
                 # no dropout: attention branch + MLP branch + residual in one pass
+                output = self._mlp_added(residual, x2, attention_output, attention_bias)
+                if output is not None:
+                    return output
                 mlp_output, mlp_bias = self.mlp(x2)
                 return bias_add_residual_pair(attention_output, attention_bias, mlp_output, mlp_bias, residual)
             if attention_bias is not None:
@@ -242,5 +294,10 @@ class TransformerLayer(torch.nn.Module):
         attention_output, attention_bias = self._attend(self.input_layernorm(x), attention_mask, layer_past)
         attention_output = bias_dropout_fn(attention_output, bias=attention_bias, residual=residual,
                                            prob=self.hidden_dropout)
-        mlp_output, mlp_bias = self.mlp(self.post_attention_layernorm(attention_output))
+        normed = self.post_attention_layernorm(attention_output)
+        if self.hidden_dropout == 0.0 or not self.training:
+            output = self._mlp_added(attention_output, normed)
+            if output is not None:
+                return output
+        mlp_output, mlp_bias = self.mlp(normed)
         return bias_dropout_fn(mlp_output, bias=mlp_bias, residual=attention_output, prob=self.hidden_dropout)

@@ -74,3 +74,92 @@ def test_everything_else_goes_to_the_library():
     with torch.autocast("cuda", dtype=torch.float16):
         assert not fused_linear._few_rows(x, w, None)
     assert torch.func.vmap(lambda v: linear(v, w))(x).shape == (4, 32)
+
+
+SHAPES = pytest.mark.parametrize("rows,n,k", [(1, 32, 32), (16, 64, 544), (5, 4160, 96), (17, 9248, 160), (3, 96, 4128), (32, 1056, 11008), (16, 12352, 800)])
+
+
+@SHAPES
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_with_the_activation(rows, n, k, dtype):
+    """The bits of the product and the activation called one after the other."""
+    from megatron.fused_kernels import _hotpath as hp
+    from megatron.model import fused_linear
+    from megatron.model.activations import Gated_Activation, bias_gelu_impl
+
+    x, w = util.randn((rows, k), dtype, seed=1).to(DEV), util.randn((n, k), dtype, seed=2, std=1.0 / math.sqrt(k)).to(DEV)
+    b = util.randn((n + 1,), dtype, seed=3).to(DEV)
+    native, most = hp.native(), (32, 32)
+    product = native.linear(x, w, None, *most)
+    for bias in (b[1:], b[:-1], None):
+        # (an aligned bias: the activation's kernel for others rounds its product with the gate once, to fp16)
+        want = bias_gelu_impl(product, torch.zeros_like(b[1:]) if bias is None else bias.clone())
+        assert torch.equal(native.linear_act(x, w, bias, fused_linear.BIAS_GELU, *most), want)
+    for kind in ("swiglu", "geglu", "reglu", "glu", "bilinear"):
+        gate = Gated_Activation(kind)
+        assert torch.equal(native.linear_act(x, w, None, gate._code, *most), gate(product))
+    assert native.linear_act(x, w, b[1:], 0, *most) is NotImplemented and native.linear_act(x, w, None, 5, *most) is NotImplemented
+    assert native.linear_act(x, w[:16], None, 0, *most) is NotImplemented
+
+
+@SHAPES
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_with_the_residual_addition(rows, n, k, dtype):
+    from megatron.fused_kernels import _hotpath as hp
+    from megatron.model.fused_bias_dropout import bias_add_residual_pair, bias_dropout_add_fused_inference
+
+    x, w = util.randn((rows, 1, k), dtype, seed=1).to(DEV), util.randn((n, k), dtype, seed=2, std=1.0 / math.sqrt(k)).to(DEV)
+    r, x1 = util.randn((rows, 1, n), dtype, seed=3).to(DEV), util.randn((rows, 1, n), dtype, seed=4).to(DEV)
+    b, b1 = util.randn((n + 1,), dtype, seed=5).to(DEV)[1:], util.randn((n,), dtype, seed=6).to(DEV)
+    native, most = hp.native(), (32, 32)
+    product = native.linear(x, w, None, *most)
+    for bias in (b, None):
+        assert torch.equal(native.linear_add(x, w, bias, None, None, r, *most), bias_dropout_add_fused_inference(product, bias, r, 0.0))
+        for bias1 in (b1, None):
+            assert torch.equal(native.linear_add(x, w, bias, x1, bias1, r, *most), bias_add_residual_pair(x1, bias1, product, bias, r))
+    for bad in (r[:, :, 1:], r.float(), r.reshape(rows, n), r.transpose(0, 2)):
+        assert native.linear_add(x, w, b, None, None, bad, *most) is NotImplemented or bad.shape == r.shape and bad.is_contiguous()
+    assert native.linear_add(x, w, b, None, b1, r, *most) is NotImplemented
+
+
+@pytest.mark.parametrize("style", ["gelu", "swiglu"])
+def test_a_layer_takes_them_unless_somebody_looks(style):
+    """One layer's step: the same bits by separate launches, which is what it makes while a module inside is watched."""
+    import types
+
+    from megatron.model.transformer_layer import TransformerLayer
+
+    gelu = style == "gelu"
+    args = types.SimpleNamespace(
+        hidden_size=256, num_attention_heads=4, num_kv_heads=4, seq_length=64, precision="bfloat16", pos_emb="rotary", rotary_pct=1.0,
+        rotary_emb_base=10000, rope_fusion=True, norm="layernorm" if gelu else "rmsnorm", layernorm_epsilon=1e-5, rms_norm_epsilon=1e-6,
+        activation=style, bias_gelu_fusion=True, onnx_safe=False, scaled_upper_triang_masked_softmax_fusion=True,
+        scaled_masked_softmax_fusion=False, attention_softmax_in_fp32=True, attention_dropout=0.0, hidden_dropout=0.0,
+        bias_dropout_fusion=True, gpt_j_residual=gelu, use_bias_in_mlp=gelu, use_bias_in_attn_linear=gelu)
+    torch.manual_seed(0)
+    with torch.device(DEV):
+        layer = TransformerLayer(args, lambda s, m: s.masked_fill_(m, -10000.0), 1, rotary=True, use_cache=True)
+    layer = layer.bfloat16().eval()
+    x, past = util.randn((1, 3, 256), torch.bfloat16, seed=1).to(DEV), util.randn((2, 9, 3, 4, 64), torch.bfloat16, seed=2).to(DEV)
+    mask = torch.zeros((1, 1, 1, 10), dtype=torch.bool, device=DEV)
+    seen = []
+
+    def step(x=x):
+        layer.layer_past = None
+        with torch.no_grad():
+            return layer(x, mask, layer_past=past)
+
+    want = step()
+    assert layer.mlp._activated(x) is None   # gradients are wanted here
+    with torch.no_grad():
+        assert layer.mlp._activated(x) is not None and layer.mlp.add_to(x, x) is not None
+    for module in (layer.mlp, layer.mlp.linear1, layer.mlp.linear2):
+        handle = module.register_forward_hook(lambda m, i, o: seen.append(m))
+        assert torch.equal(step(), want) and seen[-1] is module
+        handle.remove()
+    layer.mlp.linear1.forward = lambda v: (torch.nn.functional.linear(v, layer.mlp.linear1.weight) * 0, layer.mlp.linear1.bias)
+    assert not torch.equal(step(), want)
+    del layer.mlp.linear1.forward
+    assert torch.equal(step(), want)
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert layer.mlp._activated(x) is None

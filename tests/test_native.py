@@ -19,7 +19,8 @@ CALLS = {"layer_norm": ("x", None, None, 1e-5), "layer_norm_pair": ("x", None, N
          "rotary": ("x", "x", "x", "x", 0), "split_rotary": ("x", "x", "x", 0, 0, 0), "add_residual": ("x", None, None),
          "add_residual_pair": ("x", None, "x", None, "x"), "causal_attention": ("x", "x", "x", 1.0, -1, True),
          "masked_attention": ("x", "x", "x", "x", 1.0, -1e4, True), "decode_attention": ("x", "x", "x", "x", "x", 1.0, -1e4, True),
-         "append_to_cache": ("x", "x", None), "linear": ("x", "x", None, 16, 32)}
+         "append_to_cache": ("x", "x", None), "linear": ("x", "x", None, 16, 32),
+         "linear_act": ("x", "x", None, 0, 16, 32), "linear_add": ("x", "x", None, None, None, "x", 16, 32)}
 
 
 @pytest.mark.parametrize("name", CALLS)

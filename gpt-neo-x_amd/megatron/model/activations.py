@@ -102,10 +102,11 @@ class GeLUFunction(torch.autograd.Function):
 
 def bias_gelu_impl(input, bias):
     """``GeLUFunction.apply(input, bias)``."""
-    if not _hp._is_compiling():
-        y = _hp.native().bias_gelu(input, bias)
-        if y is not NotImplemented:
-            return y
+    if not torch.jit.is_scripting():
+        if not _hp._is_compiling():
+            y = _hp.native().bias_gelu(input, bias)
+            if y is not NotImplemented:
+                return y
     return GeLUFunction.apply(input, bias)
 
 

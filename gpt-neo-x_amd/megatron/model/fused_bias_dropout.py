@@ -153,10 +153,11 @@ def bias_add_residual_pair(x1: Tensor, bias1: Optional[Tensor], x2: Tensor, bias
     attention and MLP branches (three ``bias_dropout_add`` calls in ParallelTransformerLayer.forward,
     megatron/model/transformer.py:1229-1250) when dropout is off, in one kernel and with the reference's
     roundings."""
-    if not _hp._is_compiling():
-        out = _hp.native().add_residual_pair(x1, bias1, x2, bias2, residual)
-        if out is not NotImplemented:
-            return out
+    if not torch.jit.is_scripting():
+        if not _hp._is_compiling():
+            out = _hp.native().add_residual_pair(x1, bias1, x2, bias2, residual)
+            if out is not NotImplemented:
+                return out
     return _BiasAddResidualPair.apply(x1, bias1, x2, bias2, residual)
 
 

@@ -214,10 +214,11 @@ class LayerNorm(torch.nn.Module):
         if input.device.type != "cuda":
             # off the GPU: torch's own LayerNorm, which is the reference's class (megatron/model/norms.py:16)
             return torch.nn.functional.layer_norm(input, self.normalized_shape, self.weight, self.bias, self.eps)
-        if not _hp._is_compiling():
-            y = _hp.native().layer_norm(input, self.weight, self.bias, self.eps)
-            if y is not NotImplemented:
-                return y
+        if not torch.jit.is_scripting():
+            if not _hp._is_compiling():
+                y = _hp.native().layer_norm(input, self.weight, self.bias, self.eps)
+                if y is not NotImplemented:
+                    return y
         return _LayerNormFunction.apply(input, self.weight, self.bias, self.eps)
 
     def extra_repr(self):
@@ -308,10 +309,11 @@ class RMSNorm(torch.nn.Module):
         if x.device.type != "cuda":
             return self._forward_torch(x)
         mode = 0 if self.fused_eps else 1
-        if not _hp._is_compiling():
-            y = _hp.native().rms_norm(x, self.scale, self.offset, self.eps, mode, self.d if self.partial_size is None else self.partial_size)
-            if y is not NotImplemented:
-                return y
+        if not torch.jit.is_scripting():
+            if not _hp._is_compiling():
+                y = _hp.native().rms_norm(x, self.scale, self.offset, self.eps, mode, self.d if self.partial_size is None else self.partial_size)
+                if y is not NotImplemented:
+                    return y
         return _RMSNormFunction.apply(x, self.scale, self.offset, self.eps, mode, self.partial_size)
 
     def _forward_torch(self, x):

@@ -232,6 +232,10 @@ class SelfAttention(torch.nn.Module):
         return query, key, value
 
 
+# what the sum of the feed forward block's launch stands for; any other function set on the layer is called
+_FUSED_ADDS = (bias_dropout_add_fused_train, bias_dropout_add_fused_inference)
+
+
 class TransformerLayer(torch.nn.Module):
     """``ParallelTransformerLayer.forward`` (megatron/model/transformer.py:1179-1321) on one GPU.
     Input and output ``[s, b, h]``."""
@@ -295,7 +299,7 @@ class TransformerLayer(torch.nn.Module):
         attention_output = bias_dropout_fn(attention_output, bias=attention_bias, residual=residual,
                                            prob=self.hidden_dropout)
         normed = self.post_attention_layernorm(attention_output)
-        if self.hidden_dropout == 0.0 or not self.training:
+        if bias_dropout_fn in _FUSED_ADDS and (self.hidden_dropout == 0.0 or not self.training):
             output = self._mlp_added(attention_output, normed)
             if output is not None:
                 return output

@@ -43,3 +43,22 @@ def test_a_missing_module_is_an_error(monkeypatch):
     monkeypatch.delattr(sys.modules["megatron.fused_kernels"], "_native", raising=False)
     with pytest.raises(ImportError, match="_native.so"):
         hp.native()
+
+
+def test_what_could_be_scripted_still_can():
+    """TorchScript takes the modules and functions around the native calls as it did, and leaves those out."""
+    from megatron.model.activations import bias_gelu_impl
+    from megatron.model.fused_bias_dropout import bias_add_residual_pair
+    from megatron.model.norms import LayerNorm, RMSNorm
+
+    x = torch.randn((3, 64), generator=torch.Generator().manual_seed(0))
+    for module in (LayerNorm(64), RMSNorm(64)):
+        for grad in (True, False):
+            with torch.set_grad_enabled(grad):
+                assert torch.equal(torch.jit.script(module)(x), module(x))
+
+    def activation(x, b):
+        return bias_gelu_impl(x, b)
+
+    for f in (activation, bias_add_residual_pair):
+        torch.jit.script(f)

@@ -940,15 +940,25 @@ PyObject* py_append_to_cache(PyObject*, PyObject* const* args, Py_ssize_t count)
     END_HANDLE_TH_ERRORS
 }
 
-// Whether x W^T is one of few rows that nobody differentiates, the operands as the kernels read them
-bool few_rows(const Tensor& x, const Tensor& w, const MaybeTensor& b, int64_t most, int64_t most_split)
+// Whether nobody differentiates x W^T, the operands as the kernels read them
+bool rows_ready(const Tensor& x, const Tensor& w, const MaybeTensor& b)
 {
     if (followed() || at::autocast::is_autocast_enabled(at::kCUDA) || x.dim() < 1 || w.dim() != 2 || !is_half(x) || !alike(x, w)) return false;
     const int64_t n = w.size(0), k = w.size(1);
-    return x.size(-1) == k && x.numel() <= (std::min(n, k) <= 2048 || k > 4096 ? most_split : most) * k && k % 32 == 0 && k <= 16384 &&
-           n % 16 == 0 && n <= (1 << 24) && w.is_contiguous() && x.is_contiguous() && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
-           reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0 &&
+    return x.size(-1) == k && k % 32 == 0 && k <= 16384 && n % 16 == 0 && n <= (1 << 24) && w.is_contiguous() && x.is_contiguous() &&
+           reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 && reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0 &&
            (!b || (b->dim() == 1 && b->size(0) == n && alike(*b, x) && b->is_contiguous() && !wants_grad({&*b}))) && !wants_grad({&x, &w});
+}
+
+bool are_few(const Tensor& x, const Tensor& w, int64_t most, int64_t most_split)
+{
+    const int64_t n = w.size(0), k = w.size(1);
+    return x.numel() <= (std::min(n, k) <= 2048 || k > 4096 ? most_split : most) * k;
+}
+
+bool few_rows(const Tensor& x, const Tensor& w, const MaybeTensor& b, int64_t most, int64_t most_split)
+{
+    return rows_ready(x, w, b) && are_few(x, w, most, most_split);
 }
 
 Tensor new_rows(const Tensor& x, int64_t width)
@@ -965,11 +975,17 @@ PyObject* py_linear(PyObject*, PyObject* const* args, Py_ssize_t count)
     Tensor x, w;
     MaybeTensor b;
     int64_t most, most_split;
-    if (!take_all(args, count, x, w, b, most, most_split) || !few_rows(x, w, b, most, most_split)) return not_here();
+    if (!take_all(args, count, x, w, b, most, most_split) || !rows_ready(x, w, b)) return not_here();
+    const int64_t n = w.size(0), k = w.size(1), rows = x.numel() / k;
+    const bool few = are_few(x, w, most, most_split);
+    if (!few && (!nhp_linear_tiles_pay(rows, n, k) || (b && reinterpret_cast<uintptr_t>(b->data_ptr()) % 16))) return not_here();
     const at::NoGradGuard no_grad;
     const c10::DeviceGuard guard(x.device());
-    const int64_t n = w.size(0), k = w.size(1), rows = x.numel() / k;
     Tensor y = new_rows(x, n);
+    if (!few) {
+        check(nhp_linear_tiles(y.data_ptr(), x.data_ptr(), w.data_ptr(), ptr(b), rows, n, k, type_code(x.scalar_type()), stream_of(x)), "linear");
+        return THPVariable_Wrap(y);
+    }
     const Tensor ws = bytes(nhp_linear_decode_workspace_bytes(rows, n, k), x);
     check(nhp_linear_decode(y.data_ptr(), x.data_ptr(), w.data_ptr(), ptr(b), ptr(ws), rows, n, k, type_code(x.scalar_type()), stream_of(x)), "linear");
     return THPVariable_Wrap(y);

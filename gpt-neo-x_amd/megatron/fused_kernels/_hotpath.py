@@ -101,6 +101,8 @@ def _declare(lib):
         "nhp_linear_decode_act": ([vp] * 5 + [i64] * 3 + [ci, ci, vp], ci),
         "nhp_linear_decode_add": ([vp] * 8 + [i64] * 3 + [ci, vp], ci),
         "nhp_linear_decode_workspace_bytes": ([i64] * 3, i64),
+        "nhp_linear_tiles": ([vp] * 4 + [i64] * 3 + [ci, vp], ci),
+        "nhp_linear_tiles_pay": ([i64] * 3, ci),
         "nhp_kv_cache_append": ([vp] * 5 + [i64] * 5 + [p64] * 4 + [ci, vp], ci),
         "nhp_layernorm_bwd_noalloc": ([vp, vp, vp, vp, vp, vp, vp, vp, i64, i64, ci, ci, vp], ci),
     }

@@ -18,7 +18,9 @@ Where the line lies. On the GPU, weights not in any cache, us here / library:
     [4096, 11008]  20.2 / 37.6  20.5 / 37.9  22.2 / 37.9   23.9 / 31.2   24.8 / 30.8
     [4096, 14336]  24.6 / 25.8  25.2 / 25.9  26.8 / 26.9   28.7 / 31.2   30.7 / 33.4
 Up to 16 rows the kernel is ahead everywhere, up to 32 where a side has at most 2048 features or where four workgroups share the
-contraction (more than 4096 features); in between the library catches up."""
+contraction (more than 4096 features); in between the library catches up.
+
+More rows than that (a short prompt, many sequences) go to csrc/linear_tiles.hip where it is ahead; its table and rule stand there."""
 from typing import Optional
 
 import torch
@@ -33,10 +35,26 @@ MAX_FEATURES = 16384
 BIAS_GELU = 16   # NHP_LINEAR_BIAS_GELU; gates go by their codes
 
 
+def _are_few(x, weight):
+    n, k = weight.shape
+    return x.numel() <= (MAX_ROWS_NARROW if min(n, k) <= 2048 or k > 4096 else MAX_ROWS) * k
+
+
 def _few_rows(x, weight, bias):
+    return _are_few(x, weight) and _rows_ready(x, weight, bias)
+
+
+def _some_rows(x, weight, bias):
+    """More rows that csrc/linear_tiles.hip takes (its rule stands there)."""
+    n, k = weight.shape
+    return (not _are_few(x, weight) and _rows_ready(x, weight, bias) and _hp.lib().nhp_linear_tiles_pay(x.numel() // k, n, k)
+            and (bias is None or bias.data_ptr() % 16 == 0))
+
+
+def _rows_ready(x, weight, bias):
     n, k = weight.shape
     dtype = x.dtype
-    return (x.numel() <= (MAX_ROWS_NARROW if min(n, k) <= 2048 or k > 4096 else MAX_ROWS) * k and x.is_cuda and x.dim() > 0 and x.size(-1) == k and x.numel() > 0
+    return (x.is_cuda and x.dim() > 0 and x.size(-1) == k and x.numel() > 0
             and (dtype is torch.bfloat16 or dtype is torch.float16) and weight.dtype is dtype and weight.device == x.device
             and k % 32 == 0 and k <= MAX_FEATURES and n % 16 == 0 and 0 < n <= 1 << 24 and weight.is_contiguous()
             and x.is_contiguous()
@@ -46,8 +64,8 @@ def _few_rows(x, weight, bias):
 
 
 def linear(x, weight, bias: Optional[torch.Tensor] = None):
-    """``torch.nn.functional.linear``; in inference with few rows of a 16-bit type by one kernel (two with more than 4096
-    features). Scripted, compiled, exported or traced over proxies it is torch's: the sizes below would become conditions."""
+    """``torch.nn.functional.linear``; in inference with up to some hundred rows of a 16-bit type by one kernel (two with few rows
+    and more than 4096 features). Scripted, compiled, exported or traced over proxies it is torch's: the sizes below would become conditions."""
     if torch.jit.is_scripting():
         return F.linear(x, weight, bias)
     else:
@@ -61,12 +79,18 @@ def _linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor])
         if y is not NotImplemented:
             return y
     if (_hp._is_compiling() or _hp._tracing_state() is not None or not isinstance(x, torch.Tensor) or not isinstance(weight, torch.Tensor)
-            or weight.dim() != 2 or not _few_rows(x, weight, bias)):
+            or weight.dim() != 2 or not (_few_rows(x, weight, bias) or _some_rows(x, weight, bias))):
         return F.linear(x, weight, bias)
     n, k = weight.shape
     rows = x.numel() // k
     y = torch.empty(x.shape[:-1] + (n,), dtype=x.dtype, device=x.device)
     lib = _hp.lib()
+    if not _are_few(x, weight):
+        with _hp.device_guard(x):
+            rc = lib.nhp_linear_tiles(y.data_ptr(), x.data_ptr(), weight.data_ptr(), None if bias is None else bias.data_ptr(), rows, n,
+                                      k, _hp.dtype_code(x, "linear"), _hp.stream_of(x))
+        _hp.check(rc, "linear")
+        return y
     scratch = lib.nhp_linear_decode_workspace_bytes(rows, n, k)
     workspace = torch.empty(scratch, dtype=torch.uint8, device=x.device) if scratch else None
     with _hp.device_guard(x):

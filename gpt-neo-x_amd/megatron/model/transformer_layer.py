@@ -3,7 +3,7 @@
 The data flow of GPT-NeoX's ``ParallelTransformerLayer`` (megatron/model/transformer.py:962-1321)
 with ``ParallelSelfAttention`` (:326-959) and ``ParallelMLP`` (:93-196) inside, without the
 model-parallel layers: every linear layer is a plain ``torch.nn.functional.linear`` (library
-GEMM; for the few rows of a decoding step nhp_linear_decode) that hands its bias on instead of
+GEMM; without a gradient nhp_linear_decode for few rows, nhp_linear_tiles for a short prompt) that hands its bias on instead of
 adding it (``skip_bias_add``), and everything between the GEMMs is one of the fused kernels:
 
     norm                      nhp_layernorm / nhp_rmsnorm (the two norms of the parallel-residual layout: nhp_layernorm_pair)

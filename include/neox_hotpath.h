@@ -788,6 +788,13 @@ int nhp_linear_decode_add(void* y, const void* x, const void* weight, const void
                           const void* residual, void* workspace, int64_t rows, int64_t out_features, int64_t in_features, int dtype,
                           void* stream);
 
+/* The same product for more rows (a short prompt, many sequences; the same layers of megatron/model/transformer.py), one launch
+ * without a workspace. in_features a multiple of 64 and at most 65536, out_features of 16, at most 2^24 tiles of 64 x 64; all contiguous, bias 16-byte aligned too. _pay: whether it is the
+ * faster way on MI355X (0 for sizes that it does not take). */
+int nhp_linear_tiles_pay(int64_t rows, int64_t out_features, int64_t in_features);
+int nhp_linear_tiles(void* y, const void* x, const void* weight, const void* bias, int64_t rows, int64_t out_features,
+                     int64_t in_features, int dtype, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

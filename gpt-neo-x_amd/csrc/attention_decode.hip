@@ -16,13 +16,18 @@
 // key/value head) pairs the waves of a workgroup take two or four neighbouring heads, whose rows of a position lie side by
 // side, and with fewer of them the keys of a pair are cut into parts, which a second kernel merges (decode_plan).
 //
-// Measured (us, bf16, without the prefetch and with one head per workgroup before; copy: read and written bytes at 5.1 TB/s):
-//   16 sequences of 2047, 32 heads of 128      221 -> 204 (copy 210)     32 of 1000, 32 heads of 128   221 -> 192 (206)
-//   32 of 2000, 8 heads of keys of 128          90 -> 85 (103)           20 of 2000, 32 heads of 80    328 -> 231 (161)
-//   9 of 2000, 32 heads of 128                 163 -> 119 (116)          5 of 3000, 32 heads of 128    119 -> 91 (96)
-//   1 of 8000, 32 heads of 128                  58 -> 57 (51)            4 of 300, 8 heads of keys      14 -> 11 (2)
+// Measured (us, bf16, without the prefetch and with one head per workgroup before; copy: read and written bytes at 5.1 TB/s;
+// cards, and runs on one card, differ by up to 8 %):
+//   16 sequences of 2047, 32 heads of 128      223 -> 196 (copy 210)     32 of 1000, 32 heads of 128   225 -> 186 (206)
+//   32 of 2000, 8 heads of keys of 128          94 -> 89 (103)           20 of 2000, 32 heads of 80    328 -> 212 (161)
+//   9 of 2000, 32 heads of 128                 161 -> 114 (116)          5 of 3000, 32 heads of 128    126 -> 94 (96)
+//   1 of 8000, 32 heads of 128                  59 -> 58 (51)            4 of 300, 8 heads of keys      14 -> 11 (2)
+// The registers of the prefetch leave room for two workgroups on a CU instead of three: 24 of 200 to 400, 32 heads of 128, which are
+// three for each CU, take longer (34 -> 39, 59 -> 66); a variant without it is as fast there and slower in between.
 // (Concatenations 949 us and attention 118 us for the first of them, before there was such a kernel.)
 #include "attention.hpp"
+
+#include <cmath>
 
 namespace nhp {
 
@@ -44,6 +49,10 @@ struct Yes {
 };
 struct No {
     static constexpr bool value = false;
+};
+template <int N>
+struct Index {
+    static constexpr int value = N;
 };
 
 // Combines the lanes l, l ^ 16, l ^ 32, l ^ 48.
@@ -68,15 +77,27 @@ struct DecodeGeo {
     static constexpr int kWaveBytes = kValueBytes > kSumBytes ? kValueBytes : kSumBytes;
 };
 
-// NQ: tiles of 16 queries; NH: key/value heads of a workgroup, one or several waves each. (With two tiles of queries the
-// registers for what is on its way are there for one workgroup per CU only.)
+// Workgroups of a CU that the registers leave room for: with four sums of 128 features, or two with twice the heads, there is one.
+// (Two with six registers spilled: [16 sequences of 2047, 32 heads of 128] 206 -> 208 us, [24 of 1000] 156 -> 170.)
+constexpr int decode_blocks_per_cu(int head_dim, int heads) { return heads == 4 || (heads == 2 && head_dim == 128) ? 1 : 2; }
+
+// NQ: tiles of 16 queries; NH: key/value heads of a workgroup, one or several waves each.
+//
+// The keys of a head (of its split) always go into four sums, the 32 of chunk c into sum c % 4, whichever waves take them: a wave
+// keeps NH of the four. So the result does not depend on NH. With one sum for each wave two heads per workgroup had two sums and
+// four heads one, and the fewer there are the further off is the result: the probability of a sum's first maximum is 1, which has no
+// error in 16 bits. Relative error against 64 bits, bf16, 128 features: [16 sequences of 2047, 32 heads] 2.312e-3 with four sums
+// and 2.324e-3 with two, [64 of 400, 32 heads] 2.251e-3 and with one 2.324e-3. It costs 0 to 3 % of the time.
 template <int DT, int HD, int NQ, int NH>
-__global__ void __launch_bounds__(256, NQ == 1 ? 2 : 1) attn_decode_kernel(AttnDecodeArgs a)
+__global__ void __launch_bounds__(256, decode_blocks_per_cu(HD, NH)) attn_decode_kernel(AttnDecodeArgs a)
 {
     using G = DecodeGeo<HD>;
+    // With two tiles of queries the registers for what is on its way are there up to 64 features; beyond, two workgroups on a CU
+    // without it are faster than one with it (512 pairs of 1000 keys, 20 queries, 128 features: 98 us, 107).
+    constexpr bool kAhead = NQ == 1 || HD == 64;
     constexpr int kKeyWaves = 4 / NH, kKeys = 32 * kKeyWaves;   // waves that share a head's keys, and what they take in a round
     __shared__ __attribute__((aligned(1024))) char lds[4 * G::kWaveBytes];
-    __shared__ float wave_m[4][NQ * 16], wave_l[4][NQ * 16];
+    __shared__ float part_m[4][NH][NQ * 16], part_l[4][NH][NQ * 16];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g = lane >> 4;
     const int pairs = a.batch * a.kv_heads;
@@ -115,15 +136,17 @@ __global__ void __launch_bounds__(256, NQ == 1 ? 2 : 1) attn_decode_kernel(AttnD
         else return base + (value_row(i) * st + value_col(i));
     };
 
-    f32x4 o[NQ][G::kTiles];
-    float m[NQ], l[NQ];
+    f32x4 sums_o[NH][NQ][G::kTiles];
+    float sums_m[NH][NQ], sums_l[NH][NQ];
 #pragma unroll
-    for (int n = 0; n < NQ; ++n) {
-        m[n] = kFarBelow;
-        l[n] = 0.0f;
+    for (int i = 0; i < NH; ++i)
 #pragma unroll
-        for (int d = 0; d < G::kTiles; ++d) o[n][d] = f32x4{};
-    }
+        for (int n = 0; n < NQ; ++n) {
+            sums_m[i][n] = kFarBelow;
+            sums_l[i][n] = 0.0f;
+#pragma unroll
+            for (int d = 0; d < G::kTiles; ++d) sums_o[i][n][d] = f32x4{};
+        }
 
     // bytes 4 g .. 4 g + 3 of each 16 keys of this lane's query; the last ones of a row are read as the four bytes that end it
     auto read_mask = [&](int key0, uint32_t (&hidden)[NQ][2]) {
@@ -171,9 +194,12 @@ __global__ void __launch_bounds__(256, NQ == 1 ? 2 : 1) attn_decode_kernel(AttnD
         }
         read_mask(key0, hidden);
     };
-    // Stores and multiplies them; `whole`: all 32 exist.
-    auto use = [&](auto whole, int key0, Keys& kf, Values& vf, Hidden& hidden) {
+    // Stores and multiplies them; `whole`: all 32 exist, `sum_index`: the wave's sum that takes them.
+    auto use = [&](auto whole, auto sum_index, int key0, Keys& kf, Values& vf, Hidden& hidden) {
         constexpr bool kWhole = decltype(whole)::value;
+        auto& o = sums_o[decltype(sum_index)::value];
+        auto& m = sums_m[decltype(sum_index)::value];
+        auto& l = sums_l[decltype(sum_index)::value];
         asm volatile("" : "+s"(key0));
         uint16_t *kd = ko + (int64_t)key0 * a.out_s, *vd = vo + (int64_t)key0 * a.out_s;
 #pragma unroll
@@ -247,69 +273,106 @@ __global__ void __launch_bounds__(256, NQ == 1 ? 2 : 1) attn_decode_kernel(AttnD
     };
     int key0 = key_lo + wave / NH * 32;
     const int last_whole = min(a.past, key_hi) - 32;
-    Keys kf[2];
-    Values vf[2];
-    Hidden hidden[2];
-    if (key0 <= last_whole) {
+    Keys kf[kAhead ? 2 : 1];
+    Values vf[kAhead ? 2 : 1];
+    Hidden hidden[kAhead ? 2 : 1];
+    // one chunk, the next of this wave being asked for first; the i-th of a turn of the loop
+    auto step = [&](auto index) {
+        constexpr int i = decltype(index)::value, now = i & 1, next = now ^ 1;
+        if (key0 + kKeys <= last_whole) load(key0 + kKeys, kf[next], vf[next], hidden[next]);
+        use(Yes{}, Index<i % NH>{}, key0, kf[now], vf[now], hidden[now]);
+        key0 += kKeys;
+        return key0 <= last_whole;
+    };
+    if constexpr (!kAhead) {
+        for (; key0 <= last_whole; key0 += kKeys) {
+            load(key0, kf[0], vf[0], hidden[0]);
+            use(Yes{}, Index<0>{}, key0, kf[0], vf[0], hidden[0]);
+        }
+    } else if (key0 <= last_whole) {
         load(key0, kf[0], vf[0], hidden[0]);
-        for (;;) {
-            if (key0 + kKeys <= last_whole) load(key0 + kKeys, kf[1], vf[1], hidden[1]);
-            use(Yes{}, key0, kf[0], vf[0], hidden[0]);
-            key0 += kKeys;
-            if (key0 > last_whole) break;
-            if (key0 + kKeys <= last_whole) load(key0 + kKeys, kf[0], vf[0], hidden[0]);
-            use(Yes{}, key0, kf[1], vf[1], hidden[1]);
-            key0 += kKeys;
-            if (key0 > last_whole) break;
+        if constexpr (NH < 4) {
+            while (step(Index<0>{}) && step(Index<1>{})) {}
+        } else {
+            while (step(Index<0>{}) && step(Index<1>{}) && step(Index<2>{}) && step(Index<3>{})) {}
         }
     }
     for (; key0 < key_hi; key0 += kKeys) {
         load_last(key0, kf[0], vf[0], hidden[0]);
-        use(No{}, key0, kf[0], vf[0], hidden[0]);
-    }
-
-    // the four waves' sums, 16 queries at a time
-#pragma unroll
-    for (int n = 0; n < NQ; ++n) {
-        l[n] = reduce_columns<OpSum>(l[n]);
-        if (g == 0) {
-            wave_m[wave][n * 16 + r16] = m[n];
-            wave_l[wave][n * 16 + r16] = l[n];
+        const int sum = (key0 - key_lo) / kKeys % NH;
+        if (sum == 0) use(No{}, Index<0>{}, key0, kf[0], vf[0], hidden[0]);
+        if constexpr (NH > 1)
+            if (sum == 1) use(No{}, Index<1>{}, key0, kf[0], vf[0], hidden[0]);
+        if constexpr (NH > 2) {
+            if (sum == 2) use(No{}, Index<2>{}, key0, kf[0], vf[0], hidden[0]);
+            if (sum == 3) use(No{}, Index<3>{}, key0, kf[0], vf[0], hidden[0]);
         }
     }
+
+    // the four sums of each head, 16 queries at a time: in LDS as many as there are waves for a head
+#pragma unroll
+    for (int i = 0; i < NH; ++i)
+#pragma unroll
+        for (int n = 0; n < NQ; ++n) {
+            const float l = reduce_columns<OpSum>(sums_l[i][n]);
+            if (g == 0) {
+                part_m[i * kKeyWaves + wave / NH][wave % NH][n * 16 + r16] = sums_m[i][n];
+                part_l[i * kKeyWaves + wave / NH][wave % NH][n * 16 + r16] = l;
+            }
+        }
+    const int r = tid >> 4, c = tid & 15;
 #pragma unroll
     for (int n = 0; n < NQ; ++n) {
-        __syncthreads();
-        float* sums = reinterpret_cast<float*>(mine);
+        const int row = n * 16 + r;
+        const bool mine_too = c < G::kChunks && row < rows;
+        float big[NH], total[NH], acc[NH][8];
 #pragma unroll
-        for (int d = 0; d < G::kTiles; ++d) *reinterpret_cast<f32x4*>(sums + r16 * G::kSumRow + d * 16 + 4 * g) = o[n][d];
-        __syncthreads();
-        for (int item = tid; item < NH * 256; item += 256) {
-            const int hh = item >> 8, r = (item >> 4) & 15, c = item & 15, row = n * 16 + r;
-            if (c >= G::kChunks || row >= rows) continue;
-            const int pr = pair0 + hh, b2 = pr / a.kv_heads, hk2 = pr % a.kv_heads;
-            float big = kFarBelow, total = 0.0f, acc[8] = {};
+        for (int hh = 0; hh < NH; ++hh) {
+            big[hh] = kFarBelow;
+            total[hh] = 0.0f;
 #pragma unroll
-            for (int w = 0; w < kKeyWaves; ++w) big = fmaxf(big, wave_m[w * NH + hh][row]);
+            for (int j = 0; j < 8; ++j) acc[hh][j] = 0.0f;
+        }
 #pragma unroll
-            for (int w = 0; w < kKeyWaves; ++w) {
-                const float f = exp2_raw(wave_m[w * NH + hh][row] - big);
-                total = fmaf(wave_l[w * NH + hh][row], f, total);
-                const float* p = reinterpret_cast<const float*>(lds + (w * NH + hh) * G::kWaveBytes) + r * G::kSumRow + c * 8;
+        for (int i = 0; i < NH; ++i) {
+            if (i > 0 && key_lo + i * kKeys >= key_hi) break;   // no keys in these sums
+            __syncthreads();
+            float* sums = reinterpret_cast<float*>(mine);
 #pragma unroll
-                for (int j = 0; j < 8; ++j) acc[j] = fmaf(p[j], f, acc[j]);
+            for (int d = 0; d < G::kTiles; ++d) *reinterpret_cast<f32x4*>(sums + r16 * G::kSumRow + d * 16 + 4 * g) = sums_o[i][n][d];
+            __syncthreads();
+            if (!mine_too) continue;
+#pragma unroll
+            for (int hh = 0; hh < NH; ++hh) {
+                if (i == 0)
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) big[hh] = fmaxf(big[hh], part_m[s][hh][row]);
+#pragma unroll
+                for (int w = 0; w < kKeyWaves; ++w) {
+                    const int s = i * kKeyWaves + w;
+                    const float f = exp2_raw(part_m[s][hh][row] - big[hh]);
+                    total[hh] = fmaf(part_l[s][hh][row], f, total[hh]);
+                    const float* p = reinterpret_cast<const float*>(lds + (w * NH + hh) * G::kWaveBytes) + r * G::kSumRow + c * 8;
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) acc[hh][j] = fmaf(p[j], f, acc[hh][j]);
+                }
             }
-            if (a.splits == 1) {
-                const float inv = 1.0f / total;
+        }
+        if (!mine_too) continue;
 #pragma unroll
-                for (int j = 0; j < 8; ++j) acc[j] *= inv;
+        for (int hh = 0; hh < NH; ++hh) {
+            const int pr = pair0 + hh, b2 = pr / a.kv_heads, hk2 = pr % a.kv_heads;
+            if (a.splits == 1) {
+                const float inv = 1.0f / total[hh];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) acc[hh][j] *= inv;
                 uint16_t* op = a.o + row / a.group * a.o_s + b2 * a.o_b + (hk2 * a.group + row % a.group) * a.o_h;
-                *reinterpret_cast<u32x4*>(op + c * 8) = pack8<DT>(acc);
+                *reinterpret_cast<u32x4*>(op + c * 8) = pack8<DT>(acc[hh]);
             } else {
                 const int64_t at = ((int64_t)split * pairs + pr) * rows + row;
-                *reinterpret_cast<f32x4*>(a.part_o + at * HD + c * 8) = f32x4{acc[0], acc[1], acc[2], acc[3]};
-                *reinterpret_cast<f32x4*>(a.part_o + at * HD + c * 8 + 4) = f32x4{acc[4], acc[5], acc[6], acc[7]};
-                if (c == 0) *reinterpret_cast<f32x2*>(a.part_ml + at * 2) = f32x2{big, total};
+                *reinterpret_cast<f32x4*>(a.part_o + at * HD + c * 8) = f32x4{acc[hh][0], acc[hh][1], acc[hh][2], acc[hh][3]};
+                *reinterpret_cast<f32x4*>(a.part_o + at * HD + c * 8 + 4) = f32x4{acc[hh][4], acc[hh][5], acc[hh][6], acc[hh][7]};
+                if (c == 0) *reinterpret_cast<f32x2*>(a.part_ml + at * 2) = f32x2{big[hh], total[hh]};
             }
         }
     }
@@ -369,42 +432,60 @@ __global__ void __launch_bounds__(256) cache_append_kernel(CacheArgs a)
     *reinterpret_cast<u32x4*>(a.out + (value ? a.items * 8 : 0) + i * 8) = load16(p + c * 8);
 }
 
-// Heads of a workgroup and workgroups of a pair of batch entry and key/value head.
+// Heads of a workgroup and workgroups of a pair of batch entry and key/value head: the cheapest of those that are open.
 //
-// Heads: four or two where that leaves about one workgroup for each CU (1024 pairs of 128 features, 4 / 2 / 1 heads: 192 / 212
-// / 217 us, 768: 161 / 164 / 172, 512: 199 / 204 / 221, of which the first needs a second kernel, 384: 165 / 162 / 171, 288: 147
-// / 125 / 121), earlier where rows of 160 or 192 bytes end within a cache line (640 pairs of 80 features: 231 / 251 / 304).
+// Splits: at least as many as give each CU a workgroup with 256 keys (each has four sums, and with less the result is further off:
+// 192 pairs of 500 keys 2.17e-3 with two splits, 2.24e-3 with one), at most as many as have 128 keys. With more than 16 queries a
+// pair, beyond eight splits, 256 keys, since the second kernel has 16 KB of each to read (32 queries, 8 pairs of 4000 keys: 16
+// splits 25.4 us, 32 splits 30.4; 16 pairs of 2000: 8 splits 20.6, 16 splits 22.3).
 //
-// Workgroups: few, but so many that they go evenly on 256 CUs, with 256 keys at least (128 where there are less workgroups than
-// CUs). More of them cost the cache's bandwidth and the second kernel (256 pairs of 2000 keys: 85 us with one each, 89 with two;
-// 12 pairs of 200 keys: 6.2, 7.4), uneven ones leave CUs idle (288 pairs: 154 us with one each, 130 with two, 121 with four;
-// 160: 115 with two, 96 with four; 32 of 300: 14 with two, 11 with three).
+// Heads: two from 320 pairs and four from 640, for caches that are long enough: 768 keys, 256 where a row has less than the 256
+// bytes of 128 features (24 sequences of 600, 32 heads of 128: 85 us with one, 94 with four; 20 of 500, 32 heads of 80: 68 with one,
+// 55 with two and four splits), and unsplit four heads of 128 from 256 keys on (1024 pairs of 500: 97 -> 92). From 1024 pairs on also
+// for caches so short that waves would be idle: 32 keys are one wave's, 64 two waves'.
+//
+// Time, us: what a copy of the bytes takes at 5 TB/s, 7 or 14 % less with two or four heads and another 7 % less where rows end
+// within a cache line; times the unevenness (rounds of 256 workgroups over those there are) to the power of 0.6, because the
+// bandwidth of an idle CU goes to the others in part (288 pairs of 2000 keys, 1 / 2 / 4 / 8 splits: 153 / 129 / 121 / 120 us); and
+// 0.2 for each round and head, twice that where one workgroup fills a CU, 1 for the second kernel, 0.2 for each split. Against
+// the best plan that was measured, 84 sizes of 32 to 2048 pairs, 30 to 3000 keys and 64 to 128 features: 2 % behind on average,
+// 14 % at most.
 struct DecodePlan {
     int heads_per_block, splits, keys_per_split;
 };
+static bool decode_heads_open(int heads, int64_t pairs, int64_t sk, int64_t hd, int64_t splits)
+{
+    if (heads == 2) return (pairs >= 320 && sk >= (hd < 128 ? 256 : 768)) || (pairs >= 1024 && sk <= 64 && hd < 128);
+    if (heads == 4) return (pairs >= 640 && (sk >= 768 || (sk >= 256 && hd == 128 && splits == 1))) || (pairs >= 1024 && sk <= 32);
+    return true;
+}
 static DecodePlan decode_plan(int64_t batch, int64_t kv_heads, int64_t rows, int64_t sk, int64_t hd)
 {
-    const int64_t pairs = batch * kv_heads;
-    const bool whole_lines = hd % 64 == 0;
-    int heads = 1;
-    if (rows <= 16 && kv_heads % 4 == 0 && pairs >= (whole_lines ? 640 : 512)) heads = 4;
-    else if (rows <= 16 && kv_heads % 2 == 0 && pairs >= 384) heads = 2;
-    const int64_t groups = pairs / heads, most = sk <= 256 ? 1 : (sk + 127) / 128;
-    int64_t splits = 1, best = 0;
-    for (int64_t s = 1; s <= most && s <= 256; ++s) {
-        const int64_t blocks = groups * s, rounds = (blocks + 255) / 256;
-        if (s > 1 && rounds > 1 && sk < s * 256) break;
-        // rounds of workgroups against their number (192 of them, or 160 with four heads, need no second kernel), and in
-        // hundredths 3 for the second kernel and 1 for each split
-        const bool full = s == 1 && rounds == 1 && blocks >= (heads == 4 ? 160 : 192);
-        const int64_t cost = (full ? 1000 : rounds * 256 * 1000 / blocks) * (100 + (s > 1 ? 3 + s : 0));
-        if (s == 1 || cost < best) {
-            best = cost;
-            splits = s;
+    const int64_t pairs = batch * kv_heads, by_256 = (sk + 255) / 256, for_all = (256 + pairs - 1) / pairs;
+    const int64_t least = for_all < by_256 ? for_all : by_256;
+    int64_t most = sk <= 256 ? 1 : (sk + 127) / 128;
+    if (rows > 16 && most > 8) most = by_256 > 8 ? by_256 : 8;
+    if (most > least + 7) most = least + 7;   // more have never been the best, and the host waits for this
+    const double copy = (double)(pairs * sk * hd * 8) / 5e6;
+    DecodePlan plan{1, 1, 0};
+    double best = 0.0;
+    for (int heads = 1; heads <= (rows <= 16 ? 4 : 1); heads *= 2) {
+        if (kv_heads % heads) break;
+        const double gain = (heads == 1 ? 1.0 : heads == 2 ? 0.93 : 0.86) * (heads > 1 && hd % 64 ? 0.93 : 1.0);
+        for (int64_t s = least; s <= most; ++s) {
+            const int64_t keys = ((sk + s - 1) / s + 127) / 128 * 128, splits = (sk + keys - 1) / keys;   // none of them empty
+            if (!decode_heads_open(heads, pairs, sk, hd, splits)) continue;
+            const int64_t blocks = pairs / heads * splits, rounds = (blocks + 255) / 256;
+            const double us = copy * gain * std::pow((double)(rounds * 256) / (double)blocks, 0.6) +
+                              (decode_blocks_per_cu((int)hd, heads) == 1 ? 0.4 : 0.2) * (double)(rounds * heads) +
+                              (splits > 1 ? 1.0 + 0.2 * (double)splits : 0.0);
+            if (plan.keys_per_split == 0 || us < best) {
+                best = us;
+                plan = {heads, (int)splits, (int)keys};
+            }
         }
     }
-    const int64_t keys = ((sk + splits - 1) / splits + 127) / 128 * 128;
-    return {heads, (int)((sk + keys - 1) / keys), (int)keys};   // no empty split
+    return plan;
 }
 
 template <int DT, int HD>

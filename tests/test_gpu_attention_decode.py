@@ -58,6 +58,32 @@ def test_many_sequences(hn, past, sq, b, np_, nkv):
     assert rel_err(out.view(sq, b, np_, hn), textbook(q, k, v, mask, -10000.0)) <= limit(torch.bfloat16, 2)
 
 
+@pytest.mark.parametrize("hn", [64, 80, 96, 128])
+@pytest.mark.parametrize("past,sq,b,np_,nkv", [(767, 1, 160, 4, 4), (768, 1, 176, 4, 4), (800, 2, 100, 8, 4), (830, 1, 192, 2, 2), (911, 9, 192, 4, 2)])
+def test_many_long_sequences(hn, past, sq, b, np_, nkv):
+    """Two and four heads of keys per workgroup, whole and with their keys cut into parts, the last of them down to one key."""
+    from megatron.model.fused_attention import decode_attention
+
+    q, k, v, layer_past = cached(torch.bfloat16, past, sq, b, np_, nkv, hn)
+    mask = hidden(sq, past + sq).view(1, 1, sq, past + sq)
+    out, present = decode_attention(q, k[past:], v[past:], layer_past, mask, 1 / math.sqrt(hn), -10000.0, merged=True)
+    assert torch.equal(present, torch.stack((k, v)))
+    assert rel_err(out.view(sq, b, np_, hn), textbook(q, k, v, mask, -10000.0)) <= limit(torch.bfloat16, 2)
+
+
+@pytest.mark.parametrize("hn,heads,b", [(64, 32, 32), (96, 32, 32), (128, 32, 16)])
+def test_sums_do_not_depend_on_the_heads_of_a_workgroup(hn, heads, b):
+    """With two or four heads per workgroup the same bits as with one, which is what 256 pairs get (8 sequences of 32 heads): the
+    fewer sums a head's keys go into, the further off is the result."""
+    from megatron.model.fused_attention import decode_attention
+
+    q, k, v, layer_past = cached(torch.bfloat16, 800, 1, b, heads, heads, hn)
+    mask = torch.zeros((1, 1, 1, 801), dtype=torch.bool, device=DEV)
+    out, _ = decode_attention(q, k[800:], v[800:], layer_past, mask, 1 / math.sqrt(hn), -10000.0, merged=True)
+    few, _ = decode_attention(q[:, :8], k[800:, :8], v[800:, :8], layer_past[:, :, :8], mask, 1 / math.sqrt(hn), -10000.0, merged=True)
+    assert torch.equal(out[:, :8], few)
+
+
 def test_nan_and_infinite_keys_stay_where_they_are():
     """A value that is not finite reaches the queries that see it and no others; the cache keeps it."""
     from megatron.model.fused_attention import decode_attention

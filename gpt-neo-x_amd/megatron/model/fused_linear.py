@@ -74,7 +74,7 @@ def linear(x, weight, bias: Optional[torch.Tensor] = None):
 
 @torch.jit.unused
 def _linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> torch.Tensor:
-    if not _hp._is_compiling():
+    if isinstance(x, torch.Tensor) and x.is_cuda and not _hp._is_compiling():
         y = _hp.native().linear(x, weight, bias, MAX_ROWS, MAX_ROWS_NARROW)
         if y is not NotImplemented:
             return y

@@ -100,7 +100,7 @@ class MLP(torch.nn.Module):
 
     def _few_rows(self, x):
         """Whether ``x`` may be few rows that nobody differentiates (the launches ask closely)."""
-        return (not _hp._is_compiling() and not torch.is_grad_enabled() and isinstance(x, torch.Tensor) and x.dim() > 0
+        return (not _hp._is_compiling() and not torch.is_grad_enabled() and isinstance(x, torch.Tensor) and x.is_cuda and x.dim() > 0
                 and x.numel() <= fused_linear.MAX_ROWS_NARROW * x.size(-1))
 
     def add_to(self, residual, x, other=None, other_bias=None):

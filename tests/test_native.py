@@ -45,6 +45,28 @@ def test_a_missing_module_is_an_error(monkeypatch):
         hp.native()
 
 
+def test_what_works_without_a_gpu_needs_no_module(monkeypatch):
+    """Linear layers, a feed forward block of torch's activations and the norms, on tensors that are not on a GPU."""
+    import types
+
+    from megatron.model.fused_linear import linear
+    from megatron.model.norms import LayerNorm, RMSNorm
+    from megatron.model.transformer_layer import MLP, Linear
+
+    def missing():
+        raise ImportError("not built")
+
+    monkeypatch.setattr(hp, "native", missing)
+    x = torch.randn((3, 512))
+    mlp = MLP(types.SimpleNamespace(activation="silu", hidden_size=512, intermediate_size=1536))
+    mlp.linear2 = Linear(1536, 512, skip_bias_add=True)
+    for grad in (True, False):
+        with torch.set_grad_enabled(grad):
+            assert torch.equal(linear(x, mlp.linear1.weight), torch.nn.functional.linear(x, mlp.linear1.weight))
+            assert Linear(512, 64)(x)[0].shape == (3, 64) and LayerNorm(512)(x).shape == RMSNorm(512)(x).shape == x.shape
+            assert mlp(x)[0].shape == x.shape and mlp.add_to(x, x) is None
+
+
 def test_what_could_be_scripted_still_can():
     """TorchScript takes the modules and functions around the native calls as it did, and leaves those out."""
     from megatron.model.activations import bias_gelu_impl

@@ -18,6 +18,7 @@ then has to reduce.
 import torch
 
 from ..fused_kernels import _hotpath as _hp
+from .fused_attention import as_written
 
 
 def _as_rows(t, cols, what):
@@ -209,6 +210,7 @@ class _GatedActivationFunction(torch.autograd.Function):
         return din, dbias, None
 
 
+@as_written
 class Gated_Activation(torch.nn.Module):
     """``x, gate = x.chunk(2, dim=-1); activation_func(gate + bias_2) * (x + bias_1)``
     (megatron/model/transformer.py:186-206). ``activation_func`` is one of the functions ``get_activation``

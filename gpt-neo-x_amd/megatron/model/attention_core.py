@@ -175,6 +175,7 @@ class _CausalContextGemm(torch.autograd.Function):
         return grad_probs, grad_value, None, None, None
 
 
+@fused_attention.as_written
 class CoreAttention(torch.nn.Module):
     """Unfused ("global") attention on top of the fused softmax.
 

@@ -10,7 +10,6 @@ Layouts as in ``CoreAttention``: q ``[sq, b, np, hn]``, k and v ``[sk, b, nkv, h
 strides with contiguous features.
 """
 import ctypes
-import functools
 
 import torch
 from torch.nn.modules.module import _has_any_global_hook
@@ -186,18 +185,27 @@ def plain(*tensors):
     return not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors)) and not _hp.followed(*tensors)
 
 
-@functools.lru_cache(maxsize=8)
-def _methods(cls):
-    return frozenset(name for name, member in vars(cls).items() if callable(member) or isinstance(member, (property, staticmethod)))
+_AS_WRITTEN = {}
+_CALL = torch.nn.Module.__call__
+
+
+def as_written(cls):
+    """Class decorator: remembers what the class consists of, for ``untouched``."""
+    cls.__annotations__   # torch.jit would make it later
+    members = dict(vars(cls))
+    methods = (name for name, member in members.items() if callable(member) or isinstance(member, (property, staticmethod)))
+    _AS_WRITTEN[cls] = members, frozenset(methods) | {"_call_impl", "_compiled_call_impl"}
+    return cls
 
 
 def untouched(module, cls):
-    """Whether ``module`` is a ``cls`` as it stands: no subclass, none of its methods replaced, no hooks. Whoever put such a
-    thing there wants the tensors that pass through the module, so it has to be called, with those tensors; so does torch
-    while it compiles."""
+    """Whether ``module`` is a ``cls`` as it stands in its file (the class is marked ``as_written``): no subclass, nothing of the
+    class replaced or added, none of its methods replaced in the module, no hooks, not compiled. Whoever put such a thing there
+    wants the tensors that pass through the module, so it has to be called, with those tensors; so does torch while it compiles."""
     own = module.__dict__
-    return (not _hp._is_compiling() and type(module) is cls and own.keys().isdisjoint(_methods(cls))
-            and not (own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or own["_backward_pre_hooks"]
+    members, methods = _AS_WRITTEN[cls]
+    return (not _hp._is_compiling() and type(module) is cls and own.keys().isdisjoint(methods) and vars(cls) == members
+            and torch.nn.Module.__call__ is _CALL and not (own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or own["_backward_pre_hooks"]
                      or _has_any_global_hook()))
 
 

@@ -44,6 +44,7 @@ from torch import nn
 from ..fused_kernels import _hotpath as _hp
 from ..fused_kernels import load_fused_kernels
 from . import dropout_rng
+from .fused_attention import as_written
 
 
 class SoftmaxFusionTypes(enum.Enum):
@@ -259,6 +260,7 @@ def _fill_value(mask_func, dtype=torch.float32):
     return fill if taken else None
 
 
+@as_written
 class FusedScaleMaskSoftmax(nn.Module):
     """Scaling, masking and softmax of attention scores ``[b, np, sq, sk]``.
 

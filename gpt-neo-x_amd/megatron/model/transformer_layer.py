@@ -38,6 +38,7 @@ from .norms import get_norm, layer_norm_pair
 from .positional_embeddings import AliBi, RotaryEmbedding
 
 
+@fused_attention.as_written
 class Linear(torch.nn.Module):
     """``y = x W^T (+ b)``; with ``skip_bias_add`` the bias is returned beside the product instead of being
     added (what the reference's Column/RowParallelLinear do, megatron/mpu/layers.py), so that the next fused
@@ -56,6 +57,7 @@ class Linear(torch.nn.Module):
         return linear(x, self.weight, self.bias), None
 
 
+@fused_attention.as_written
 class MLP(torch.nn.Module):
     """``ParallelMLP`` (megatron/model/transformer.py:93-196): h -> ffn -> activation -> h, the second bias handed on."""
 
@@ -84,7 +86,7 @@ class MLP(torch.nn.Module):
 
     def _activated(self, x):
         """The activated intermediate for the few rows of a decoding step, in the launch of the first product, or None."""
-        if not fused_attention.untouched(self.linear1, Linear):
+        if not (fused_attention.untouched(self.linear1, Linear) and self.linear1.skip_bias_add):
             return None
         bias = self.linear1.bias
         if self.is_gated:
@@ -107,7 +109,8 @@ class MLP(torch.nn.Module):
         """``residual + mlp(x)`` or ``residual + ((other + other_bias) + mlp(x))`` for the few rows of a decoding step, the
         activation and the addition each in the launch of a product; None for anything else, and where somebody looks at the
         modules."""
-        if not self._few_rows(x) or not (fused_attention.untouched(self, MLP) and fused_attention.untouched(self.linear2, Linear)):
+        if not self._few_rows(x) or not (fused_attention.untouched(self, MLP) and fused_attention.untouched(self.linear2, Linear)
+                                         and self.linear2.skip_bias_add):
             return None
         intermediate = self._activated(x)
         if intermediate is None:
@@ -232,8 +235,9 @@ class SelfAttention(torch.nn.Module):
         return query, key, value
 
 
-# what the sum of the feed forward block's launch stands for; any other function set on the layer is called
+# what the sum of the feed forward block's launch stands for; any other function set on the layer or in this module is called
 _FUSED_ADDS = (bias_dropout_add_fused_train, bias_dropout_add_fused_inference)
+_FUSED_PAIR = bias_add_residual_pair
 
 
 class TransformerLayer(torch.nn.Module):
@@ -283,9 +287,10 @@ class TransformerLayer(torch.nn.Module):
             attention_output, attention_bias = self._attend(x1, attention_mask, layer_past)
             if self.bias_dropout_fusion and (self.hidden_dropout == 0.0 or not self.training):
                 # no dropout: attention branch + MLP branch + residual in one pass
-                output = self._mlp_added(residual, x2, attention_output, attention_bias)
-                if output is not None:
-                    return output
+                if bias_add_residual_pair is _FUSED_PAIR:
+                    output = self._mlp_added(residual, x2, attention_output, attention_bias)
+                    if output is not None:
+                        return output
                 mlp_output, mlp_bias = self.mlp(x2)
                 return bias_add_residual_pair(attention_output, attention_bias, mlp_output, mlp_bias, residual)
             if attention_bias is not None:

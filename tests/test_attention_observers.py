@@ -133,3 +133,82 @@ def test_a_layer_attention_compiles_whole(past):
         (want, want_present), _ = attention(*args)
         (got, present), _ = torch.compile(attention, fullgraph=True, backend="eager")(*args)
     assert torch.allclose(got, want, atol=1e-6) and torch.equal(present, want_present)
+
+
+class OnGpu(torch.Tensor):
+    """Says that it is on a GPU, for what is asked before the first launch."""
+    is_cuda = True
+
+
+class Launches:
+    """Stands for the extension module."""
+
+    def linear_act(self, x, *args):
+        return x
+
+    def linear_add(self, *args):
+        return "one launch"
+
+
+def few_rows():
+    from megatron.model.transformer_layer import MLP
+
+    mlp = MLP(types.SimpleNamespace(activation="swiglu", hidden_size=512, use_bias_in_mlp=False))
+    return mlp, torch.randn((1, 1, 512)).as_subclass(OnGpu)
+
+
+REPLACED = {
+    "forward of the class": lambda m, mlp: m.setattr(type(mlp), "forward", lambda self, x: None),
+    "forward of the linear layers": lambda m, mlp: m.setattr(type(mlp.linear1), "forward", lambda self, x: None),
+    "forward of the gate": lambda m, mlp: m.setattr(type(mlp.activation_func), "forward", lambda self, x: None),
+    "call of the class": lambda m, mlp: m.setattr(type(mlp), "__call__", lambda self, x: None, raising=False),
+    "call of every module": lambda m, mlp: m.setattr(torch.nn.Module, "__call__", lambda self, x: None),
+    "compiled": lambda m, mlp: m.setattr(mlp.linear2, "_compiled_call_impl", lambda self, x: None, raising=False),
+    "bias added in the layer": lambda m, mlp: m.setattr(mlp.linear2, "skip_bias_add", False),
+    "another layer": lambda m, mlp: mlp.__setattr__("linear1", torch.nn.Linear(512, 512)),
+}
+
+
+@pytest.mark.parametrize("who", REPLACED)
+def test_a_decoding_step_calls_what_was_replaced(who, monkeypatch):
+    """The launches of few rows stand for the classes of this package as they are written."""
+    from megatron.fused_kernels import _hotpath
+
+    monkeypatch.setattr(_hotpath, "native", Launches)
+    mlp, x = few_rows()
+    with torch.no_grad():
+        assert mlp.add_to(x, x) == "one launch"
+        REPLACED[who](monkeypatch, mlp)
+        assert mlp.add_to(x, x) is None
+
+
+@pytest.mark.parametrize("who", ["softmax", "core"])
+def test_attention_classes_that_were_replaced_are_called(who, monkeypatch):
+    c = core()
+    assert scale(c) is not None and fused_attention.untouched(c, CoreAttention)
+    monkeypatch.setattr(FusedScaleMaskSoftmax if who == "softmax" else CoreAttention, "forward", lambda *a, **k: None)
+    assert scale(c) is None if who == "softmax" else not fused_attention.untouched(c, CoreAttention)
+
+
+@pytest.mark.parametrize("replaced", [False, True])
+def test_a_replaced_addition_of_both_branches_is_called(replaced, monkeypatch):
+    """In the parallel layout, where the attention's output is added in the launch of the feed forward block."""
+    from megatron.model import transformer_layer as layers
+
+    class Layer(layers.TransformerLayer):
+        def _attend(self, x, attention_mask, layer_past):
+            return x, None
+
+        def _mlp_added(self, *args):
+            return "one launch"
+
+    args = types.SimpleNamespace(norm="layernorm", layernorm_epsilon=1e-5, hidden_size=128, num_attention_heads=2, seq_length=16, precision="fp32",
+                                 pos_emb="none", activation="silu", intermediate_size=768, gpt_j_residual=True, gpt_j_tied=True, hidden_dropout=0.0,
+                                 scaled_upper_triang_masked_softmax_fusion=False, scaled_masked_softmax_fusion=False)
+    layer = Layer(args, lambda s, m: s, 1).eval()
+    layer.mlp = torch.nn.Identity()
+    layer.mlp.forward = lambda x: (x, None)
+    if replaced:
+        monkeypatch.setattr(layers, "bias_add_residual_pair", lambda *a: "the sum")
+    with torch.no_grad():
+        assert layer(torch.randn((2, 1, 128)), None) == ("the sum" if replaced else "one launch")

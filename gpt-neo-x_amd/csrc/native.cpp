@@ -1049,4 +1049,16 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, kMethods, 
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__native() { return PyModule_Create(&kModule); }
+// BUILT_FOR: the versions of torch, of Python and of the library's interface that this file was compiled against
+PyMODINIT_FUNC PyInit__native()
+{
+    PyObject* module = PyModule_Create(&kModule);
+    if (!module) return nullptr;
+    PyObject* versions = Py_BuildValue("(ssi)", NHP_TORCH_VERSION, Py_STRINGIFY(PY_MAJOR_VERSION) "." Py_STRINGIFY(PY_MINOR_VERSION), NHP_ABI_VERSION);
+    if (!versions || PyModule_AddObject(module, "BUILT_FOR", versions) < 0) {
+        Py_XDECREF(versions);
+        Py_DECREF(module);
+        return nullptr;
+    }
+    return module;
+}

@@ -1405,7 +1405,7 @@ int nhp_rope_freqs_qk_bwd(void* q_out, void* k_out, const void* q_in, const void
                                q_out_stride, k_out_stride, dtype, stream);
 }
 
-int nhp_abi_version(void) { return 1; }
+int nhp_abi_version(void) { return NHP_ABI_VERSION; }
 
 const char* nhp_status_string(int status)
 {

@@ -35,7 +35,7 @@ def load(neox_args=None):
     """Build (if needed) and load the kernels.
 
     ``neox_args`` is only consulted for ``rank`` to decide verbosity, as in the
-    reference. Raises if the build or the load fails.
+    reference. Raises if the build or the load fails, and if what is built is for other versions.
     """
     verbose = True if neox_args is None else (getattr(neox_args, "rank", 0) == 0)
     if not (os.path.exists(_hotpath.LIB_PATH) and os.path.exists(_hotpath.NATIVE_PATH)):
@@ -43,6 +43,7 @@ def load(neox_args=None):
             print(f"building {_hotpath.LIB_PATH} for gfx950 ...", flush=True)
         _hotpath.build(verbose=verbose)
     _hotpath.lib()
+    _hotpath.native()
     _register_extension_modules()
 
 

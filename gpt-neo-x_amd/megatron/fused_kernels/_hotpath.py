@@ -6,6 +6,7 @@ is raised, there is no fallback of any kind.
 import ctypes
 import os
 import subprocess
+import sys
 import threading
 
 import torch
@@ -26,7 +27,7 @@ _lib = None
 
 def build(force=False, verbose=False):
     """Compile the HIP sources for gfx950 with hipcc (``make`` in csrc/)."""
-    cmd = ["make", "-C", CSRC_DIR, "-j4"] + (["-B"] if force else [])
+    cmd = ["make", "-C", CSRC_DIR, "-j4", f"PYTHON={sys.executable}"] + (["-B"] if force else [])
     out = None if verbose else subprocess.DEVNULL
     subprocess.run(cmd, check=True, stdout=out, stderr=None if verbose else subprocess.PIPE)
     return LIB_PATH
@@ -145,7 +146,7 @@ _native = None
 
 def native():
     """The extension module with the host side of the most frequent calls (csrc/native.cpp); raises ImportError when it is
-    absent. Its functions return NotImplemented for operands that they leave to the caller. Not to be called while torch
+    absent or built for another torch, Python or library than the running ones. Its functions return NotImplemented for operands that they leave to the caller. Not to be called while torch
     compiles: it does not see through them."""
     global _native
     if _native is None:
@@ -153,6 +154,9 @@ def native():
             from . import _native as module   # links libneox_hotpath.so beside it
         except ImportError as e:
             raise ImportError(f"cannot load {NATIVE_PATH}: {e}") from e
+        built, running = getattr(module, "BUILT_FOR", None), (str(torch.__version__), "%d.%d" % sys.version_info[:2], ABI_VERSION)
+        if built != running:
+            raise ImportError(f"{NATIVE_PATH} is built for {built}, but torch, Python and the library's interface are {running}; rebuild it")
         _native = module
     return _native
 

@@ -48,6 +48,7 @@ typedef enum nhp_status {
 } nhp_status;
 
 /* Library ABI version (bumped when a signature changes). */
+#define NHP_ABI_VERSION 1
 int nhp_abi_version(void);
 
 /* Static, human readable text for an nhp_status value. Never NULL. */

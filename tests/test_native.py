@@ -45,6 +45,34 @@ def test_a_missing_module_is_an_error(monkeypatch):
         hp.native()
 
 
+@pytest.mark.parametrize("built", [("2.9.1+rocm6.4", None, None), (None, "3.11", None), (None, None, 0), None])
+def test_a_module_built_for_something_else_is_an_error(built, monkeypatch):
+    """Torch's C++ interface holds for one version: such a module is not called, neither by the layers nor after ``load``."""
+    import sys
+    import types
+
+    import megatron.fused_kernels as fk
+
+    fits = hp.native().BUILT_FOR
+    assert fits == (torch.__version__, "%d.%d" % sys.version_info[:2], hp.lib().nhp_abi_version())
+    other = types.SimpleNamespace() if built is None else types.SimpleNamespace(BUILT_FOR=tuple(b if b is not None else f for b, f in zip(built, fits)))
+    monkeypatch.setattr(hp, "_native", None)
+    monkeypatch.setattr(fk, "_native", other, raising=False)
+    for call in (hp.native, fk.load):
+        with pytest.raises(ImportError, match="rebuild"):
+            call()
+    assert hp._native is None
+
+
+def test_the_build_is_for_the_running_python(monkeypatch):
+    import sys
+
+    seen = []
+    monkeypatch.setattr(hp.subprocess, "run", lambda cmd, **kw: seen.append(cmd))
+    hp.build()
+    assert f"PYTHON={sys.executable}" in seen[0]
+
+
 def test_what_works_without_a_gpu_needs_no_module(monkeypatch):
     """Linear layers, a feed forward block of torch's activations and the norms, on tensors that are not on a GPU."""
     import types

@@ -657,6 +657,18 @@ bool wants_grad(std::initializer_list<const Tensor*> tensors)
 // --------------------------------------------------------------------------------------------------------- entry points
 PyObject* not_here() { Py_RETURN_NOTIMPLEMENTED; }
 
+// What `work` returns, other Python threads running meanwhile: an allocation may wait for the driver and a launch for a queue
+// that is full. What comes back into Python (hooks on saved tensors, anomaly mode) takes the lock by itself. (0.2 us a call.)
+template <typename F>
+auto unlocked(F work)
+{
+    struct Lock {
+        PyThreadState* const state = PyEval_SaveThread();
+        ~Lock() { PyEval_RestoreThread(state); }
+    } lock;
+    return work();
+}
+
 PyObject* pack(const variable_list& tensors)
 {
     PyObject* tuple = PyTuple_New((Py_ssize_t)tensors.size());
@@ -676,7 +688,7 @@ PyObject* py_layer_norm(PyObject*, PyObject* const* args, Py_ssize_t count)
     if (followed() || !take_all(args, count, x, w, b, eps) || x.dim() < 1 || type_code(x.scalar_type()) < 0 ||
         !parameters_fit(x, {&w, &b}, x.size(-1), pcode))
         return not_here();
-    return THPVariable_Wrap(LayerNormNode::apply(x, w, b, eps, (int64_t)pcode));
+    return THPVariable_Wrap(unlocked([&] { return LayerNormNode::apply(x, w, b, eps, (int64_t)pcode); }));
     END_HANDLE_TH_ERRORS
 }
 
@@ -691,7 +703,7 @@ PyObject* py_layer_norm_pair(PyObject*, PyObject* const* args, Py_ssize_t count)
     if (followed() || !take_all(args, count, x, w1, b1, w2, b2, eps) || x.dim() < 1 || type_code(x.scalar_type()) < 0 ||
         !parameters_fit(x, {&w1, &b1, &w2, &b2}, x.size(-1), pcode))
         return not_here();
-    return pack(LayerNormPairNode::apply(x, w1, b1, w2, b2, eps, (int64_t)pcode));
+    return pack(unlocked([&] { return LayerNormPairNode::apply(x, w1, b1, w2, b2, eps, (int64_t)pcode); }));
     END_HANDLE_TH_ERRORS
 }
 
@@ -707,7 +719,7 @@ PyObject* py_rms_norm(PyObject*, PyObject* const* args, Py_ssize_t count)
     if (followed() || !take_all(args, count, x, s, o, eps, mode, stat) || x.dim() < 1 || type_code(x.scalar_type()) < 0 ||
         !parameters_fit(x, {&s, &o}, x.size(-1), pcode) || mode < 0 || mode > 2 || stat < 1 || stat > x.size(-1))
         return not_here();
-    return THPVariable_Wrap(RMSNormNode::apply(x, s, o, eps, mode, stat, (int64_t)pcode));
+    return THPVariable_Wrap(unlocked([&] { return RMSNormNode::apply(x, s, o, eps, mode, stat, (int64_t)pcode); }));
     END_HANDLE_TH_ERRORS
 }
 
@@ -719,7 +731,7 @@ PyObject* py_bias_gelu(PyObject*, PyObject* const* args, Py_ssize_t count)
     MaybeTensor b;
     if (followed() || !take_all(args, count, x, b) || x.dim() < 1 || type_code(x.scalar_type()) < 0) return not_here();
     if (b && (b->dim() != 1 || b->size(0) != x.size(-1) || !alike(*b, x))) return not_here();
-    return THPVariable_Wrap(BiasGeluNode::apply(x, b));
+    return THPVariable_Wrap(unlocked([&] { return BiasGeluNode::apply(x, b); }));
     END_HANDLE_TH_ERRORS
 }
 
@@ -730,7 +742,7 @@ PyObject* py_gated(PyObject*, PyObject* const* args, Py_ssize_t count)
     Tensor x;
     int64_t act;
     if (followed() || !take_all(args, count, x, act) || x.dim() < 1 || x.size(-1) % 2 || type_code(x.scalar_type()) < 0) return not_here();
-    return THPVariable_Wrap(GatedNode::apply(x, act));
+    return THPVariable_Wrap(unlocked([&] { return GatedNode::apply(x, act); }));
     END_HANDLE_TH_ERRORS
 }
 
@@ -743,7 +755,7 @@ PyObject* py_causal_softmax(PyObject*, PyObject* const* args, Py_ssize_t count)
     int64_t window;
     if (followed() || !take_all(args, count, x, scale, window) || x.dim() != 4 || x.size(2) != x.size(3) || !is_half(x) || !x.is_contiguous())
         return not_here();
-    return THPVariable_Wrap(CausalSoftmaxNode::apply(x, scale, window));
+    return THPVariable_Wrap(unlocked([&] { return CausalSoftmaxNode::apply(x, scale, window); }));
     END_HANDLE_TH_ERRORS
 }
 
@@ -757,7 +769,7 @@ PyObject* py_masked_softmax(PyObject*, PyObject* const* args, Py_ssize_t count)
         mask.element_size() != 1 || mask.device() != x.device() || x.size(2) < 2 || (mask.size(0) != 1 && mask.size(0) != x.size(0)) ||
         mask.size(1) != 1 || mask.size(2) != x.size(2) || mask.size(3) != x.size(3))
         return not_here();
-    return THPVariable_Wrap(MaskedSoftmaxNode::apply(x, mask, scale));
+    return THPVariable_Wrap(unlocked([&] { return MaskedSoftmaxNode::apply(x, mask, scale); }));
     END_HANDLE_TH_ERRORS
 }
 
@@ -771,7 +783,7 @@ PyObject* py_rotary(PyObject*, PyObject* const* args, Py_ssize_t count)
         !alike(q, k) || q.size(0) != k.size(0) || q.size(1) != k.size(1) || q.size(3) != k.size(3) ||
         !tables_fit(cos, sin, q, q.size(3), q.size(0), offset))
         return not_here();
-    return pack(RotaryNode::apply(q, k, table_rows(cos, offset, q.size(0)), table_rows(sin, offset, q.size(0))));
+    return pack(unlocked([&] { return RotaryNode::apply(q, k, table_rows(cos, offset, q.size(0)), table_rows(sin, offset, q.size(0))); }));
     END_HANDLE_TH_ERRORS
 }
 
@@ -786,7 +798,7 @@ PyObject* py_split_rotary(PyObject*, PyObject* const* args, Py_ssize_t count)
         return not_here();
     const int64_t divided = heads == 0 ? 3 : heads + 2 * kv_heads, hn = mixed.size(-1) / divided;
     if (mixed.size(-1) % divided || !tables_fit(cos, sin, mixed, hn, mixed.size(0), offset)) return not_here();
-    return pack(SplitRotaryNode::apply(mixed, table_rows(cos, offset, mixed.size(0)), table_rows(sin, offset, mixed.size(0)), heads, kv_heads));
+    return pack(unlocked([&] { return SplitRotaryNode::apply(mixed, table_rows(cos, offset, mixed.size(0)), table_rows(sin, offset, mixed.size(0)), heads, kv_heads); }));
     END_HANDLE_TH_ERRORS
 }
 
@@ -801,7 +813,7 @@ PyObject* py_add_residual(PyObject*, PyObject* const* args, Py_ssize_t count)
     if (followed() || !take_all(args, count, x, b, r) || x.dim() < 1 || type_code(x.scalar_type()) < 0 || !bias_fits(b, x) ||
         (r && (r->sizes() != x.sizes() || !alike(*r, x))))
         return not_here();
-    return THPVariable_Wrap(AddResidualNode::apply(x, b, r));
+    return THPVariable_Wrap(unlocked([&] { return AddResidualNode::apply(x, b, r); }));
     END_HANDLE_TH_ERRORS
 }
 
@@ -814,7 +826,7 @@ PyObject* py_add_residual_pair(PyObject*, PyObject* const* args, Py_ssize_t coun
     if (followed() || !take_all(args, count, x1, b1, x2, b2, r) || x1.dim() < 1 || type_code(x1.scalar_type()) < 0 || !bias_fits(b1, x1) ||
         !bias_fits(b2, x1) || x2.sizes() != x1.sizes() || !alike(x2, x1) || r.sizes() != x1.sizes() || !alike(r, x1))
         return not_here();
-    return THPVariable_Wrap(AddResidualPairNode::apply(x1, b1, x2, b2, r));
+    return THPVariable_Wrap(unlocked([&] { return AddResidualPairNode::apply(x1, b1, x2, b2, r); }));
     END_HANDLE_TH_ERRORS
 }
 
@@ -827,7 +839,7 @@ PyObject* py_causal_attention(PyObject*, PyObject* const* args, Py_ssize_t count
     int64_t window;
     bool merged;
     if (followed() || !take_all(args, count, q, k, v, scale, window, merged) || !attention_fits(q, k, v)) return not_here();
-    return THPVariable_Wrap(CausalAttentionNode::apply(q, k, v, scale, window, merged, wants_grad({&q, &k, &v})));
+    return THPVariable_Wrap(unlocked([&] { return CausalAttentionNode::apply(q, k, v, scale, window, merged, wants_grad({&q, &k, &v})); }));
     END_HANDLE_TH_ERRORS
 }
 
@@ -843,19 +855,21 @@ PyObject* py_masked_attention(PyObject*, PyObject* const* args, Py_ssize_t count
     if (mask.scalar_type() != at::kBool || mask.device() != q.device() || mask.dim() != 4 || (mask.size(0) != 1 && mask.size(0) != b) ||
         mask.size(1) != 1 || mask.size(2) != sq || mask.size(3) != sk || sk > 65536 || mask.size(0) * sq >= (1 << 26))
         return not_here();
-    const at::NoGradGuard no_grad;
-    const c10::DeviceGuard guard(q.device());
-    q = readable(q);
-    k = readable(k);
-    v = readable(v);
-    mask = mask.contiguous();
-    const Tensor bits = at::empty({mask.size(0), sq, (sk + 63) / 64}, q.options().dtype(at::kLong));
-    auto [out, out_strides] = new_context(q, merged);
-    check(nhp_attention_mask_bits(bits.data_ptr(), mask.data_ptr(), mask.size(0), sq, sk, stream_of(q)), "masked_attention");
-    check(nhp_attention_fwd_keep(out.data_ptr(), nullptr, nullptr, q.data_ptr(), k.data_ptr(), v.data_ptr(), bits.data_ptr(), mask.size(0),
-                                 (float)fill, (float)scale, -1, b, q.size(2), k.size(2), sq, sk, q.size(3), Strides3(q).s, Strides3(k).s,
-                                 Strides3(v).s, out_strides.s, type_code(q.scalar_type()), stream_of(q)), "masked_attention");
-    return THPVariable_Wrap(out);
+    return THPVariable_Wrap(unlocked([&] {
+        const at::NoGradGuard no_grad;
+        const c10::DeviceGuard guard(q.device());
+        q = readable(q);
+        k = readable(k);
+        v = readable(v);
+        mask = mask.contiguous();
+        const Tensor bits = at::empty({mask.size(0), sq, (sk + 63) / 64}, q.options().dtype(at::kLong));
+        auto [out, out_strides] = new_context(q, merged);
+        check(nhp_attention_mask_bits(bits.data_ptr(), mask.data_ptr(), mask.size(0), sq, sk, stream_of(q)), "masked_attention");
+        check(nhp_attention_fwd_keep(out.data_ptr(), nullptr, nullptr, q.data_ptr(), k.data_ptr(), v.data_ptr(), bits.data_ptr(), mask.size(0),
+                                     (float)fill, (float)scale, -1, b, q.size(2), k.size(2), sq, sk, q.size(3), Strides3(q).s, Strides3(k).s,
+                                     Strides3(v).s, out_strides.s, type_code(q.scalar_type()), stream_of(q)), "masked_attention");
+        return out;
+    }));
     END_HANDLE_TH_ERRORS
 }
 
@@ -898,22 +912,24 @@ PyObject* py_decode_attention(PyObject*, PyObject* const* args, Py_ssize_t count
     if (k.size(0) != sq || sk < 4 || sq * (np / nkv) > 32 || mask.scalar_type() != at::kBool || mask.device() != q.device() || mask.dim() != 4 ||
         (mask.size(0) != 1 && mask.size(0) != b) || mask.size(1) != 1 || mask.size(2) != sq || mask.size(3) != sk)
         return not_here();
-    const at::NoGradGuard no_grad;
-    const c10::DeviceGuard guard(q.device());
-    q = readable(q);
-    k = readable(k);
-    v = readable(v);
-    if (mask.stride(3) != 1) mask = mask.contiguous();
-    auto [out, out_strides] = new_context(q, merged);
-    Tensor present = at::empty({2, sk, b, nkv, hn}, k.options());
-    const Tensor ws = bytes(nhp_attention_decode_workspace_bytes(b, np, nkv, sq, n, hn), q);
-    const char* keys = static_cast<const char*>(past.data_ptr());
-    const Strides3 ps = past_strides(past);
-    check(nhp_attention_decode(out.data_ptr(), present.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), keys, keys + 2 * past.stride(0),
-                               mask.data_ptr(), mask.size(0) > 1 ? mask.stride(0) : 0, mask.stride(2), (float)fill, ptr(ws), (float)scale, b, np,
-                               nkv, sq, n, hn, out_strides.s, Strides3(q).s, Strides3(k).s, Strides3(v).s, ps.s, ps.s,
-                               type_code(q.scalar_type()), stream_of(q)), "decode_attention");
-    return pack({out, present});
+    return pack(unlocked([&] {
+        const at::NoGradGuard no_grad;
+        const c10::DeviceGuard guard(q.device());
+        q = readable(q);
+        k = readable(k);
+        v = readable(v);
+        if (mask.stride(3) != 1) mask = mask.contiguous();
+        auto [out, out_strides] = new_context(q, merged);
+        Tensor present = at::empty({2, sk, b, nkv, hn}, k.options());
+        const Tensor ws = bytes(nhp_attention_decode_workspace_bytes(b, np, nkv, sq, n, hn), q);
+        const char* keys = static_cast<const char*>(past.data_ptr());
+        const Strides3 ps = past_strides(past);
+        check(nhp_attention_decode(out.data_ptr(), present.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), keys, keys + 2 * past.stride(0),
+                                   mask.data_ptr(), mask.size(0) > 1 ? mask.stride(0) : 0, mask.stride(2), (float)fill, ptr(ws), (float)scale, b, np,
+                                   nkv, sq, n, hn, out_strides.s, Strides3(q).s, Strides3(k).s, Strides3(v).s, ps.s, ps.s,
+                                   type_code(q.scalar_type()), stream_of(q)), "decode_attention");
+        return variable_list{out, present};
+    }));
     END_HANDLE_TH_ERRORS
 }
 
@@ -925,18 +941,20 @@ PyObject* py_append_to_cache(PyObject*, PyObject* const* args, Py_ssize_t count)
     MaybeTensor past;
     if (followed() || !take_all(args, count, k, v, past) || wants_grad({&k, &v}) || !cache_fits(k, v, past ? past->size(1) : 0)) return not_here();
     if (past && (!continues(*past, k) || !rows_readable(*past) || wants_grad({&*past}))) return not_here();
-    const at::NoGradGuard no_grad;
-    const c10::DeviceGuard guard(k.device());
-    k = readable(k);
-    v = readable(v);
-    const int64_t n = past ? past->size(1) : 0, sq = k.size(0), b = k.size(1), nkv = k.size(2), hn = k.size(3);
-    Tensor present = at::empty({2, n + sq, b, nkv, hn}, k.options());
-    const char* keys = past ? static_cast<const char*>(past->data_ptr()) : nullptr;
-    const Strides3 ps = past ? past_strides(*past) : Strides3(0, 0, 0);
-    check(nhp_kv_cache_append(present.data_ptr(), k.data_ptr(), v.data_ptr(), keys, past ? keys + 2 * past->stride(0) : nullptr, b, nkv, sq, n, hn,
-                              Strides3(k).s, Strides3(v).s, past ? ps.s : nullptr, past ? ps.s : nullptr, type_code(k.scalar_type()), stream_of(k)),
-          "append_to_cache");
-    return THPVariable_Wrap(present);
+    return THPVariable_Wrap(unlocked([&] {
+        const at::NoGradGuard no_grad;
+        const c10::DeviceGuard guard(k.device());
+        k = readable(k);
+        v = readable(v);
+        const int64_t n = past ? past->size(1) : 0, sq = k.size(0), b = k.size(1), nkv = k.size(2), hn = k.size(3);
+        Tensor present = at::empty({2, n + sq, b, nkv, hn}, k.options());
+        const char* keys = past ? static_cast<const char*>(past->data_ptr()) : nullptr;
+        const Strides3 ps = past ? past_strides(*past) : Strides3(0, 0, 0);
+        check(nhp_kv_cache_append(present.data_ptr(), k.data_ptr(), v.data_ptr(), keys, past ? keys + 2 * past->stride(0) : nullptr, b, nkv, sq, n, hn,
+                                  Strides3(k).s, Strides3(v).s, past ? ps.s : nullptr, past ? ps.s : nullptr, type_code(k.scalar_type()), stream_of(k)),
+              "append_to_cache");
+        return present;
+    }));
     END_HANDLE_TH_ERRORS
 }
 
@@ -979,16 +997,18 @@ PyObject* py_linear(PyObject*, PyObject* const* args, Py_ssize_t count)
     const int64_t n = w.size(0), k = w.size(1), rows = x.numel() / k;
     const bool few = are_few(x, w, most, most_split);
     if (!few && (!nhp_linear_tiles_pay(rows, n, k) || (b && reinterpret_cast<uintptr_t>(b->data_ptr()) % 16))) return not_here();
-    const at::NoGradGuard no_grad;
-    const c10::DeviceGuard guard(x.device());
-    Tensor y = new_rows(x, n);
-    if (!few) {
-        check(nhp_linear_tiles(y.data_ptr(), x.data_ptr(), w.data_ptr(), ptr(b), rows, n, k, type_code(x.scalar_type()), stream_of(x)), "linear");
-        return THPVariable_Wrap(y);
-    }
-    const Tensor ws = bytes(nhp_linear_decode_workspace_bytes(rows, n, k), x);
-    check(nhp_linear_decode(y.data_ptr(), x.data_ptr(), w.data_ptr(), ptr(b), ptr(ws), rows, n, k, type_code(x.scalar_type()), stream_of(x)), "linear");
-    return THPVariable_Wrap(y);
+    return THPVariable_Wrap(unlocked([&] {
+        const at::NoGradGuard no_grad;
+        const c10::DeviceGuard guard(x.device());
+        Tensor y = new_rows(x, n);
+        if (!few) {
+            check(nhp_linear_tiles(y.data_ptr(), x.data_ptr(), w.data_ptr(), ptr(b), rows, n, k, type_code(x.scalar_type()), stream_of(x)), "linear");
+            return y;
+        }
+        const Tensor ws = bytes(nhp_linear_decode_workspace_bytes(rows, n, k), x);
+        check(nhp_linear_decode(y.data_ptr(), x.data_ptr(), w.data_ptr(), ptr(b), ptr(ws), rows, n, k, type_code(x.scalar_type()), stream_of(x)), "linear");
+        return y;
+    }));
     END_HANDLE_TH_ERRORS
 }
 
@@ -1002,14 +1022,16 @@ PyObject* py_linear_act(PyObject*, PyObject* const* args, Py_ssize_t count)
     if (!take_all(args, count, x, w, b, act, most, most_split) || !few_rows(x, w, b, most, most_split)) return not_here();
     const bool gated = act != NHP_LINEAR_BIAS_GELU;
     if (gated && (b || w.size(0) % 32 || act < NHP_GATE_SWISH || act > NHP_GATE_IDENTITY)) return not_here();
-    const at::NoGradGuard no_grad;
-    const c10::DeviceGuard guard(x.device());
-    const int64_t n = w.size(0), k = w.size(1), rows = x.numel() / k;
-    Tensor y = new_rows(x, gated ? n / 2 : n);
-    const Tensor ws = bytes(nhp_linear_decode_workspace_bytes(rows, n, k), x);
-    check(nhp_linear_decode_act(y.data_ptr(), x.data_ptr(), w.data_ptr(), ptr(b), ptr(ws), rows, n, k, (int)act, type_code(x.scalar_type()),
-                                stream_of(x)), "linear and activation");
-    return THPVariable_Wrap(y);
+    return THPVariable_Wrap(unlocked([&] {
+        const at::NoGradGuard no_grad;
+        const c10::DeviceGuard guard(x.device());
+        const int64_t n = w.size(0), k = w.size(1), rows = x.numel() / k;
+        Tensor y = new_rows(x, gated ? n / 2 : n);
+        const Tensor ws = bytes(nhp_linear_decode_workspace_bytes(rows, n, k), x);
+        check(nhp_linear_decode_act(y.data_ptr(), x.data_ptr(), w.data_ptr(), ptr(b), ptr(ws), rows, n, k, (int)act, type_code(x.scalar_type()),
+                                    stream_of(x)), "linear and activation");
+        return y;
+    }));
     END_HANDLE_TH_ERRORS
 }
 
@@ -1028,13 +1050,15 @@ PyObject* py_linear_add(PyObject*, PyObject* const* args, Py_ssize_t count)
         if (r.size(i) != x.size(i)) return not_here();
     if (x1 && (x1->sizes() != r.sizes() || !alike(*x1, x) || !x1->is_contiguous() || wants_grad({&*x1}))) return not_here();
     if (b1 && (b1->dim() != 1 || b1->size(0) != n || !alike(*b1, x) || !b1->is_contiguous() || wants_grad({&*b1}))) return not_here();
-    const at::NoGradGuard no_grad;
-    const c10::DeviceGuard guard(x.device());
-    Tensor y = new_rows(x, n);
-    const Tensor ws = bytes(nhp_linear_decode_workspace_bytes(rows, n, k), x);
-    check(nhp_linear_decode_add(y.data_ptr(), x.data_ptr(), w.data_ptr(), ptr(b), ptr(x1), ptr(b1), r.data_ptr(), ptr(ws), rows, n, k,
-                                type_code(x.scalar_type()), stream_of(x)), "linear and residual");
-    return THPVariable_Wrap(y);
+    return THPVariable_Wrap(unlocked([&] {
+        const at::NoGradGuard no_grad;
+        const c10::DeviceGuard guard(x.device());
+        Tensor y = new_rows(x, n);
+        const Tensor ws = bytes(nhp_linear_decode_workspace_bytes(rows, n, k), x);
+        check(nhp_linear_decode_add(y.data_ptr(), x.data_ptr(), w.data_ptr(), ptr(b), ptr(x1), ptr(b1), r.data_ptr(), ptr(ws), rows, n, k,
+                                    type_code(x.scalar_type()), stream_of(x)), "linear and residual");
+        return y;
+    }));
     END_HANDLE_TH_ERRORS
 }
 

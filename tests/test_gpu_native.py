@@ -368,3 +368,33 @@ def test_another_stream_and_thread():
     [t.join() for t in threads]
     assert not failed
     assert all(torch.equal(a, b) for result in got for a, b in zip(result, want))
+
+
+def test_other_threads_run_during_a_call():
+    """Allocations and launches leave the interpreter's lock to others. The calls follow each other without any of this thread's
+    own bytecode in between, where it would hand over the lock anyway."""
+    import collections
+    import itertools
+    import threading
+    import time
+
+    from megatron.fused_kernels import _hotpath as hp
+
+    x, w, rows = randn((8, 64), BF16, 1), randn((64, 64), BF16, 2), randn((64,), BF16, 3)
+    with torch.no_grad():
+        for call, args in ((hp.native().layer_norm, (x, rows, rows, 1e-5)), (hp.native().linear, (x, w, None, 16, 32))):
+            ticks, stop = [], threading.Event()
+
+            def tick():
+                while not stop.is_set():
+                    ticks.append(time.perf_counter())
+
+            other = threading.Thread(target=tick)
+            other.start()
+            start = time.perf_counter()
+            collections.deque(itertools.starmap(call, itertools.repeat(args, 5000)), maxlen=0)
+            end = time.perf_counter()
+            stop.set()
+            other.join()
+            quarters = {int(4 * (t - start) / (end - start)) for t in ticks if start <= t < end}
+            assert {1, 2} <= quarters, (quarters, end - start)

@@ -7,22 +7,39 @@
 // the steps in turn are up to 15 % faster with 2048 features, but add up in another order than a pass with gradients does: here the
 // features come one after the other, and the results were the library's bit for bit at all 86 sizes compared (bf16, 33 to 512 rows).
 //
-// Measured, weights not in any cache, us here / library, whose call costs the host 25 us besides, this one 5; sizes in brackets
-// are not taken:
-//   rows           33             64             96             128            192            256            320            512
-//   [768, 768]     5.1 / 4.9      5.3 / 5.8      5.3 / 5.0      5.3 / 4.8      5.5 / 5.0      5.3 / 7.0      5.5 / 7.0      5.5 / 7.3
-//   [2304, 768]    5.4 / 7.1      5.5 / 7.5      5.6 / 7.2      5.5 / 8.1      5.8 / 7.6      5.7 / 7.7      6.0 / 7.7      7.3 / 8.6
-//   [4096, 1024]   6.3 / 8.3      6.5 / 8.7      6.5 / 9.1      6.6 / 9.3      6.8 / 10.6     6.9 / 9.1      8.3 / 9.9      8.9 / 10.5
-//   [2048, 2048]   [10.2 / 8.6]   [10.2 / 8.9]   [10.2 / 8.6]   [10.2 / 8.6]   [10.2 / 9.4]   10.3 / 9.6     10.4 / 10.5    10.8 / 11.1
-//   [3072, 2048]   [10.2 / 8.8]   [10.2 / 9.1]   [10.3 / 9.6]   [10.3 / 11.8]  10.4 / 15.9    10.6 / 10.9    10.9 / 10.9    [13.1 / 13.6]
-//   [6144, 2048]   [10.7 / 9.7]   [10.8 / 9.7]   12.4 / 14.2    12.7 / 15.6    [13.4 / 16.5]  [13.7 / 19.1]  [19.5 / 17.6]  [25.9 / 20.3]
-//   [8192, 2048]   14.1 / 15.0    14.9 / 15.0    12.8 / 14.9    13.2 / 16.1    [20.1 / 22.7]  [20.7 / 25.2]
-//   [7680, 2560]   [15.5 / 16.1]  [17.8 / 16.0]  16.3 / 17.7    16.9 / 19.4    [26.8 / 25.1]  [26.0 / 31.0]  -              [45.1 / 30.8]
-//   [4096, 4096]   [19.1 / 12.6]  [20.1 / 14.2]  19.9 / 22.1    21.3 / 24.5    21.1 / 32.5    21.4 / 23.1    [33.2 / 25.8]  [33.7 / 29.6]
-//   [768, 3072]    [15.4 / 9.6]   [15.3 / 9.8]   [15.6 / 7.7]   [15.4 / 8.0]   [15.5 / 8.7]   [15.4 / 8.9]   -              [14.7 / 12.0]
-//   [2048, 8192]   [36.5 / 13.5]  [36.9 / 21.4]  [35.0 / 20.1]  [36.0 / 20.5]  [36.4 / 26.4]  [36.4 / 26.9]  -              [37.4 / 34.2]
-// A whole layer, no gradient, us here / with the library: 768 features 132 / 204 at 40 to 512 rows, 1024 features 133 / 202; 2048 (16
-// heads) 155 / 203 at 100, 182 / 202 at 200; 4096 (gated) 187 / 212 at 100, 200 / 212 at 200.
+// Measured, weights not in any cache (340 MB of them in turn), us here/library, whose call costs the host 25 us besides, this one 5;
+// sizes in brackets are not taken, those with a dash were not looked at:
+//   rows            33          64          96          128         192         256         320         512         1024        2048        4096
+//   [16, 768]       4.5/5.1     4.6/6.6     4.6/6.9     4.6/7.3     4.5/8.6     4.7/8.0     4.7/4.9     4.7/4.9     4.8/4.9     4.8/4.9     4.9/5.0
+//   [256, 768]      4.9/9.9     5.0/9.8     5.0/12.5    5.0/12.2    5.1/15.6    5.1/17.5    5.1/6.7     5.1/6.7     5.1/6.9     5.2/7.1     5.4/7.5
+//   [768, 768]      5.7/8.9     6.1/9.4     5.7/8.9     6.0/8.9     6.1/9.0     5.9/8.6     6.1/8.6     5.9/9.0     6.0/9.3     8.2/10.5    [13.4/12.3]
+//   [2304, 768]     5.8/9.2     6.3/9.5     5.9/9.1     6.2/10.2    6.4/9.5     6.2/9.7     6.5/9.7     8.1/10.4    [11.7/12.3] [18.4/15.9] -
+//   [128, 1024]     5.7/7.8     5.8/8.2     5.8/7.9     5.9/7.8     5.9/7.8     6.0/7.8     6.0/7.9     6.0/7.9     6.0/8.0     6.0/8.0     6.2/8.5
+//   [1024, 1024]    6.7/10.9    7.2/11.3    6.8/10.7    7.1/10.7    7.0/10.6    7.0/10.3    7.0/11.0    7.0/10.7    7.1/11.2    11.1/12.2   [21.5/14.4]
+//   [4096, 1024]    6.9/11.2    7.5/11.7    7.0/12.0    7.4/12.3    7.4/13.2    7.4/12.0    10.5/12.7   11.2/13.1   [20.1/14.5] -           -
+//   [512, 512]      4.1/6.4     4.1/6.8     4.1/7.6     4.1/7.7     4.2/6.3     4.2/6.4     4.2/6.4     4.2/6.5     4.3/7.0     4.5/7.2     6.3/8.4
+//   [2048, 64]      2.5/3.5     2.6/3.7     2.6/4.1     2.6/4.2     2.6/3.6     2.6/3.7     2.7/3.9     2.8/4.0     3.3/4.8     [5.2/5.9]   -
+//   [2048, 2048]    -           -           -           -           -           11.4/11.9   11.4/12.8   11.5/12.7   -           -           -
+//   [3072, 2048]    -           -           -           -           11.8/21.5   11.8/13.2   11.8/13.2   -           -           -           -
+//   [6144, 2048]    -           -           12.4/14.2   13.0/15.5   [19.3/22.2] -           -           -           -           -           -
+//   [8192, 2048]    14.2/15.2   14.8/14.8   14.6/15.6   15.3/16.7   -           -           -           -           -           -           -
+//   [2560, 2560]    -           -           -           -           [15.1/14.4] 15.1/16.1   15.1/16.0   -           -           -           -
+//   [7680, 2560]    [16.9/17.5] [18.4/17.6] 16.8/18.4   18.0/20.2   -           -           -           -           -           -           -
+//   [2048, 4096]    -           -           -           -           -           20.2/16.1   20.3/21.6   20.5/21.2   -           -           -
+//   [4096, 4096]    -           -           20.0/22.4   21.5/24.8   21.5/33.3   21.4/22.8   -           -           -           -           -
+//   [6144, 4096]    -           -           21.5/23.5   22.8/25.9   [35.0/33.8] -           -           -           -           -           -
+// Behind the library on the GPU, and taken for the host's time all the same:
+//  - up to 160 tiles with more than 3584 features, where the library splits the contraction at some numbers of rows:
+//    [4096, 4096] at 80 rows 19.6/17.1, at 112 20.6/17.1, [3072, 4096] at 160 19.6/16.8, [2048, 4096] at 256 20.2/16.1,
+//  - 128 tiles with 2048 rows of weights or 112 of x beyond 2048 features, by up to 7 %: [2048, 2560] at 256 14.8/13.8,
+//  - with weights that stay in the caches (16 sets of them in turn) [768, 768] up to 192 rows, 5.5/5.0, [256, 768] at
+//    320 and 768 rows, 5.6/5.0, and 128 to 144 tiles of 2048 features, [2048, 2048] at 256 10.5/9.9, [3072, 2048] at 160 10.5/9.5.
+// The host is what a program waits for that does not capture its layers: a layer of 4096 features (gated) without gradient at 70 / 120
+// rows takes 221 / 208 us here and 273 / 228 with [4096, 4096] left to the library; in a captured graph 176 / 179 and 173 / 176. With
+// all products the library's and the former host path, 349 / 301 and 172 / 175.
+// Other whole layers, step by step / captured, before this kernel and the native calls -> here: 768 features, 40 rows, 298 / 56 ->
+// 150 / 51; 1024, 100 rows, 269 / 71 -> 144 / 60; 2048 (16 heads), 100 rows, 273 / 87 -> 167 / 84, 200 rows 270 / 107 -> 198 / 105;
+// 4096 (gated), 200 rows, 312 / 213 -> 207 / 207.
 #include "attention.hpp"
 
 namespace nhp {
@@ -137,10 +154,11 @@ static int64_t linear_tiles(int64_t rows, int64_t out_features)
 
 extern "C" {
 
-// Contractions of up to 1024 features as long as all tiles run at once (two a CU); longer ones where a tile has a CU to itself and at
-// least half of the CUs have one, and beyond 2048 features where the weights are read for more than one row of tiles. Outside of
-// that the library is ahead on the GPU or the two take turns (table above): with fewer tiles it splits the contraction, with more
-// its larger ones read less.
+// Contractions of up to 1024 features as long as all tiles run at once, two a CU (beyond one a CU up to 4096 rows: [128, 1024] at
+// 16384 is 11.9 us, 10.3 in the library); longer ones where a tile has a CU to itself and at least half of the CUs have one, and
+// beyond 2048 features where the weights are read for more than one row of tiles. Outside of that the library is ahead or the two
+// take turns: with fewer tiles it splits the contraction, with more its larger ones read less. Where the rule takes sizes for the
+// host's time only, the table above says so.
 int nhp_linear_tiles_pay(int64_t rows, int64_t out_features, int64_t in_features)
 {
     using namespace nhp;
@@ -148,7 +166,7 @@ int nhp_linear_tiles_pay(int64_t rows, int64_t out_features, int64_t in_features
         in_features % kTileStep)
         return 0;
     const int64_t tiles = linear_tiles(rows, out_features);
-    if (in_features <= 1024) return tiles <= 512;
+    if (in_features <= 1024) return tiles <= 256 || (tiles <= 512 && rows <= 4096);
     return in_features <= 4096 && tiles >= 128 && tiles <= 256 && (in_features <= 2048 || rows > kTileRows);
 }
 

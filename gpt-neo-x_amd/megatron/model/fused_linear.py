@@ -17,8 +17,10 @@ Where the line lies. On the GPU, weights not in any cache, us here / library:
     [2560, 10240]  14.3 / 19.5  14.8 / 19.4  15.8 / 19.6   17.8 / 22.3   18.2 / 22.4
     [4096, 11008]  20.2 / 37.6  20.5 / 37.9  22.2 / 37.9   23.9 / 31.2   24.8 / 30.8
     [4096, 14336]  24.6 / 25.8  25.2 / 25.9  26.8 / 26.9   28.7 / 31.2   30.7 / 33.4
-Up to 16 rows the kernel is ahead everywhere, up to 32 where a side has at most 2048 features or where four workgroups share the
-contraction (more than 4096 features); in between the library catches up.
+Up to 16 rows the kernel is ahead everywhere, up to 28 where a side has at most 2048 features and up to 32 where four workgroups
+share the contraction (more than 4096 features; [8192, 8192] 32.5 / 31.2); in between the library catches up. At 29 to 32 rows with a
+side of at most 2048 features and more than 2048 in it is up to 9 % ahead on the GPU ([1024, 4096] 12.8 / 11.9, [1536, 3072] 10.4 /
+10.1); these are taken for the 20 us that its call costs the host.
 
 More rows than that (a short prompt, many sequences) go to csrc/linear_tiles.hip where it is ahead; its table and rule stand there."""
 from typing import Optional

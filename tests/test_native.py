@@ -112,3 +112,10 @@ def test_what_could_be_scripted_still_can():
 
     for f in (activation, bias_add_residual_pair):
         torch.jit.script(f)
+
+
+@pytest.mark.parametrize("rows,n,k,taken", [(4096, 512, 512, True), (4097, 512, 512, False), (8192, 256, 768, False), (4096, 256, 768, True),
+                                            (16384, 16, 768, True), (16385, 16, 768, False), (16384, 128, 1024, False), (2048, 1024, 1024, True)])
+def test_many_rows_of_narrow_layers(rows, n, k, taken):
+    """Where tiles share the CUs the rule of nhp_linear_tiles ends with the rows that were measured."""
+    assert bool(hp.lib().nhp_linear_tiles_pay(rows, n, k)) == taken

@@ -94,6 +94,10 @@ class MLP(torch.nn.Module):
                 return None
             act = self.activation_func._code
         elif self.activation_func is bias_gelu_impl:
+            # (the activation's kernel for a bias that is not aligned rounds its last product to fp16 at once, the launch to fp32
+            # first: the bits of a layer would depend on which of them it takes)
+            if bias is not None and bias.dtype is torch.float16 and (_hp.followed(bias) or bias.data_ptr() % 16):
+                return None
             act = fused_linear.BIAS_GELU
         else:
             return None

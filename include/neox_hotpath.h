@@ -778,7 +778,8 @@ int64_t nhp_linear_decode_workspace_bytes(int64_t rows, int64_t out_features, in
 int nhp_linear_decode(void* y, const void* x, const void* weight, const void* bias, void* workspace, int64_t rows,
                       int64_t out_features, int64_t in_features, int dtype, void* stream);
 /* The same with what follows such a layer (ParallelMLP and the residual additions, megatron/model/transformer.py:171-184 and
- * :1229-1250), rounded as by the separate calls (the product to the storage type first).
+ * :1229-1250), rounded as by the separate calls (the product to the storage type first); the
+ * GeLU of an fp16 bias that is not 16-byte aligned as that of an aligned one.
  * _act: act = NHP_LINEAR_BIAS_GELU: y = nhp_bias_gelu_fwd of the product, bias may be NULL; a NHP_GATE_*: nhp_gated_act_fwd of it,
  * y [rows, out_features / 2], out_features a multiple of 32, bias NULL. _add: nhp_bias_add_residual of the product, or with x1
  * [rows, out_features] nhp_bias_add_residual_pair(x1, bias1, product, bias); x1 and bias1 may be NULL. */

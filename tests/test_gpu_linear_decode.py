@@ -163,3 +163,20 @@ def test_a_layer_takes_them_unless_somebody_looks(style):
     assert torch.equal(step(), want)
     with torch.autocast("cuda", dtype=torch.float16):
         assert layer.mlp._activated(x) is None
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_an_unaligned_bias_gives_the_bits_of_separate_launches(dtype):
+    """The parameters of a layer may be slices of one buffer."""
+    import types
+
+    from megatron.model.transformer_layer import MLP
+
+    mlp = MLP(types.SimpleNamespace(activation="gelu", bias_gelu_fusion=True, hidden_size=768)).to(DEV).to(dtype)
+    x, buffer = util.randn((16, 1, 768), dtype, seed=1).to(DEV), util.randn((3073,), dtype, seed=2).to(DEV)
+    mlp.linear1.bias = torch.nn.Parameter(buffer[1:])
+    with torch.no_grad():
+        mlp.linear1.weight.copy_(util.randn((3072, 768), dtype, seed=3, std=0.05))
+        got = mlp(x)[0]
+        mlp.linear1.register_forward_hook(lambda module, inputs, output: None)
+        assert torch.equal(got, mlp(x)[0])

@@ -186,7 +186,8 @@ def plain(*tensors):
 
 
 _AS_WRITTEN = {}
-_CALL = torch.nn.Module.__call__
+_Module = torch.nn.Module
+_CALL = _Module.__call__
 
 
 def as_written(cls):
@@ -194,7 +195,7 @@ def as_written(cls):
     cls.__annotations__   # torch.jit would make it later
     members = dict(vars(cls))
     methods = (name for name, member in members.items() if callable(member) or isinstance(member, (property, staticmethod)))
-    _AS_WRITTEN[cls] = members, frozenset(methods) | {"_call_impl", "_compiled_call_impl"}
+    _AS_WRITTEN[cls] = vars(cls), members, frozenset(methods) | {"_call_impl", "_compiled_call_impl"}
     return cls
 
 
@@ -202,10 +203,16 @@ def untouched(module, cls):
     """Whether ``module`` is a ``cls`` as it stands in its file (the class is marked ``as_written``): no subclass, nothing of the
     class replaced or added, none of its methods replaced in the module, no hooks, not compiled. Whoever put such a thing there
     wants the tensors that pass through the module, so it has to be called, with those tensors; so does torch while it compiles."""
+    return not _hp._is_compiling() and as_it_stands(module, cls)
+
+
+def as_it_stands(module, cls):
+    """``untouched`` for a caller that knows that torch is not compiling."""
     own = module.__dict__
-    members, methods = _AS_WRITTEN[cls]
-    return (not _hp._is_compiling() and type(module) is cls and own.keys().isdisjoint(methods) and vars(cls) == members
-            and torch.nn.Module.__call__ is _CALL and not (own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or own["_backward_pre_hooks"]
+    now, members, methods = _AS_WRITTEN[cls]
+    return (type(module) is cls and own.keys().isdisjoint(methods) and now == members
+            and _Module.__call__ is _CALL
+            and not (own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or own["_backward_pre_hooks"]
                      or _has_any_global_hook()))
 
 

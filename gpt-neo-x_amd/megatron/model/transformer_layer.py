@@ -85,12 +85,13 @@ class MLP(torch.nn.Module):
         self.linear2 = Linear(ffn_dim_in, hidden, bias=use_bias, skip_bias_add=True)
 
     def _activated(self, x):
-        """The activated intermediate for the few rows of a decoding step, in the launch of the first product, or None."""
-        if not (fused_attention.untouched(self.linear1, Linear) and self.linear1.skip_bias_add):
+        """The activated intermediate for the few rows of a decoding step (``_few_rows``), in the launch of the first product, or None."""
+        linear1 = self.linear1
+        if not (fused_attention.as_it_stands(linear1, Linear) and linear1.skip_bias_add):
             return None
-        bias = self.linear1.bias
+        bias = linear1.bias
         if self.is_gated:
-            if not fused_attention.untouched(self.activation_func, Gated_Activation):
+            if not fused_attention.as_it_stands(self.activation_func, Gated_Activation):
                 return None
             act = self.activation_func._code
         elif self.activation_func is bias_gelu_impl:
@@ -101,7 +102,7 @@ class MLP(torch.nn.Module):
             act = fused_linear.BIAS_GELU
         else:
             return None
-        y = _hp.native().linear_act(x, self.linear1.weight, bias, act, fused_linear.MAX_ROWS, fused_linear.MAX_ROWS_NARROW)
+        y = _hp.native().linear_act(x, linear1.weight, bias, act, fused_linear.MAX_ROWS, fused_linear.MAX_ROWS_NARROW)
         return None if y is NotImplemented else y
 
     def _few_rows(self, x):
@@ -113,17 +114,18 @@ class MLP(torch.nn.Module):
         """``residual + mlp(x)`` or ``residual + ((other + other_bias) + mlp(x))`` for the few rows of a decoding step, the
         activation and the addition each in the launch of a product; None for anything else, and where somebody looks at the
         modules."""
-        if not self._few_rows(x) or not (fused_attention.untouched(self, MLP) and fused_attention.untouched(self.linear2, Linear)
-                                         and self.linear2.skip_bias_add):
+        linear2 = self.linear2
+        if not self._few_rows(x) or not (fused_attention.as_it_stands(self, MLP) and fused_attention.as_it_stands(linear2, Linear)
+                                         and linear2.skip_bias_add):
             return None
         intermediate = self._activated(x)
         if intermediate is None:
             return None
-        y = _hp.native().linear_add(intermediate, self.linear2.weight, self.linear2.bias, other, other_bias, residual,
+        y = _hp.native().linear_add(intermediate, linear2.weight, linear2.bias, other, other_bias, residual,
                                     fused_linear.MAX_ROWS, fused_linear.MAX_ROWS_NARROW)
         if y is not NotImplemented:
             return y
-        output, bias = self.linear2(intermediate)
+        output, bias = linear2(intermediate)
         if other is None:
             return bias_dropout_add_fused_inference(output, bias, residual, 0.0)
         return bias_add_residual_pair(other, other_bias, output, bias, residual)
@@ -204,9 +206,9 @@ class SelfAttention(torch.nn.Module):
                     query, key = apply_rotary_to_query_key(query, key, self.rotary_emb, rotary_ndims=self.rotary_ndims,
                                                            rope_fusion=False, bf16=self.bf16, layer_past=layer_past)
         past = layer_past if layer_past is not None and layer_past.numel() > 0 else None
-        call = None
-        if self.use_cache and past is not None and fused_attention.untouched(self.core, CoreAttention):
-            call = self.core._cached_call(query, key, value, attention_mask, past)
+        call, core = None, self.core
+        if self.use_cache and past is not None and fused_attention.untouched(core, CoreAttention):
+            call = core._cached_call(query, key, value, attention_mask, past)
         if call is not None:
             context, present = fused_attention.checked_decode_attention(query, key, value, past, *call, merged=True)
         else:
@@ -221,7 +223,7 @@ class SelfAttention(torch.nn.Module):
                     value = torch.cat((past_value.type_as(value), value), dim=0)
                 present = torch.stack((key, value)) if self.use_cache else None
             # [sq, b, np * hn], written in that layout by the attention kernel or the context GEMM
-            context = self.core(query, key, value, attention_mask, merged_heads=True)
+            context = core(query, key, value, attention_mask, merged_heads=True)
         output, bias = self.dense(context)
         return ([output, present] if self.use_cache else output), bias
 

@@ -12,9 +12,13 @@
 // tile is that of the sums). Loaded straight into the registers in the instruction's order, a load touched 64 bytes of 16
 // rows, half a cache line of each; here it takes whole lines of 8 rows. us, 16 rows, weights that are not in any cache,
 // half lines -> here (a kernel that only reads as many bytes):
-//   [22016, 4096] 43.9 -> 37.5 (27.5)   [12288, 4096] 26.2 -> 22.5 (16.1)   [4096, 11008] 27.9 -> 22.0 (14.5)
-//   [7680, 2560] 16.0 -> 11.5           [768, 3072] 8.6 -> 6.5              [4096, 4096] 12.2 -> 11.4 (6.4)
-// A ring of 6 or 7 pieces, or two workgroups per CU, are no faster; reading x costs 2 to 3 us of it (one row: 33.7, 20.2).
+//   [22016, 4096] 44.3 -> 38.1 (27.5)   [12288, 4096] 26.3 -> 23.1 (16.1)   [4096, 11008] 28.2 -> 23.1 (14.5)
+//   [7680, 2560] 16.6 -> 12.3           [768, 3072] 8.8 -> 7.4              [4096, 4096] 12.6 -> 12.0 (6.4)
+// A ring of 6 or 7 pieces, or two workgroups per CU, are no faster; reading x costs 2 to 3 us of it (one row: 34.6, 21.1).
+//
+// The contraction of a workgroup goes into sixteen sums of consecutive features, two to a wave, which are added up one after the
+// other: the order of sixteen waves with a sum each, as which this kernel began, so the results stay what they were. Against one sum
+// a wave it costs 0.1 us, 0.5 to 0.9 with more than 16 rows ([22016, 4096] 37.7 and 38.1, 32 rows 42.2 and 43.3).
 //
 // Rows of the matrix instruction (16 x 16 x 32) are weight rows, its columns the rows of x. A lane takes 16 consecutive
 // bytes of its row per instruction and x in the same order, which the contraction does not mind.
@@ -40,8 +44,10 @@ struct LinearArgs {
 // (a layer of 768 features, one sequence: a step 100 -> 91 us; 4096 features, gated, 16 sequences: 312 -> 307).
 enum LinearEnd { kPlainRows, kGeluRows, kGatedRows, kAddRows };
 
-constexpr int kLinearWaves = 8, kLinearBlocks = 256, kLinearSteps = 16;   // steps of 32 features that a wave has at most
-constexpr int kLinearWhole = kLinearSteps * kLinearWaves * 32, kLinearSplits = 4;   // features of an unsplit product; splits beyond
+constexpr int kLinearWaveBits = 3, kLinearWaves = 1 << kLinearWaveBits, kLinearBlocks = 256;
+constexpr int kLinearSteps = 16;   // steps of 32 features that a wave has at most
+constexpr int kLinearSplitBits = 2, kLinearSplits = 1 << kLinearSplitBits;   // of a product with more features than the next
+constexpr int kLinearWhole = kLinearSteps * kLinearWaves * 32;
 constexpr int kRing = 4, kPieceBytes = 2048;   // pieces of 16 rows x 64 features in LDS for each wave
 
 template <int N>
@@ -107,13 +113,15 @@ template <int DT, int MT, int END>
 __global__ void __launch_bounds__(64 * kLinearWaves) linear_decode_kernel(LinearArgs a)
 {
     __shared__ __attribute__((aligned(1024))) char ring[kLinearWaves * kRing * kPieceBytes];
-    __shared__ float sums[2][kLinearWaves][16 * MT][17];
+    __shared__ float sums[2][2 * kLinearWaves][16 * MT][17];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g = lane >> 4;
-    const int split = blockIdx.x % a.splits, first_tile = blockIdx.x / a.splits, stride = gridDim.x / a.splits;
+    const int split_bits = a.splits == 1 ? 0 : kLinearSplitBits;
+    const int split = blockIdx.x & (a.splits - 1), first_tile = blockIdx.x >> split_bits, stride = gridDim.x >> split_bits;
     // groups of 32 features are dealt out evenly to the waves of all splits, a wave's being consecutive
-    const int groups = a.k / 32, shares = kLinearWaves * a.splits, share = split * kLinearWaves + wave;
-    const int lo = __builtin_amdgcn_readfirstlane(groups * share / shares), count = __builtin_amdgcn_readfirstlane(groups * (share + 1) / shares - lo);
+    const int groups = a.k / 32, share = split * kLinearWaves + wave, share_bits = kLinearWaveBits + split_bits;
+    const int lo = groups * share >> share_bits, count = (groups * (share + 1) >> share_bits) - lo;
+    const int mid = (groups * (2 * share + 1) >> (share_bits + 1)) - lo;   // steps of the wave's first sum
     constexpr int kParts = END == kGatedRows ? 2 : 1;   // tiles of a result: its values, its gates
     const int tiles = a.n / 16 / kParts, pieces = (count + 1) / 2;
 
@@ -164,9 +172,17 @@ __global__ void __launch_bounds__(64 * kLinearWaves) linear_decode_kernel(Linear
     for (int tile = first_tile; tile < tiles; tile += stride) {
         float value = 0.0f;   // kGatedRows: the first of the two sums
         for (int part = 0; part < kParts; ++part) {
-            f32x4 acc[MT];
+            f32x4 acc[2][MT];
 #pragma unroll
-            for (int r = 0; r < MT; ++r) acc[r] = f32x4{};
+            for (int r = 0; r < MT; ++r) acc[0][r] = acc[1][r] = f32x4{};
+            auto multiply = [&](const u32x4& w, int step) {   // (a constant after unrolling)
+                if (step < mid)
+#pragma unroll
+                    for (int r = 0; r < MT; ++r) acc[0][r] = mma16<DT>(w, x[r][step], acc[0][r]);
+                else
+#pragma unroll
+                    for (int r = 0; r < MT; ++r) acc[1][r] = mma16<DT>(w, x[r][step], acc[1][r]);
+            };
 #pragma unroll
             for (int p = 0; p < kLinearSteps / 2; ++p) {
                 if (p >= pieces) continue;
@@ -177,23 +193,23 @@ __global__ void __launch_bounds__(64 * kLinearWaves) linear_decode_kernel(Linear
                 const char* f = frag + at * kPieceBytes;
                 at = at + 1 == kRing ? 0 : at + 1;
                 const u32x4 w_lo = lds_read16(f + ((g ^ sw) << 4)), w_hi = lds_read16(f + (((4 + g) ^ sw) << 4));
-#pragma unroll
-                for (int r = 0; r < MT; ++r) acc[r] = mma16<DT>(w_lo, x[r][2 * p], acc[r]);
-                if (2 * p + 1 < count)
-#pragma unroll
-                    for (int r = 0; r < MT; ++r) acc[r] = mma16<DT>(w_hi, x[r][2 * p + 1], acc[r]);
+                multiply(w_lo, 2 * p);
+                if (2 * p + 1 < count) multiply(w_hi, 2 * p + 1);
             }
 #pragma unroll
             for (int r = 0; r < MT; ++r)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) sums[buf][wave][r * 16 + r16][4 * g + j] = acc[r][j];
+                for (int j = 0; j < 4; ++j) {
+                    sums[buf][2 * wave][r * 16 + r16][4 * g + j] = acc[0][r][j];
+                    sums[buf][2 * wave + 1][r * 16 + r16][4 * g + j] = acc[1][r][j];
+                }
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
             // (a wave is at most one tile ahead of those that add up here: the other half of the sums is free)
             const int row = tid >> 4, col = tid & 15;
             if (row < a.m && row < 16 * MT) {
                 float v = 0.0f;
 #pragma unroll
-                for (int s = 0; s < kLinearWaves; ++s) v += sums[buf][s][row][col];
+                for (int s = 0; s < 2 * kLinearWaves; ++s) v += sums[buf][s][row][col];
                 if (a.splits > 1) {
                     a.parts[((int64_t)split * a.m + row) * a.n + (tile + part * tiles) * 16 + col] = v;
                 } else if (part + 1 < kParts) {

@@ -180,3 +180,30 @@ def test_an_unaligned_bias_gives_the_bits_of_separate_launches(dtype):
         got = mlp(x)[0]
         mlp.linear1.register_forward_hook(lambda module, inputs, output: None)
         assert torch.equal(got, mlp(x)[0])
+
+
+@pytest.mark.parametrize("rows", [1, 16, 20])
+@pytest.mark.parametrize("splits", [1, 4])
+def test_the_order_of_the_sums(rows, splits):
+    """Sixteen sums of consecutive features each, added up one after the other, in each of the splits, and those. Whole numbers, whose
+    products add up without rounding; the sixth sum takes the fifth, which is 2^18 times the size of the others, away again."""
+    from megatron.fused_kernels import _hotpath as hp
+
+    shares, each, n = 16 * splits, 128, 48
+    g = torch.Generator().manual_seed(0)
+    x, w = (torch.randint(-4, 5, (r, shares, each), generator=g).double() for r in (rows, n))
+    w[:, 4] *= 2.0 ** 18
+    w[:, 5], x[:, 5] = -w[:, 4], x[:, 4]
+    sums = torch.einsum("rsk,nsk->srn", x, w).float().view(splits, 16, rows, n)
+    want = torch.zeros((rows, n))
+    for part in sums:
+        v = torch.zeros_like(want)
+        for s in part:
+            v = v + s
+        want = want + v if splits > 1 else v
+    x, w = (t.reshape(t.size(0), -1).bfloat16().to(DEV) for t in (x, w))
+    y, scratch = torch.empty((rows, n), dtype=torch.bfloat16, device=DEV), torch.empty((4 * splits * rows * n,), dtype=torch.uint8, device=DEV)
+    hp.check(hp.lib().nhp_linear_decode(y.data_ptr(), x.data_ptr(), w.data_ptr(), None, scratch.data_ptr(), rows, n, shares * each, hp.BF16,
+                                        hp.stream_of(x)), "linear")
+    exact = torch.einsum("rk,nk->rn", x.double().cpu(), w.double().cpu())
+    assert torch.equal(y.cpu(), want.bfloat16()) and not torch.equal(y.cpu(), exact.bfloat16())

@@ -372,7 +372,7 @@ def test_another_stream_and_thread():
 
 def test_other_threads_run_during_a_call():
     """Allocations and launches leave the interpreter's lock to others. The calls follow each other without any of this thread's
-    own bytecode in between, where it would hand over the lock anyway."""
+    own bytecode in between, where it would hand over the lock anyway (one that is left to a busy thread comes back after 5 ms)."""
     import collections
     import itertools
     import threading
@@ -392,7 +392,7 @@ def test_other_threads_run_during_a_call():
             other = threading.Thread(target=tick)
             other.start()
             start = time.perf_counter()
-            collections.deque(itertools.starmap(call, itertools.repeat(args, 5000)), maxlen=0)
+            collections.deque(itertools.starmap(call, itertools.repeat(args, 100)), maxlen=0)
             end = time.perf_counter()
             stop.set()
             other.join()

@@ -4,23 +4,23 @@ The reference's Column / RowParallelLinear (megatron/mpu/layers.py) call the lib
 few of them the product is a single read of the weights, and the library's call alone takes the host 25 us (this one 4).
 
 Where the line lies. On the GPU, weights not in any cache, us here / library:
-    rows           1            4            16            24            32
-    [2304, 768]    3.7 / 5.1    3.7 / 5.2    3.8 / 5.2     4.3 / 7.0     4.4 / 7.0
-    [2048, 2048]   5.0 / 11.0   4.9 / 11.0   5.7 / 10.9    7.1 / 10.9    7.8 / 11.1
-    [1024, 4096]   6.5 / 14.6   6.6 / 14.4   8.5 / 14.4    11.1 / 14.2   12.6 / 11.8
-    [4096, 4096]   9.4 / 15.5   9.8 / 15.4   10.9 / 15.5   13.1 / 13.2   14.6 / 13.1
-    [12288, 4096]  20.5 / 27.5  21.0 / 28.3  22.7 / 28.3   24.9 / 23.5   26.7 / 24.2
-    [22016, 4096]  34.2 / 51.7  34.9 / 52.1  37.5 / 52.5   40.2 / 43.4   42.1 / 43.9
-    [6144, 4096]   13.1 / 15.6  13.5 / 15.6  15.3 / 15.5   17.5 / 16.0   18.7 / 16.3
-    [7680, 2560]   10.1 / 12.0  10.2 / 12.0  11.6 / 11.9   13.0 / 12.6   14.2 / 12.9
-    [5120, 5120]   14.1 / 14.4  14.4 / 14.9  15.1 / 17.4   16.2 / 20.2   16.8 / 20.6
-    [2560, 10240]  14.3 / 19.5  14.8 / 19.4  15.8 / 19.6   17.8 / 22.3   18.2 / 22.4
-    [4096, 11008]  20.2 / 37.6  20.5 / 37.9  22.2 / 37.9   23.9 / 31.2   24.8 / 30.8
-    [4096, 14336]  24.6 / 25.8  25.2 / 25.9  26.8 / 26.9   28.7 / 31.2   30.7 / 33.4
+    rows           1            4            16           24           32
+    [2304, 768]    3.8 / 6.3    3.9 / 6.4    3.9 / 6.4    4.7 / 9.3    4.8 / 9.2
+    [2048, 2048]   5.1 / 10.9   5.1 / 11.0   6.0 / 11.0   7.4 / 11.0   8.3 / 11.3
+    [1024, 4096]   6.4 / 14.4   6.8 / 14.5   8.6 / 14.4   11.5 / 14.2  12.9 / 11.9
+    [4096, 4096]   9.8 / 15.8   9.9 / 15.9   11.7 / 15.9  14.6 / 14.1  15.7 / 14.0
+    [12288, 4096]  20.4 / 27.5  20.8 / 28.9  22.6 / 28.7  25.1 / 24.6  26.9 / 24.7
+    [22016, 4096]  34.0 / 51.8  34.8 / 52.0  37.6 / 52.5  40.4 / 44.8  42.3 / 45.2
+    [6144, 4096]   13.4 / 15.8  13.5 / 16.1  15.5 / 15.9  17.9 / 16.3  19.4 / 17.0
+    [7680, 2560]   10.4 / 12.4  10.5 / 12.3  11.6 / 12.7  13.5 / 13.2  15.0 / 13.3
+    [5120, 5120]   14.5 / 14.8  14.8 / 15.2  15.5 / 17.9  17.3 / 20.5  17.8 / 20.9
+    [2560, 10240]  14.6 / 19.7  15.0 / 19.5  16.2 / 20.1  18.3 / 22.5  19.6 / 22.6
+    [4096, 11008]  20.9 / 38.5  21.2 / 38.9  22.8 / 38.8  25.0 / 32.5  26.2 / 31.9
+    [4096, 14336]  24.9 / 26.8  25.5 / 26.7  27.3 / 27.3  29.6 / 32.0  31.0 / 34.0
 Up to 16 rows the kernel is ahead everywhere, up to 28 where a side has at most 2048 features and up to 32 where four workgroups
-share the contraction (more than 4096 features; [8192, 8192] 32.5 / 31.2); in between the library catches up. At 29 to 32 rows with a
-side of at most 2048 features and more than 2048 in it is up to 9 % ahead on the GPU ([1024, 4096] 12.8 / 11.9, [1536, 3072] 10.4 /
-10.1); these are taken for the 20 us that its call costs the host.
+share the contraction (more than 4096 features; [8192, 8192] 33.1 / 31.3); in between the library catches up. At 29 to 32 rows with a
+side of at most 2048 features and more than 2048 in the library is up to 14 % ahead on the GPU ([2048, 4096] 13.8 / 12.1, [1536, 3072]
+10.7 / 10.1); these are taken for the 20 us that its call costs the host.
 
 More rows than that (a short prompt, many sequences) go to csrc/linear_tiles.hip where it is ahead; its table and rule stand there."""
 from typing import Optional

@@ -157,6 +157,13 @@ def few_rows():
     return mlp, torch.randn((1, 1, 512)).as_subclass(OnGpu)
 
 
+def own_linear_layers(m, mlp):
+    from megatron.model import transformer_layer as layers
+
+    m.setattr(layers, "Linear", type("Own", (layers.Linear,), {}))
+    mlp.linear1, mlp.linear2 = layers.Linear(512, 512, bias=False, skip_bias_add=True), layers.Linear(256, 512, bias=False, skip_bias_add=True)
+
+
 REPLACED = {
     "forward of the class": lambda m, mlp: m.setattr(type(mlp), "forward", lambda self, x: None),
     "forward of the linear layers": lambda m, mlp: m.setattr(type(mlp.linear1), "forward", lambda self, x: None),
@@ -165,6 +172,7 @@ REPLACED = {
     "call of every module": lambda m, mlp: m.setattr(torch.nn.Module, "__call__", lambda self, x: None),
     "compiled": lambda m, mlp: m.setattr(mlp.linear2, "_compiled_call_impl", lambda self, x: None, raising=False),
     "bias added in the layer": lambda m, mlp: m.setattr(mlp.linear2, "skip_bias_add", False),
+    "another class of linear layers": lambda m, mlp: own_linear_layers(m, mlp),
     "another layer": lambda m, mlp: mlp.__setattr__("linear1", torch.nn.Linear(512, 512)),
 }
 

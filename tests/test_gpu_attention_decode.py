@@ -48,7 +48,7 @@ def test_decode(dtype, hn, past, sq, b, np_, nkv):
 @pytest.mark.parametrize("past", [3, 31, 32, 63, 64, 65, 97, 128, 161, 300])
 @pytest.mark.parametrize("sq,b,np_,nkv", [(1, 160, 4, 4), (1, 128, 4, 4), (2, 97, 8, 4), (1, 192, 2, 2), (9, 192, 4, 2), (1, 131, 3, 3)])
 def test_many_sequences(hn, past, sq, b, np_, nkv):
-    """One, two and four heads of keys per workgroup; rounds of 32 keys that a wave has one, two or several of."""
+    """One and two heads of keys per workgroup; rounds of 32 keys that a wave has one, two or several of."""
     from megatron.model.fused_attention import decode_attention
 
     q, k, v, layer_past = cached(torch.bfloat16, past, sq, b, np_, nkv, hn)
